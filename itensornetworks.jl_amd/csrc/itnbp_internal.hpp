@@ -152,6 +152,7 @@ struct itnbp_net {
   DevBuf scratch, tasks, stats, partials, red, aux;
   DevBuf mdesc;          // per message: offset (long long) and chi (int), for device-side initialisation
   DevBuf apply_ws;       // itnbp_apply_gates: launch items, gates, LDS-kernel work, outputs (grows, kept)
+  DevBuf apply_big;      // itnbp_apply_gates: the split pipeline's workspace (kept up to a bound)
   void* fast = nullptr;  // state of the specialised pipeline (k_fast.hip)
   void* small = nullptr; // state of the per-vertex small-chi kernel (k_vertex.hip)
 };

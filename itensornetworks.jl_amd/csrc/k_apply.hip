@@ -25,91 +25,14 @@
 #include <string>
 #include <vector>
 
+#include "itnbp_apply.hpp"
 #include "itnbp_ops.hpp"
 
 namespace {
 
-typedef double f64x4 __attribute__((ext_vector_type(4)));
-
-constexpr int AP_XY = 8192;   // max E * n (external size x d chi_b) per side
-// tall-skinny QR (E >= 4 n, n <= 16): the stacked R factors (4n x n) and the
-// heads and betas of their reflectors, per side, after the side's reflectors
-constexpr int AP_QRX = 4 * 16 * 16 + 4 * 16;
-constexpr int AP_SIDE = AP_XY + AP_QRX;  // global scratch per side of a gate
-constexpr int AP_TH = 32;     // max rows/cols of Theta (r d)
-constexpr int AP_ENV = 8;     // max external bond dimension
-constexpr int AP_MAXEXT = 3;  // max external bonds per side (degree 4)
-constexpr int AP_SITE_D = 16; // max physical dimension of a one-site gate
-// the global-memory variant (k_apply_gates<true>) for bonds past the LDS limits:
-// every per-bond matrix in a global workspace, one workgroup per bond
-constexpr int AP_ENV_BIG = 32;    // max external bond dimension
-constexpr int AP_N_BIG = 64;      // max d chi_b
-constexpr int AP_TH_BIG = 128;    // max rows/cols of Theta
-constexpr int AP_KEEP_BIG = 64;   // max kept rank (the growth cap of itnbp_apply_gates)
-constexpr int AP_F_BIG = AP_TH_BIG * AP_KEEP_BIG;  // R factor, then the left / right factor
-// LDS of the small vectors (rot, four reflector-head vectors, the singular
-// values, the block reduction), rounded up to 256 bytes
-constexpr int AP_BIG_SMALL = (4 * 32 + 4 * AP_N_BIG + AP_TH_BIG + 16 + 31) & ~31;
-
-struct ApplyItem {
-  int u, v;      // vertices
-  int ju, jv;    // bond axis at u, v
-  long long gate;  // offset of the (d_u d_v)^2 gate
-  int slot;
-  int chib_in;     // bond dimension before the call (the layout may be grown past it)
-};
-
-struct ApplyParams {
-  int maxdim;         // <= 0: none (still capped by the bond dimension)
-  double cutoff;      // < 0: none
-  int normalize;
-  double eig_cutoff;  // map_eigvals cutoff (10 eps)
-  int max_keep;       // stride of the singular value output
-  // per-phase timestamps (wall clock; 16 slots per gate, slot 8 the SVD's
-  // sweep count), or null; ITNBP_APPLY_PHASES=1
-  unsigned long long* ts = nullptr;
-  // global-memory variant: per-gate workspace stride and the sizes of its
-  // side matrices (QR of each side: E n; work: E max(n, d keep)), in doubles
-  long long big_stride = 0, big_q = 0, big_x = 0;
-};
-
 // thread 0 of the workgroup records the end of phase ph (0: start)
 __device__ inline void phase_mark(const ApplyParams& prm, int ph) {
   if (prm.ts && threadIdx.x == 0) prm.ts[blockIdx.x * 16 + ph] = wall_clock64();
-}
-
-__device__ inline double wave_sum_d(double v) {
-  for (int m = 32; m > 0; m >>= 1) v += __shfl_xor(v, m);
-  return v;
-}
-
-__device__ double block_sum_d(double v, double* red) {
-  v = wave_sum_d(v);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  double s = 0;
-  for (int i = 0; i < (int)(blockDim.x >> 6); ++i) s += red[i];
-  __syncthreads();
-  return s;
-}
-
-// Round-robin pairing: step st of a cyclic sweep over n (even) indices.
-__device__ inline void rr_pair(int n, int st, int i, int& p, int& q) {
-  // positions 0..n-1; position 0 fixed, others rotate
-  // (pos - 1 + st) < 2 (n - 1): one conditional subtraction instead of a modulo
-  auto at = [&](int pos) {
-    if (pos == 0) return 0;
-    const int x = pos - 1 + st;
-    return 1 + (x >= n - 1 ? x - (n - 1) : x);
-  };
-  p = at(i);
-  q = at(n - 1 - i);
-  if (p > q) {
-    int t = p;
-    p = q;
-    q = t;
-  }
 }
 
 // sqrt(M) and M^{-1/2} of a symmetrised chi x chi message (column-major in
@@ -234,151 +157,6 @@ __device__ inline void wave_sync_ap() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// sqrt(M) and M^{-1/2} of a symmetrised chi x chi message for chi <= AP_ENV_BIG
-// (the global-memory variant), by one wave with the matrices in LDS (wk:
-// ENVB_WORK doubles per wave): cyclic two-sided Jacobi with the round-robin
-// pairs of rr_pair, the rotations of a step derived by the first ne / 2 lanes
-// and then applied to the rows, the columns and V; the stopping rule of
-// env_roots_wave (off-diagonal mass below 1e-30 of the diagonal's, or no
-// longer decreasing, at most 40 sweeps) and its eigenvalue truncation
-// (map_eigvals, src/apply.jl:9-25).  S and Si row-major, ld chi.
-constexpr int ENVB_LD = AP_ENV_BIG + 1;
-constexpr int ENVB_WORK = 2 * AP_ENV_BIG * ENVB_LD + 4 * AP_ENV_BIG;
-__device__ void env_roots_big(const double* M, int chi, double cutoff, double* S, double* Si, double* wk) {
-  const int l = threadIdx.x & 63;
-  double* A = wk;
-  double* V = A + AP_ENV_BIG * ENVB_LD;
-  double* rc = V + AP_ENV_BIG * ENVB_LD;  // per pair of a step: c, s, p, q
-  double* rs = rc + AP_ENV_BIG / 2;
-  int* rp = reinterpret_cast<int*>(rs + AP_ENV_BIG / 2);
-  int* rq = rp + AP_ENV_BIG / 2;
-  int* rank = rq + AP_ENV_BIG / 2;        // rank of each eigenvalue by |lambda|
-  int* byr = rank + AP_ENV_BIG;           // the eigenvalue of each rank
-  for (int o = l; o < chi * chi; o += 64) {
-    const int i = o / chi, j = o - i * chi;
-    A[i * ENVB_LD + j] = 0.5 * (M[i + chi * j] + M[j + chi * i]);
-    V[i * ENVB_LD + j] = i == j ? 1.0 : 0.0;
-  }
-  wave_sync_ap();
-  const int ne = chi + (chi & 1), np = ne / 2;
-  double prev = INFINITY;
-  for (int sweep = 0; sweep < 40 && chi > 1; ++sweep) {
-    double off = 0, dg = 0;
-    for (int o = l; o < chi * chi; o += 64) {
-      const int i = o / chi, j = o - i * chi;
-      const double a = A[i * ENVB_LD + j];
-      if (i != j)
-        off += a * a;
-      else
-        dg += a * a;
-    }
-    off = wave_sum_d(off);
-    dg = wave_sum_d(dg);
-    if (off <= 1e-30 * dg || off == 0.0 || off >= prev) break;
-    prev = off;
-    for (int st = 0; st < ne - 1; ++st) {
-      if (l < np) {
-        int p, q;
-        rr_pair(ne, st, l, p, q);
-        double c = 1, sn = 0;
-        if (q < chi) {
-          const double apq = A[p * ENVB_LD + q];
-          if (apq != 0.0) {
-            const double zeta = (A[q * ENVB_LD + q] - A[p * ENVB_LD + p]) / (2 * apq);
-            const double t = (zeta >= 0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1 + zeta * zeta));
-            c = 1 / sqrt(1 + t * t);
-            sn = c * t;
-          }
-        }
-        rc[l] = c;
-        rs[l] = sn;
-        rp[l] = p;
-        rq[l] = q;
-      }
-      wave_sync_ap();
-      for (int o = l; o < np * chi; o += 64) {  // rows: A <- J^T A
-        const int i = o / chi, col = o - i * chi;
-        const int p = rp[i], q = rq[i];
-        if (q >= chi) continue;
-        const double c = rc[i], sn = rs[i];
-        const double ap = A[p * ENVB_LD + col], aq = A[q * ENVB_LD + col];
-        A[p * ENVB_LD + col] = c * ap - sn * aq;
-        A[q * ENVB_LD + col] = sn * ap + c * aq;
-      }
-      wave_sync_ap();
-      for (int o = l; o < np * chi; o += 64) {  // columns: A <- A J, V <- V J
-        const int i = o / chi, row = o - i * chi;
-        const int p = rp[i], q = rq[i];
-        if (q >= chi) continue;
-        const double c = rc[i], sn = rs[i];
-        const double ap = A[row * ENVB_LD + p], aq = A[row * ENVB_LD + q];
-        A[row * ENVB_LD + p] = c * ap - sn * aq;
-        A[row * ENVB_LD + q] = sn * ap + c * aq;
-        const double vp = V[row * ENVB_LD + p], vq = V[row * ENVB_LD + q];
-        V[row * ENVB_LD + p] = c * vp - sn * vq;
-        V[row * ENVB_LD + q] = sn * vp + c * vq;
-      }
-      wave_sync_ap();
-    }
-  }
-  // truncation: rank |lambda| descending (ties by index); drop from the small
-  // end while the dropped weight / total <= cutoff (keep >= 1)
-  if (l < chi) {
-    const double wl = fabs(A[l * ENVB_LD + l]);
-    int r = 0;
-    for (int m = 0; m < chi; ++m) {
-      const double wm = fabs(A[m * ENVB_LD + m]);
-      if (wm > wl || (wm == wl && m < l)) ++r;
-    }
-    rank[l] = r;
-    byr[r] = l;
-  }
-  wave_sync_ap();
-  double tot = 0;
-  for (int m = 0; m < chi; ++m) tot += fabs(A[m * ENVB_LD + m]);
-  int keep = chi;
-  double disc = 0;
-  while (keep > 1 && tot > 0) {
-    const int m = byr[keep - 1];
-    const double x = fabs(A[m * ENVB_LD + m]);
-    if ((disc + x) / tot > cutoff) break;
-    disc += x;
-    --keep;
-  }
-  // S[i][j] = sum_m V[i][m] V[j][m] sqrt(l_m) over the kept m, Si with 1 / sqrt
-  for (int o = l; o < chi * chi; o += 64) {
-    const int i = o / chi, j = o - i * chi;
-    double sv = 0, siv = 0;
-    for (int m = 0; m < chi; ++m) {
-      if (rank[m] >= keep) continue;
-      const double sq = sqrt(A[m * ENVB_LD + m]);  // NaN for a kept negative eigenvalue
-      const double vv = V[i * ENVB_LD + m] * V[j * ENVB_LD + m];
-      sv += vv * sq;
-      siv += vv / sq;
-    }
-    S[i * chi + j] = sv;
-    Si[i * chi + j] = siv;
-  }
-  wave_sync_ap();
-}
-
-// Exact x / d and x % d by a multiply-high: m = ceil(2^sh / d) with
-// sh = 32 + ceil(log2 d), q = (x m) >> sh, exact for every x < 2^31 (x d <
-// 2^sh, and x m fits 64 bits); the integer divisions of the index arithmetic
-// otherwise cost ~30 instructions each, and the flat element loops of this
-// kernel run one wave per SIMD with nothing to hide them behind.
-struct FastDiv {  // an aggregate, so that a SideGeom can live in LDS
-  unsigned d, sh;
-  unsigned long long m;
-  __device__ unsigned div(unsigned x) const { return (unsigned)(((unsigned long long)x * m) >> sh); }
-  __device__ unsigned mod(unsigned x) const { return x - div(x) * d; }
-};
-__device__ inline FastDiv fast_div(unsigned d) {
-  unsigned sh = 32;
-  while ((1ull << (sh - 32)) < d) ++sh;
-  return FastDiv{d, sh, ((1ull << sh) + d - 1) / d};
-}
-
 struct SideGeom {
   int d, k, j, chib, E, n, r;
   int dims[ITNBP_MAXR];
@@ -460,43 +238,6 @@ __device__ void ext_mode_product(const SideGeom& g, int pa, const double* X, dou
         acc += X[(lo + stride * (b + chi * hi)) + (long long)g.E * c] * m;
       }
     Y[idx] = acc;
-  }
-  __syncthreads();
-}
-
-// The same mode product for the global-memory variant, one fibre per thread:
-// a thread loads the chi entries of one (lo, hi, column) fibre once and writes
-// all chi outputs, with Mt (transposed if asked) staged in LDS at ms (CH x CH;
-// every lane of a wave reads the same entry).  The per-output form above
-// reloads each fibre chi times, which from global memory costs more than the
-// multiply-adds.
-template <int CH>
-__device__ void ext_mode_product_fibre(const SideGeom& g, int pa, const double* X, double* Y, int cols,
-                                       const double* Mt, bool transpose, double* ms) {
-  const int stride = (int)g.fst[pa].d;
-  const int chi = g.dims[g.ext[pa]];
-  for (int i = threadIdx.x; i < chi * chi; i += blockDim.x) {
-    const int b = i / chi, b2 = i - b * chi;
-    ms[b * CH + b2] = transpose ? Mt[b2 * chi + b] : Mt[b * chi + b2];
-  }
-  __syncthreads();
-  const int per = g.E / chi;  // fibres per column
-  const FastDiv fper = fast_div((unsigned)per);
-  const int nfib = per * cols;
-  for (int f = threadIdx.x; f < nfib; f += blockDim.x) {
-    const int c = (int)fper.div(f), r = f - c * per;
-    const int hi = (int)g.fst[pa].div(r), lo = r - hi * stride;
-    const long long base = (long long)g.E * c + lo + (long long)stride * chi * hi;
-    double x[CH];
-#pragma unroll
-    for (int b = 0; b < CH; ++b) x[b] = b < chi ? X[base + (long long)stride * b] : 0.0;
-#pragma unroll 4
-    for (int b2 = 0; b2 < chi; ++b2) {
-      double acc = 0;
-#pragma unroll
-      for (int b = 0; b < CH; ++b) acc += x[b] * ms[b * CH + b2];
-      Y[base + (long long)stride * b2] = acc;
-    }
   }
   __syncthreads();
 }
@@ -693,86 +434,6 @@ __device__ void wave_apply_q16(const double* V, int ldv, int rows, int n, const 
   }
 }
 
-// One-sided Jacobi SVD of A (M x N, column-major, M >= N) in place:
-// A <- U diag(s), V (N x N column-major) accumulated unless V is null.  A pair is rotated while
-// |<a_p, a_q>| > tol |a_p| |a_q| with tol = 8 eps sqrt(M), the rounding error
-// of the inner product itself, and while both columns are above the rounding
-// level of A (|a|^2 > eps^2 ||A||_F^2): a column at that level is zero to
-// working precision, and rotating it against its rounding noise would keep
-// the sweeps going.  The pairs of a step are disjoint and each group of G
-// threads reads and writes only its own rows of its pair, so a step needs one
-// barrier (before the next step's pairing).  Returns the number of sweeps.
-__device__ int jacobi_svd(double* A, int M, int N, double* V, double* rot, double* red) {
-  const int tid = threadIdx.x;
-  if (V)
-    for (int i = tid; i < N * N; i += blockDim.x) V[i] = (i % N == i / N) ? 1.0 : 0.0;
-  double fro = 0;
-  for (int i = tid; i < M * N; i += blockDim.x) fro += A[i] * A[i];
-  fro = block_sum_d(fro, red);
-  if (N == 1) return 0;
-  const int ne = N + (N & 1);
-  const double tol = 8 * 2.220446049250313e-16 * sqrt((double)M);
-  const double floor2 = 2.220446049250313e-16 * 2.220446049250313e-16 * fro;
-  int sweep = 0;
-  for (; sweep < 60; ++sweep) {
-    int rotated = 0;
-    for (int st = 0; st < ne - 1; ++st) {
-      // each pair handled by a group of G threads
-      // (the largest power of two <= 64 with G npair <= blockDim.x: every pair
-      // has a group for N <= 2 blockDim.x)
-      const int npair = ne / 2;
-      int G = 64;
-      while (G > 1 && G * npair > (int)blockDim.x) G >>= 1;
-      const int pi = tid / G, gl = tid % G;
-      double alpha = 0, beta = 0, gamma = 0;
-      int p = 0, q = 0;
-      const bool active = pi < npair;
-      if (active) {
-        rr_pair(ne, st, pi, p, q);
-        if (q < N) {
-          for (int i = gl; i < M; i += G) {
-            const double ap = A[i + (long long)M * p], aq = A[i + (long long)M * q];
-            alpha += ap * ap;
-            beta += aq * aq;
-            gamma += ap * aq;
-          }
-        }
-      }
-      for (int m = G / 2; m > 0; m >>= 1) {
-        alpha += __shfl_xor(alpha, m);
-        beta += __shfl_xor(beta, m);
-        gamma += __shfl_xor(gamma, m);
-      }
-      double c = 1, s = 0;
-      if (active && q < N && alpha > floor2 && beta > floor2 && fabs(gamma) > tol * sqrt(alpha * beta)) {
-        const double zeta = (beta - alpha) / (2 * gamma);
-        const double t = (zeta >= 0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1 + zeta * zeta));
-        c = 1 / sqrt(1 + t * t);
-        s = c * t;
-        rotated = 1;
-      }
-      if (active && q < N && s != 0.0) {
-        for (int i = gl; i < M; i += G) {
-          const double ap = A[i + (long long)M * p], aq = A[i + (long long)M * q];
-          A[i + (long long)M * p] = c * ap - s * aq;
-          A[i + (long long)M * q] = s * ap + c * aq;
-        }
-        if (V)
-          for (int i = gl; i < N; i += G) {
-            const double vp = V[i + N * p], vq = V[i + N * q];
-            V[i + N * p] = c * vp - s * vq;
-            V[i + N * q] = s * vp + c * vq;
-          }
-      }
-      __syncthreads();
-    }
-    // a barrier that also tells every thread whether any pair rotated (no
-    // shared flag to reset, so no thread can see the next sweep's reset)
-    if (!__syncthreads_or(rotated)) break;
-  }
-  return sweep + 1;
-}
-
 // Householder QR with column pivoting of A (M x N column-major in LDS,
 // N <= M <= 32) by one wave with A in registers, keeping R only: on return A's
 // top N x N upper triangle holds R with A P = Q R, and perm[j] is the original
@@ -939,68 +600,6 @@ __device__ int wave_jacobi_svd32(double* A, int M, int N, double* V) {
   return sweep + 1;
 }
 
-// ---- Gram-based QR of a side, global-memory variant ----------------------
-// The QR of a tall side enters simple_update_bp only through R (in Theta) and
-// Q (in the rebuild), and any factorisation X = Q R with orthonormal Q gives
-// the same psi' (R changes by an orthogonal factor that Theta's SVD absorbs).
-// Here: G = X^T X = V diag(l) V^T (one-sided Jacobi of the symmetric G),
-// directions with l <= n eps l_max dropped (rank r); X1 = X T with
-// T = V_r diag(l_r)^{-1/2}; G1 = X1^T X1 = R1^T R1 (Cholesky, G1 ~ I); then
-// R = R1 diag(l_r)^{1/2} V_r^T (r x n) and Q = X Tq, Tq = T R1^{-1}: the
-// second Gram removes the first one's loss of orthogonality (the scheme of
-// CholeskyQR2).  Directions of X below ~sqrt(n eps) of its largest singular
-// value are dropped, as rank-deficient ones.  Every step streams X through
-// the workgroup from global memory a fixed number of times, where the
-// column-by-column Householder QR reads it once per column.
-
-// G = X^T X (n x n, ld n, in LDS) of X (E x n column-major, global), the rows
-// staged through `tile` (tile_cap doubles of LDS) in chunks, the products on
-// the FP64 matrix cores: wave w owns the 16-row block w of G and its four
-// 16 x 16 tiles (n <= 64), v_mfma_f64_16x16x4f64 with A[i][k] = X[e + k][16 w + i]
-// and B[k][j] = X[e + k][16 bj + j] for four rows e.. e + 3 per step (rows past
-// the chunk and columns past n read as zero); D[4 v + l / 16][l % 16] is value
-// v of lane l
-__device__ void gram_rows(const double* X, long long E, int n, double* G, double* tile, int tile_cap) {
-  const int tid = threadIdx.x, l = tid & 63, wv = tid >> 6, li = l & 15, lk = l >> 4;
-  const int ld = tile_cap / n;  // rows of a chunk + 1 (odd pitch against bank conflicts)
-  const int cr = (ld & 1) ? ld - 1 : ld - 2;
-  const int pitch = cr + 1;
-  f64x4 acc[4];
-#pragma unroll
-  for (int t = 0; t < 4; ++t) acc[t] = f64x4{0, 0, 0, 0};
-  const int ri = 16 * wv + li;  // this lane's row of G (A operand column of X)
-  for (long long e0 = 0; e0 < E; e0 += cr) {
-    const int rows = (int)((E - e0) < cr ? (E - e0) : cr);
-    __syncthreads();  // the previous chunk is consumed
-    for (int idx = tid; idx < rows * n; idx += blockDim.x) {
-      const int c = idx / rows, rr = idx - c * rows;
-      tile[c * pitch + rr] = X[e0 + rr + E * c];
-    }
-    __syncthreads();
-    if (16 * wv < n)
-      for (int k0 = 0; k0 < rows; k0 += 4) {
-        const int rr = k0 + lk;
-        const bool rin = rr < rows;
-        const double av = (rin && ri < n) ? tile[ri * pitch + rr] : 0.0;
-#pragma unroll
-        for (int bj = 0; bj < 4; ++bj) {
-          const int cj = 16 * bj + li;
-          const double bv = (rin && cj < n) ? tile[cj * pitch + rr] : 0.0;
-          acc[bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, acc[bj], 0, 0, 0);
-        }
-      }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int bj = 0; bj < 4; ++bj)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int row = 16 * wv + 4 * v + lk, col = 16 * bj + li;
-      if (row < n && col < n) G[row + n * col] = acc[bj][v];
-    }
-  __syncthreads();
-}
-
 // out[e + E j] = sum_c X[e + E c] W[c + n j] for j < m (n <= 64), W (n x m,
 // ld n) in LDS, on the FP64 matrix cores: wave w takes the 16-row blocks
 // w, w + 4, ..; a block's A operands (A[i][k] = X[e0 + i][4 s + k], lane
@@ -1039,116 +638,9 @@ __device__ void rows_times(const double* X, long long E, int n, const double* W,
   __syncthreads();
 }
 
-// The factorisation above for one side.  X (E x n, global) is left unchanged;
-// Xw (E x n, global) is work; lds: 4 n^2 + 4 n doubles of LDS (>= 4 AP_N_BIG^2
-// + ...); R (r x n, ld r) and Tq (n x r, ld n) to global, lam: n doubles of
-// LDS.  Returns r.
-__device__ int gram_qr(const double* X, long long E, int n, double* Xw, double* lds, int lds_cap, double* lam,
-                       int* keep_idx, double* R, double* Tq, double* rot, double* red) {
-  const int tid = threadIdx.x;
-  double* G = lds;             // n x n: G, then U diag(l); then G1 / R1 (r x r)
-  double* V = G + n * n;       // n x n
-  double* T = V + n * n;       // n x r
-  double* work = T + n * n;    // Gram staging
-  const int wcap = lds_cap - 3 * n * n;
-  __shared__ int s_rank;
-  gram_rows(X, E, n, G, T, lds_cap - 2 * n * n);
-  if (n <= 32) {
-    // one wave, QR-preconditioned (as for Theta): G P = Q R, Jacobi on R^T ->
-    // U_x diag(l); G's eigenvectors are P U_x, its eigenvalues the column norms
-    __shared__ int gperm[32];
-    double* Xr = T;  // free until T is built
-    if (tid < 64) wave_qrcp32(G, n, n, gperm);
-    __syncthreads();
-    for (int i = tid; i < n * n; i += blockDim.x) {
-      const int row = i % n, col = i / n;
-      Xr[i] = col <= row ? G[col + n * row] : 0.0;
-    }
-    __syncthreads();
-    if (tid < 64) wave_jacobi_svd32<false>(Xr, n, n, nullptr);
-    __syncthreads();
-    for (int j = tid; j < n; j += blockDim.x) {
-      double t = 0;
-      for (int i = 0; i < n; ++i) t += Xr[i + n * j] * Xr[i + n * j];
-      lam[j] = sqrt(t);
-    }
-    __syncthreads();
-    for (int idx = tid; idx < n * n; idx += blockDim.x) {
-      const int i = idx % n, j = idx / n;
-      V[gperm[i] + n * j] = lam[j] > 0 ? Xr[i + n * j] / lam[j] : 0.0;
-    }
-    __syncthreads();
-  } else {
-    jacobi_svd(G, n, n, V, rot, red);
-    // eigenvalues of the PSD G: the column norms of U diag(l)
-    for (int j = tid; j < n; j += blockDim.x) {
-      double t = 0;
-      for (int i = 0; i < n; ++i) t += G[i + n * j] * G[i + n * j];
-      lam[j] = sqrt(t);
-    }
-    __syncthreads();
-  }
-  if (tid == 0) {
-    double lmax = 0;
-    for (int j = 0; j < n; ++j) lmax = lam[j] > lmax ? lam[j] : lmax;
-    int r = 0;
-    for (int j = 0; j < n; ++j)
-      if (lam[j] > n * 2.220446049250313e-16 * lmax) keep_idx[r++] = j;
-    if (r == 0) keep_idx[r++] = 0;  // X = 0: one zero direction, R = 0
-    s_rank = r;
-  }
-  __syncthreads();
-  const int r = s_rank;
-  for (int idx = tid; idx < n * r; idx += blockDim.x) {
-    const int c = idx % n, k = idx / n;
-    const double l = lam[keep_idx[k]];
-    T[idx] = l > 0 ? V[c + n * keep_idx[k]] / sqrt(l) : 0.0;
-  }
-  __syncthreads();
-  rows_times(X, E, n, T, r, Xw);  // X1 = X T
-  gram_rows(Xw, E, r, G, work, wcap);  // G1 = X1^T X1 (r x r, ld r)
-  // Cholesky G1 = R1^T R1 in place (upper triangle, ld r); a non-positive pivot
-  // (a zero column of X1) gives a unit diagonal and a zero row
-  for (int k = 0; k < r; ++k) {
-    const double pkk = G[k + r * k];
-    const double piv = pkk > 0 ? sqrt(pkk) : 0.0;
-    __syncthreads();
-    for (int j = k + tid; j < r; j += blockDim.x)
-      G[k + r * j] = j == k ? (piv > 0 ? piv : 1.0) : (piv > 0 ? G[k + r * j] / piv : 0.0);
-    __syncthreads();
-    const int m = r - k - 1;
-    for (int idx = tid; idx < m * m; idx += blockDim.x) {
-      const int i = k + 1 + idx % m, j = k + 1 + idx / m;
-      if (i <= j) G[i + r * j] -= G[k + r * i] * G[k + r * j];
-    }
-    __syncthreads();
-  }
-  // R = R1 diag(l_r)^{1/2} V_r^T
-  for (int idx = tid; idx < r * n; idx += blockDim.x) {
-    const int i = idx % r, c = idx / r;
-    double t = 0;
-    for (int k = i; k < r; ++k) t += G[i + r * k] * sqrt(lam[keep_idx[k]]) * V[c + n * keep_idx[k]];
-    R[i + r * c] = t;
-  }
-  // Tq = T R1^{-1}: forward substitution along each row of T
-  for (int c = tid; c < n; c += blockDim.x)
-    for (int j = 0; j < r; ++j) {
-      double t = T[c + n * j];
-      for (int k = 0; k < j; ++k) t -= Tq[c + n * k] * G[k + r * j];
-      Tq[c + n * j] = t / G[j + r * j];
-    }
-  __syncthreads();
-  return r;
-}
-
-// BIG = false: the side matrices (E n <= AP_XY) and every small matrix in LDS,
-// the Householder reflectors of each side saved to `work` (2 AP_SIDE doubles
-// per gate).  BIG = true: the same steps with every matrix in a global
-// workspace of prm.big_stride doubles per gate at `work` (layout below), for
-// external bonds up to AP_ENV_BIG, d chi_b <= AP_N_BIG and Theta up to
-// AP_TH_BIG square; LDS holds the geometry, the vectors and the environment
-// eigenproblems.
-template <bool BIG>
+// The side matrices (E n <= AP_XY) and every small matrix in LDS, the
+// Householder reflectors of each side saved to `work` (2 AP_SIDE doubles per
+// gate).
 __global__ __launch_bounds__(256) void k_apply_gates(const ApplyItem* __restrict__ items,
                                                      const VDesc* __restrict__ vds,
                                                      double* __restrict__ psi,
@@ -1158,44 +650,19 @@ __global__ __launch_bounds__(256) void k_apply_gates(const ApplyItem* __restrict
                                                      double* __restrict__ truncerr,
                                                      double* __restrict__ svals, int* __restrict__ kept,
                                                      int* __restrict__ status) {
-  constexpr int TH = BIG ? AP_TH_BIG : AP_TH;           // rows/cols of Theta
-  constexpr int ENV = BIG ? AP_ENV_BIG : AP_ENV;        // external bond dimension
-  constexpr int RS = ENV * ENV;                         // one environment root
-  static_assert(4 * ENVB_WORK <= AP_TH_BIG * AP_TH_BIG, "environment work must fit the Theta area");
-  static_assert(2 * AP_F_BIG >= AP_TH_BIG * AP_TH_BIG, "a copy of Theta must fit the R factors' area");
+  constexpr int TH = AP_TH;             // rows/cols of Theta
+  constexpr int RS = AP_ENV * AP_ENV;   // one environment root
   extern __shared__ __align__(16) double sm[];
-  double *X, *Y, *Ru, *Rv, *roots, *small, *A, *VV, *scr_u, *scr_v;
-  double *tq_u = nullptr, *tq_v = nullptr;  // BIG: Q = X Tq of each side
-  if constexpr (BIG) {
-    // per gate in global memory: QR of side u (E_u n_u), of side v, two work
-    // matrices (E max(n, d keep)), the R / factor matrices, V of the SVD
-    // (when it does not fit in LDS beside Theta), the roots; in LDS the small
-    // vectors, the matrix of a mode product and Theta / U diag(s)
-    double* w = work + (long long)blockIdx.x * prm.big_stride;
-    scr_u = w;
-    scr_v = scr_u + prm.big_q;
-    X = scr_v + prm.big_q;
-    Y = X + prm.big_x;
-    Ru = Y + prm.big_x;
-    Rv = Ru + AP_F_BIG;
-    VV = Rv + AP_F_BIG;
-    roots = VV + AP_TH_BIG * AP_TH_BIG;
-    tq_u = roots + 2 * AP_MAXEXT * 2 * RS;
-    tq_v = tq_u + AP_N_BIG * AP_N_BIG;
-    small = sm;
-    A = sm + AP_BIG_SMALL + AP_ENV_BIG * AP_ENV_BIG;
-  } else {
-    X = sm;                       // AP_XY: QR, then SVD workspace
-    Y = X + AP_XY;                // AP_XY: mode-product partner, rebuild
-    Ru = Y + AP_XY;               // 1024: R_u (r x n), then the left factor
-    Rv = Ru + 1024;               // 1024: R_v, then the right factor
-    roots = Rv + 1024;            // 2 sides x AP_MAXEXT x (sqrt, inv sqrt) x AP_ENV^2
-    small = roots + 2 * AP_MAXEXT * 2 * RS;
-    A = X;                        // Theta, then U diag(s)
-    VV = X + 1024;                // V of the SVD
-    scr_u = work + (long long)blockIdx.x * 2 * AP_SIDE;
-    scr_v = scr_u + AP_SIDE;
-  }
+  double* X = sm;               // AP_XY: QR, then SVD workspace
+  double* Y = X + AP_XY;        // AP_XY: mode-product partner, rebuild
+  double* Ru = Y + AP_XY;       // 1024: R_u (r x n), then the left factor
+  double* Rv = Ru + 1024;       // 1024: R_v, then the right factor
+  double* roots = Rv + 1024;    // 2 sides x AP_MAXEXT x (sqrt, inv sqrt) x AP_ENV^2
+  double* small = roots + 2 * AP_MAXEXT * 2 * RS;
+  double* A = X;                // Theta, then U diag(s)
+  double* VV = X + 1024;        // V of the SVD
+  double* scr_u = work + (long long)blockIdx.x * 2 * AP_SIDE;
+  double* scr_v = scr_u + AP_SIDE;
   double* rot = small;
   double* vh = rot + 4 * 32;
   double* beta = vh + AP_N_BIG;
@@ -1203,12 +670,9 @@ __global__ __launch_bounds__(256) void k_apply_gates(const ApplyItem* __restrict
   double* betav = vhv + AP_N_BIG;
   double* svec = betav + AP_N_BIG;
   double* red = svec + TH;
-  double* ms = small + AP_BIG_SMALL;  // BIG: the matrix of a mode product
-  double* envw = A;                   // BIG: ENVB_WORK doubles per wave, phase 1 only
   __shared__ int sh_keep;
   __shared__ int order[TH];
-  __shared__ int gkeep[BIG ? AP_N_BIG : 1];  // BIG: the directions the Gram QR keeps
-  __shared__ int qgemm[2];                    // LDS kernel: side rebuilt as X R^{-1} F
+  __shared__ int qgemm[2];  // side rebuilt as X R^{-1} F
 
   const ApplyItem it = items[blockIdx.x];
   const int tid = threadIdx.x;
@@ -1239,10 +703,7 @@ __global__ __launch_bounds__(256) void k_apply_gates(const ApplyItem* __restrict
       const VDesc& V = vds[side == 0 ? it.u : it.v];
       const int a = g.ext[pa];
       double* S = roots + ((side * AP_MAXEXT + pa) * 2) * RS;
-      if constexpr (BIG)
-        env_roots_big(msg + V.in_msg[a], g.dims[a], prm.eig_cutoff, S, S + RS, envw + wv * ENVB_WORK);
-      else
-        env_roots_wave(msg + V.in_msg[a], g.dims[a], prm.eig_cutoff, S, S + RS);
+      env_roots_wave(msg + V.in_msg[a], g.dims[a], prm.eig_cutoff, S, S + RS);
     }
     __syncthreads();
   }
@@ -1261,10 +722,7 @@ __global__ __launch_bounds__(256) void k_apply_gates(const ApplyItem* __restrict
     double* oth = Y;
     for (int pa = 0; pa < g.next; ++pa) {
       const double* S = roots + ((side * AP_MAXEXT + pa) * 2) * RS;
-      if constexpr (BIG)
-        ext_mode_product_fibre<ENV>(g, pa, cur, oth, g.n, S, false, ms);
-      else
-        ext_mode_product<ENV>(g, pa, cur, oth, g.n, S, false);
+      ext_mode_product<AP_ENV>(g, pa, cur, oth, g.n, S, false);
       double* t = cur;
       cur = oth;
       oth = t;
@@ -1277,13 +735,11 @@ __global__ __launch_bounds__(256) void k_apply_gates(const ApplyItem* __restrict
     double* bts = side == 0 ? beta : betav;
     double* R = side == 0 ? Ru : Rv;
     double* scr = side == 0 ? scr_u : scr_v;
-    if (!BIG) {
-      // X itself, for a rebuild by Q = X R^{-1} (kept if the side qualifies)
-      for (int i = tid; i < g.E * g.n; i += blockDim.x) scr[i] = X[i];
-      __syncthreads();
-    }
+    // X itself, for a rebuild by Q = X R^{-1} (kept if the side qualifies)
+    for (int i = tid; i < g.E * g.n; i += blockDim.x) scr[i] = X[i];
+    __syncthreads();
     if (side == 0) phase_mark(prm, 11);
-    if (!BIG && tsqr_ok(g)) {
+    if (tsqr_ok(g)) {
       // the stacked R factors S (4n x n) in Y, which is free after the copy to X
       const int n4 = 4 * g.n, wv = tid >> 6;
       double* S = Y;
@@ -1305,45 +761,33 @@ __global__ __launch_bounds__(256) void k_apply_gates(const ApplyItem* __restrict
       }
       for (int i = tid; i < n4 * g.n; i += blockDim.x) qx[i] = S[i];
     } else {
-      if constexpr (BIG) {
-        // the Gram QR: X unchanged, Y as work, the rank r replaces min(E, n)
-        const int r = gram_qr(X, g.E, g.n, Y, A, AP_TH_BIG * AP_TH_BIG, svec, gkeep, R, side == 0 ? tq_u : tq_v,
-                              rot, red);
-        if (tid == 0) sgeo[side].r = r;
-        __syncthreads();
-      } else {
-        householder_qr(X, g.E, g.n, vhs, bts, red);
-        for (int idx = tid; idx < g.r * g.n; idx += blockDim.x) {
-          const int i = idx % g.r, c = idx / g.r;
-          R[i + g.r * c] = (i <= c) ? X[i + (long long)g.E * c] : 0.0;  // R[i][c], column-major (ld r)
-        }
+      householder_qr(X, g.E, g.n, vhs, bts, red);
+      for (int idx = tid; idx < g.r * g.n; idx += blockDim.x) {
+        const int i = idx % g.r, c = idx / g.r;
+        R[i + g.r * c] = (i <= c) ? X[i + (long long)g.E * c] : 0.0;  // R[i][c], column-major (ld r)
       }
     }
     if (side == 0) phase_mark(prm, 12);
-    if constexpr (BIG) {
-      for (int i = tid; i < g.E * g.n; i += blockDim.x) scr[i] = X[i];
+    // a tall side whose R has no diagonal entry below 1e-5 of its largest
+    // keeps X and R: the rebuild's Q [F; 0] is then X (R^{-1} F), one small
+    // product, instead of applying the n reflectors (latency-bound), with an
+    // orthogonality error ~eps cond(X); other sides keep their reflectors
+    __syncthreads();  // R is complete
+    if (tid == 0) {
+      bool ok = g.E >= g.n;
+      double dmax = 0, dmin = INFINITY;
+      for (int j = 0; j < g.n && ok; ++j) {
+        const double dj = fabs(R[j + g.r * j]);
+        dmax = dj > dmax ? dj : dmax;
+        dmin = dj < dmin ? dj : dmin;
+      }
+      qgemm[side] = ok && dmax > 0 && isfinite(dmax) && dmin >= 1e-5 * dmax;
+    }
+    __syncthreads();
+    if (qgemm[side]) {
+      for (int i = tid; i < g.n * g.n; i += blockDim.x) scr[AP_XY + i] = R[i];  // ld n (r = n)
     } else {
-      // a tall side whose R has no diagonal entry below 1e-5 of its largest
-      // keeps X and R: the rebuild's Q [F; 0] is then X (R^{-1} F), one small
-      // product, instead of applying the n reflectors (latency-bound), with an
-      // orthogonality error ~eps cond(X); other sides keep their reflectors
-      __syncthreads();  // R is complete
-      if (tid == 0) {
-        bool ok = g.E >= g.n;
-        double dmax = 0, dmin = INFINITY;
-        for (int j = 0; j < g.n && ok; ++j) {
-          const double dj = fabs(R[j + g.r * j]);
-          dmax = dj > dmax ? dj : dmax;
-          dmin = dj < dmin ? dj : dmin;
-        }
-        qgemm[side] = ok && dmax > 0 && isfinite(dmax) && dmin >= 1e-5 * dmax;
-      }
-      __syncthreads();
-      if (qgemm[side]) {
-        for (int i = tid; i < g.n * g.n; i += blockDim.x) scr[AP_XY + i] = R[i];  // ld n (r = n)
-      } else {
-        for (int i = tid; i < g.E * g.n; i += blockDim.x) scr[i] = X[i];  // the reflectors
-      }
+      for (int i = tid; i < g.E * g.n; i += blockDim.x) scr[i] = X[i];  // the reflectors
     }
     __syncthreads();
     if (side == 0) phase_mark(prm, 13);
@@ -1357,8 +801,6 @@ __global__ __launch_bounds__(256) void k_apply_gates(const ApplyItem* __restrict
   const double* G = gates + it.gate;
   const bool tr = Mr < Nc;
   const int M = tr ? Nc : Mr, N = tr ? Mr : Nc;
-  if constexpr (BIG)
-    if (M * N + N * N <= AP_TH_BIG * AP_TH_BIG) VV = A + M * N;  // else in the global workspace
   for (int idx = tid; idx < Mr * Nc; idx += blockDim.x) {
     const int row = idx % Mr, col = idx / Mr;
     const int ru = row % gu.r, sup = row / gu.r;
@@ -1378,53 +820,34 @@ __global__ __launch_bounds__(256) void k_apply_gates(const ApplyItem* __restrict
   __syncthreads();
   phase_mark(prm, 3);
   // 4. SVD
-  // Theta up to 32 x 32 (QR-preconditioned one-sided Jacobi, one wave):
+  // QR-preconditioned one-sided Jacobi, one wave (Theta is at most 32 x 32):
   // Theta P = Q R by a pivoted Householder QR, then Jacobi on X = R^T in
   // registers, X <- U_x diag(s) (R^T = U_x S V_x^T, so Theta = (Q V_x) S (P U_x)^T):
   // V_Theta = P U_x, and the kept U_Theta s = Theta V_Theta from a copy of
   // Theta, so neither Q nor V_x is formed.  The pivoting grades X's columns and
-  // halves the sweeps (7 instead of 13-14 on a config-2 Theta).  Larger Theta
-  // (global-memory variant): the workgroup's Jacobi on Theta, V accumulated.
+  // halves the sweeps (7 instead of 13-14 on a config-2 Theta).
   int nsweeps = 0;
-  const bool pre = M <= 32;
-  double* Th0 = A + 2048;  // pre: a copy of Theta, then X = R^T at Th0 + 1024
+  double* Th0 = A + 2048;  // a copy of Theta, then X = R^T at Th0 + 1024
   double* Xr = Th0 + 1024;
   __shared__ int perm[TH];
-  if (pre) {
-    for (int i = tid; i < M * N; i += blockDim.x) Th0[i] = A[i];
-    __syncthreads();
-    if (tid < 64) wave_qrcp32(A, M, N, perm);
-    __syncthreads();
-    for (int i = tid; i < N * N; i += blockDim.x) {
-      const int row = i % N, col = i / N;
-      Xr[i] = col <= row ? A[col + M * row] : 0.0;  // X[row][col] = R[col][row]
-    }
-    __syncthreads();
-    if (tid < 64) nsweeps = wave_jacobi_svd32<false>(Xr, N, N, nullptr);
-    __syncthreads();
-  } else {
-    if constexpr (BIG) {
-      // Theta > 32 x 32 (global-memory variant): V of the kept columns from a
-      // copy of Theta afterwards, as for the preconditioned path, which spares
-      // the rotation of V (N x N, in global memory at N = 128) in every step;
-      // the copy goes where R_u and R_v were (free once Theta is built)
-      for (int i = tid; i < M * N; i += blockDim.x) Ru[i] = A[i];
-      __syncthreads();
-      nsweeps = jacobi_svd(A, M, N, nullptr, rot, red);
-    } else {
-      nsweeps = jacobi_svd(A, M, N, VV, rot, red);
-    }
+  for (int i = tid; i < M * N; i += blockDim.x) Th0[i] = A[i];
+  __syncthreads();
+  if (tid < 64) wave_qrcp32(A, M, N, perm);
+  __syncthreads();
+  for (int i = tid; i < N * N; i += blockDim.x) {
+    const int row = i % N, col = i / N;
+    Xr[i] = col <= row ? A[col + M * row] : 0.0;  // X[row][col] = R[col][row]
   }
+  __syncthreads();
+  if (tid < 64) nsweeps = wave_jacobi_svd32<false>(Xr, N, N, nullptr);
+  __syncthreads();
   if (prm.ts && tid == 0) {
     prm.ts[blockIdx.x * 16 + 8] = (unsigned long long)nsweeps;
-    prm.ts[blockIdx.x * 16 + 9] = (unsigned long long)((!BIG && tsqr_ok(gu)) + (!BIG && tsqr_ok(gv)));
+    prm.ts[blockIdx.x * 16 + 9] = (unsigned long long)(tsqr_ok(gu) + tsqr_ok(gv));
   }
   for (int j = tid; j < N; j += blockDim.x) {
     double s = 0;
-    if (pre)
-      for (int i = 0; i < N; ++i) s += Xr[i + N * j] * Xr[i + N * j];
-    else
-      for (int i = 0; i < M; ++i) s += A[i + M * j] * A[i + M * j];
+    for (int i = 0; i < N; ++i) s += Xr[i + N * j] * Xr[i + N * j];
     svec[j] = sqrt(s);
   }
   __syncthreads();
@@ -1467,35 +890,22 @@ __global__ __launch_bounds__(256) void k_apply_gates(const ApplyItem* __restrict
   // finite, is left untouched (the host reports the error); every write to psi
   // comes after this point
   if (keep < 0) return;
-  if (BIG && !pre) {
-    // the kept right singular vectors: V_o = Theta^T A_o / s_o^2 (zero for s_o = 0)
-    for (int idx = tid; idx < N * keep; idx += blockDim.x) {
-      const int i = idx % N, o = order[idx / N];
-      const double s2 = svec[o] * svec[o];
-      double t = 0;
-      for (int r = 0; r < M; ++r) t += Ru[r + (long long)M * i] * A[r + (long long)M * o];
-      VV[i + N * o] = s2 > 0 ? t / s2 : 0.0;
-    }
-    __syncthreads();
+  // the kept singular vectors: V_o = P U_x,o = P X_o / s_o, then
+  // A_o = U_o s_o = Theta V_o (a zero singular value gets zero columns, which
+  // its sqrt(s) = 0 factor multiplies anyway)
+  for (int idx = tid; idx < N * keep; idx += blockDim.x) {
+    const int i = idx % N, o = order[idx / N];
+    const double so = svec[o];
+    VV[perm[i] + N * o] = so > 0 ? Xr[i + N * o] / so : 0.0;
   }
-  if (pre) {
-    // the kept singular vectors: V_o = P U_x,o = P X_o / s_o, then
-    // A_o = U_o s_o = Theta V_o (a zero singular value gets zero columns, which
-    // its sqrt(s) = 0 factor multiplies anyway)
-    for (int idx = tid; idx < N * keep; idx += blockDim.x) {
-      const int i = idx % N, o = order[idx / N];
-      const double so = svec[o];
-      VV[perm[i] + N * o] = so > 0 ? Xr[i + N * o] / so : 0.0;
-    }
-    __syncthreads();
-    for (int idx = tid; idx < M * keep; idx += blockDim.x) {
-      const int r = idx % M, o = order[idx / M];
-      double t = 0;
-      for (int i = 0; i < N; ++i) t += Th0[r + M * i] * VV[i + N * o];
-      A[r + M * o] = t;
-    }
-    __syncthreads();
+  __syncthreads();
+  for (int idx = tid; idx < M * keep; idx += blockDim.x) {
+    const int r = idx % M, o = order[idx / M];
+    double t = 0;
+    for (int i = 0; i < N; ++i) t += Th0[r + M * i] * VV[i + N * o];
+    A[r + M * o] = t;
   }
+  __syncthreads();
   // left factor Lf (Mr x keep) = U sqrt(S) into Ru, right factor Rf (Nc x keep) = V sqrt(S) into Rv;
   // A = U diag(s) (M x N), V = VV (N x N); if transposed, Theta = VV S U^T
   for (int idx = tid; idx < Mr * keep; idx += blockDim.x) {
@@ -1515,26 +925,13 @@ __global__ __launch_bounds__(256) void k_apply_gates(const ApplyItem* __restrict
   // 5. rebuild both sides: Y = [F as r x (d keep); 0], apply Q, then M^{-1/2};
   //    the largest-magnitude entry of every new-bond slice of psi_u' (first in
   //    column-major order) is made positive and the same sign applied to psi_v'
-  __shared__ double bond_sign[BIG ? AP_KEEP_BIG : AP_TH];
+  __shared__ double bond_sign[TH];
   for (int side = 0; side < 2; ++side) {
     const SideGeom& g = side == 0 ? gu : gv;
     const double* F = side == 0 ? Ru : Rv;  // rows (r_i, s), r fastest
     const double* scr = side == 0 ? scr_u : scr_v;
     const int cols = g.d * keep;  // column c' = s + d b'
-    if constexpr (BIG) {
-      // Q [F] = X Tq F: W = Tq F (n x cols) in the Theta area (free once the
-      // factors are out), then Y = X W with X (psi with sqrt(env)) from scr
-      const double* Tq = side == 0 ? tq_u : tq_v;
-      for (int idx = tid; idx < g.n * cols; idx += blockDim.x) {
-        const int c = idx % g.n, cc = idx / g.n;
-        const int b = cc / g.d, s = cc - b * g.d;
-        double t = 0;
-        for (int k = 0; k < g.r; ++k) t += Tq[c + g.n * k] * F[(k + g.r * s) + (long long)(g.r * g.d) * b];
-        A[idx] = t;
-      }
-      __syncthreads();
-      rows_times(scr, g.E, g.n, A, cols, Y);
-    } else if (qgemm[side]) {
+    if (qgemm[side]) {
       // W = R^{-1} F (n x cols, back substitution per column) in LDS X, Y = X_side W
       const double* Rg = scr + AP_XY;
       for (int cc = tid; cc < cols; cc += blockDim.x) {
@@ -1585,10 +982,7 @@ __global__ __launch_bounds__(256) void k_apply_gates(const ApplyItem* __restrict
     double* oth = X;
     for (int pa = 0; pa < g.next; ++pa) {
       const double* Si = roots + ((side * AP_MAXEXT + pa) * 2 + 1) * RS;
-      if constexpr (BIG)
-        ext_mode_product_fibre<ENV>(g, pa, cur, oth, cols, Si, true, ms);
-      else
-        ext_mode_product<ENV>(g, pa, cur, oth, cols, Si, true);
+      ext_mode_product<AP_ENV>(g, pa, cur, oth, cols, Si, true);
       double* t = cur;
       cur = oth;
       oth = t;
@@ -1677,17 +1071,12 @@ __global__ __launch_bounds__(256) void k_apply_site(const int* __restrict__ vert
   for (long long i = threadIdx.x; i < V.D; i += blockDim.x) t[i] *= sc;
 }
 
-// dynamic LDS of k_apply_gates<false> / <true>: the matrices (LDS variant
-// only), then rot, four reflector-head vectors, the singular values, the
-// block reduction and (global-memory variant) one environment work area per wave
+// dynamic LDS of k_apply_gates: the matrices, then rot, four reflector-head
+// vectors, the singular values and the block reduction
 size_t apply_lds_bytes() {
   return sizeof(double) * (2 * AP_XY + 2 * 1024 + 2 * AP_MAXEXT * 2 * AP_ENV * AP_ENV + 4 * 32 + 4 * AP_N_BIG +
                            AP_TH + 16);
 }
-size_t apply_big_lds_bytes() {
-  return sizeof(double) * (AP_BIG_SMALL + AP_ENV_BIG * AP_ENV_BIG + AP_TH_BIG * AP_TH_BIG);
-}
-
 // per-side sizes of a bond for the kernel limits: E (external size), n = d chi_b
 // (the bond as it is), cols = d chi (the bond's layout during the call)
 struct SideSize {
@@ -1698,13 +1087,6 @@ SideSize side_size(const itnbp_net* net, int x, int e, const std::vector<int>& c
   for (int a = net->inc_ptr[x]; a < net->inc_ptr[x + 1]; ++a)
     if (net->inc_edge[a] != e) z.E *= chi[net->inc_edge[a]];
   return z;
-}
-
-// global workspace of k_apply_gates<true> per gate, in doubles, for side
-// matrices of q = E n and x = E max(n, cols) doubles
-long long big_stride(long long q, long long x) {
-  return 2 * q + 2 * x + 2LL * AP_F_BIG + (long long)AP_TH_BIG * AP_TH_BIG +
-         2LL * AP_MAXEXT * 2 * AP_ENV_BIG * AP_ENV_BIG + 2LL * AP_N_BIG * AP_N_BIG;
 }
 
 // Checks the call and fills the launch items; goff receives the number of gate
@@ -1730,7 +1112,7 @@ long long theta_rank_bound(const itnbp_net* net, int e) {
 // kept rank must fit the bond as it is.
 //
 // With big non-null, a bond past the LDS kernel's limits that fits those of
-// the global-memory variant is marked (*big)[i] = 1 instead of refused.
+// the split pipeline is marked (*big)[i] = 1 instead of refused.
 int prepare_apply(itnbp_net* net, int n, const int* edge_ids, int maxdim, double cutoff, double* svals,
                   int max_keep, const std::vector<int>& chi, bool fixed_bonds, std::vector<ApplyItem>& items,
                   long long& goff, std::vector<char>* big = nullptr) {
@@ -1777,7 +1159,7 @@ int prepare_apply(itnbp_net* net, int n, const int* edge_ids, int maxdim, double
       else if (r * z.n > 1024) lds_why = "apply: R factor larger than 1024";
     }
     if (lds_why) {
-      // the global-memory variant: external bonds <= 32, d chi_b <= 64, Theta <= 128 x 128
+      // the split pipeline: external bonds <= 32, d chi_b <= 64, Theta <= 128 x 128
       bool fits = big != nullptr;
       for (int side = 0; side < 2 && fits; ++side) {
         const int x = side == 0 ? u : v;
@@ -1851,16 +1233,19 @@ ApplyBufs carve_apply_bufs(char* base, int n, long long goff, int mk) {
   return b;
 }
 
-// upload, one launch, read-back; every device buffer comes from b
-// upload, the launches, read-back; every device buffer but the global-memory
-// variant's workspace comes from b.  Gates marked in big run on
-// k_apply_gates<true> after the others, in chunks whose workspace fits the
-// device's free memory (at most 16 GiB).
+// Upload, the launches, read-back; every device buffer but the split
+// pipeline's workspace comes from b.  Gates marked in big run on the split
+// pipeline after the others, in chunks whose workspace fits the device's free
+// memory (at most 16 GiB).  The network keeps a workspace of up to
+// APPLY_BIG_KEEP bytes for its next call (a round is a call per colour class,
+// and an allocation of this size costs more than a launch sequence at small
+// bonds); a larger one is freed at the end of the call.
+constexpr size_t APPLY_BIG_KEEP = 256ULL << 20;
 int run_apply(itnbp_net* net, int n, const std::vector<ApplyItem>& items_in, const double* gates, long long goff,
               int maxdim, double cutoff, int normalize, double* truncerr, double* svals, int mk, int* kept,
               const ApplyBufs& b, const std::vector<char>* big = nullptr) {
   itnbp_ctx* ctx = net->ctx;
-  // the LDS kernel's gates first, then the global-memory variant's (every
+  // the LDS kernel's gates first, then the split pipeline's (every
   // output is indexed by the gate's slot, so the order is free)
   std::vector<ApplyItem> items;
   items.reserve(n);
@@ -1888,7 +1273,7 @@ int run_apply(itnbp_net* net, int n, const std::vector<ApplyItem>& items_in, con
   prm.eig_cutoff = 10 * 2.220446049250313e-16;
   prm.max_keep = mk;
   const size_t lds = apply_lds_bytes();
-  hipError_t ea = hipFuncSetAttribute((const void*)k_apply_gates<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
+  hipError_t ea = hipFuncSetAttribute((const void*)k_apply_gates, hipFuncAttributeMaxDynamicSharedMemorySize,
                                       (int)lds);
   if (ea != hipSuccess)
     return itnbp_fail(ctx, ITNBP_ERR_HIP, std::string("apply: LDS attribute: ") + hipGetErrorString(ea));
@@ -1899,99 +1284,76 @@ int run_apply(itnbp_net* net, int n, const std::vector<ApplyItem>& items_in, con
     ITNBP_HIPCHK(ctx, hipMemsetAsync(tsb.p, 0, (size_t)n * 16 * sizeof(unsigned long long), ctx->stream));
     prm.ts = (unsigned long long*)tsb.p;
   }
-  DevBuf bw;
-  std::unique_ptr<DevBuf, void (*)(DevBuf*)> bw_guard(&bw, [](DevBuf* x) { free_buf(*x); });
-  // the global-memory variant's workspace first, so that a failed allocation
-  // leaves every tensor of the call untouched
-  ApplyParams pb = prm;
-  int chunk = 1;
-  size_t lds_big = 0;
+  // the split pipeline's workspace first, so that a failed allocation leaves
+  // every tensor of the call untouched
+  std::vector<int> chunk_end;  // ends of the launch sequences of items [nl, n)
   if (nb > 0) {
-    // side matrices of the largest gate: E n for the QR, E max(n, d chi) for the work
-    long long q = 1, xs = 1;
-    for (int i = nl; i < n; ++i)
-      for (int side = 0; side < 2; ++side) {
-        const VDesc& V = net->vdesc[side == 0 ? items[i].u : items[i].v];
-        const int j = side == 0 ? items[i].ju : items[i].jv;
-        long long E = 1;
-        for (int a = 1; a <= V.k; ++a)
-          if (a != j) E *= V.dims[a];
-        const long long nn = (long long)V.dims[0] * items[i].chib_in, cols = (long long)V.dims[0] * V.dims[j];
-        q = std::max(q, E * nn);
-        xs = std::max(xs, E * std::max(nn, cols));
-      }
-    pb.big_q = q;
-    pb.big_x = xs;
-    pb.big_stride = (big_stride(q, xs) + 31) & ~31LL;
     size_t fr = 0, tot = 0;
     if (hipMemGetInfo(&fr, &tot) != hipSuccess) fr = 0;
-    const size_t budget = std::min<size_t>(fr / 2, 16ULL << 30);
-    const long long per = pb.big_stride * 8;
-    chunk = (int)std::max<long long>(1, std::min<long long>(nb, (long long)(budget / (size_t)per)));
-    ITNBP_RETCHK(ensure_buf(ctx, bw, (size_t)chunk * per));
-    lds_big = apply_big_lds_bytes();
-    hipError_t eb = hipFuncSetAttribute((const void*)k_apply_gates<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)lds_big);
-    if (eb != hipSuccess)
-      return itnbp_fail(ctx, ITNBP_ERR_HIP, std::string("apply: LDS attribute: ") + hipGetErrorString(eb));
+    const size_t budget = std::min<size_t>(fr / 2 + net->apply_big.bytes, 16ULL << 30);
+    size_t most = 0;
+    for (int c0 = nl; c0 < n;) {
+      int c1 = c0 + 1;
+      size_t bytes = apply_big_bytes(net, items.data() + c0, 1);
+      while (c1 < n) {
+        const size_t more = apply_big_bytes(net, items.data() + c0, c1 + 1 - c0);
+        if (more > budget) break;
+        bytes = more;
+        ++c1;
+      }
+      most = std::max(most, bytes);
+      chunk_end.push_back(c1);
+      c0 = c1;
+    }
+    ITNBP_RETCHK(ensure_buf(ctx, net->apply_big, most));
   }
   const int pm0 = prof_mark(ctx);
   if (nl > 0)
-    hipLaunchKernelGGL(k_apply_gates<false>, dim3(nl), dim3(256), lds, ctx->stream, (const ApplyItem*)b.items,
+    hipLaunchKernelGGL(k_apply_gates, dim3(nl), dim3(256), lds, ctx->stream, (const ApplyItem*)b.items,
                        net->d_vdesc, (double*)net->d_psi, net->d_msg[net->cur], (const double*)b.gates, prm,
                        b.work, b.te, svals ? b.sv : nullptr, b.kept, b.st);
   hipError_t ek = hipGetLastError();
   prof_add(ctx, "apply_gates", pm0, prof_mark(ctx));
   if (ek == hipSuccess && nb > 0) {
-    const int pm1 = prof_mark(ctx);
-    for (int c0 = nl; c0 < n && ek == hipSuccess; c0 += chunk) {
-      const int cn = std::min(chunk, n - c0);
-      pb.ts = prm.ts ? prm.ts + (size_t)c0 * 16 : nullptr;
-      hipLaunchKernelGGL(k_apply_gates<true>, dim3(cn), dim3(256), lds_big, ctx->stream,
-                         (const ApplyItem*)b.items + c0, net->d_vdesc, (double*)net->d_psi, net->d_msg[net->cur],
-                         (const double*)b.gates, pb, (double*)bw.p, b.te, svals ? b.sv : nullptr, b.kept, b.st);
-      ek = hipGetLastError();
+    int c0 = nl;
+    for (int c1 : chunk_end) {
+      const int rc = apply_big_run(net, items.data() + c0, c1 - c0, b.gates, prm, net->apply_big.p, b.te,
+                                   svals ? b.sv : nullptr, b.kept, b.st);
+      if (rc != ITNBP_OK) {
+        (void)hipStreamSynchronize(ctx->stream);
+        return rc;
+      }
+      c0 = c1;
     }
-    prof_add(ctx, "apply_gates_global", pm1, prof_mark(ctx));
   }
   if (prm.ts && ek == hipSuccess) {
-    // mean duration of every phase over the gates that ran to the end, in us,
-    // for the LDS kernel's gates [0, nl) and the global-memory variant's [nl, n)
+    // mean duration of every phase over the LDS kernel's gates that ran to the end, in us
     std::vector<unsigned long long> ts((size_t)n * 16);
     int khz = 0;
     ek = hipMemcpyAsync(ts.data(), prm.ts, ts.size() * 8, hipMemcpyDeviceToHost, ctx->stream);
     if (ek == hipSuccess) ek = hipStreamSynchronize(ctx->stream);
     if (ek == hipSuccess) ek = hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ctx->device);
-    for (int part = 0; part < 2 && ek == hipSuccess && khz > 0; ++part) {
-      const int i0 = part == 0 ? 0 : nl, i1 = part == 0 ? nl : n;
-      double mean[7] = {0, 0, 0, 0, 0, 0, 0}, sweeps = 0, tsq = 0;
-      int cnt = 0;
-      for (int i = i0; i < i1; ++i) {
-        const unsigned long long* t = &ts[(size_t)i * 16];
-        if (!t[7]) continue;
-        ++cnt;
-        for (int p = 0; p < 7; ++p) mean[p] += (double)(t[p + 1] - t[p]) * 1e3 / khz;
-        sweeps += (double)t[8];
-        tsq += (double)t[9];
-      }
-      if (cnt == 0) continue;
-      const double c = cnt;
-      double sub[3] = {0, 0, 0}, load = 0;
-      for (int i = i0; i < i1; ++i) {
-        const unsigned long long* t = &ts[(size_t)i * 16];
-        if (!t[7] || !t[13]) continue;
-        load += (double)(t[10] - t[1]) * 1e3 / khz;
-        for (int p = 0; p < 3; ++p) sub[p] += (double)(t[11 + p] - t[10 + p]) * 1e3 / khz;
-      }
-      const char* what = part == 0 ? "LDS kernel" : "global-memory variant";
-      fprintf(stderr, "  %s, side u of qr (us): psi load %.1f, mode products %.1f, factorisation %.1f, save %.1f\n",
-              what, load / c, sub[0] / c, sub[1] / c, sub[2] / c);
-      fprintf(stderr,
-              "apply phases, %s (us, mean over %d gates): roots %.1f, qr %.1f (%.2f tall-skinny sides), theta %.1f, "
-              "svd %.1f (%.1f sweeps), factors %.1f, rebuild_u %.1f, rebuild_v %.1f\n",
-              what, cnt, mean[0] / c, mean[1] / c, tsq / c, mean[2] / c, mean[3] / c, sweeps / c, mean[4] / c,
-              mean[5] / c, mean[6] / c);
+    double mean[7] = {0, 0, 0, 0, 0, 0, 0}, sub[3] = {0, 0, 0}, load = 0, sweeps = 0, tsq = 0;
+    int cnt = 0;
+    for (int i = 0; i < nl && ek == hipSuccess && khz > 0; ++i) {
+      const unsigned long long* t = &ts[(size_t)i * 16];
+      if (!t[7]) continue;
+      ++cnt;
+      for (int p = 0; p < 7; ++p) mean[p] += (double)(t[p + 1] - t[p]) * 1e3 / khz;
+      sweeps += (double)t[8];
+      tsq += (double)t[9];
+      if (!t[13]) continue;
+      load += (double)(t[10] - t[1]) * 1e3 / khz;
+      for (int p = 0; p < 3; ++p) sub[p] += (double)(t[11 + p] - t[10 + p]) * 1e3 / khz;
     }
+    const double c = cnt;
+    if (cnt > 0)
+      fprintf(stderr,
+              "  side u of qr (us): psi load %.1f, mode products %.1f, factorisation %.1f, save %.1f\n"
+              "apply phases (us, mean over %d gates): roots %.1f, qr %.1f (%.2f tall-skinny sides), theta %.1f, "
+              "svd %.1f (%.1f sweeps), factors %.1f, rebuild_u %.1f, rebuild_v %.1f\n",
+              load / c, sub[0] / c, sub[1] / c, sub[2] / c, cnt, mean[0] / c, mean[1] / c, tsq / c, mean[2] / c,
+              mean[3] / c, sweeps / c, mean[4] / c, mean[5] / c, mean[6] / c);
   }
   std::vector<int> st(n);
   std::vector<int> kp(n);
@@ -2003,6 +1365,7 @@ int run_apply(itnbp_net* net, int n, const std::vector<ApplyItem>& items_in, con
     return itnbp_fail(ctx, ITNBP_ERR_HIP, "apply: workspace layout");
   if (ek == hipSuccess) ek = hipMemcpyAsync(dn.data(), b.te, dn.size(), hipMemcpyDeviceToHost, ctx->stream);
   if (ek == hipSuccess) ek = hipStreamSynchronize(ctx->stream);
+  if (net->apply_big.bytes > APPLY_BIG_KEEP) free_buf(net->apply_big);
   if (ek != hipSuccess) return itnbp_fail(ctx, ITNBP_ERR_HIP, std::string("apply: ") + hipGetErrorString(ek));
   std::memcpy(truncerr, dn.data(), (size_t)n * 8);
   if (svals) std::memcpy(svals, dn.data() + sz[3], (size_t)n * mk * 8);
