@@ -142,7 +142,23 @@ int plan_tasks(itnbp_net* net, const std::vector<OcTask>& tasks, int acc_f64, Ta
   const int eb = acc_f64 ? 8 : 4;
   std::vector<OcTask> small[3], large;
   const size_t lds_cls[3] = {32 * 1024, 64 * 1024, 160 * 1024};
+  // message updates with every bond <= 16 and the site tensor in LDS: the site
+  // kernel, in launches of similar LDS need
+  std::vector<SiteTask> site[SITE_CLASSES];
+  const bool use_site = site_enabled();
   for (const auto& t : tasks) {
+    const VDesc& V = net->vdesc[t.v];
+    if (use_site && !t.s_open && t.j > 0 && t.absorb_mask == (((1 << (V.k + 1)) - 2) & ~(1 << t.j)) &&
+        site_fits(V, eb)) {
+      const int o = (t.j < V.k || V.k == 1) ? 0 : 1;  // the open bond is p (with q = p + 1) or, for the last bond, q
+      SiteTask st = site_task(V, t.j - o, 1 << o);
+      st.out[o] = t.out_off;
+      st.old[o] = t.old_off;
+      st.slot[o] = t.slot;
+      st.normalize[o] = t.normalize;
+      site[site_class(V.D, eb)].push_back(st);
+      continue;
+    }
     const size_t b = oc_small_lds_bytes(net->vdesc[t.v], t, eb);
     if (b == 0) {
       large.push_back(t);
@@ -150,6 +166,19 @@ int plan_tasks(itnbp_net* net, const std::vector<OcTask>& tasks, int acc_f64, Ta
     }
     const int c = b <= lds_cls[0] ? 0 : b <= lds_cls[1] ? 1 : 2;
     small[c].push_back(t);
+  }
+  for (const auto& sc : site) {
+    if (sc.empty()) continue;
+    LaunchGroup lg{};
+    lg.kind = 2;
+    lg.begin = plan.sites.size();
+    lg.count = sc.size();
+    long long dmax = 1;
+    for (const auto& t : sc) dmax = std::max<long long>(dmax, t.D);
+    lg.threads = site_threads(dmax);
+    lg.lds = site_lds_bytes(dmax, eb);
+    plan.sites.insert(plan.sites.end(), sc.begin(), sc.end());
+    plan.groups.push_back(lg);
   }
   for (int c = 0; c < 3; ++c) {
     if (small[c].empty()) continue;
@@ -193,13 +222,22 @@ int plan_tasks(itnbp_net* net, const std::vector<OcTask>& tasks, int acc_f64, Ta
   return ITNBP_OK;
 }
 
-// upload the task table (synchronously) and size the scratch buffers
+// bytes of the open-contraction tasks in the task buffer; the site tasks follow
+static size_t plan_site_offset(const TaskPlan& plan) {
+  return (plan.tasks.size() * sizeof(OcTask) + 255) & ~(size_t)255;
+}
+
+// upload the task tables (synchronously) and size the scratch buffers
 int upload_plan(itnbp_net* net, const TaskPlan& plan, DevBuf& taskbuf) {
   itnbp_ctx* ctx = net->ctx;
-  if (plan.tasks.empty()) return ITNBP_OK;
-  RETCHK(ensure_buf(ctx, taskbuf, plan.tasks.size() * sizeof(OcTask)));
-  HIPCHK(ctx, hipMemcpyAsync(taskbuf.p, plan.tasks.data(), plan.tasks.size() * sizeof(OcTask),
-                             hipMemcpyHostToDevice, ctx->stream));
+  if (plan.tasks.empty() && plan.sites.empty()) return ITNBP_OK;
+  const size_t so = plan_site_offset(plan), sb = plan.sites.size() * sizeof(SiteTask);
+  RETCHK(ensure_buf(ctx, taskbuf, so + sb));
+  if (!plan.tasks.empty())
+    HIPCHK(ctx, hipMemcpyAsync(taskbuf.p, plan.tasks.data(), plan.tasks.size() * sizeof(OcTask),
+                               hipMemcpyHostToDevice, ctx->stream));
+  if (sb)
+    HIPCHK(ctx, hipMemcpyAsync((char*)taskbuf.p + so, plan.sites.data(), sb, hipMemcpyHostToDevice, ctx->stream));
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
   if (plan.scratch_bytes) RETCHK(ensure_buf(ctx, net->scratch, plan.scratch_bytes));
   if (plan.partial_bytes) RETCHK(ensure_buf(ctx, net->partials, plan.partial_bytes));
@@ -221,6 +259,11 @@ int launch_plan(itnbp_net* net, const TaskPlan& plan, size_t g0, size_t g1, cons
       HIPCHK(ctx, launch_oc_small(psi_dtype, plan.acc_f64, net->d_vdesc, d_tasks + lg.begin, (int)lg.count,
                                   psi, msg_in, out, d_stats, lg.lds, s));
       if (main) prof_add(ctx, "oc_small", e0, prof_mark(ctx));
+    } else if (lg.kind == 2) {
+      const SiteTask* sites = (const SiteTask*)((const char*)d_tasks + plan_site_offset(plan));
+      HIPCHK(ctx, launch_site(psi_dtype, plan.acc_f64, sites + lg.begin, (int)lg.count, psi, msg_in, out, d_stats, 0, 1,
+                              lg.threads, lg.lds, nullptr, nullptr, 0, s));
+      if (main) prof_add(ctx, "site", e0, prof_mark(ctx));
     } else {
       HIPCHK(ctx, launch_oc_large(psi_dtype, plan.acc_f64, net->d_vdesc, d_tasks + lg.begin,
                                   plan.tasks.data() + lg.begin, net->vdesc.data(), (int)lg.count, psi,

@@ -75,23 +75,6 @@ __device__ inline void rr_pair(int n, int st, int i, int& p, int& q) {
   }
 }
 
-// Exact x / d and x % d by a multiply-high: m = ceil(2^sh / d) with
-// sh = 32 + ceil(log2 d), q = (x m) >> sh, exact for every x < 2^31 (x d <
-// 2^sh, and x m fits 64 bits); the integer divisions of the index arithmetic
-// otherwise cost ~30 instructions each, and the flat element loops of this
-// kernel run one wave per SIMD with nothing to hide them behind.
-struct FastDiv {  // an aggregate, so that a SideGeom can live in LDS
-  unsigned d, sh;
-  unsigned long long m;
-  __host__ __device__ unsigned div(unsigned x) const { return (unsigned)(((unsigned long long)x * m) >> sh); }
-  __host__ __device__ unsigned mod(unsigned x) const { return x - div(x) * d; }
-};
-__host__ __device__ inline FastDiv fast_div(unsigned d) {
-  unsigned sh = 32;
-  while ((1ull << (sh - 32)) < d) ++sh;
-  return FastDiv{d, sh, ((1ull << sh) + d - 1) / d};
-}
-
 // One-sided Jacobi SVD of A (M x N, column-major, M >= N) in place:
 // A <- U diag(s), V (N x N column-major) accumulated unless V is null.  A pair is rotated while
 // |<a_p, a_q>| > tol |a_p| |a_q| with tol = 8 eps sqrt(M), the rounding error

@@ -47,6 +47,23 @@ __device__ inline TA load_as(const float* p, long long i) { return (TA)p[i]; }
 template <typename TA>
 __device__ inline TA load_as(const bf16_t* p, long long i) { return (TA)bf16_to_f32(p[i]); }
 
+// Exact x / d and x % d by a multiply-high: m = ceil(2^sh / d) with
+// sh = 32 + ceil(log2 d), q = (x m) >> sh, exact for every x < 2^31 (x d <
+// 2^sh, and x m fits 64 bits); the integer divisions of the index arithmetic
+// otherwise cost ~30 instructions each, and flat element loops at one or two
+// waves per SIMD have little to hide them behind.
+struct FastDiv {  // an aggregate, so that a SideGeom can live in LDS
+  unsigned d, sh;
+  unsigned long long m;
+  __host__ __device__ unsigned div(unsigned x) const { return (unsigned)(((unsigned long long)x * m) >> sh); }
+  __host__ __device__ unsigned mod(unsigned x) const { return x - div(x) * d; }
+};
+__host__ __device__ inline FastDiv fast_div(unsigned d) {
+  unsigned sh = 32;
+  while ((1ull << (sh - 32)) < d) ++sh;
+  return FastDiv{d, sh, ((1ull << sh) + d - 1) / d};
+}
+
 // Device-side description of one site tensor and the messages flowing into it.
 struct VDesc {
   long long psi_off;           // element offset of psi_v in the psi buffer
@@ -81,19 +98,13 @@ struct MsgStat {
 };
 
 struct LaunchGroup {
-  int kind;          // 0: small (LDS) path, 1: large (global scratch) path
+  int kind;          // 0: small (LDS) path, 1: large (global scratch) path, 2: site kernel (k_site.hip)
   size_t begin, count;
-  size_t lds;        // small: dynamic LDS bytes
+  size_t lds;        // small, site: dynamic LDS bytes
+  int threads;       // site: workgroup size
   long long maxD;    // large: scratch stride
   int nsplit;        // large: split-K factor
   long long part_stride;
-};
-
-struct TaskPlan {
-  std::vector<OcTask> tasks;
-  std::vector<LaunchGroup> groups;
-  size_t scratch_bytes = 0, partial_bytes = 0;
-  int acc_f64 = 1;
 };
 
 struct DevBuf {

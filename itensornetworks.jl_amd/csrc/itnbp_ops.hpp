@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "itnbp_internal.hpp"
+#include "itnbp_site.hpp"
 
 int itnbp_fail(itnbp_ctx* ctx, int code, const std::string& msg);
 int ensure_buf(itnbp_ctx* ctx, DevBuf& b, size_t bytes);

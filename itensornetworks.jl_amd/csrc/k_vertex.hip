@@ -1,19 +1,18 @@
-// Per-vertex eigenbasis message update for small bond dimensions (every
-// chi <= 16, the site tensor resident in LDS).  One workgroup computes all k
-// outgoing messages of a vertex in a Jacobi sweep
+// Jacobi sweeps of the sites whose bonds are all <= 16: the sites whose tensor
+// fits in LDS as tasks of k_site.hip, two messages per task, and the larger ones
+// by the per-vertex eigenbasis kernels below
 // (updated_message, src/caches/abstractbeliefpropagationcache.jl:225-239):
 //
-//   1. psi_v -> LDS;
-//   2. every incoming message M_c (symmetric) -> M_c = U_c diag(l_c) U_c^T by a
+//   1. every incoming message M_c (symmetric) -> M_c = U_c diag(l_c) U_c^T by a
 //      wave-level cyclic Jacobi (the four waves take one bond each);
-//   3. psi_v rotated in place into the eigenbasis of every bond (fibre by fibre);
-//   4. per bond c: T'_c[r, r'] = sum over the fibres along c of
+//   2. psi_v rotated into the eigenbasis of every bond (fibre by fibre) in a
+//      scratch tensor in global memory;
+//   3. per bond c: T'_c[r, r'] = sum over the fibres along c of
 //      prod_{e != c} l_e[r_e] Y[.., r, ..] Y[.., r', ..];
-//   5. T_c = U_c T'_c U_c^T, symmetrised, normalised, message_diff / residual.
+//   4. T_c = U_c T'_c U_c^T, symmetrised, normalised, message_diff / residual.
 //
 // That is d prod(chi) (k chi + k chi) multiply-adds per vertex for all k
-// messages, versus k (k - 1) chi d prod(chi) for k independent contractions, and
-// psi is read from HBM once per vertex instead of once per message.  The
+// messages, versus k (k - 1) chi d prod(chi) for k independent contractions.  The
 // absorbed form is recovered exactly for any orthogonal U_c (eigenvalues of
 // either sign), so the result is the reference's update for symmetric messages.
 #include <algorithm>
@@ -203,8 +202,7 @@ __device__ inline double block_sum(double v, double* red) {
   return s;
 }
 
-// LDS carve-up (bytes): fixed part, the fibre tables (FMAX weights and base
-// offsets), then Y[D] in TA
+// fixed LDS (bytes), with one Jacobi work area per wave
 constexpr size_t SV_FIXED = (size_t)ITNBP_MAXK * SV_LD * SV_LD * 8   // U_c
                             + 4 * SV_LD * SV_LD * 8                   // Jacobi work, one per wave
                             + (size_t)ITNBP_MAXK * SV_MAXCHI * 8      // l_c
@@ -213,325 +211,18 @@ constexpr size_t SV_FIXED = (size_t)ITNBP_MAXK * SV_LD * SV_LD * 8   // U_c
                             + 2 * SV_LD * SV_LD * 8                   // T', U T'
                             + 64;                                     // block reduction
 
-// One site's update (the task tk) by the whole workgroup; k_vertex_eig runs
-// one task per workgroup, k_vertex_eig_queue a persistent grid that takes
-// tasks from a queue.
-template <typename TS, typename TA, typename TM>
-__device__ __forceinline__ void vertex_eig_task(const VDesc* __restrict__ vdesc, const SmallTask* __restrict__ tk,
-                                                const TS* __restrict__ psi, const TM* msg_in, TM* msg_out,
-                                                MsgStat* __restrict__ stats, int normalize, int fmax,
-                                                double* __restrict__ seeds, int warm,
-                                                const int* __restrict__ active,
-                                                const long long* __restrict__ sweep_ctr) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  double* Us = reinterpret_cast<double*>(smem);
-  double* As = Us + ITNBP_MAXK * SV_LD * SV_LD;
-  double* lam = As + 4 * SV_LD * SV_LD;
-  double* rc = lam + ITNBP_MAXK * SV_MAXCHI;
-  double* rs = rc + 32;
-  int* rp = reinterpret_cast<int*>(rs + 32);
-  int* rq = rp + 32;
-  double* gpart = reinterpret_cast<double*>(rq + 32);
-  double* Tp = gpart + SV_THREADS;
-  double* X = Tp + SV_LD * SV_LD;
-  double* red = X + SV_LD * SV_LD;
-  double* fw = reinterpret_cast<double*>(smem + SV_FIXED);
-  int* fb = reinterpret_cast<int*>(fw + fmax);
-  TA* Y = reinterpret_cast<TA*>(smem + SV_FIXED + (((size_t)fmax * 12 + 15) & ~(size_t)15));
-
-  __shared__ int dims[ITNBP_MAXR], strides[ITNBP_MAXR];
-  // batched update: a finished instance's messages were carried over already
-  if (active && !active[tk->inst]) return;
-  if (sweep_ctr) warm = (*sweep_ctr % 16) != 0;
-  const VDesc* V = vdesc + tk->v;
-  const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63;
-  const int k = V->k, D = V->D;
-  if (tid == 0) {
-    int s = 1;
-    for (int a = 0; a <= k; ++a) {
-      dims[a] = V->dims[a];
-      strides[a] = s;
-      s *= dims[a];
-    }
-  }
-  __syncthreads();
-  // 1. psi -> LDS
-  const TS* src = psi + V->psi_off;
-  for (int i = tid; i < D; i += SV_THREADS) Y[i] = load_as<TA>(src, i);
-  // 2. eigendecompositions, one bond per wave
-  for (int a = wv; a < k; a += 4)
-    bond_eigh(msg_in + V->in_msg[a + 1], dims[a + 1], As + wv * SV_LD * SV_LD, Us + a * SV_LD * SV_LD,
-              lam + a * SV_MAXCHI, seeds + (long long)tk->useed[a] * SEED_LD * SEED_LD, warm, rc + 8 * wv,
-              rs + 8 * wv, rp + 8 * wv, rq + 8 * wv);
-  __syncthreads();
-  // 3. rotate every bond: Y <- Y x_c U_c (in place, one fibre per thread)
-  for (int a = 0; a < k; ++a) {
-    const int n = dims[a + 1], st = strides[a + 1];
-    const int F = D / n;
-    const double* U = Us + a * SV_LD * SV_LD;
-    if (n <= 8) {
-      // U in registers (zero-padded to 8 x 8), read once per bond
-      TA u[8][8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-#pragma unroll
-        for (int r = 0; r < 8; ++r) u[j][r] = (j < n && r < n) ? (TA)U[j * SV_LD + r] : (TA)0;
-      for (int f = tid; f < F; f += SV_THREADS) {
-        const int base = (f % st) + (f / st) * st * n;
-        TA x[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) x[j] = j < n ? Y[base + j * st] : (TA)0;
-#pragma unroll
-        for (int r = 0; r < 8; ++r) {
-          TA acc = 0;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) acc += u[j][r] * x[j];
-          if (r < n) Y[base + r * st] = acc;
-        }
-      }
-      __syncthreads();
-      continue;
-    }
-    for (int f = tid; f < F; f += SV_THREADS) {
-      const int base = (f % st) + (f / st) * st * n;
-      TA x[SV_MAXCHI];
-#pragma unroll
-      for (int j = 0; j < SV_MAXCHI; ++j) x[j] = j < n ? Y[base + j * st] : (TA)0;
-      for (int r = 0; r < n; ++r) {
-        TA acc = 0;
-#pragma unroll
-        for (int j = 0; j < SV_MAXCHI; ++j)
-          if (j < n) acc += (TA)U[j * SV_LD + r] * x[j];
-        Y[base + r * st] = acc;
-      }
-    }
-    __syncthreads();
-  }
-  // 4-5. per bond: weighted Gram, rotate back, normalise, statistics
-  for (int a = 0; a < k; ++a) {
-    const int n = dims[a + 1], st = strides[a + 1], nn = n * n;
-    const int F = D / n;
-    // fibre table: base offset and weight prod_{b != a} l_b of every fibre along a
-    for (int f = tid; f < F; f += SV_THREADS) {
-      const int base = (f % st) + (f / st) * st * n;
-      double w = 1.0;
-      for (int b = 0; b < k; ++b)
-        if (b != a) w *= lam[b * SV_MAXCHI + (base / strides[b + 1]) % dims[b + 1]];
-      fb[f] = base;
-      fw[f] = w;
-    }
-    __syncthreads();
-    if (n <= 8) {
-      // lane (r, gq) of wave wv: row r = l & 7 of T' over the fibres of group
-      // wv * 8 + gq (gq = l >> 3), all n columns at once; fibre groups summed with
-      // shuffles inside the wave, then across the four waves
-      const int r = l & 7, gg = wv * 8 + (l >> 3);
-      double acc8[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) acc8[j] = 0;
-      if (r < n) {
-        // four fibres per step, their loads issued together
-        int f = gg;
-        for (; f + 96 < F; f += 128) {
-          int b[4];
-          double wy[4], y[4][8];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            b[i] = fb[f + 32 * i];
-            wy[i] = fw[f + 32 * i];
-          }
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) y[i][j] = j < n ? (double)Y[b[i] + j * st] : 0.0;
-            wy[i] *= (double)Y[b[i] + r * st];
-          }
-#pragma unroll
-          for (int j = 0; j < 8; ++j) acc8[j] += (wy[0] * y[0][j] + wy[1] * y[1][j]) + (wy[2] * y[2][j] + wy[3] * y[3][j]);
-        }
-        for (; f < F; f += 32) {
-          const int b = fb[f];
-          const double wy = fw[f] * (double)Y[b + r * st];
-#pragma unroll
-          for (int j = 0; j < 8; ++j)
-            if (j < n) acc8[j] += wy * (double)Y[b + j * st];
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        for (int m = 8; m < 64; m <<= 1) acc8[j] += __shfl_xor(acc8[j], m);
-      if (l < 8) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) gpart[wv * 64 + l * 8 + j] = acc8[j];
-      }
-      __syncthreads();
-      if (tid < nn) {
-        const int rr = tid % n, r2 = tid / n;
-        Tp[rr * SV_LD + r2] = (gpart[rr * 8 + r2] + gpart[64 + rr * 8 + r2]) +
-                              (gpart[128 + rr * 8 + r2] + gpart[192 + rr * 8 + r2]);
-      }
-      __syncthreads();
-    }
-    // T' = sum_f w_f y_f y_f^T on the FP64 matrix cores: v_mfma_f64_16x16x4f64
-    // with A[i][k] = w_f Y[f, i] and B[k][j] = Y[f, j] for the four fibres
-    // f = 4 b + k of a fibre block b (lane i + 16 k loads Y[f, i] once; rows and
-    // columns >= n are zero); wave wv takes the blocks b = wv (mod 4), two
-    // accumulators in turn so that consecutive MFMAs do not wait on each other.
-    // D[4 v + l / 16][l % 16] is value v of lane l; the four waves' partial
-    // Grams meet in the Jacobi work area (idle after step 2) and are summed in
-    // a fixed order.  (For n <= 8 the VALU form above is faster: three
-    // quarters of the 16 x 16 tile would be padding.)
-    if (n > 8) {
-      const int li = l & 15, lk = l >> 4;
-      f64x4 acc0 = {0, 0, 0, 0}, acc1 = {0, 0, 0, 0};
-      const int nblk = (F + 3) >> 2;
-      int b4 = wv;
-      for (; b4 + 4 < nblk; b4 += 8) {
-        const int f0 = 4 * b4 + lk, f1 = f0 + 16;
-        double y0 = 0, y1 = 0, w0 = 0, w1 = 0;
-        if (li < n) {
-          if (f0 < F) {
-            y0 = (double)Y[fb[f0] + li * st];
-            w0 = fw[f0];
-          }
-          if (f1 < F) {
-            y1 = (double)Y[fb[f1] + li * st];
-            w1 = fw[f1];
-          }
-        }
-        acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64(w0 * y0, y0, acc0, 0, 0, 0);
-        acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64(w1 * y1, y1, acc1, 0, 0, 0);
-      }
-      for (; b4 < nblk; b4 += 4) {
-        const int f0 = 4 * b4 + lk;
-        double y0 = 0, w0 = 0;
-        if (li < n && f0 < F) {
-          y0 = (double)Y[fb[f0] + li * st];
-          w0 = fw[f0];
-        }
-        acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64(w0 * y0, y0, acc0, 0, 0, 0);
-      }
-      double* part = As;  // 4 x 256 doubles
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int row = 4 * v + lk;
-        if (row < n && li < n) part[wv * 256 + row * 16 + li] = acc0[v] + acc1[v];
-      }
-      __syncthreads();
-      if (tid < nn) {
-        const int rr = tid % n, r2 = tid / n;
-        Tp[rr * SV_LD + r2] = (part[rr * 16 + r2] + part[256 + rr * 16 + r2]) +
-                              (part[512 + rr * 16 + r2] + part[768 + rr * 16 + r2]);
-      }
-      __syncthreads();
-    }
-    const double* U = Us + a * SV_LD * SV_LD;
-    if (tid < nn) {
-      const int b = tid % n, rr = tid / n;
-      double s = 0;
-      for (int r = 0; r < n; ++r) s += U[b * SV_LD + r] * Tp[r * SV_LD + rr];
-      X[b * SV_LD + rr] = s;  // (U T')[b][r']
-    }
-    __syncthreads();
-    double tv = 0;
-    if (tid < nn) {
-      const int i = tid % n, j = tid / n;  // message layout M[i + n j]
-      double sij = 0, sji = 0;
-      for (int r = 0; r < n; ++r) {
-        sij += X[i * SV_LD + r] * U[j * SV_LD + r];
-        sji += X[j * SV_LD + r] * U[i * SV_LD + r];
-      }
-      tv = 0.5 * (sij + sji);
-    }
-    const double n2 = block_sum(tv * tv, red);
-    const double nrm = sqrt(n2);
-    const double sc = (normalize && nrm != 0.0) ? 1.0 / nrm : 1.0;
-    const long long off = tk->out[a];
-    double dot = 0, o2 = 0, d2 = 0, bad = 0;
-    if (tid < nn) {
-      const double nv = tv * sc;
-      const double ov = (double)msg_in[off + tid];
-      if (!isfinite(nv)) bad = 1;
-      dot = ov * nv;
-      o2 = ov * ov;
-      d2 = (nv - ov) * (nv - ov);
-      msg_out[off + tid] = (TM)nv;
-    }
-    dot = block_sum(dot, red);
-    o2 = block_sum(o2, red);
-    d2 = block_sum(d2, red);
-    bad = block_sum(bad, red);
-    const int slot = tk->slot[a];
-    if (tid == 0 && slot >= 0) {
-      const double nn2 = n2 * sc * sc;
-      MsgStat stt;
-      stt.diff = 1.0 - (dot * dot) / (o2 * nn2);
-      stt.res2 = nn2 > 0 ? d2 / nn2 : 0.0;
-      stt.norm = nrm;
-      stt.bad = (bad > 0 || !isfinite(nrm)) ? 1.0 : 0.0;
-      stats[slot] = stt;
-    }
-    __syncthreads();
-  }
-}
-
-template <typename TS, typename TA, typename TM>
-__global__ __launch_bounds__(SV_THREADS) void k_vertex_eig(const VDesc* __restrict__ vdesc,
-                                                          const SmallTask* __restrict__ tasks,
-                                                          const TS* __restrict__ psi, const TM* msg_in,
-                                                          TM* msg_out, MsgStat* __restrict__ stats,
-                                                          int normalize, int fmax, double* __restrict__ seeds,
-                                                          int warm, const int* __restrict__ active,
-                                                          const long long* __restrict__ sweep_ctr) {
-  vertex_eig_task<TS, TA, TM>(vdesc, tasks + blockIdx.x, psi, msg_in, msg_out, stats, normalize, fmax, seeds, warm,
-                              active, sweep_ctr);
-}
-
-// Persistent form: a grid of resident workgroups takes the (cost-sorted) tasks
-// in order from a device counter that k_queue_reset clears before the launch;
-// every workgroup leaves once the counter has passed ntasks, so the grid
-// drains without any wait on another workgroup.
-template <typename TS, typename TA, typename TM>
-__global__ __launch_bounds__(SV_THREADS) void k_vertex_eig_queue(const VDesc* __restrict__ vdesc,
-                                                                const SmallTask* __restrict__ tasks, int ntasks,
-                                                                int* __restrict__ queue, const TS* __restrict__ psi,
-                                                                const TM* msg_in, TM* msg_out,
-                                                                MsgStat* __restrict__ stats, int normalize, int fmax,
-                                                                double* __restrict__ seeds, int warm,
-                                                                const int* __restrict__ active,
-                                                                const long long* __restrict__ sweep_ctr) {
-  __shared__ int next;
-  for (;;) {
-    if (threadIdx.x == 0) next = atomicAdd(queue, 1);
-    __syncthreads();
-    const int t = next;
-    __syncthreads();  // every thread has read next before thread 0 takes the following task
-    if (t >= ntasks) return;
-    vertex_eig_task<TS, TA, TM>(vdesc, tasks + t, psi, msg_in, msg_out, stats, normalize, fmax, seeds, warm, active,
-                                sweep_ctr);
-    __syncthreads();  // the task's last LDS reads come before the next task's writes
-  }
-}
-
-// clears the task counter of k_vertex_eig_queue (a kernel, so that it can sit
-// in a captured graph; one lane writes)
-__global__ void k_queue_reset(int* __restrict__ queue) {
-  if (threadIdx.x == 0) queue[0] = 0;
-}
-
-// The same update for sites whose tensor does not fit in LDS (every chi <= 16,
-// e.g. chi = 12 or 16 at degree 4): psi is copied into a scratch tensor Y in
-// global memory (L2 / Infinity Cache resident while the workgroup works on it),
-// rotated there in place fibre by fibre, and every weighted Gram streams Y
-// through LDS in tiles of FT fibres (base offsets and weights computed by the
-// loader).  Steps 2 and 5 are those of k_vertex_eig.  The tile size is a
-// template parameter; the batched update's autotuner times the VB_TILES
+// The update of a site whose tensor does not fit in LDS (every chi <= 16, e.g.
+// chi = 12 or 16 at degree 4): psi is rotated into a scratch tensor Y in global
+// memory (L2 / Infinity Cache resident while the workgroup works on it), in
+// place fibre by fibre, and every weighted Gram streams Y through LDS in tiles
+// of FT fibres (base offsets and weights computed by the loader).  The tile size
+// is a template parameter; the batched update's autotuner times the VB_TILES
 // variants and keeps the fastest, VB_FT otherwise.
 constexpr int VB_FT = 192;
 constexpr int VB_TILES[3] = {160, 192, 256};
-// fixed LDS of k_vertex_big: that of k_vertex_eig without the Jacobi work
-// areas, which alias the Gram tile (idle while the messages are decomposed), so
-// that four FP32 workgroups share a CU
+// fixed LDS of k_vertex_big: without the Jacobi work areas, which alias the
+// Gram tile (idle while the messages are decomposed), so that four FP32
+// workgroups share a CU
 constexpr size_t VB_FIXED = SV_FIXED - 4 * SV_LD * SV_LD * 8;
 static_assert(160 * SV_LD * sizeof(float) >= 4 * SV_LD * SV_LD * 8, "Jacobi work must fit in the tile area");
 
@@ -960,11 +651,19 @@ __global__ __launch_bounds__(SV_THREADS) void k_vertex_big_mfma(const VDesc* __r
   }
 }
 
+constexpr int QUEUE_STRIDE = 64;
+
 struct SmallState {
-  std::vector<SmallTask> tasks;
+  // LDS-resident sites: tasks of k_site.hip in launches of similar LDS need
+  std::vector<SiteTask> tasks;
+  int nsites = 0;  // sites the tasks cover
   DevBuf d_tasks;
-  size_t lds = 0;
-  int fmax = 0;  // largest fibre count over the tasks' bonds
+  struct Launch {
+    int begin, count, threads;
+    size_t lds;
+    int grid;  // resident workgroups of the persistent form (0: not yet sized)
+  };
+  std::vector<Launch> launches;
   // sites too large for LDS: k_vertex_big with scratch tensors
   std::vector<SmallTask> big;
   DevBuf d_big, ybuf;
@@ -983,19 +682,18 @@ struct SmallState {
   // k_vertex_big variant the autotuner chose (0: none yet) and for which flavour
   int ft = 0;
   bool ft_f32 = false;
-  // persistent small-site launch (k_vertex_eig_queue): its task counter, its
-  // grid of resident workgroups (0: not yet sized), and the autotuner's choice
-  // between it and one workgroup per task (-1: untuned, one per task)
+  // persistent form of the LDS-resident launches: a task counter each
+  // (QUEUE_STRIDE ints apart), and the autotuner's choice between it and one
+  // workgroup per task (-1: untuned, one per task)
   DevBuf queue;
-  int queue_grid = 0;
-  int eig_queue = -1;
+  int site_queue = -1;
 };
 
 // ITNBP_VERTEX_QUEUE=0/1 forces the small-site launch form, else the
 // autotuner's choice, else one workgroup per task
 bool use_queue(const SmallState* st) {
   if (const char* e = getenv("ITNBP_VERTEX_QUEUE")) return atoi(e) != 0;
-  return st->eig_queue == 1;
+  return st->site_queue == 1;
 }
 
 // the k_vertex_big variant of a launch: ITNBP_VERTEX_BIG_TILE=<tile> forces
@@ -1063,52 +761,34 @@ hipError_t launch_big_ft(int ft, itnbp_net* net, SmallState* st, const void* psi
 }
 
 // the LDS-resident sites: one workgroup per task, or the persistent queue form
-template <typename TS, typename TA, typename TM>
-hipError_t launch_small(itnbp_net* net, SmallState* st, const void* psi, const void* msg_in, void* msg_out,
-                        MsgStat* stats, int normalize, double* seeds, int warm, bool queue, hipStream_t stream) {
-  const int ntasks = (int)st->tasks.size();
-  if (!queue || !st->queue.p) {
-    auto kern = k_vertex_eig<TS, TA, TM>;
-    hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)st->lds);
+hipError_t launch_small(itnbp_net* net, SmallState* st, int acc_f64, const void* psi, int psi_dtype,
+                        const void* msg_in, void* msg_out, MsgStat* stats, int normalize, bool queue,
+                        hipStream_t stream) {
+  for (size_t i = 0; i < st->launches.size(); ++i) {
+    SmallState::Launch& L = st->launches[i];
+    int* q = queue && st->queue.p ? (int*)st->queue.p + i * QUEUE_STRIDE : nullptr;
+    if (q && L.grid == 0) {
+      // every workgroup of the grid resident at once
+      int per_cu = 0;
+      hipError_t e = site_queue_occupancy(psi_dtype, acc_f64, L.threads, L.lds, &per_cu);
+      if (e != hipSuccess) return e;
+      L.grid = std::max(1, std::min(L.count, std::max(1, per_cu) * net->ctx->num_cu));
+    }
+    hipError_t e = launch_site(psi_dtype, acc_f64, (const SiteTask*)st->d_tasks.p + L.begin, L.count, psi, msg_in,
+                               msg_out, stats, 1, normalize, L.threads, L.lds, st->active, q, L.grid, stream);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3((unsigned)ntasks), dim3(SV_THREADS), st->lds, stream, (const VDesc*)net->d_vdesc,
-                       (const SmallTask*)st->d_tasks.p, (const TS*)psi, (const TM*)msg_in, (TM*)msg_out, stats,
-                       normalize, st->fmax, seeds, warm, st->active, st->sweep_ctr);
-    return hipGetLastError();
   }
-  auto kern = k_vertex_eig_queue<TS, TA, TM>;
-  hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)st->lds);
-  if (e != hipSuccess) return e;
-  if (st->queue_grid == 0) {
-    // every workgroup of the grid resident at once
-    int per_cu = 0;
-    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)kern, SV_THREADS, st->lds);
-    if (e != hipSuccess) return e;
-    st->queue_grid = std::max(1, std::min(ntasks, std::max(1, per_cu) * net->ctx->num_cu));
-  }
-  hipLaunchKernelGGL(k_queue_reset, dim3(1), dim3(64), 0, stream, (int*)st->queue.p);
-  hipLaunchKernelGGL(kern, dim3((unsigned)st->queue_grid), dim3(SV_THREADS), st->lds, stream,
-                     (const VDesc*)net->d_vdesc, (const SmallTask*)st->d_tasks.p, ntasks, (int*)st->queue.p,
-                     (const TS*)psi, (const TM*)msg_in, (TM*)msg_out, stats, normalize, st->fmax, seeds, warm,
-                     st->active, st->sweep_ctr);
-  return hipGetLastError();
+  return hipSuccess;
 }
 
 template <typename TS, typename TA, typename TM>
-hipError_t launch_impl(itnbp_net* net, SmallState* st, const void* psi, const void* msg_in, void* msg_out,
+hipError_t launch_big_sites(itnbp_net* net, SmallState* st, const void* psi, const void* msg_in, void* msg_out,
                        MsgStat* stats, int normalize) {
   const int warm = (st->sweeps % 16) != 0 ? 1 : 0;
   double* seeds = (double*)st->seeds.p;
-  // the big sites (the longest workgroups) first, so that the LDS-resident
-  // sites fill in behind them
   if (!st->big.empty()) {
     hipError_t e = launch_big_ft<TS, TA, TM>(big_variant<TA>(st), net, st, psi, msg_in, msg_out, stats, normalize,
                                             seeds, warm, net->ctx->stream);
-    if (e != hipSuccess) return e;
-  }
-  if (!st->tasks.empty()) {
-    hipError_t e = launch_small<TS, TA, TM>(net, st, psi, msg_in, msg_out, stats, normalize, seeds, warm,
-                                            use_queue(st), net->ctx->stream);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
@@ -1179,31 +859,22 @@ int small_prepare(itnbp_net* net, const std::vector<int>& seq, int acc_f64, std:
   }
   st->tasks.clear();
   st->big.clear();
+  st->launches.clear();
+  st->nsites = 0;
   st->ytotal = 0;
-  st->lds = 0;
-  st->fmax = 0;
   st->sweeps = 0;
   if (!small_path_enabled(net)) return ITNBP_OK;
   std::vector<int> pos(2 * net->ne, -1);
   for (size_t i = 0; i < seq.size(); ++i) pos[seq[i]] = (int)i;
   const size_t eb = acc_f64 ? 8 : 4;
-  int dmax_all = 0;
+  std::vector<SiteTask> site[SITE_CLASSES];
   for (int v = 0; v < net->nv; ++v) {
     const VDesc& V = net->vdesc[v];
     if (V.k < 1 || V.k > ITNBP_MAXK) continue;
     bool ok = true;
-    int nmin = SV_MAXCHI;
-    for (int a = 1; a <= V.k && ok; ++a) {
-      ok = V.dims[a] <= SV_MAXCHI;
-      nmin = std::min(nmin, V.dims[a]);
-    }
+    for (int a = 1; a <= V.k && ok; ++a) ok = V.dims[a] <= SV_MAXCHI;
     if (!ok) continue;
-    // one LDS carve-up serves every task of the launch: the largest fibre table
-    // and the largest site tensor
-    const int fmax = std::max(st->fmax, V.D / std::max(1, nmin));
-    const int dmax = std::max(dmax_all, V.D);
-    const size_t lds = SV_FIXED + (((size_t)fmax * 12 + 15) & ~(size_t)15) + (size_t)dmax * eb;
-    const bool fits = lds + 256 <= 160 * 1024;  // + the static LDS of the kernel
+    const bool fits = site_fits(V, (int)eb);
     SmallTask t{};
     t.v = v;
     t.inst = st->vinst.empty() ? 0 : st->vinst[v];
@@ -1221,17 +892,28 @@ int small_prepare(itnbp_net* net, const std::vector<int>& seq, int acc_f64, std:
     if (!ok) continue;
     for (int a = 0; a < V.k; ++a) handled[t.slot[a]] = 1;
     if (fits) {
-      st->tasks.push_back(t);
-      st->fmax = fmax;
-      dmax_all = dmax;
-      st->lds = lds;
+      // pairs of neighbouring bonds, both messages of a pair from one task; the
+      // last of an odd number of bonds as the second of a pair of its own
+      ++st->nsites;
+      for (int p = 1; p <= V.k; p += 2) {
+        const int q = p < V.k ? p : (V.k == 1 ? 1 : p - 1), want = p < V.k ? 3 : (V.k == 1 ? 1 : 2);
+        SiteTask s = site_task(V, q, want);
+        s.inst = t.inst;
+        for (int o = 0; o < 2; ++o)
+          if ((want >> o) & 1) {
+            s.out[o] = s.old[o] = t.out[q + o - 1];
+            s.slot[o] = t.slot[q + o - 1];
+            s.normalize[o] = 1;
+          }
+        site[site_class(V.D, (int)eb)].push_back(s);
+      }
     } else {
       t.yoff = st->ytotal;
       st->ytotal += V.D;
       st->big.push_back(t);
     }
   }
-  // costliest sites first (rotations and Grams both scale as D x sum of the
+  // costliest sites first (mode products and Grams both scale as D x sum of the
   // bond dimensions), so that the hardware dispatcher starts the long
   // workgroups early and the short ones fill in behind them
   auto cost = [&](const SmallTask& t) {
@@ -1240,10 +922,24 @@ int small_prepare(itnbp_net* net, const std::vector<int>& seq, int acc_f64, std:
     for (int a = 1; a <= V.k; ++a) s += V.dims[a];
     return (long long)V.D * s;
   };
-  auto by_cost = [&](const SmallTask& x, const SmallTask& y) { return cost(x) > cost(y); };
-  std::stable_sort(st->tasks.begin(), st->tasks.end(), by_cost);
-  std::stable_sort(st->big.begin(), st->big.end(), by_cost);
-  if (!st->tasks.empty() || !st->big.empty())
+  auto site_cost = [](const SiteTask& t) {
+    long long s = (long long)(t.np + t.nq) * (t.want == 3 ? 2 : 1);
+    for (int m = 0; m < t.nmode; ++m) s += t.mode[m].n;
+    return (long long)t.D * s;
+  };
+  std::stable_sort(st->big.begin(), st->big.end(),
+                   [&](const SmallTask& x, const SmallTask& y) { return cost(x) > cost(y); });
+  for (int c = SITE_CLASSES - 1; c >= 0; --c) {
+    if (site[c].empty()) continue;
+    std::stable_sort(site[c].begin(), site[c].end(),
+                     [&](const SiteTask& x, const SiteTask& y) { return site_cost(x) > site_cost(y); });
+    long long dmax = 1;
+    for (const SiteTask& s : site[c]) dmax = std::max<long long>(dmax, s.D);
+    st->launches.push_back(SmallState::Launch{(int)st->tasks.size(), (int)site[c].size(), site_threads(dmax),
+                                              site_lds_bytes(dmax, (int)eb), 0});
+    st->tasks.insert(st->tasks.end(), site[c].begin(), site[c].end());
+  }
+  if (!st->big.empty())
     ITNBP_RETCHK(ensure_buf(ctx, st->seeds, (size_t)std::max(1, 2 * net->ne) * SEED_LD * SEED_LD * 8));
   if (!st->big.empty()) {
     ITNBP_RETCHK(ensure_buf(ctx, st->d_big, st->big.size() * sizeof(SmallTask)));
@@ -1253,10 +949,9 @@ int small_prepare(itnbp_net* net, const std::vector<int>& seq, int acc_f64, std:
     ITNBP_HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
   }
   if (!st->tasks.empty()) {
-    ITNBP_RETCHK(ensure_buf(ctx, st->queue, 256));
-    st->queue_grid = 0;
-    ITNBP_RETCHK(ensure_buf(ctx, st->d_tasks, st->tasks.size() * sizeof(SmallTask)));
-    ITNBP_HIPCHK(ctx, hipMemcpyAsync(st->d_tasks.p, st->tasks.data(), st->tasks.size() * sizeof(SmallTask),
+    ITNBP_RETCHK(ensure_buf(ctx, st->queue, SITE_CLASSES * QUEUE_STRIDE * sizeof(int)));
+    ITNBP_RETCHK(ensure_buf(ctx, st->d_tasks, st->tasks.size() * sizeof(SiteTask)));
+    ITNBP_HIPCHK(ctx, hipMemcpyAsync(st->d_tasks.p, st->tasks.data(), st->tasks.size() * sizeof(SiteTask),
                                      hipMemcpyHostToDevice, ctx->stream));
     ITNBP_HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
   }
@@ -1276,18 +971,16 @@ void small_set_batch(itnbp_net* net, const std::vector<int>& vinst, const int* a
 
 // Times one launch of the LDS-resident sites in each form (one workgroup per
 // task; the persistent queue) on scratch outputs and keeps the faster.
-template <typename TS, typename TA, typename TM>
-int autotune_small(itnbp_net* net, SmallState* st, const void* psi, const void* msg_in, int normalize) {
+static int autotune_small(itnbp_net* net, SmallState* st, int acc_f64, const void* psi, int psi_dtype,
+                          const void* msg_in, int normalize) {
   itnbp_ctx* ctx = net->ctx;
-  DevBuf out, stats, seeds;
+  DevBuf out, stats;
   auto cleanup = [&]() {
     free_buf(out);
     free_buf(stats);
-    free_buf(seeds);
   };
-  int rc = ensure_buf(ctx, out, (size_t)net->msg_total * sizeof(TM));
+  int rc = ensure_buf(ctx, out, (size_t)net->msg_total * (acc_f64 ? 8 : 4));
   if (rc == ITNBP_OK) rc = ensure_buf(ctx, stats, sizeof(MsgStat) * (size_t)std::max(1, 2 * net->ne));
-  if (rc == ITNBP_OK) rc = ensure_buf(ctx, seeds, st->seeds.bytes);
   if (rc != ITNBP_OK) {
     cleanup();
     return rc;
@@ -1298,8 +991,8 @@ int autotune_small(itnbp_net* net, SmallState* st, const void* psi, const void* 
     for (int q = 0; q < 2; ++q) {
       hipError_t e = hipEventRecord(ctx->ev0, ctx->stream);
       if (e == hipSuccess)
-        e = launch_small<TS, TA, TM>(net, st, psi, msg_in, out.p, (MsgStat*)stats.p, normalize, (double*)seeds.p, 0,
-                                     q == 1, ctx->stream);
+        e = launch_small(net, st, acc_f64, psi, psi_dtype, msg_in, out.p, (MsgStat*)stats.p, normalize, q == 1,
+                         ctx->stream);
       if (e == hipSuccess) e = hipEventRecord(ctx->ev1, ctx->stream);
       if (e == hipSuccess) e = hipEventSynchronize(ctx->ev1);
       float ms = 0;
@@ -1314,27 +1007,14 @@ int autotune_small(itnbp_net* net, SmallState* st, const void* psi, const void* 
       }
     }
   cleanup();
-  st->eig_queue = best_q;
+  st->site_queue = best_q;
   return ITNBP_OK;
 }
 
 int small_autotune(itnbp_net* net, int acc_f64, const void* psi, int psi_dtype, const void* msg_in, int normalize) {
   SmallState* st = small_of(net);
   if (st && !st->tasks.empty() && st->queue.p) {
-    int rc;
-    if (acc_f64) {
-      switch (psi_dtype) {
-        case ITNBP_F64: rc = autotune_small<double, double, double>(net, st, psi, msg_in, normalize); break;
-        case ITNBP_F32: rc = autotune_small<float, double, double>(net, st, psi, msg_in, normalize); break;
-        default: rc = autotune_small<bf16_t, double, double>(net, st, psi, msg_in, normalize); break;
-      }
-    } else {
-      switch (psi_dtype) {
-        case ITNBP_F64: rc = autotune_small<double, float, float>(net, st, psi, msg_in, normalize); break;
-        case ITNBP_F32: rc = autotune_small<float, float, float>(net, st, psi, msg_in, normalize); break;
-        default: rc = autotune_small<bf16_t, float, float>(net, st, psi, msg_in, normalize); break;
-      }
-    }
+    const int rc = autotune_small(net, st, acc_f64, psi, psi_dtype, msg_in, normalize);
     if (rc != ITNBP_OK) return rc;
   }
   if (!st || st->big.empty()) return ITNBP_OK;
@@ -1372,7 +1052,7 @@ const char* small_big_kind(itnbp_net* net) {
 
 int small_task_count(itnbp_net* net) {
   SmallState* st = small_of(net);
-  return st ? (int)(st->tasks.size() + st->big.size()) : 0;
+  return st ? st->nsites + (int)st->big.size() : 0;
 }
 
 int small_sweep(itnbp_net* net, int acc_f64, const void* psi, int psi_dtype, const void* msg_in, void* msg_out,
@@ -1381,20 +1061,26 @@ int small_sweep(itnbp_net* net, int acc_f64, const void* psi, int psi_dtype, con
   SmallState* st = small_of(net);
   if (!st || (st->tasks.empty() && st->big.empty())) return ITNBP_OK;
   const int e0 = prof_mark(ctx);
-  hipError_t e;
-  if (acc_f64) {
-    switch (psi_dtype) {
-      case ITNBP_F64: e = launch_impl<double, double, double>(net, st, psi, msg_in, msg_out, stats, normalize); break;
-      case ITNBP_F32: e = launch_impl<float, double, double>(net, st, psi, msg_in, msg_out, stats, normalize); break;
-      default: e = launch_impl<bf16_t, double, double>(net, st, psi, msg_in, msg_out, stats, normalize); break;
-    }
-  } else {
-    switch (psi_dtype) {
-      case ITNBP_F64: e = launch_impl<double, float, float>(net, st, psi, msg_in, msg_out, stats, normalize); break;
-      case ITNBP_F32: e = launch_impl<float, float, float>(net, st, psi, msg_in, msg_out, stats, normalize); break;
-      default: e = launch_impl<bf16_t, float, float>(net, st, psi, msg_in, msg_out, stats, normalize); break;
+  hipError_t e = hipSuccess;
+  // the big sites (the longest workgroups) first, so that the LDS-resident
+  // sites fill in behind them
+  if (!st->big.empty()) {
+    if (acc_f64) {
+      switch (psi_dtype) {
+        case ITNBP_F64: e = launch_big_sites<double, double, double>(net, st, psi, msg_in, msg_out, stats, normalize); break;
+        case ITNBP_F32: e = launch_big_sites<float, double, double>(net, st, psi, msg_in, msg_out, stats, normalize); break;
+        default: e = launch_big_sites<bf16_t, double, double>(net, st, psi, msg_in, msg_out, stats, normalize); break;
+      }
+    } else {
+      switch (psi_dtype) {
+        case ITNBP_F64: e = launch_big_sites<double, float, float>(net, st, psi, msg_in, msg_out, stats, normalize); break;
+        case ITNBP_F32: e = launch_big_sites<float, float, float>(net, st, psi, msg_in, msg_out, stats, normalize); break;
+        default: e = launch_big_sites<bf16_t, float, float>(net, st, psi, msg_in, msg_out, stats, normalize); break;
+      }
     }
   }
+  if (e == hipSuccess && !st->tasks.empty())
+    e = launch_small(net, st, acc_f64, psi, psi_dtype, msg_in, msg_out, stats, normalize, use_queue(st), ctx->stream);
   prof_add(ctx, "vertex_eig", e0, prof_mark(ctx));
   ITNBP_HIPCHK(ctx, e);
   ++st->sweeps;
