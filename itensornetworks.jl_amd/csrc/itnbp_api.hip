@@ -15,6 +15,7 @@
 #include <complex>
 #include <cstdio>
 #include <cstring>
+#include <numeric>
 #include <exception>
 #include <new>
 #include <string>
@@ -292,10 +293,6 @@ int run_tasks(itnbp_net* net, const std::vector<OcTask>& tasks, int acc_f64, con
 // ---------------------------------------------------------------------------
 namespace {
 
-std::vector<std::pair<int, int>> sequential_runs(const itnbp_net* net, const std::vector<int>& seq) {
-  return itnbp_graph::sequential_runs(topo_of(net), seq);
-}
-
 struct Phase {
   int acc_f64;
   const void* psi;
@@ -318,11 +315,16 @@ int sweep_phase(itnbp_net* net, const std::vector<int>& seq, const itnbp_update_
   double* d_red = (double*)net->red.p;
   const size_t eb = ph.acc_f64 ? 8 : 4;
   const bool partial = (o->schedule == ITNBP_SCHED_PARALLEL) && n != 2 * net->ne;
+  // launches: all messages, or the levels of a sequential sweep (a default sweep
+  // of a 9x7 grid has 28 levels where its consecutive independent messages make
+  // 191 launches: the branches of a spanning tree do not wait for each other)
   std::vector<std::pair<int, int>> runs;
+  std::vector<int> order(n);
   if (o->schedule == ITNBP_SCHED_PARALLEL) {
     runs.push_back({0, n});
+    std::iota(order.begin(), order.end(), 0);
   } else {
-    runs = sequential_runs(net, seq);
+    itnbp_graph::sequential_levels(topo_of(net), seq, order, runs);
   }
   // the specialised pipeline produces the messages of its bulk vertices; the
   // generic plan everything else
@@ -348,8 +350,10 @@ int sweep_phase(itnbp_net* net, const std::vector<int>& seq, const itnbp_update_
   for (auto& r : runs) {
     std::vector<OcTask> rt;
     rt.reserve(r.second - r.first);
-    for (int i = r.first; i < r.second; ++i)
+    for (int k = r.first; k < r.second; ++k) {
+      const int i = order[k];
       if (!handled[i]) rt.push_back(message_task(net, seq[i], i, true, o->normalize));
+    }
     RETCHK(plan_tasks(net, rt, ph.acc_f64, plan));
     run_groups.push_back(plan.groups.size());
   }

@@ -186,6 +186,36 @@ std::vector<std::pair<int, int>> sequential_runs(const Topo& t, const std::vecto
   return runs;
 }
 
+void sequential_levels(const Topo& t, const std::vector<int>& seq, std::vector<int>& order,
+                       std::vector<std::pair<int, int>>& bounds) {
+  const size_t n = seq.size();
+  // levels of the last update and of the last read of every message so far
+  std::vector<int> wrote(2 * (size_t)t.ne, -1), read(2 * (size_t)t.ne, -1), level(n);
+  int depth = 0;
+  for (size_t i = 0; i < n; ++i) {
+    const int m = seq[i], u = msg_src(t, m), v = msg_dst(t, m);
+    int l = std::max(wrote[m], read[m]) + 1;
+    for (int a = t.inc_ptr[u]; a < t.inc_ptr[u + 1]; ++a) {
+      const int in = msg_id_into(t, t.inc_edge[a], u);
+      if (msg_src(t, in) != v) l = std::max(l, wrote[in] + 1);
+    }
+    for (int a = t.inc_ptr[u]; a < t.inc_ptr[u + 1]; ++a) {
+      const int in = msg_id_into(t, t.inc_edge[a], u);
+      if (msg_src(t, in) != v) read[in] = std::max(read[in], l);
+    }
+    wrote[m] = l;
+    level[i] = l;
+    depth = std::max(depth, l + 1);
+  }
+  std::vector<int> at(depth + 1, 0);
+  for (int l : level) ++at[l + 1];
+  for (int l = 0; l < depth; ++l) at[l + 1] += at[l];
+  bounds.clear();
+  for (int l = 0; l < depth; ++l) bounds.push_back({at[l], at[l + 1]});
+  order.assign(n, 0);
+  for (size_t i = 0; i < n; ++i) order[at[level[i]]++] = (int)i;
+}
+
 int check_sequence(const Topo& t, const std::vector<char>& is_set, const std::vector<int>& seq, bool sequential,
                    bool need_old, std::string& err) {
   std::vector<char> set(is_set);

@@ -66,6 +66,16 @@ void default_sequence(const Topo& t, bool parallel, std::vector<int>& seq);
 // give the result of the one-by-one sequential update.
 std::vector<std::pair<int, int>> sequential_runs(const Topo& t, const std::vector<int>& seq);
 
+// Launch levels of a sequential sweep: positions of seq grouped so that no
+// message of a level reads another one of it (or repeats it), every message
+// comes in a later level than the earlier messages of seq that it reads, that
+// read it or that it repeats, and in the earliest such level.  Updating level
+// after level gives the result of the one-by-one update exactly: positions that
+// trade places do not depend on each other.  order lists the positions level
+// by level; level i is order[bounds[i].first .. bounds[i].second).
+void sequential_levels(const Topo& t, const std::vector<int>& seq, std::vector<int>& order,
+                       std::vector<std::pair<int, int>>& bounds);
+
 // The errors update(bpc) raises for a sequence: an id out of range
 // (ITNBP_ERR_ARG), an incoming message read before it was set, or, with
 // need_old, a message without a previous value (ITNBP_ERR_STATE).  is_set has

@@ -19,6 +19,7 @@
 #include <algorithm>
 #include <cmath>
 #include <memory>
+#include <numeric>
 #include <string>
 #include <vector>
 
@@ -354,8 +355,10 @@ int lnet_update(itnbp_lnet* L, const itnbp_update_opts* o, itnbp_update_result* 
     return itnbp_fail(ctx, rc, why);
   const size_t nseq = seq.size();
   ITNBP_RETCHK(ensure_buf(ctx, L->stats, nseq * sizeof(MsgStat)));
-  const auto runs = seqsched ? itnbp_graph::sequential_runs(tp, seq)
-                             : std::vector<std::pair<int, int>>{{0, (int)nseq}};
+  std::vector<std::pair<int, int>> runs{{0, (int)nseq}};
+  std::vector<int> order(nseq);
+  std::iota(order.begin(), order.end(), 0);
+  if (seqsched) itnbp_graph::sequential_levels(tp, seq, order, runs);
   std::vector<MsgStat> hs(nseq);
   itnbp_update_result r{};
   ITNBP_HIPCHK(ctx, hipEventRecord(ctx->ev0, ctx->stream));
@@ -366,13 +369,13 @@ int lnet_update(itnbp_lnet* L, const itnbp_update_opts* o, itnbp_update_result* 
       ITNBP_HIPCHK(ctx, hipMemcpyAsync(nxt, cur, L->msg_total * L->es, hipMemcpyDeviceToDevice, ctx->stream));
     for (const auto& run : runs) {
       std::vector<LTask> tasks;
-      for (int i = run.first; i < run.second; ++i) {
-        const int m = seq[i];
+      for (int k = run.first; k < run.second; ++k) {
+        const int i = order[k], m = seq[i];
         tasks.push_back(message_task_l(L, m, i, L->msg_set[m] != 0, o->normalize));
       }
       ITNBP_RETCHK(run_layer_tasks(L, tasks, cur, nxt, (MsgStat*)L->stats.p));
       if (seqsched)
-        for (int i = run.first; i < run.second; ++i) L->msg_set[seq[i]] = 1;
+        for (int k = run.first; k < run.second; ++k) L->msg_set[seq[order[k]]] = 1;
     }
     if (!seqsched) {
       L->cur = 1 - L->cur;
