@@ -145,19 +145,19 @@ int plan_tasks(itnbp_net* net, const std::vector<OcTask>& tasks, int acc_f64, Ta
   const size_t lds_cls[3] = {32 * 1024, 64 * 1024, 160 * 1024};
   // message updates with every bond <= 16 and the site tensor in LDS: the site
   // kernel, in launches of similar LDS need
-  std::vector<SiteTask> site[SITE_CLASSES];
+  std::vector<SiteTask> site;
   const bool use_site = site_enabled();
   for (const auto& t : tasks) {
     const VDesc& V = net->vdesc[t.v];
     if (use_site && !t.s_open && t.j > 0 && t.absorb_mask == (((1 << (V.k + 1)) - 2) & ~(1 << t.j)) &&
         site_fits(V, eb)) {
       const int o = (t.j < V.k || V.k == 1) ? 0 : 1;  // the open bond is p (with q = p + 1) or, for the last bond, q
-      SiteTask st = site_task(V, t.j - o, 1 << o);
+      SiteTask st = site_task(V, t.j - o, 1 << o, eb);
       st.out[o] = t.out_off;
       st.old[o] = t.old_off;
       st.slot[o] = t.slot;
       st.normalize[o] = t.normalize;
-      site[site_class(V.D, eb)].push_back(st);
+      site.push_back(st);
       continue;
     }
     const size_t b = oc_small_lds_bytes(net->vdesc[t.v], t, eb);
@@ -168,19 +168,17 @@ int plan_tasks(itnbp_net* net, const std::vector<OcTask>& tasks, int acc_f64, Ta
     const int c = b <= lds_cls[0] ? 0 : b <= lds_cls[1] ? 1 : 2;
     small[c].push_back(t);
   }
-  for (const auto& sc : site) {
-    if (sc.empty()) continue;
+  for (const SiteLaunch& L : site_group(site, eb, ctx->num_cu)) {
     LaunchGroup lg{};
     lg.kind = 2;
-    lg.begin = plan.sites.size();
-    lg.count = sc.size();
-    long long dmax = 1;
-    for (const auto& t : sc) dmax = std::max<long long>(dmax, t.D);
-    lg.threads = site_threads(dmax);
-    lg.lds = site_lds_bytes(dmax, eb);
-    plan.sites.insert(plan.sites.end(), sc.begin(), sc.end());
+    lg.begin = plan.sites.size() + L.begin;
+    lg.count = L.count;
+    lg.threads = L.threads;
+    lg.lds = L.lds;
+    lg.staged = L.staged;
     plan.groups.push_back(lg);
   }
+  plan.sites.insert(plan.sites.end(), site.begin(), site.end());
   for (int c = 0; c < 3; ++c) {
     if (small[c].empty()) continue;
     LaunchGroup lg{};
@@ -263,7 +261,7 @@ int launch_plan(itnbp_net* net, const TaskPlan& plan, size_t g0, size_t g1, cons
     } else if (lg.kind == 2) {
       const SiteTask* sites = (const SiteTask*)((const char*)d_tasks + plan_site_offset(plan));
       HIPCHK(ctx, launch_site(psi_dtype, plan.acc_f64, sites + lg.begin, (int)lg.count, psi, msg_in, out, d_stats, 0, 1,
-                              lg.threads, lg.lds, nullptr, nullptr, 0, s));
+                              lg.threads, lg.lds, lg.staged, nullptr, nullptr, 0, s));
       if (main) prof_add(ctx, "site", e0, prof_mark(ctx));
     } else {
       HIPCHK(ctx, launch_oc_large(psi_dtype, plan.acc_f64, net->d_vdesc, d_tasks + lg.begin,

@@ -102,6 +102,7 @@ struct LaunchGroup {
   size_t begin, count;
   size_t lds;        // small, site: dynamic LDS bytes
   int threads;       // site: workgroup size
+  bool staged;       // site: psi staged in LDS
   long long maxD;    // large: scratch stride
   int nsplit;        // large: split-K factor
   long long part_stride;

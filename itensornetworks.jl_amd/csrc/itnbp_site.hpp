@@ -22,11 +22,14 @@ struct SiteTask {
   long long old[2];      // previous messages out (-1: none to compare with)
   int slot[2];           // statistics slots (-1: none)
   int normalize[2];
-  FastDiv fsp;           // stride of bond p
+  FastDiv fsp;           // stride sp of bond p in the site tensor
+  int sps, Ds;           // its padded stride in LDS, and the elements of the padded tensor
   struct Mode {
     long long msg;
-    int n, pad;
-    FastDiv fst;         // stride of the bond
+    int n, nfib, pst;    // dimension, fibres, padded stride
+    int above;           // the bond lies above p
+    FastDiv fst;         // stride in the site tensor
+    FastDiv fg;          // below p: sp / (stride n)
   } mode[ITNBP_MAXK - 1];
 };
 
@@ -42,21 +45,31 @@ struct TaskPlan {
 bool site_fits(const VDesc& V, int elem_bytes);
 // task of vertex V for the messages on bond axis p and p + 1 (1-based; want as
 // above); out, old, slot and normalize are left to the caller
-SiteTask site_task(const VDesc& V, int p, int want);
+SiteTask site_task(const VDesc& V, int p, int want, int elem_bytes);
 // ITNBP_DISABLE_VERTEX=1 keeps message updates on the generic kernels
 bool site_enabled();
-// launches group tasks of similar LDS need: below 2048 elements (256 threads),
-// then site tensors of at most 40, 80 and 160 KB (4, 2 and 1 workgroups per CU)
+// Launches of a set of tasks.  While the tasks whose two tensors (P and psi) fit
+// in LDS are no more than the CUs, each has a CU to itself: one launch of them,
+// with psi staged in LDS (shortest task: no global load after the first).  More
+// tasks than that are bound by throughput: psi is read from global memory a second
+// time, so that more workgroups share a CU, in launches of similar LDS need (below
+// 2048 elements 256 threads; P of at most 40, 80 and 160 KB 512 threads).  16x16
+// chi = 8 (512 tasks) 46 us a sweep staged, 39 us unstaged; heavy-hex 9x7 FP32 (188
+// tasks) 15 us staged, 31 us unstaged.
 constexpr int SITE_CLASSES = 4;
-int site_class(long long D, int elem_bytes);
-// threads and dynamic LDS of a launch whose largest task has D elements
-int site_threads(long long D);
-size_t site_lds_bytes(long long D, int elem_bytes);
+struct SiteLaunch {
+  size_t begin, count;
+  int threads;
+  size_t lds;
+  bool staged;
+};
+// reorders the tasks launch by launch, the costliest first
+std::vector<SiteLaunch> site_group(std::vector<SiteTask>& tasks, int elem_bytes, int num_cu);
 // queue != null: a persistent grid of `grid` workgroups takes the n tasks in
 // order from the counter at queue (cleared by the launch); active: skip the
 // tasks of finished instances
 hipError_t launch_site(int psi_dtype, int acc_f64, const SiteTask* d_tasks, int n, const void* psi, const void* msg_in,
-                       void* msg_out, MsgStat* stats, int sym, int normalize, int threads, size_t lds, const int* active, int* queue,
-                       int grid, hipStream_t s);
+                       void* msg_out, MsgStat* stats, int sym, int normalize, int threads, size_t lds, bool staged, const int* active,
+                       int* queue, int grid, hipStream_t s);
 // resident workgroups of the persistent form on the current device
-hipError_t site_queue_occupancy(int psi_dtype, int acc_f64, int threads, size_t lds, int* per_cu);
+hipError_t site_queue_occupancy(int psi_dtype, int acc_f64, int threads, size_t lds, bool staged, int* per_cu);

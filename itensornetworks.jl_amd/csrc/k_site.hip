@@ -21,14 +21,15 @@
 // The eigenbasis form this replaces (rotate every bond into its message's
 // eigenvectors, weighted Grams) needs a Jacobi eigendecomposition per message
 // first, a serial chain of some 30 us per workgroup, and ran one workgroup per
-// site.  Bound: latency of the LDS and MFMA chains; blocks of bonds <= 8 leave half
-// of each 16 x 16 tile idle in the mode products and the absorptions.
-// One Jacobi sweep, eigenbasis form -> this: 16x16 PEPS chi = 8 FP64 103 -> 42 us,
-// heavy-hex 9x7 chi 5..16 FP32 189 -> 31 us, 8x8 chi = 4 FP64 40 -> 9 us (two launches
-// where the sites fall into two classes).  A sequential run of a 9x7 chi 3..8 PEPS
-// takes 10 us a launch, 21 us on the generic LDS kernel.
+// site.  Bound: a fixed chain of about 6 us (launch, task, inputs, stores), then LDS
+// and MFMA latency; blocks of bonds <= 8 leave half of each 16 x 16 tile idle in the
+// mode products and the absorptions.
+// One Jacobi sweep, eigenbasis form -> this: 16x16 PEPS chi = 8 FP64 103 -> 39 us
+// (two launches), heavy-hex 9x7 chi 5..16 FP32 189 -> 15 us, 8x8 chi = 4 FP64 40 -> 9
+// us.  A level of a sequential sweep of a 9x7 chi 3..8 PEPS takes 13 us.
 #include <algorithm>
 #include <cstdlib>
+#include <vector>
 
 #include "itnbp_site.hpp"
 
@@ -61,129 +62,201 @@ __device__ inline double site_wave_sum(double v) {
   return v;
 }
 
-// P[.. b' ..] = sum_b src[.. b ..] K[b][b'] on one bond (n <= 16), 16 fibres per
-// MFMA column set and two sets in flight per wave
-template <typename TA, typename TSrc, typename TM>
-__device__ inline void site_mode(const SiteTask::Mode& md, int D, const TSrc* src, TA* P, const TM* msg_in) {
-  const int l = threadIdx.x & 63, li = l & 15, lk = l >> 4, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  const int n = md.n, st = (int)md.fst.d, nk = (n + 3) >> 2;
-  const TM* K = msg_in + md.msg;
-  TA a[4];
-  const int r = Mf<TA>::a_row(li);
+// A operand of a product with the message at msg (n x n, column-major):
+// A[b'][b] = M[b][b'] for output row b' = a_row(lane) and K-steps b = 4 q + l / 16
+template <typename TA, typename TM>
+__device__ inline void site_msg(const TM* msg_in, long long msg, int n, TA (&a)[4]) {
+  const int l = threadIdx.x & 63, lk = l >> 4, r = Mf<TA>::a_row(l & 15);
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const int b = 4 * q + lk;
-    a[q] = (b < n && r < n) ? (TA)K[b + n * r] : (TA)0;
+    a[q] = (b < n && r < n) ? (msg < 0 ? (TA)1 : (TA)msg_in[msg + b + n * r]) : (TA)0;
   }
-  const int nfib = D / n, ngrp = (nfib + 15) >> 4;
+}
+
+// LDS layout of a site tensor: the stride of bond p padded from sp to sps, so that
+// element a sits at a + (sps - sp) (a / sp).  Blocks and fibres along outer bonds
+// otherwise step by powers of two of 32 and more elements (chi = 4, 8, 16), which
+// puts the lanes of a load on one or two banks (site_task picks the padding).
+
+// P[.. b' ..] = sum_b src[.. b ..] M[b][b'] on one bond (n <= 16), 16 fibres per
+// MFMA column set and two sets in flight per wave; src in LDS, or psi itself.
+// FULL: no remainder in the bond or the fibres, so no lane is masked.
+template <typename TA, bool LDS, bool FULL, typename TSrc>
+__device__ inline void site_mode_body(const SiteTask* __restrict__ tk, const SiteTask::Mode& md, const TA (&a)[4],
+                                      const TSrc* src, TA* P) {
+  const int l = threadIdx.x & 63, li = l & 15, lk = l >> 4, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int n = md.n, st = (int)md.fst.d, pst = md.pst, nk = (n + 3) >> 2, above = md.above;
+  const int nfib = md.nfib, ngrp = (nfib + 15) >> 4, pad = tk->sps - (int)tk->fsp.d;
+  int off[4], goff[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int b = 4 * q + lk < n ? 4 * q + lk : 0;
+    off[q] = pst * b;
+    goff[q] = st * b;
+  }
   for (int g0 = wv; g0 < ngrp; g0 += 2 * nw) {
     TA x[2][4];
     int base[2];
     bool in[2];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      const int f = 16 * (g0 + u * nw) + li;
-      in[u] = f < nfib;
-      base[u] = in[u] ? f + (int)md.fst.div(f) * st * (n - 1) : 0;
+      const int f0 = 16 * (g0 + u * nw) + li;
+      in[u] = FULL ? g0 + u * nw < ngrp : f0 < nfib;
+      const int f = in[u] ? f0 : 0;
+      const int hi = (int)md.fst.div(f), lo = f - hi * st;
+      base[u] = above ? lo + pad * (int)tk->fsp.div(lo) + pst * n * hi : lo + st * n * hi + pad * (int)md.fg.div(hi);
+      const int gb = lo + st * n * hi;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int b = 4 * q + lk;
-        x[u][q] = (q < nk && in[u] && b < n) ? load_as<TA>(src, base[u] + st * b) : (TA)0;
-      }
+      for (int q = 0; q < 4; ++q)
+        if (q < nk) {
+          const TA t = load_as<TA>(src, LDS ? base[u] + off[q] : gb + goff[q]);
+          x[u][q] = FULL || (in[u] && 4 * q + lk < n) ? t : (TA)0;
+        }
     }
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
+      if (FULL && u == 1 && !in[1]) continue;
       typename Mf<TA>::V acc = {0, 0, 0, 0};
 #pragma unroll
       for (int q = 0; q < 4; ++q)
         if (q < nk) acc = Mf<TA>::mma(a[q], x[u][q], acc);
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int b2 = 4 * v + lk;
-        if (v < nk && in[u] && b2 < n) P[base[u] + st * b2] = acc[v];
-      }
+      for (int v = 0; v < 4; ++v)
+        if (v < nk && (FULL || (in[u] && 4 * v + lk < n))) P[base[u] + off[v]] = acc[v];
     }
   }
 }
 
-template <typename TS, typename TA, typename TM>
+template <typename TA, bool LDS, typename TSrc>
+__device__ inline void site_mode(const SiteTask* __restrict__ tk, int m, const TA (&a)[4], const TSrc* src, TA* P) {
+  const SiteTask::Mode& md = tk->mode[m];
+  if (((md.n & 3) | (md.nfib & 15)) == 0)
+    site_mode_body<TA, LDS, true>(tk, md, a, src, P);
+  else
+    site_mode_body<TA, LDS, false>(tk, md, a, src, P);
+}
+
+// The blocks of a pair.  Lane column li is index li % 2^lsh of block li / 2^lsh of
+// the tile.  FULL: tiles without remainder.  ld(at, gl): psi at LDS position at /
+// element gl.
+template <bool FULL, typename TA, typename F>
+__device__ inline void site_blocks(const SiteTask* __restrict__ tk, const TA* P, const TA (&mp)[4], const TA (&mq)[4],
+                                   F ld, f64x4& tp, f64x4& tq) {
+  const int l = threadIdx.x & 63, li = l & 15, lk = l >> 4, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int np = tk->np, nq = tk->nq, want = tk->want, lsh = tk->lsh, nb = tk->nb;
+  const int sp = (int)tk->fsp.d, sq = sp * np, sps = tk->sps, sqs = sps * np;
+  const int pk = 16 >> lsh, idx = li & ((1 << lsh) - 1), blk = li >> lsh;
+  const int npk = (nb + pk - 1) >> (4 - lsh);
+  // one output: x = its bond as the lane column, b = the other bond as K-row
+  auto output = [&](int base, int gb, bool in, int nx, int nbb, int sx, int sb, int gx, int gbb, const TA(&m)[4],
+                    f64x4& acc) {
+    const int kb = (nbb + 3) >> 2;
+    TA x[4], y[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (q < kb) {
+        const int b = 4 * q + lk;
+        const bool ok = FULL || (in && idx < nx && b < nbb);
+        const int at = base + (ok ? sx * idx + sb * b : 0);
+        x[q] = P[at];
+        y[q] = ld(at, gb + (ok ? gx * idx + gbb * b : 0));
+        if (!ok) x[q] = y[q] = (TA)0;
+      }
+    typename Mf<TA>::V d = {0, 0, 0, 0};
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (q < kb) d = Mf<TA>::mma(m[q], x[q], d);
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+      if (v < kb) acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)d[v], (double)y[v], acc, 0, 0, 0);
+  };
+  for (int t = wv; t < npk; t += nw) {
+    const int r0 = t * pk + blk;
+    const bool in = FULL || r0 < nb;
+    const int r = in ? r0 : 0;
+    const int hi = (int)tk->fsp.div(r), lo = r - hi * sp;
+    const int base = lo + hi * (sqs * nq), gb = lo + hi * (sq * nq);
+    if (want & 1) output(base, gb, in, np, nq, sps, sqs, sp, sq, mq, tp);
+    if (want & 2) output(base, gb, in, nq, np, sqs, sps, sq, sp, mp, tq);
+  }
+}
+
+// STAGE: psi is staged in LDS as well (behind P)
+template <bool STAGE, typename TS, typename TA, typename TM>
 __device__ __forceinline__ void site_run(const SiteTask* __restrict__ tk, const TS* __restrict__ psi_all,
                                          const TM* msg_in, TM* msg_out, MsgStat* __restrict__ stats, int sym,
                                          int normalize, unsigned char* smem) {
-  TA* P = reinterpret_cast<TA*>(smem);
-  const int tid = threadIdx.x, l = tid & 63, li = l & 15, lk = l >> 4, wv = tid >> 6, nw = blockDim.x >> 6;
-  const int D = tk->D;
-  const TS* psi = psi_all + tk->psi_off;
-  // 1. mode products
-  if (tk->nmode == 0)
-    for (int i = tid; i < D; i += blockDim.x) P[i] = load_as<TA>(psi, i);
-  for (int m = 0; m < tk->nmode; ++m) {
-    if (m == 0)
-      site_mode<TA>(tk->mode[0], D, psi, P, msg_in);
-    else
-      site_mode<TA>(tk->mode[m], D, P, P, msg_in);
-    if (m + 1 < tk->nmode) __syncthreads();
-  }
-  // 2. blocks: lane column li is index li % 2^lsh of block li / 2^lsh of the tile
-  const int np = tk->np, nq = tk->nq, want = tk->want, lsh = tk->lsh, nb = tk->nb;
-  const int sp = (int)tk->fsp.d, sq = sp * np;
-  const int pk = 16 >> lsh, idx = li & ((1 << lsh) - 1), blk = li >> lsh;
-  const int kp = (np + 3) >> 2, kq = (nq + 3) >> 2;
-  TA mq[4], mp[4];
+  // the task's cache lines, all at once: its fields are read one by one below,
+  // and each first touch of a line would be a round trip of its own
   {
-    const int r = Mf<TA>::a_row(li);
+    const int* w = reinterpret_cast<const int*>(tk);
+    int touch = 0;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int b = 4 * q + lk;
-      mq[q] = (b < nq && r < nq) ? (tk->mq < 0 ? (TA)1 : (TA)msg_in[tk->mq + b + nq * r]) : (TA)0;
-      mp[q] = (b < np && r < np) ? (TA)msg_in[tk->mp + b + np * r] : (TA)0;
-    }
+    for (int i = 0; i < (int)sizeof(SiteTask) / 4; i += 16) touch += w[i];
+    asm volatile("" ::"s"(touch));
   }
-  __syncthreads();
+  const int tid = threadIdx.x, l = tid & 63, li = l & 15, lk = l >> 4, wv = tid >> 6, nw = blockDim.x >> 6;
+  const int D = tk->D, nmode = tk->nmode, want = tk->want;
+  const int np = tk->np, nq = tk->nq;
+  TA* P = reinterpret_cast<TA*>(smem);
+  TA* Y = P + tk->Ds;
+  const int sp = (int)tk->fsp.d, pad = tk->sps - sp;
+  const TS* psi = psi_all + tk->psi_off;
+  // everything the task reads from global memory is asked for at once: psi, the
+  // messages in, and (waves 0 and 1) the previous messages out
+  TA a[4], mp[4], mq[4];
+  if (nmode > 0) site_msg(msg_in, tk->mode[0].msg, tk->mode[0].n, a);
+  site_msg(msg_in, tk->mp, np, mp);
+  site_msg(msg_in, tk->mq, nq, mq);
+  double ov[4] = {0, 0, 0, 0};
+  const int fin = wv < 2 && ((want >> wv) & 1);  // this wave finishes output wv
+  const long long old = fin ? tk->old[wv] : -1;
+  const int no = wv == 0 ? np : nq;
+  if (old >= 0)
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if (l + 64 * c < no * no) ov[c] = (double)msg_in[old + l + 64 * c];
+  if constexpr (STAGE) {
+#pragma unroll 4
+    for (int i = tid; i < D; i += blockDim.x) Y[i + pad * (int)tk->fsp.div(i)] = load_as<TA>(psi, i);
+    __syncthreads();
+  }
+  // 1. mode products
+  if (nmode == 0) {
+    if constexpr (STAGE)
+      P = Y;
+    else
+      for (int i = tid; i < D; i += blockDim.x) P[i + pad * (int)tk->fsp.div(i)] = load_as<TA>(psi, i);
+  }
+  for (int m = 0; m < nmode; ++m) {
+    TA an[4] = {0, 0, 0, 0};
+    if (m + 1 < nmode) site_msg(msg_in, tk->mode[m + 1].msg, tk->mode[m + 1].n, an);
+    if (m > 0)
+      site_mode<TA, true>(tk, m, a, P, P);
+    else if constexpr (STAGE)
+      site_mode<TA, true>(tk, 0, a, Y, P);
+    else
+      site_mode<TA, false>(tk, 0, a, psi, P);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) a[q] = an[q];
+  }
+  if (!STAGE && nmode == 0) __syncthreads();
+  // 2. blocks
+  auto ld = [&](int at, int gl) -> TA {
+    if constexpr (STAGE)
+      return Y[at];
+    else
+      return load_as<TA>(psi, gl);
+  };
   f64x4 tp = {0, 0, 0, 0}, tq = {0, 0, 0, 0};
-  const int npk = (nb + pk - 1) / pk;
-  for (int t = wv; t < npk; t += nw) {
-    const int r = t * pk + blk;
-    const bool in = r < nb;
-    const int base = in ? r + (int)tk->fsp.div(r) * sp * (np * nq - 1) : 0;
-    if (want & 1) {
-      TA x[4], y[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int b = 4 * q + lk;
-        const bool ok = q < kq && in && idx < np && b < nq;
-        const int at = base + sp * idx + sq * b;
-        x[q] = ok ? P[at] : (TA)0;
-        y[q] = ok ? load_as<TA>(psi, at) : (TA)0;
-      }
-      typename Mf<TA>::V d = {0, 0, 0, 0};
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        if (q < kq) d = Mf<TA>::mma(mq[q], x[q], d);
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-        if (v < kq) tp = __builtin_amdgcn_mfma_f64_16x16x4f64((double)d[v], (double)y[v], tp, 0, 0, 0);
-    }
-    if (want & 2) {
-      TA x[4], y[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int b = 4 * q + lk;
-        const bool ok = q < kp && in && idx < nq && b < np;
-        const int at = base + sp * b + sq * idx;
-        x[q] = ok ? P[at] : (TA)0;
-        y[q] = ok ? load_as<TA>(psi, at) : (TA)0;
-      }
-      typename Mf<TA>::V d = {0, 0, 0, 0};
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        if (q < kp) d = Mf<TA>::mma(mp[q], x[q], d);
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-        if (v < kp) tq = __builtin_amdgcn_mfma_f64_16x16x4f64((double)d[v], (double)y[v], tq, 0, 0, 0);
-    }
-  }
-  __syncthreads();  // P is read; its place takes the partial T
+  const int lsh = tk->lsh, pk = 16 >> lsh;
+  if (np == (1 << lsh) && nq == np && np >= 4 && (tk->nb & (pk - 1)) == 0)
+    site_blocks<true, TA>(tk, P, mp, mq, ld, tp, tq);
+  else
+    site_blocks<false, TA>(tk, P, mp, mq, ld, tp, tq);
+  __syncthreads();  // P and psi are read; their place takes the partial T
   // 3. red[wave][output][row * 16 + col]
   double* red = reinterpret_cast<double*>(smem);
 #pragma unroll
@@ -198,10 +271,10 @@ __device__ __forceinline__ void site_run(const SiteTask* __restrict__ tk, const 
     red[e] = s;
   }
   __syncthreads();
-  if (wv < 2 && ((want >> wv) & 1)) {
-    const int n = wv == 0 ? np : nq, nn = n * n;
+  if (fin) {
+    const int n = no, nn = n * n;
     const double* T = red + wv * 256;
-    const long long off = tk->out[wv], old = tk->old[wv];
+    const long long off = tk->out[wv];
     double tv[4], n2 = 0;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
@@ -230,10 +303,9 @@ __device__ __forceinline__ void site_run(const SiteTask* __restrict__ tk, const 
         const double nv = tv[c] * sc;
         if (!isfinite(nv)) bad = 1;
         if (old >= 0) {
-          const double ov = (double)msg_in[old + e];
-          dot += ov * nv;
-          o2 += ov * ov;
-          d2 += (nv - ov) * (nv - ov);
+          dot += ov[c] * nv;
+          o2 += ov[c] * ov[c];
+          d2 += (nv - ov[c]) * (nv - ov[c]);
         }
         msg_out[off + e] = (TM)nv;
       }
@@ -255,23 +327,23 @@ __device__ __forceinline__ void site_run(const SiteTask* __restrict__ tk, const 
   }
 }
 
-template <typename TS, typename TA, typename TM>
-__global__ __launch_bounds__(512) void k_site(const SiteTask* __restrict__ tasks, const TS* __restrict__ psi,
+template <bool STAGE, typename TS, typename TA, typename TM>
+__global__ __launch_bounds__(STAGE ? 1024 : 512) void k_site(const SiteTask* __restrict__ tasks, const TS* __restrict__ psi,
                                               const TM* msg_in, TM* msg_out, MsgStat* __restrict__ stats, int sym,
                                               int normalize, const int* __restrict__ active) {
   extern __shared__ __align__(16) unsigned char smem[];
   const SiteTask* tk = tasks + blockIdx.x;
   // batched update: a finished instance's messages were carried over already
   if (active && !active[tk->inst]) return;
-  site_run<TS, TA, TM>(tk, psi, msg_in, msg_out, stats, sym, normalize, smem);
+  site_run<STAGE, TS, TA, TM>(tk, psi, msg_in, msg_out, stats, sym, normalize, smem);
 }
 
 // Persistent form: a grid of resident workgroups takes the (cost-sorted) tasks
 // in order from a device counter that k_site_reset clears before the launch;
 // every workgroup leaves once the counter has passed ntasks, so the grid
 // drains without any wait on another workgroup.
-template <typename TS, typename TA, typename TM>
-__global__ __launch_bounds__(512) void k_site_queue(const SiteTask* __restrict__ tasks, int ntasks,
+template <bool STAGE, typename TS, typename TA, typename TM>
+__global__ __launch_bounds__(STAGE ? 1024 : 512) void k_site_queue(const SiteTask* __restrict__ tasks, int ntasks,
                                                     int* __restrict__ queue, const TS* __restrict__ psi,
                                                     const TM* msg_in, TM* msg_out, MsgStat* __restrict__ stats,
                                                     int sym, int normalize, const int* __restrict__ active) {
@@ -284,7 +356,7 @@ __global__ __launch_bounds__(512) void k_site_queue(const SiteTask* __restrict__
     __syncthreads();  // every thread has read next before thread 0 takes the following task
     if (t >= ntasks) return;
     if (!(active && !active[tasks[t].inst])) 
-      site_run<TS, TA, TM>(tasks + t, psi, msg_in, msg_out, stats, sym, normalize, smem);
+      site_run<STAGE, TS, TA, TM>(tasks + t, psi, msg_in, msg_out, stats, sym, normalize, smem);
     __syncthreads();  // the task's last LDS reads come before the next task's writes
   }
 }
@@ -295,19 +367,19 @@ __global__ void k_site_reset(int* __restrict__ queue) {
   if (threadIdx.x == 0) queue[0] = 0;
 }
 
-template <typename TS, typename TA, typename TM>
+template <bool STAGE, typename TS, typename TA, typename TM>
 hipError_t launch_impl(const SiteTask* d_tasks, int n, const void* psi, const void* msg_in, void* msg_out,
                        MsgStat* stats, int sym, int normalize, int threads, size_t lds, const int* active, int* queue, int grid,
                        hipStream_t s) {
   if (!queue) {
-    auto kern = k_site<TS, TA, TM>;
+    auto kern = k_site<STAGE, TS, TA, TM>;
     hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kern, dim3((unsigned)n), dim3((unsigned)threads), lds, s, d_tasks, (const TS*)psi,
                        (const TM*)msg_in, (TM*)msg_out, stats, sym, normalize, active);
     return hipGetLastError();
   }
-  auto kern = k_site_queue<TS, TA, TM>;
+  auto kern = k_site_queue<STAGE, TS, TA, TM>;
   hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k_site_reset, dim3(1), dim3(64), 0, s, queue);
@@ -316,9 +388,9 @@ hipError_t launch_impl(const SiteTask* d_tasks, int n, const void* psi, const vo
   return hipGetLastError();
 }
 
-template <typename TS, typename TA, typename TM>
+template <bool STAGE, typename TS, typename TA, typename TM>
 hipError_t occ_impl(int threads, size_t lds, int* per_cu) {
-  auto kern = k_site_queue<TS, TA, TM>;
+  auto kern = k_site_queue<STAGE, TS, TA, TM>;
   hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
   return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, (const void*)kern, threads, lds);
@@ -331,26 +403,74 @@ bool site_enabled() {
   return !(e && e[0] == '1');
 }
 
+namespace {
+// LDS elements of one padded site tensor, by its elements alone (an upper bound:
+// site_task keeps the padding within it)
+long long site_pad(long long D) { return D + D / 8 + 32; }
+constexpr size_t SITE_LDS = 160 * 1024 - 256;  // less the static LDS of the persistent form
+}  // namespace
+
+bool site_stageable(long long D, int elem_bytes) { return (size_t)(2 * site_pad(D) * elem_bytes) <= SITE_LDS; }
+
 int site_class(long long D, int elem_bytes) {
-  const long long b = D * elem_bytes;
+  const size_t b = (size_t)site_pad(D) * elem_bytes;
   return D < 2048 ? 0 : b <= 40 * 1024 ? 1 : b <= 80 * 1024 ? 2 : 3;
 }
 
-int site_threads(long long D) { return D >= 2048 ? 512 : 256; }
+int site_threads(long long D, bool staged) { return D < 2048 ? 256 : staged && D >= 4096 ? 1024 : 512; }
 
-size_t site_lds_bytes(long long D, int elem_bytes) {
-  const size_t red = (size_t)(site_threads(D) / 64) * 512 * 8;
-  return std::max((size_t)D * elem_bytes, red);
+size_t site_lds_bytes(long long D, int elem_bytes, bool staged) {
+  const size_t red = (size_t)(site_threads(D, staged) / 64) * 512 * 8;
+  return std::max((size_t)site_pad(D) * elem_bytes * (staged ? 2 : 1), red);
 }
 
 bool site_fits(const VDesc& V, int elem_bytes) {
   if (V.k < 1 || V.k > ITNBP_MAXK) return false;
   for (int a = 1; a <= V.k; ++a)
     if (V.dims[a] > SITE_MAXCHI) return false;
-  return site_lds_bytes(V.D, elem_bytes) + 256 <= 160 * 1024;  // + the static LDS of the persistent form
+  return site_lds_bytes(V.D, elem_bytes, false) <= SITE_LDS;
 }
 
-SiteTask site_task(const VDesc& V, int p, int want) {
+namespace {
+// Padding of bond p's LDS stride sp: among paddings that grow the tensor by at
+// most an eighth, the smallest with the fewest LDS cycles for the two operand
+// loads of a block (lane column (block, index) x 4 K-rows), counted as the most
+// lanes on one bank of elem_bytes.
+int site_padding(int sp, int np, int nq, int lsh, int elem_bytes) {
+  struct Key {
+    int sp, np, nq, pad;
+  };
+  static thread_local std::vector<Key> known[2];
+  std::vector<Key>& seen = known[elem_bytes == 8];
+  for (const Key& k : seen)
+    if (k.sp == sp && k.np == np && k.nq == nq) return k.pad;
+  const int banks = 256 / elem_bytes, pk = 16 >> lsh;
+  int best = 0, best_cost = 1 << 30;
+  for (int pad = 0; pad <= sp / 8 && pad < banks; ++pad) {
+    const int s1 = sp + pad, s2 = s1 * np;
+    int cost = 0;
+    for (int o = 0; o < 2; ++o) {
+      int hit[64] = {0}, most = 0;
+      const int ni = o == 0 ? np : nq, nk = o == 0 ? nq : np, si = o == 0 ? s1 : s2, sk = o == 0 ? s2 : s1;
+      for (int blk = 0; blk < pk; ++blk)
+        for (int i = 0; i < ni; ++i)
+          for (int b = 0; b < std::min(4, nk); ++b) {
+            const int base = blk % sp + blk / sp * s2 * nq;
+            most = std::max(most, ++hit[(base + i * si + b * sk) % banks]);
+          }
+      cost += most;
+    }
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = pad;
+    }
+  }
+  if (seen.size() < 512) seen.push_back(Key{sp, np, nq, best});
+  return best;
+}
+}  // namespace
+
+SiteTask site_task(const VDesc& V, int p, int want, int elem_bytes) {
   SiteTask t{};
   t.D = V.D;
   t.psi_off = V.psi_off;
@@ -362,18 +482,26 @@ SiteTask site_task(const VDesc& V, int p, int want) {
   int lsh = 0;
   while ((1 << lsh) < std::max(t.np, t.nq)) ++lsh;
   t.lsh = lsh;
+  int sp = V.dims[0];
+  for (int a = 1; a < p; ++a) sp *= V.dims[a];
+  t.fsp = fast_div((unsigned)sp);
+  t.sps = sp + site_padding(sp, t.np, t.nq, lsh, elem_bytes);
+  t.Ds = V.D / sp * t.sps;
   t.mp = V.in_msg[p];
   t.mq = q ? V.in_msg[q] : -1;
   t.slot[0] = t.slot[1] = -1;
   t.old[0] = t.old[1] = -1;
   int st = V.dims[0];
   for (int a = 1; a <= V.k; ++a) {
-    if (a == p) t.fsp = fast_div((unsigned)st);
     if (a != p && a != q) {
       SiteTask::Mode& m = t.mode[t.nmode++];
       m.n = V.dims[a];
+      m.nfib = V.D / m.n;
       m.fst = fast_div((unsigned)st);
       m.msg = V.in_msg[a];
+      m.above = a > p;
+      m.pst = m.above ? st / sp * t.sps : st;
+      m.fg = fast_div((unsigned)(m.above ? 1 : sp / (st * m.n)));
     }
     st *= V.dims[a];
   }
@@ -381,11 +509,14 @@ SiteTask site_task(const VDesc& V, int p, int want) {
 }
 
 hipError_t launch_site(int psi_dtype, int acc_f64, const SiteTask* d_tasks, int n, const void* psi, const void* msg_in,
-                       void* msg_out, MsgStat* stats, int sym, int normalize, int threads, size_t lds, const int* active, int* queue,
-                       int grid, hipStream_t s) {
+                       void* msg_out, MsgStat* stats, int sym, int normalize, int threads, size_t lds, bool staged, const int* active,
+                       int* queue, int grid, hipStream_t s) {
   if (n <= 0) return hipSuccess;
-#define SITE_GO(TS, TA) \
-  launch_impl<TS, TA, TA>(d_tasks, n, psi, msg_in, msg_out, stats, sym, normalize, threads, lds, active, queue, grid, s)
+#define SITE_GO(TS, TA)                                                                                              \
+  (staged ? launch_impl<true, TS, TA, TA>(d_tasks, n, psi, msg_in, msg_out, stats, sym, normalize, threads, lds,     \
+                                          active, queue, grid, s)                                                    \
+          : launch_impl<false, TS, TA, TA>(d_tasks, n, psi, msg_in, msg_out, stats, sym, normalize, threads, lds,    \
+                                           active, queue, grid, s))
   if (acc_f64) switch (psi_dtype) {
       case ITNBP_F64: return SITE_GO(double, double);
       case ITNBP_F32: return SITE_GO(float, double);
@@ -399,15 +530,45 @@ hipError_t launch_site(int psi_dtype, int acc_f64, const SiteTask* d_tasks, int 
 #undef SITE_GO
 }
 
-hipError_t site_queue_occupancy(int psi_dtype, int acc_f64, int threads, size_t lds, int* per_cu) {
+hipError_t site_queue_occupancy(int psi_dtype, int acc_f64, int threads, size_t lds, bool staged, int* per_cu) {
+#define SITE_OCC(TS, TA) \
+  (staged ? occ_impl<true, TS, TA, TA>(threads, lds, per_cu) : occ_impl<false, TS, TA, TA>(threads, lds, per_cu))
   if (acc_f64) switch (psi_dtype) {
-      case ITNBP_F64: return occ_impl<double, double, double>(threads, lds, per_cu);
-      case ITNBP_F32: return occ_impl<float, double, double>(threads, lds, per_cu);
-      default: return occ_impl<bf16_t, double, double>(threads, lds, per_cu);
+      case ITNBP_F64: return SITE_OCC(double, double);
+      case ITNBP_F32: return SITE_OCC(float, double);
+      default: return SITE_OCC(bf16_t, double);
     }
   switch (psi_dtype) {
-    case ITNBP_F64: return occ_impl<double, float, float>(threads, lds, per_cu);
-    case ITNBP_F32: return occ_impl<float, float, float>(threads, lds, per_cu);
-    default: return occ_impl<bf16_t, float, float>(threads, lds, per_cu);
+    case ITNBP_F64: return SITE_OCC(double, float);
+    case ITNBP_F32: return SITE_OCC(float, float);
+    default: return SITE_OCC(bf16_t, float);
   }
+#undef SITE_OCC
+}
+
+std::vector<SiteLaunch> site_group(std::vector<SiteTask>& tasks, int elem_bytes, int num_cu) {
+  std::vector<SiteTask> cls[SITE_CLASSES + 1];  // the staged ones first
+  size_t nst = 0;
+  for (const SiteTask& t : tasks) nst += site_stageable(t.D, elem_bytes);
+  const bool stage = nst <= (size_t)num_cu;
+  for (const SiteTask& t : tasks)
+    cls[stage && site_stageable(t.D, elem_bytes) ? 0 : 1 + site_class(t.D, elem_bytes)].push_back(t);
+  auto cost = [](const SiteTask& t) {
+    long long s = (long long)(t.np + t.nq) * (t.want == 3 ? 2 : 1);
+    for (int m = 0; m < t.nmode; ++m) s += t.mode[m].n;
+    return (long long)t.D * s;
+  };
+  std::vector<SiteLaunch> out;
+  tasks.clear();
+  for (int c : {4, 3, 2, 1, 0}) {
+    if (cls[c].empty()) continue;
+    std::stable_sort(cls[c].begin(), cls[c].end(),
+                     [&](const SiteTask& x, const SiteTask& y) { return cost(x) > cost(y); });
+    long long dmax = 1;
+    for (const SiteTask& t : cls[c]) dmax = std::max<long long>(dmax, t.D);
+    const bool st = c == 0;
+    out.push_back(SiteLaunch{tasks.size(), cls[c].size(), site_threads(dmax, st), site_lds_bytes(dmax, elem_bytes, st), st});
+    tasks.insert(tasks.end(), cls[c].begin(), cls[c].end());
+  }
+  return out;
 }

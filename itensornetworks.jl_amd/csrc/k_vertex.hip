@@ -658,12 +658,8 @@ struct SmallState {
   std::vector<SiteTask> tasks;
   int nsites = 0;  // sites the tasks cover
   DevBuf d_tasks;
-  struct Launch {
-    int begin, count, threads;
-    size_t lds;
-    int grid;  // resident workgroups of the persistent form (0: not yet sized)
-  };
-  std::vector<Launch> launches;
+  std::vector<SiteLaunch> launches;
+  int queue_grid[SITE_CLASSES + 1] = {0};  // resident workgroups of the persistent form (0: not yet sized)
   // sites too large for LDS: k_vertex_big with scratch tensors
   std::vector<SmallTask> big;
   DevBuf d_big, ybuf;
@@ -765,17 +761,17 @@ hipError_t launch_small(itnbp_net* net, SmallState* st, int acc_f64, const void*
                         const void* msg_in, void* msg_out, MsgStat* stats, int normalize, bool queue,
                         hipStream_t stream) {
   for (size_t i = 0; i < st->launches.size(); ++i) {
-    SmallState::Launch& L = st->launches[i];
+    const SiteLaunch& L = st->launches[i];
     int* q = queue && st->queue.p ? (int*)st->queue.p + i * QUEUE_STRIDE : nullptr;
-    if (q && L.grid == 0) {
+    if (q && st->queue_grid[i] == 0) {
       // every workgroup of the grid resident at once
       int per_cu = 0;
-      hipError_t e = site_queue_occupancy(psi_dtype, acc_f64, L.threads, L.lds, &per_cu);
+      hipError_t e = site_queue_occupancy(psi_dtype, acc_f64, L.threads, L.lds, L.staged, &per_cu);
       if (e != hipSuccess) return e;
-      L.grid = std::max(1, std::min(L.count, std::max(1, per_cu) * net->ctx->num_cu));
+      st->queue_grid[i] = std::max(1, std::min((int)L.count, std::max(1, per_cu) * net->ctx->num_cu));
     }
-    hipError_t e = launch_site(psi_dtype, acc_f64, (const SiteTask*)st->d_tasks.p + L.begin, L.count, psi, msg_in,
-                               msg_out, stats, 1, normalize, L.threads, L.lds, st->active, q, L.grid, stream);
+    hipError_t e = launch_site(psi_dtype, acc_f64, (const SiteTask*)st->d_tasks.p + L.begin, (int)L.count, psi, msg_in,
+                               msg_out, stats, 1, normalize, L.threads, L.lds, L.staged, st->active, q, st->queue_grid[i], stream);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
@@ -867,7 +863,6 @@ int small_prepare(itnbp_net* net, const std::vector<int>& seq, int acc_f64, std:
   std::vector<int> pos(2 * net->ne, -1);
   for (size_t i = 0; i < seq.size(); ++i) pos[seq[i]] = (int)i;
   const size_t eb = acc_f64 ? 8 : 4;
-  std::vector<SiteTask> site[SITE_CLASSES];
   for (int v = 0; v < net->nv; ++v) {
     const VDesc& V = net->vdesc[v];
     if (V.k < 1 || V.k > ITNBP_MAXK) continue;
@@ -897,7 +892,7 @@ int small_prepare(itnbp_net* net, const std::vector<int>& seq, int acc_f64, std:
       ++st->nsites;
       for (int p = 1; p <= V.k; p += 2) {
         const int q = p < V.k ? p : (V.k == 1 ? 1 : p - 1), want = p < V.k ? 3 : (V.k == 1 ? 1 : 2);
-        SiteTask s = site_task(V, q, want);
+        SiteTask s = site_task(V, q, want, (int)eb);
         s.inst = t.inst;
         for (int o = 0; o < 2; ++o)
           if ((want >> o) & 1) {
@@ -905,7 +900,7 @@ int small_prepare(itnbp_net* net, const std::vector<int>& seq, int acc_f64, std:
             s.slot[o] = t.slot[q + o - 1];
             s.normalize[o] = 1;
           }
-        site[site_class(V.D, (int)eb)].push_back(s);
+        st->tasks.push_back(s);
       }
     } else {
       t.yoff = st->ytotal;
@@ -922,23 +917,10 @@ int small_prepare(itnbp_net* net, const std::vector<int>& seq, int acc_f64, std:
     for (int a = 1; a <= V.k; ++a) s += V.dims[a];
     return (long long)V.D * s;
   };
-  auto site_cost = [](const SiteTask& t) {
-    long long s = (long long)(t.np + t.nq) * (t.want == 3 ? 2 : 1);
-    for (int m = 0; m < t.nmode; ++m) s += t.mode[m].n;
-    return (long long)t.D * s;
-  };
   std::stable_sort(st->big.begin(), st->big.end(),
                    [&](const SmallTask& x, const SmallTask& y) { return cost(x) > cost(y); });
-  for (int c = SITE_CLASSES - 1; c >= 0; --c) {
-    if (site[c].empty()) continue;
-    std::stable_sort(site[c].begin(), site[c].end(),
-                     [&](const SiteTask& x, const SiteTask& y) { return site_cost(x) > site_cost(y); });
-    long long dmax = 1;
-    for (const SiteTask& s : site[c]) dmax = std::max<long long>(dmax, s.D);
-    st->launches.push_back(SmallState::Launch{(int)st->tasks.size(), (int)site[c].size(), site_threads(dmax),
-                                              site_lds_bytes(dmax, (int)eb), 0});
-    st->tasks.insert(st->tasks.end(), site[c].begin(), site[c].end());
-  }
+  st->launches = site_group(st->tasks, (int)eb, net->ctx->num_cu);
+  std::fill(st->queue_grid, st->queue_grid + SITE_CLASSES + 1, 0);
   if (!st->big.empty())
     ITNBP_RETCHK(ensure_buf(ctx, st->seeds, (size_t)std::max(1, 2 * net->ne) * SEED_LD * SEED_LD * 8));
   if (!st->big.empty()) {
@@ -949,7 +931,7 @@ int small_prepare(itnbp_net* net, const std::vector<int>& seq, int acc_f64, std:
     ITNBP_HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
   }
   if (!st->tasks.empty()) {
-    ITNBP_RETCHK(ensure_buf(ctx, st->queue, SITE_CLASSES * QUEUE_STRIDE * sizeof(int)));
+    ITNBP_RETCHK(ensure_buf(ctx, st->queue, (SITE_CLASSES + 1) * QUEUE_STRIDE * sizeof(int)));
     ITNBP_RETCHK(ensure_buf(ctx, st->d_tasks, st->tasks.size() * sizeof(SiteTask)));
     ITNBP_HIPCHK(ctx, hipMemcpyAsync(st->d_tasks.p, st->tasks.data(), st->tasks.size() * sizeof(SiteTask),
                                      hipMemcpyHostToDevice, ctx->stream));
