@@ -155,6 +155,307 @@ __device__ inline int jacobi_svd(double* A, int M, int N, double* V, double* rot
   return sweep + 1;
 }
 
+// ---- SVD of Theta -----------------------------------------------------------
+// sum over the 8 or 16 lanes of a (half) DPP row, the same bits in every lane
+template <int CTRL>
+__device__ inline double dpp_mov_d(double x) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+__device__ inline double row8_sum(double v) {
+  v += dpp_mov_d<0xB1>(v);   // quad_perm 1 0 3 2
+  v += dpp_mov_d<0x4E>(v);   // quad_perm 2 3 0 1
+  v += dpp_mov_d<0x141>(v);  // row_half_mirror
+  return v;
+}
+__device__ inline double row16_sum(double v) {
+  v = row8_sum(v);
+  v += dpp_mov_d<0x140>(v);  // row_mirror
+  return v;
+}
+
+// 1 / sqrt(x) to a rounding error or two: the hardware estimate (~2^-23) and one
+// step of third order
+__device__ inline double rsqrt_d(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
+// The Jacobi rotation of a column pair with squared norms al, be and inner
+// product ga != 0: tan 2 theta = 2 ga / (be - al), |theta| <= pi / 4; new columns
+// c p - s q and s p + c q.  Two reciprocal roots in place of the textbook form's
+// three divisions and two roots (launches of 28 SVDs of 64 x 64: 640 -> 504 us, of
+// 10 of 128 x 128: 2.63 -> 2.05 ms).  al, be, ga of order 1 or below (the caller
+// scales), so the squares stay in range.
+__device__ inline void jacobi_rotation(double al, double be, double ga, double& c, double& s) {
+  const double d = be - al, g2 = 2 * ga;
+  const double ri = rsqrt_d(fma(d, d, g2 * g2));
+  const double c2 = fma(0.5 * fabs(d), ri, 0.5);
+  const double ci = rsqrt_d(c2);
+  c = c2 * ci;
+  const double t = 0.5 * g2 * ri * ci;
+  s = d >= 0 ? t : -t;
+}
+
+// LDS of gate_svd<NP>: X (NP x (NP + 16)) and the vectors behind it
+template <int NP>
+struct SvdLds {
+  static constexpr int LD = NP + 16;
+  double *X, *vbuf, *wmv, *svec;
+  int *wmi, *perm, *order, *skeep;
+  __device__ explicit SvdLds(double* sm) {
+    X = sm;
+    vbuf = X + NP * LD;
+    wmv = vbuf + 2 * NP;
+    svec = wmv + 16;
+    wmi = reinterpret_cast<int*>(svec + NP);
+    perm = wmi + 16;
+    order = perm + NP;
+    skeep = order + NP;
+  }
+  static constexpr size_t bytes() {
+    return sizeof(double) * ((size_t)NP * LD + 2 * NP + 16 + NP) + sizeof(int) * (16 + 2 * NP + 4);
+  }
+};
+
+// SVD and truncation of Theta (M x N, N <= M <= NP) by a workgroup of 8 NP
+// threads; thread (c, h) = (tid / 8, tid % 8) passes rows h + 8 i of column c in a
+// (zero outside).  Theta P = Q R by a Householder QR with column pivoting (the
+// column in registers, the reflector through LDS), then one-sided Jacobi on X =
+// R^T in LDS (16 lanes per column pair, one barrier per step; rotation threshold,
+// rounding floor and stopping rule of jacobi_svd), X <- U_x diag(s): V_Theta = P U_x.
+// The pivoting grades the columns and halves the sweeps.  Theta is scaled by a
+// power of two to order 1 first (exact).  On return L.X holds U_x in the kept
+// columns, L.perm the pivots, L.svec the singular values, L.order their descending order;
+// the truncation (maxdim, cutoff, the bond's layout lay) and the outputs of slot
+// are done.  Returns the kept rank, -1 if the gate is refused.  A step is bound by
+// its dependent chain (loads, reduction, rotation, barrier) up to NP = 64 and by
+// LDS bandwidth at 128.
+template <int NP>
+__device__ int gate_svd(double (&a)[NP / 8], int M, int N, const SvdLds<NP>& L, const ApplyParams& prm, int lay,
+                        int slot, double* truncerr, double* svals, int* kept, int* status) {
+  constexpr int LD = SvdLds<NP>::LD, RW = NP / 8, NW = NP / 8, RB = NP / 32;
+  constexpr double EPS = 2.220446049250313e-16;
+  double* X = L.X;
+  const int tid = threadIdx.x, c = tid >> 3, h = tid & 7;
+  double mx = 0;
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < RW; ++i) {
+    bad = bad || !isfinite(a[i]);
+    mx = fmax(mx, fabs(a[i]));
+  }
+  for (int m = 32; m > 0; m >>= 1) mx = fmax(mx, __shfl_xor(mx, m));
+  if ((tid & 63) == 0) L.wmv[tid >> 6] = mx;
+  for (int i = tid; i < NP * LD; i += 8 * NP) X[i] = 0.0;
+  if (__syncthreads_or(bad)) {  // a NaN or Inf in psi or an environment
+    if (tid == 0) {
+      truncerr[slot] = NAN;
+      if (svals)
+        for (int i = 0; i < prm.max_keep; ++i) svals[(long long)slot * prm.max_keep + i] = 0.0;
+      if (kept) kept[slot] = prm.maxdim > 0 && prm.maxdim < N ? prm.maxdim : N;
+      status[slot] = 2;
+    }
+    return -1;
+  }
+  mx = L.wmv[0];
+#pragma unroll
+  for (int q = 1; q < NW; ++q) mx = fmax(mx, L.wmv[q]);
+  const int ex = mx > 0 ? ilogb(mx) : 0;
+#pragma unroll
+  for (int i = 0; i < RW; ++i) a[i] = ldexp(a[i], -ex);
+  __syncthreads();
+  bool done = c >= N;
+  for (int j = 0; j < N; ++j) {
+    // the remaining column of largest norm over rows >= j (ties: the smaller index)
+    double part = 0;
+#pragma unroll
+    for (int i = 0; i < RW; ++i)
+      if (h + 8 * i >= j) part += a[i] * a[i];
+    double best = done ? -1.0 : row8_sum(part);
+    int bi = c;
+    for (int m = 8; m < 64; m <<= 1) {
+      const double ob = __shfl_xor(best, m);
+      const int oi = __shfl_xor(bi, m);
+      if (ob > best || (ob == best && oi < bi)) {
+        best = ob;
+        bi = oi;
+      }
+    }
+    if ((tid & 63) == 0) {
+      L.wmv[tid >> 6] = best;
+      L.wmi[tid >> 6] = bi;
+    }
+    __syncthreads();
+    best = L.wmv[0];
+    bi = L.wmi[0];
+#pragma unroll
+    for (int q = 1; q < NW; ++q) {
+      const double ob = L.wmv[q];
+      const int oi = L.wmi[q];
+      if (ob > best || (ob == best && oi < bi)) {
+        best = ob;
+        bi = oi;
+      }
+    }
+    double* v = L.vbuf + (j & 1) * NP;
+    if (c == bi) {
+#pragma unroll
+      for (int i = 0; i < RW; ++i) {
+        const int row = h + 8 * i;
+        v[row] = a[i];
+        if (row < j) X[j + LD * row] = a[i];  // X[j][row] = R[row][j]
+      }
+      if (h == 0) L.perm[j] = c;
+      done = true;
+    }
+    __syncthreads();
+    const double xjj = v[j];
+    const double nrm = sqrt(best);
+    const double alpha = xjj >= 0 ? -nrm : nrm;
+    const double v0 = xjj - alpha;
+    const double vv = best - xjj * xjj + v0 * v0;
+    const double beta = (nrm == 0.0 || vv == 0.0) ? 0.0 : 2.0 / vv;
+    if (tid == 0) X[j + LD * j] = beta != 0.0 ? alpha : xjj;
+    double dot = 0;
+#pragma unroll
+    for (int i = 0; i < RW; ++i) {
+      const int row = h + 8 * i;
+      if (row >= j) dot += (row == j ? v0 : v[row]) * a[i];
+    }
+    dot = row8_sum(dot);
+    if (!done) {
+      const double f = beta * dot;
+#pragma unroll
+      for (int i = 0; i < RW; ++i) {
+        const int row = h + 8 * i;
+        if (row >= j) a[i] -= f * (row == j ? v0 : v[row]);
+      }
+    }
+  }
+  __syncthreads();
+  // one-sided Jacobi on X (N x N, zero-padded rows)
+  const int pi = tid >> 4, gl = tid & 15;
+  double fro = 0;
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {  // group pi: columns pi, pi + NP / 2
+    const double* x = X + (pi + q * (NP / 2)) * LD;
+#pragma unroll
+    for (int m = 0; m < RB; ++m) {
+      const double2 t = *reinterpret_cast<const double2*>(x + 2 * gl + 32 * m);
+      fro += t.x * t.x + t.y * t.y;
+    }
+  }
+  fro = block_sum_d(fro, L.wmv);
+  const int ne = N + (N & 1), npair = ne / 2;
+  const double tol = 8 * EPS * sqrt((double)N);
+  const double tol2 = tol * tol, floor2 = EPS * EPS * fro;
+  for (int sweep = 0; sweep < 60 && N > 1; ++sweep) {
+    int rotated = 0;
+    for (int st = 0; st < ne - 1; ++st) {
+      if (pi < npair) {
+        int p, q;
+        rr_pair(ne, st, pi, p, q);
+        if (q < N) {
+          double* xp = X + p * LD + 2 * gl;
+          double* xq = X + q * LD + 2 * gl;
+          double2 ap[RB], aq[RB];
+          double al = 0, be = 0, ga = 0;
+#pragma unroll
+          for (int m = 0; m < RB; ++m) {
+            ap[m] = *reinterpret_cast<const double2*>(xp + 32 * m);
+            aq[m] = *reinterpret_cast<const double2*>(xq + 32 * m);
+            al += ap[m].x * ap[m].x + ap[m].y * ap[m].y;
+            be += aq[m].x * aq[m].x + aq[m].y * aq[m].y;
+            ga += ap[m].x * aq[m].x + ap[m].y * aq[m].y;
+          }
+          al = row16_sum(al);
+          be = row16_sum(be);
+          ga = row16_sum(ga);
+          // |ga| > tol |p| |q|
+          if (al > floor2 && be > floor2 && ga * ga > tol2 * al * be) {
+            double cs, sn;
+            jacobi_rotation(al, be, ga, cs, sn);
+            rotated = 1;
+#pragma unroll
+            for (int m = 0; m < RB; ++m) {
+              double2 np_, nq_;
+              np_.x = cs * ap[m].x - sn * aq[m].x;
+              np_.y = cs * ap[m].y - sn * aq[m].y;
+              nq_.x = sn * ap[m].x + cs * aq[m].x;
+              nq_.y = sn * ap[m].y + cs * aq[m].y;
+              *reinterpret_cast<double2*>(xp + 32 * m) = np_;
+              *reinterpret_cast<double2*>(xq + 32 * m) = nq_;
+            }
+          }
+        }
+      }
+      __syncthreads();
+    }
+    if (!__syncthreads_or(rotated)) break;
+  }
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int col = pi + q * (NP / 2);
+    double s = 0;
+#pragma unroll
+    for (int m = 0; m < RB; ++m) {
+      const double2 t = *reinterpret_cast<const double2*>(X + col * LD + 2 * gl + 32 * m);
+      s += t.x * t.x + t.y * t.y;
+    }
+    s = row16_sum(s);
+    if (gl == 0) L.svec[col] = sqrt(s);
+  }
+  __syncthreads();
+  if (tid < N) {  // descending order, ties by index
+    const double s = L.svec[tid];
+    int r = 0;
+    for (int m = 0; m < N; ++m)
+      if (L.svec[m] > s || (L.svec[m] == s && m < tid)) ++r;
+    L.order[r] = tid;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    double tot = 0;
+    for (int i = 0; i < N; ++i) tot += L.svec[i] * L.svec[i];
+    int keep = N;
+    if (prm.maxdim > 0 && keep > prm.maxdim) keep = prm.maxdim;
+    double disc = 0;
+    for (int i = keep; i < N; ++i) disc += L.svec[L.order[i]] * L.svec[L.order[i]];
+    if (prm.cutoff >= 0 && tot > 0) {
+      while (keep > 1 && (disc + L.svec[L.order[keep - 1]] * L.svec[L.order[keep - 1]]) / tot <= prm.cutoff) {
+        disc += L.svec[L.order[keep - 1]] * L.svec[L.order[keep - 1]];
+        --keep;
+      }
+    }
+    int st = 0;
+    if (keep > lay) st = 1;  // more than the bond's layout holds
+    if (!isfinite(ldexp(tot, 2 * ex))) st = 2;  // the weight leaves the range
+    truncerr[slot] = st == 2 ? NAN : (tot > 0 ? disc / tot : 0.0);
+    if (svals)
+      for (int i = 0; i < prm.max_keep; ++i)
+        svals[(long long)slot * prm.max_keep + i] = i < keep ? ldexp(L.svec[L.order[i]], ex) : 0.0;
+    if (kept) kept[slot] = keep;
+    status[slot] = st;
+    *L.skeep = st ? -1 : keep;
+  }
+  __syncthreads();
+  const int keep = *L.skeep;
+  if (keep < 0) return -1;
+  // the kept columns of X over their singular values; the values back at Theta's scale
+  for (int i = tid; i < N * keep; i += 8 * NP) {
+    const int row = i % N, o = L.order[i / N];
+    const double s = L.svec[o];
+    X[row + LD * o] = s > 0 ? X[row + LD * o] / s : 0.0;
+  }
+  __syncthreads();
+  if (tid < N) L.svec[tid] = ldexp(L.svec[tid], ex);
+  __syncthreads();
+  return keep;
+}
+
 // ---- the split pipeline (k_apply_big.hip) -----------------------------------
 // device workspace of nb gates (host items) of one launch sequence, in bytes
 size_t apply_big_bytes(const itnbp_net* net, const ApplyItem* items, int nb);

@@ -29,15 +29,14 @@
 // (three read + write passes, two Gram reads, rebuild, scale) and are HBM-bound
 // at chi = 32; the per-gate kernels (roots, chol, svd) are latency-bound, one
 // workgroup each.  One round with the copies in and out, against one workgroup
-// per bond through all steps: 8x8 chi = 16 (4 classes of 28 gates) 44.1 -> 9.6 ms,
-// 5x4 chi = 32 (4 classes of 6 to 10) 447 -> 28.8 ms; per class there, svd 0.64 and
-// 2.6 ms, rebuild 88 and 343 us, roots 94 and 234 us, grams 89 and 347 us, chol 81
+// per bond through all steps: 8x8 chi = 16 (4 classes of 28 gates) 44.1 -> 9.3 ms,
+// 5x4 chi = 32 (4 classes of 6 to 10) 447 -> 26.9 ms; per class there, svd 0.50 and
+// 2.05 ms, rebuild 88 and 343 us, roots 94 and 234 us, grams 89 and 347 us, chol 81
 // and 476 us, the three mode passes 50 and 124 us.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <string>
-#include <type_traits>
 #include <vector>
 
 #include "itnbp_apply.hpp"
@@ -682,265 +681,35 @@ __global__ __launch_bounds__(256) void k_gb_theta(GbWork w, const double* __rest
 }
 
 // ---- SVD ------------------------------------------------------------------------
-// sum over the 16 lanes of a DPP row, the same bits in every lane
-__device__ inline double row16_sum(double v) {
-  auto mv = [](double x, auto ctrl) {
-    constexpr int c = decltype(ctrl)::value;
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), c, 0xf, 0xf, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), c, 0xf, 0xf, true);
-    return __hiloint2double(hi, lo);
-  };
-  v += mv(v, std::integral_constant<int, 0xB1>{});   // quad_perm 1 0 3 2
-  v += mv(v, std::integral_constant<int, 0x4E>{});   // quad_perm 2 3 0 1
-  v += mv(v, std::integral_constant<int, 0x141>{});  // row_half_mirror
-  v += mv(v, std::integral_constant<int, 0x140>{});  // row_mirror
-  return v;
-}
-
-template <int NP>
-constexpr size_t gb_svd_lds() {
-  return sizeof(double) * ((size_t)NP * (NP + 16) + 2 * NP + 16 + NP) + sizeof(int) * (16 + 2 * NP + 4);
-}
-
-// Theta (M x N, N <= M <= NP) of one gate by one workgroup of 8 NP threads:
-// Theta P = Q R by a Householder QR with column pivoting (8 threads per column,
-// the column in registers, the reflector through LDS), then one-sided Jacobi on
-// X = R^T in LDS (16 lanes per column pair, one barrier per step; rotation
-// threshold, rounding floor and stopping rule of jacobi_svd), X <- U_x diag(s):
-// V_Theta = P U_x.  The pivoting grades the columns and halves the sweeps.  The
-// step is bound by its dependent chain (loads, reduction, rotation, barrier)
-// up to NP = 64 and by LDS bandwidth at 128.
+// Theta of one gate by one workgroup (gate_svd); the kept right singular vectors
+// and values go to the workspace
 template <int NP>
 __global__ __launch_bounds__(8 * NP) void k_gb_svd(GbWork w, ApplyParams prm, double* __restrict__ truncerr,
                                                    double* __restrict__ svals, int* __restrict__ kept,
                                                    int* __restrict__ status) {
   extern __shared__ __align__(16) double sm[];
-  constexpr int LD = NP + 16, RW = NP / 8, NW = NP / 8, RB = NP / 32;
-  double* X = sm;
-  double* vbuf = X + NP * LD;
-  double* wmv = vbuf + 2 * NP;
-  double* svec = wmv + 16;
-  int* wmi = reinterpret_cast<int*>(svec + NP);
-  int* perm = wmi + 16;
-  int* order = perm + NP;
-  int* skeep = order + NP;
+  const SvdLds<NP> L(sm);
   const int gt = blockIdx.x, tid = threadIdx.x;
   const GbSide& gu = w.side[2 * gt];
   const GbSide& gv = w.side[2 * gt + 1];
   const int Mr = w.info[2 * gt].r * gu.d, Nc = w.info[2 * gt + 1].r * gv.d;
   const int M = Mr < Nc ? Nc : Mr, N = Mr < Nc ? Mr : Nc;
   const double* Th = w.theta + (long long)gt * AP_TH_BIG * AP_TH_BIG;
-  const int slot = w.gate[gt].slot;
   const int c = tid >> 3, h = tid & 7;
-  double a[RW];
-  bool bad = false;
+  double a[NP / 8];
 #pragma unroll
-  for (int i = 0; i < RW; ++i) {
+  for (int i = 0; i < NP / 8; ++i) {
     const int row = h + 8 * i;
     a[i] = (c < N && row < M) ? Th[row + M * c] : 0.0;
-    bad = bad || !isfinite(a[i]);
   }
-  for (int i = tid; i < NP * LD; i += 8 * NP) X[i] = 0.0;
-  if (__syncthreads_or(bad)) {  // a NaN or Inf in psi or an environment
-    if (tid == 0) {
-      truncerr[slot] = NAN;
-      if (svals)
-        for (int i = 0; i < prm.max_keep; ++i) svals[(long long)slot * prm.max_keep + i] = 0.0;
-      if (kept) kept[slot] = N;
-      status[slot] = 2;
-      w.out[gt].keep = -1;
-    }
-    return;
-  }
-  bool done = c >= N;
-  for (int j = 0; j < N; ++j) {
-    // the remaining column of largest norm over rows >= j (ties: the smaller index)
-    double part = 0;
-#pragma unroll
-    for (int i = 0; i < RW; ++i)
-      if (h + 8 * i >= j) part += a[i] * a[i];
-    part += __shfl_xor(part, 1);
-    part += __shfl_xor(part, 2);
-    part += __shfl_xor(part, 4);
-    double best = done ? -1.0 : part;
-    int bi = c;
-    for (int m = 8; m < 64; m <<= 1) {
-      const double ob = __shfl_xor(best, m);
-      const int oi = __shfl_xor(bi, m);
-      if (ob > best || (ob == best && oi < bi)) {
-        best = ob;
-        bi = oi;
-      }
-    }
-    if ((tid & 63) == 0) {
-      wmv[tid >> 6] = best;
-      wmi[tid >> 6] = bi;
-    }
-    __syncthreads();
-    best = wmv[0];
-    bi = wmi[0];
-#pragma unroll
-    for (int q = 1; q < NW; ++q) {
-      const double ob = wmv[q];
-      const int oi = wmi[q];
-      if (ob > best || (ob == best && oi < bi)) {
-        best = ob;
-        bi = oi;
-      }
-    }
-    double* v = vbuf + (j & 1) * NP;
-    if (c == bi) {
-#pragma unroll
-      for (int i = 0; i < RW; ++i) {
-        const int row = h + 8 * i;
-        v[row] = a[i];
-        if (row < j) X[j + LD * row] = a[i];  // X[j][row] = R[row][j]
-      }
-      if (h == 0) perm[j] = c;
-      done = true;
-    }
-    __syncthreads();
-    const double xjj = v[j];
-    const double nrm = sqrt(best);
-    const double alpha = xjj >= 0 ? -nrm : nrm;
-    const double v0 = xjj - alpha;
-    const double vv = best - xjj * xjj + v0 * v0;
-    const double beta = (nrm == 0.0 || vv == 0.0) ? 0.0 : 2.0 / vv;
-    if (tid == 0) X[j + LD * j] = beta != 0.0 ? alpha : xjj;
-    double dot = 0;
-#pragma unroll
-    for (int i = 0; i < RW; ++i) {
-      const int row = h + 8 * i;
-      if (row >= j) dot += (row == j ? v0 : v[row]) * a[i];
-    }
-    dot += __shfl_xor(dot, 1);
-    dot += __shfl_xor(dot, 2);
-    dot += __shfl_xor(dot, 4);
-    if (!done) {
-      const double f = beta * dot;
-#pragma unroll
-      for (int i = 0; i < RW; ++i) {
-        const int row = h + 8 * i;
-        if (row >= j) a[i] -= f * (row == j ? v0 : v[row]);
-      }
-    }
-  }
-  __syncthreads();
-  // one-sided Jacobi on X (N x N, zero-padded rows)
-  const int pi = tid >> 4, gl = tid & 15;
-  double fro = 0;
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {  // group pi: columns pi, pi + NP / 2
-    const double* x = X + (pi + q * (NP / 2)) * LD;
-#pragma unroll
-    for (int m = 0; m < RB; ++m) {
-      const double2 t = *reinterpret_cast<const double2*>(x + 2 * gl + 32 * m);
-      fro += t.x * t.x + t.y * t.y;
-    }
-  }
-  fro = block_sum_d(fro, wmv);
-  const int ne = N + (N & 1), npair = ne / 2;
-  const double tol = 8 * EPS * sqrt((double)N);
-  const double tol2 = tol * tol, floor2 = EPS * EPS * fro;
-  for (int sweep = 0; sweep < 60 && N > 1; ++sweep) {
-    int rotated = 0;
-    for (int st = 0; st < ne - 1; ++st) {
-      if (pi < npair) {
-        int p, q;
-        rr_pair(ne, st, pi, p, q);
-        if (q < N) {
-          double* xp = X + p * LD + 2 * gl;
-          double* xq = X + q * LD + 2 * gl;
-          double2 ap[RB], aq[RB];
-          double al = 0, be = 0, ga = 0;
-#pragma unroll
-          for (int m = 0; m < RB; ++m) {
-            ap[m] = *reinterpret_cast<const double2*>(xp + 32 * m);
-            aq[m] = *reinterpret_cast<const double2*>(xq + 32 * m);
-            al += ap[m].x * ap[m].x + ap[m].y * ap[m].y;
-            be += aq[m].x * aq[m].x + aq[m].y * aq[m].y;
-            ga += ap[m].x * aq[m].x + ap[m].y * aq[m].y;
-          }
-          al = row16_sum(al);
-          be = row16_sum(be);
-          ga = row16_sum(ga);
-          if (al > floor2 && be > floor2 && fabs(ga) > tol * sqrt(al * be)) {
-            const double zeta = (be - al) / (2 * ga);
-            const double t = (zeta >= 0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1 + zeta * zeta));
-            const double cs = 1 / sqrt(1 + t * t), sn = cs * t;
-            rotated = 1;
-#pragma unroll
-            for (int m = 0; m < RB; ++m) {
-              double2 np_, nq_;
-              np_.x = cs * ap[m].x - sn * aq[m].x;
-              np_.y = cs * ap[m].y - sn * aq[m].y;
-              nq_.x = sn * ap[m].x + cs * aq[m].x;
-              nq_.y = sn * ap[m].y + cs * aq[m].y;
-              *reinterpret_cast<double2*>(xp + 32 * m) = np_;
-              *reinterpret_cast<double2*>(xq + 32 * m) = nq_;
-            }
-          }
-        }
-      }
-      __syncthreads();
-    }
-    if (!__syncthreads_or(rotated)) break;
-  }
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const int col = pi + q * (NP / 2);
-    double s = 0;
-#pragma unroll
-    for (int m = 0; m < RB; ++m) {
-      const double2 t = *reinterpret_cast<const double2*>(X + col * LD + 2 * gl + 32 * m);
-      s += t.x * t.x + t.y * t.y;
-    }
-    s = row16_sum(s);
-    if (gl == 0) svec[col] = sqrt(s);
-  }
-  __syncthreads();
-  if (tid < N) {  // descending order, ties by index
-    const double s = svec[tid];
-    int r = 0;
-    for (int m = 0; m < N; ++m)
-      if (svec[m] > s || (svec[m] == s && m < tid)) ++r;
-    order[r] = tid;
-  }
-  __syncthreads();
-  if (tid == 0) {
-    double tot = 0;
-    for (int i = 0; i < N; ++i) tot += svec[i] * svec[i];
-    int keep = N;
-    if (prm.maxdim > 0 && keep > prm.maxdim) keep = prm.maxdim;
-    double disc = 0;
-    for (int i = keep; i < N; ++i) disc += svec[order[i]] * svec[order[i]];
-    if (prm.cutoff >= 0 && tot > 0) {
-      while (keep > 1 && (disc + svec[order[keep - 1]] * svec[order[keep - 1]]) / tot <= prm.cutoff) {
-        disc += svec[order[keep - 1]] * svec[order[keep - 1]];
-        --keep;
-      }
-    }
-    int st = 0;
-    if (keep > gu.lay) st = 1;    // more than the bond's layout holds
-    if (!isfinite(tot)) st = 2;
-    truncerr[slot] = tot > 0 ? disc / tot : (st == 2 ? tot : 0.0);
-    if (svals)
-      for (int i = 0; i < prm.max_keep; ++i)
-        svals[(long long)slot * prm.max_keep + i] = i < keep ? svec[order[i]] : 0.0;
-    if (kept) kept[slot] = keep;
-    status[slot] = st;
-    w.out[gt].keep = st ? -1 : keep;
-    *skeep = st ? -1 : keep;
-  }
-  __syncthreads();
-  const int keep = *skeep;
+  const int keep = gate_svd<NP>(a, M, N, L, prm, gu.lay, w.gate[gt].slot, truncerr, svals, kept, status);
+  if (tid == 0) w.out[gt].keep = keep;
   if (keep < 0) return;
   double* Vg = w.V + (long long)gt * GB_W;
   for (int i = tid; i < N * keep; i += 8 * NP) {
-    const int row = i % N, k = i / N, o = order[k];
-    const double s = svec[o];
-    Vg[perm[row] + N * k] = s > 0 ? X[row + LD * o] / s : 0.0;
-    if (row == 0) w.sv[gt * AP_KEEP_BIG + k] = s;
+    const int row = i % N, k = i / N, o = L.order[k];
+    Vg[L.perm[row] + N * k] = L.X[row + SvdLds<NP>::LD * o];
+    if (row == 0) w.sv[gt * AP_KEEP_BIG + k] = L.svec[o];
   }
 }
 
@@ -1356,7 +1125,7 @@ int apply_big_run(itnbp_net* net, const ApplyItem* items, int nb, const double* 
   const size_t lds_gram = sizeof(double) * GB_N * GB_PITCH;
   const size_t lds_chol = sizeof(double) * (2 * GB_N * GB_LD + 256 + GB_N);
   const size_t lds_reb = sizeof(double) * (GB_N * GB_PITCH + 4 + 6 * p.lcols + p.max_w);
-  const size_t lds_svd = p.max_th <= 32 ? gb_svd_lds<32>() : p.max_th <= 64 ? gb_svd_lds<64>() : gb_svd_lds<128>();
+  const size_t lds_svd = p.max_th <= 32 ? SvdLds<32>::bytes() : p.max_th <= 64 ? SvdLds<64>::bytes() : SvdLds<128>::bytes();
   const struct {
     const void* f;
     size_t lds;
@@ -1364,7 +1133,7 @@ int apply_big_run(itnbp_net* net, const ApplyItem* items, int nb, const double* 
               {(const void*)k_gb_chol1, lds_chol},
               {(const void*)k_gb_chol2, lds_chol},
               {(const void*)k_gb_theta, 2 * GB_SQ * sizeof(double)},
-              {(const void*)k_gb_svd<128>, gb_svd_lds<128>()},
+              {(const void*)k_gb_svd<128>, SvdLds<128>::bytes()},
               {(const void*)k_gb_factors, GB_W * sizeof(double)},
               {(const void*)k_gb_rebuild, lds_reb}};
   for (const auto& a : attr)

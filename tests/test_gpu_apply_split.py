@@ -137,3 +137,29 @@ def test_cutoff_and_a_non_finite_gate():
                              g.index[bonds[0][1]], maxdim=10, normalize=True)
     for x in bonds[0]:
         np.testing.assert_allclose(new[x], ref[g.index[x]], atol=1e-10)
+
+
+@pytest.mark.parametrize("chi", [15, 16, 17, 31])  # Theta 30, 32 (one kernel), 34 and 62 (the next)
+def test_powers_of_two_change_no_bits(chi):
+    """Theta is scaled to order 1 by a power of two before its SVD: a site tensor
+    times 2^+-300 gives the same gauged tensors bit for bit, singular values and
+    all (the norms divide it out again, every step before is homogeneous)."""
+    rng = np.random.default_rng(65)
+    g = itnbp.path_graph(3)
+    psi = itnbp.random_tensornetwork(rng, np.float64, g, link_space=chi)
+    msgs = positive_messages(rng, psi)
+    bond = (2, 3)
+    gate = random_gates(rng, [bond])[0]
+    runs = []
+    for p in (0, 300, -300):
+        q = psi.copy()
+        q[2] = np.ldexp(psi[2], p)
+        bpc = itnbp.initialize_cache(q, messages=msgs)
+        sv = []
+        errs = itnbp.apply_gates_(bpc, [itnbp.Gate(gate, bond)], maxdim=chi, normalize=True,
+                                  callback=lambda singular_values, truncation_error: sv.append(singular_values))
+        new = bpc.tensornetwork()
+        runs.append((np.ldexp(sv[0], -p), new[2], new[3], errs[0]))
+    for r in runs[1:]:
+        for x, y in zip(r, runs[0]):
+            np.testing.assert_array_equal(x, y)
