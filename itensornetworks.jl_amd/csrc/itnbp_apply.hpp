@@ -444,11 +444,13 @@ __device__ int gate_svd(double (&a)[NP / 8], int M, int N, const SvdLds<NP>& L, 
   __syncthreads();
   const int keep = *L.skeep;
   if (keep < 0) return -1;
-  // the kept columns of X over their singular values; the values back at Theta's scale
+  // the kept columns of X over their singular values; the values back at Theta's
+  // scale.  A column at the rounding level was not rotated against the others, so its
+  // direction is noise with a part in theirs: zero, which Theta has along it
   for (int i = tid; i < N * keep; i += 8 * NP) {
     const int row = i % N, o = L.order[i / N];
     const double s = L.svec[o];
-    X[row + LD * o] = s > 0 ? X[row + LD * o] / s : 0.0;
+    X[row + LD * o] = s * s > floor2 ? X[row + LD * o] / s : 0.0;
   }
   __syncthreads();
   if (tid < N) L.svec[tid] = ldexp(L.svec[tid], ex);

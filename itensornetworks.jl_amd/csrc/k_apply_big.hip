@@ -22,8 +22,8 @@
 //
 // M^{-1/2} is never applied to a tall side: Q = X Tq with X = psi sqrt(M), and
 // sqrt(M) M^{-1/2} = P, which is the identity unless map_eigvals drops
-// eigenvalues, so psi' = (psi P) Tq F.  A wide side (E <= n) needs no QR: R = X,
-// Q = 1 and psi' = M^{-1/2} F.
+// eigenvalues, so psi' = (psi P) Tq F.  A wide side (E <= n) of full rank needs no
+// QR: R = X, Q = 1 and psi' = M^{-1/2} F.
 //
 // Bound: the launches over the site tensors move about 12 times their bytes
 // (three read + write passes, two Gram reads, rebuild, scale) and are HBM-bound
@@ -501,28 +501,64 @@ __device__ inline void gb_sum_parts(const GbWork& w, int side, int np, int n, do
       }
 }
 
+// X X^T of a wide side (E <= n <= 64) from R = X
+__device__ inline void gb_wide_gram(const GbWork& w, int side, double (&g)[4][4]) {
+  const GbSide& sd = w.side[side];
+  const int ti = threadIdx.x & 15, tj = threadIdx.x >> 4, E = sd.E;
+  const double* R = w.R + (long long)side * GB_SQ;
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      const int i = ti + 16 * a, j = tj + 16 * b;
+      g[a][b] = 0;
+      if (i < E && j < E)
+        for (int c = 0; c < sd.n; ++c) g[a][b] += R[i + E * c] * R[j + E * c];
+    }
+}
+
+// R <- V_r^T R (r x n) in place, V E x E in LDS
+__device__ inline void gb_wide_rank(const GbWork& w, int side, int r, const double* V, const int* keep_idx) {
+  const GbSide& g = w.side[side];
+  const int tid = threadIdx.x, E = g.E;
+  double* R = w.R + (long long)side * GB_SQ;
+  double t[16];
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    const int i = tid + 256 * q, k = i % r, c = i / r;
+    t[q] = 0;
+    if (i < r * g.n)
+      for (int e = 0; e < E; ++e) t[q] += V[e + E * keep_idx[k]] * R[e + E * c];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 16; ++q)
+    if (tid + 256 * q < r * g.n) R[tid + 256 * q] = t[q];
+}
+
 // The first factorisation of a side.  The Cholesky factor is used while its
 // pivots span at most 1e-10 (R's diagonal 1e-5, as the LDS kernel's rebuild
 // test); a side past that, rank-deficient ones among them, takes the
 // eigendecomposition G = V diag(l) V^T by one-sided Jacobi instead, dropping
 // directions with l <= n eps l_max: T = V_r l_r^{-1/2}, R0 = l_r^{1/2} V_r^T,
-// exact inverses of each other however graded l is.
+// exact inverses of each other however graded l is.  A wide side keeps R = X, Q = 1
+// unless X X^T fails the same test: then R = V_r^T X and Q = V_r with its
+// eigenvectors, so that noise directions stay out of Theta.
 __global__ __launch_bounds__(256) void k_gb_chol1(GbWork w) {
   extern __shared__ __align__(16) double sm[];
   const int side = blockIdx.x, tid = threadIdx.x;
   const GbSide& g = w.side[side];
-  const int n = g.n;
+  const int n = g.wide ? g.E : g.n;
   double* T = w.T + (long long)side * GB_SQ;
   double* R0 = w.R0 + (long long)side * GB_SQ;
-  if (g.wide) {  // R = X, Q = 1
-    double* R = w.R + (long long)side * GB_SQ;
+  if (g.wide) {  // R = X
     const double* X = w.X + g.x_off;
-    for (int i = tid; i < g.E * n; i += 256) {
+    double* R = w.R + (long long)side * GB_SQ;
+    for (int i = tid; i < g.E * g.n; i += 256) {
       const int c = i / g.E, e = i - c * g.E, b = (int)g.fd.div(c), s = c - b * g.d;
       R[i] = X[gb_nat(g, s, e, b)];
     }
-    if (tid == 0) w.info[side].r = g.E;
-    return;
+    __syncthreads();
   }
   double* U = sm;
   double* Mi = U + GB_N * GB_LD;
@@ -530,7 +566,10 @@ __global__ __launch_bounds__(256) void k_gb_chol1(GbWork w) {
   double* piv = rows + 256;
   const int nch = (g.E + GB_ROWS - 1) / GB_ROWS, np = nch < w.nsplit ? nch : w.nsplit;
   double a[4][4];
-  gb_sum_parts(w, side, np, n, a);
+  if (g.wide)
+    gb_wide_gram(w, side, a);
+  else
+    gb_sum_parts(w, side, np, n, a);
   bool bad = false;
 #pragma unroll
   for (int i = 0; i < 4; ++i)
@@ -538,7 +577,7 @@ __global__ __launch_bounds__(256) void k_gb_chol1(GbWork w) {
     for (int j = 0; j < 4; ++j) bad = bad || !isfinite(a[i][j]);
   if (__syncthreads_or(bad)) {
     // a NaN or Inf in psi or an environment: carried to Theta, which reports it
-    for (int i = tid; i < n * n; i += 256) {
+    for (int i = tid; !g.wide && i < n * n; i += 256) {
       T[i] = 0.0;
       R0[i] = NAN;
     }
@@ -552,7 +591,7 @@ __global__ __launch_bounds__(256) void k_gb_chol1(GbWork w) {
     pmax = fmax(pmax, piv[k]);
   }
   if (pmin > 1e-10 * pmax) {
-    for (int i = tid; i < n * n; i += 256) {
+    for (int i = tid; !g.wide && i < n * n; i += 256) {
       const int c = i % n, k = i / n;
       T[i] = c <= k ? Mi[k * GB_LD + c] / sqrt(piv[k]) : 0.0;  // T[c + n k]
       R0[i] = c <= k ? U[c * GB_LD + k] / sqrt(piv[c]) : 0.0;  // R0[c + n k], row c, column k
@@ -561,7 +600,10 @@ __global__ __launch_bounds__(256) void k_gb_chol1(GbWork w) {
     return;
   }
   __syncthreads();
-  gb_sum_parts(w, side, np, n, a);
+  if (g.wide)
+    gb_wide_gram(w, side, a);
+  else
+    gb_sum_parts(w, side, np, n, a);
   double* G = U;
   double* V = Mi;
 #pragma unroll
@@ -587,13 +629,19 @@ __global__ __launch_bounds__(256) void k_gb_chol1(GbWork w) {
     for (int j = 0; j < n; ++j) lmax = lam[j] > lmax ? lam[j] : lmax;
     int r = 0;
     for (int j = 0; j < n; ++j)
-      if (lam[j] > n * EPS * lmax) keep_idx[r++] = j;
+      if (lam[j] > g.n * EPS * lmax) keep_idx[r++] = j;
     if (r == 0) keep_idx[r++] = 0;  // X = 0: one zero direction, R = 0
     s_rank = r;
     w.info[side].r = r;
   }
   __syncthreads();
   const int r = s_rank;
+  if (g.wide) {  // R = V_r^T X, Q = V_r
+    double* Tq = w.Tq + (long long)side * GB_SQ;
+    for (int i = tid; i < n * r; i += 256) Tq[i] = V[i % n + n * keep_idx[i / n]];
+    gb_wide_rank(w, side, r, V, keep_idx);
+    return;
+  }
   for (int i = tid; i < n * r; i += 256) {
     const int c = i % n, k = i / n, kk = keep_idx[k];
     const double l = lam[kk];
@@ -717,7 +765,8 @@ __global__ __launch_bounds__(8 * NP) void k_gb_svd(GbWork w, ApplyParams prm, do
 // One side of a gate per workgroup: F = V sqrt(S) on the shorter side of Theta,
 // Theta V / sqrt(S) = U sqrt(S) on the taller one (rows (r, s'), r fastest); then
 // W = Tq F as n x (d keep), column s' + d b' (F is r x (d keep) in the same
-// storage).  A wide side has Q = 1: W = F with M^{-1/2} on its external bonds.
+// storage).  A wide side: W = F (rank-deficient: V_r F) with M^{-1/2} on its
+// external bonds.
 __global__ __launch_bounds__(256) void k_gb_factors(GbWork w) {
   extern __shared__ __align__(16) double F[];
   const int side = blockIdx.x, gt = side >> 1, tid = threadIdx.x;
@@ -778,6 +827,18 @@ __global__ __launch_bounds__(256) void k_gb_factors(GbWork w) {
       }
     }
     return;
+  }
+  if (r < g.E) {  // Q = V_r
+    const double* Tq = w.Tq + (long long)side * GB_SQ;
+    for (int i = tid; i < g.E * cols; i += 256) {
+      const int e = i % g.E, c = i / g.E;
+      double t = 0;
+      for (int k = 0; k < r; ++k) t += Tq[e + g.E * k] * F[k + r * c];
+      W[i] = t;
+    }
+    __syncthreads();
+    for (int i = tid; i < g.E * cols; i += 256) F[i] = W[i];
+    __syncthreads();
   }
   for (int pa = 0; pa < g.next; ++pa) {
     const double* Si = w.roots + ((long long)side * AP_MAXEXT + pa) * 3 * GB_ROOT + GB_ROOT;

@@ -163,3 +163,34 @@ def test_powers_of_two_change_no_bits(chi):
     for r in runs[1:]:
         for x, y in zip(r, runs[0]):
             np.testing.assert_array_equal(x, y)
+
+
+@pytest.mark.parametrize("chie,chib,rank,gate", [(32, 16, 5, "full"), (24, 16, 5, "full"), (32, 10, 5, "full"),
+                                                  (32, 16, None, "projector"), (32, 10, None, "projector")])
+def test_rank_deficient_pairs_keep_the_state(chie, chib, rank, gate):
+    """Without truncation the gauged pair contracts to the gate times the old one,
+    also where Theta has fewer non-zero singular values than the bond may keep: a
+    side of low rank (wide: E <= n, tall: E = 32 > n = 20), whose kept rank is the
+    rank's bound, or a gate that halves Theta's rank, whose bond keeps noise
+    values.  Bound: products of n x n factors and E-row sums, ~sqrt(n) eps each,
+    and rotations to 8 eps sqrt(N): 1e-13 is a few times their sum."""
+    rng = np.random.default_rng(66)
+    g, n = itnbp.path_graph(4), 2 * chib
+    psi = itnbp.random_tensornetwork(rng, np.float64, g, link_space=[chie, chib, chie])
+    if rank is not None:
+        for v in (2, 3):
+            t = (rng.standard_normal((chie, rank)) @ rng.standard_normal((rank, n))).reshape(chie, 2, chib)
+            psi[v] = np.asfortranarray(t.transpose(1, 0, 2) if v == 2 else t.transpose(1, 2, 0))
+    msgs = positive_messages(rng, psi)
+    Q = np.linalg.qr(rng.standard_normal((4, 4)))[0]
+    G = Q if gate == "full" else np.diag([1.0, 0.0, 0.0, 0.0])
+    bpc = itnbp.initialize_cache(psi, messages=msgs)
+    sv = []
+    itnbp.apply_gates_(bpc, [itnbp.Gate(G, (2, 3))], maxdim=2 * n, normalize=False,
+                       callback=lambda singular_values, truncation_error: sv.append(singular_values))
+    new = bpc.tensornetwork()
+    exact = np.einsum("xyst,seb,tbf->xeyf", G.reshape((2,) * 4, order="F"), psi[2], psi[3])
+    got = np.einsum("xek,ykf->xeyf", new[2], new[3])
+    assert np.linalg.norm(got - exact) <= 1e-13 * np.linalg.norm(exact)
+    if rank is not None:
+        assert len(sv[0]) == 2 * rank
