@@ -516,7 +516,7 @@ def main():
                                             "max_truncerr": max(errs.values()),
                                             "gate_build_seconds_untimed": t_gates}
         del c2
-        # a round at chi = 16 (8x8, 112 bonds): the global-memory gate kernel
+        # a round at chi = 16 (8x8, 112 bonds): the split gate pipeline
         g16 = itnbp.named_grid((8, 8))
         p16 = itnbp.random_tensornetwork(np.random.default_rng(16), np.float64, g16, link_space=16)
         c16 = itnbp.update(itnbp.initialize_cache(p16), maxiter=60, tol=1e-10, edge_sequence="parallel")

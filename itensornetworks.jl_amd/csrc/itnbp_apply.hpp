@@ -1,5 +1,5 @@
 // Declarations and device functions shared by the gate-application kernels:
-// the LDS kernel (k_apply.hip) and the split pipeline (k_apply_big.hip).
+// the LDS kernels (k_apply.hip) and the split pipeline (k_apply_big.hip).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -8,10 +8,9 @@
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 constexpr int AP_XY = 8192;   // max E * n (external size x d chi_b) per side
-// tall-skinny QR (E >= 4 n, n <= 16): the stacked R factors (4n x n) and the
-// heads and betas of their reflectors, per side, after the side's reflectors
-constexpr int AP_QRX = 4 * 16 * 16 + 4 * 16;
-constexpr int AP_SIDE = AP_XY + AP_QRX;  // global scratch per side of a gate
+// global scratch per side of a gate within the LDS limits: X of an explicit side, R,
+// Tq, the environments' M^{-1/2} and P, flags
+constexpr int AP_SIDE = AP_XY + 1024 + 1024 + 2 * 3 * 8 * 8 + 1;
 constexpr int AP_TH = 32;     // max rows/cols of Theta (r d)
 constexpr int AP_ENV = 8;     // max external bond dimension
 constexpr int AP_MAXEXT = 3;  // max external bonds per side (degree 4)
@@ -36,8 +35,8 @@ struct ApplyParams {
   int normalize;
   double eig_cutoff;  // map_eigvals cutoff (10 eps)
   int max_keep;       // stride of the singular value output
-  // per-phase timestamps (wall clock; 16 slots per gate, slot 8 the SVD's
-  // sweep count), or null; ITNBP_APPLY_PHASES=1
+  // per-phase timestamps (wall clock; 16 slots per gate), or null;
+  // ITNBP_APPLY_PHASES=1
   unsigned long long* ts = nullptr;
 };
 
@@ -153,6 +152,157 @@ __device__ inline int jacobi_svd(double* A, int M, int N, double* V, double* rot
     if (!__syncthreads_or(rotated)) break;
   }
   return sweep + 1;
+}
+
+// ---- QR of a tall side by Gram matrices ---------------------------------------
+// LDS of one elimination, n <= 16 NT
+template <int NT>
+struct CholLds {
+  static constexpr int LD = 16 * NT + 1;
+  double *U, *Mi, *rows, *piv;
+  __device__ explicit CholLds(double* sm) {
+    U = sm;
+    Mi = U + 16 * NT * LD;
+    rows = Mi + 16 * NT * LD;
+    piv = rows + 64 * NT;
+  }
+  static constexpr size_t bytes() { return sizeof(double) * (2 * 16 * NT * LD + 64 * NT + 16 * NT); }
+};
+
+// [G | 1] reduced by Gaussian elimination without exchanges, G (n x n) symmetric:
+// thread (ti, tj) = (tid % 16, tid / 16) of 256 holds elements (ti + 16 a, tj + 16 b)
+// of both halves in registers; only the pivot row goes through LDS, one barrier
+// per column.  With G = L D L^T: U[k][j >= k] = (D L^T)[k][j], Mi = L^{-1}, piv =
+// diag D.  A column whose pivot is at most thr is skipped, its piv 0.
+template <int NT>
+__device__ void chol_eliminate(double (&g)[NT][NT], int n, double thr, const CholLds<NT>& L) {
+  constexpr int NP = 16 * NT, LD = CholLds<NT>::LD;
+  const int tid = threadIdx.x, ti = tid & 15, tj = tid >> 4;
+  double m[NT][NT];
+#pragma unroll
+  for (int a = 0; a < NT; ++a)
+#pragma unroll
+    for (int b = 0; b < NT; ++b) m[a][b] = ti + 16 * a == tj + 16 * b ? 1.0 : 0.0;
+  // rows: [parity][G row (NP) | M row (NP)]
+  if (ti == 0)
+#pragma unroll
+    for (int b = 0; b < NT; ++b) {
+      L.rows[tj + 16 * b] = g[0][b];
+      L.rows[NP + tj + 16 * b] = m[0][b];
+    }
+  __syncthreads();
+  for (int k = 0; k < n; ++k) {
+    const double* rg = L.rows + (k & 1) * 2 * NP;
+    double* nx = L.rows + ((k & 1) ^ 1) * 2 * NP;
+    const double p = rg[k];
+    const bool ok = p > thr;
+    const double inv = ok ? 1 / p : 0.0;
+    if (tid < NP) {
+      L.U[k * LD + tid] = rg[tid];
+      L.Mi[k * LD + tid] = rg[NP + tid];
+      if (tid == 0) L.piv[k] = ok ? p : 0.0;
+    }
+    double gj[NT], mj[NT];
+#pragma unroll
+    for (int b = 0; b < NT; ++b) {
+      gj[b] = rg[tj + 16 * b];
+      mj[b] = rg[NP + tj + 16 * b];
+    }
+#pragma unroll
+    for (int a = 0; a < NT; ++a) {
+      const int i = ti + 16 * a;
+      if (i <= k || i >= n) continue;
+      const double f = rg[i] * inv;
+#pragma unroll
+      for (int b = 0; b < NT; ++b) {
+        g[a][b] -= f * gj[b];
+        m[a][b] -= f * mj[b];
+      }
+      if (i == k + 1)
+#pragma unroll
+        for (int b = 0; b < NT; ++b) {
+          nx[tj + 16 * b] = g[a][b];
+          nx[NP + tj + 16 * b] = m[a][b];
+        }
+    }
+    __syncthreads();
+  }
+}
+
+// One pass of the QR of a tall side, X = Q R from the Gram matrices G_p of X_p
+// (X_0 = X, X_{p+1} = X_p R_p^{-1}): on return U holds R_p and Mi its inverse
+// transposed.  Returns whether the pass was the last.
+//
+// Well-conditioned sides: two passes (CholeskyQR2), Q = X R_0^{-1} R_1^{-1} never
+// formed, orthogonal to ~eps cond(X); taken while the pivots of G_0 span at most
+// 1e-10 (R's diagonal 1e-5).  Past that the side turns explicit: each X_{p+1} is
+// stored, and the first passes factor G_p + s 1, s = 4 n eps tr G_p, which is
+// positive definite for every X and leaves X_{p+1} a condition number of at most
+// ~sqrt(eps) times X_p's (shifted CholeskyQR, Fukaya, Kannan, Nakatsukasa,
+// Yamamoto, Yanagisawa 2020); the pass after a well-conditioned G_p is the last.
+// From pass 2 columns with a pivot at most n eps max diag are dropped (zero columns
+// of Q and rows of R: directions below ~1e-20 of X).  X = Q R and Q^T Q = 1 then
+// hold to a few eps for every cond(X), rank-deficient X among them, as with
+// Householder reflectors.
+template <int NT, int PASS>
+__device__ bool chol_pass(double (&a)[NT][NT], int n, bool& expl, const CholLds<NT>& L) {
+  constexpr double EPS = 2.220446049250313e-16;
+  constexpr int LD = CholLds<NT>::LD;
+  const int tid = threadIdx.x, ti = tid & 15, tj = tid >> 4;
+  double keep[NT][NT];
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      keep[i][j] = a[i][j];
+      bad = bad || !isfinite(a[i][j]);
+      const int q = ti + 16 * i;
+      if (q == tj + 16 * j && q < n) L.piv[q] = a[i][j];
+    }
+  if (__syncthreads_or(bad)) {
+    // a NaN or Inf in psi or an environment: carried to Theta, which reports it
+    for (int i = tid; i < n * LD; i += 256) {
+      L.U[i] = NAN;
+      L.Mi[i] = 0.0;
+    }
+    __syncthreads();
+    return PASS > 0;
+  }
+  double tr = 0, mx = 0;
+  for (int k = 0; k < n; ++k) {
+    tr += L.piv[k];
+    mx = fmax(mx, L.piv[k]);
+  }
+  __syncthreads();
+  chol_eliminate<NT>(a, n, PASS < 2 ? 0.0 : n * EPS * mx, L);
+  double pmin = INFINITY, pmax = 0;
+  for (int k = 0; k < n; ++k) {
+    if (PASS < 2 || L.piv[k] > 0) pmin = fmin(pmin, L.piv[k]);
+    pmax = fmax(pmax, L.piv[k]);
+  }
+  bool fin = PASS == 3 || (PASS > 0 && (!expl || (pmin > 0.5 && pmax < 2.0)));
+  if (PASS < 2 && !fin && !(pmin > 1e-10 * pmax)) {
+    expl = true;
+    const double s = 4 * n * EPS * tr;
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const int q = ti + 16 * i;
+        a[i][j] = keep[i][j] + (q == tj + 16 * j && q < n ? s : 0.0);
+      }
+    __syncthreads();
+    chol_eliminate<NT>(a, n, 0.0, L);
+  }
+  for (int i = tid; i < n * n; i += 256) {
+    const int k = i / n, j = i - k * n;
+    const double p = L.piv[k], sc = p > 0 ? 1 / sqrt(p) : 0.0;
+    L.U[k * LD + j] = j < k ? 0.0 : L.U[k * LD + j] * sc;
+    L.Mi[k * LD + j] = j > k ? 0.0 : L.Mi[k * LD + j] * sc;
+  }
+  __syncthreads();
+  return fin;
 }
 
 // ---- SVD of Theta -----------------------------------------------------------

@@ -12,10 +12,14 @@
 //   4. psi_u' = (Q_u with M^{-1/2} on the external bonds) U sqrt(S), likewise
 //      psi_v' with sqrt(S) V^T (src/apply.jl:90-93); optional normalisation
 //      (src/apply.jl:134-137).
-// One workgroup per bond; the bonds of one launch are disjoint.  Small dense
-// linear algebra: two-sided Jacobi in registers for the environment
-// eigenproblems (one wave each), Householder QR and one-sided (Hestenes) Jacobi
-// SVD in LDS.
+// The bonds of one call are disjoint.  Within the LDS limits (external bonds <= 8,
+// a side of at most 8192 elements, Theta <= 32 x 32) a call is two launches: one
+// workgroup per side up to R, one per bond from Theta on; larger bonds run the
+// split pipeline (k_apply_big.hip).  Small dense linear algebra: two-sided Jacobi
+// in registers for the environment eigenproblems (one wave each), QR by Gram
+// matrices on the matrix cores (chol_pass), one-sided (Hestenes) Jacobi SVD in LDS
+// (gate_svd).  120 gates of a chi = 8 colour class: 910 us in one launch with
+// Householder QR and the SVD on one wave -> 77 + 225 us.
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
@@ -31,20 +35,22 @@
 namespace {
 
 // thread 0 of the workgroup records the end of phase ph (0: start)
-__device__ inline void phase_mark(const ApplyParams& prm, int ph) {
-  if (prm.ts && threadIdx.x == 0) prm.ts[blockIdx.x * 16 + ph] = wall_clock64();
+__device__ inline void phase_mark(const ApplyParams& prm, int gate, int ph) {
+  if (prm.ts && threadIdx.x == 0) prm.ts[gate * 16 + ph] = wall_clock64();
 }
 
-// sqrt(M) and M^{-1/2} of a symmetrised chi x chi message (column-major in
-// global), chi <= 8, by one wave: lane i ne + j (ne = chi rounded up to even)
-// holds A[i][j] and V[i][j] in registers.  Cyclic two-sided Jacobi with
-// round-robin pairs (rr_pair's schedule), every lane deriving the rotations of
-// its row pair and column pair from the pre-step matrix through shuffles, so a
-// step needs no LDS and no barrier; stops when the off-diagonal mass is below
-// 1e-30 of the diagonal's or stops decreasing (at most 40 sweeps).  Then the eigenvalue truncation
-// of map_eigvals (cutoff = 10 eps, src/apply.jl:9-25), recomputed identically
-// by every lane.  S and Si row-major, ld chi.
-__device__ void env_roots_wave(const double* M, int chi, double cutoff, double* S, double* Si) {
+// sqrt(M), M^{-1/2} and the projector P on the kept eigenvectors of a symmetrised
+// chi x chi message (column-major in global), chi <= 8, by one wave: lane i ne + j
+// (ne = chi rounded up to even) holds A[i][j] and V[i][j] in registers.  Cyclic
+// two-sided Jacobi with round-robin pairs (rr_pair's schedule), every lane deriving
+// the rotations of its row pair and column pair from the pre-step matrix through
+// shuffles, so a step needs no LDS and no barrier; stops when the off-diagonal mass
+// is below 1e-30 of the diagonal's or stops decreasing (at most 40 sweeps).  Then
+// the eigenvalue truncation of map_eigvals (cutoff = 10 eps, src/apply.jl:9-25),
+// recomputed identically by every lane.  M is scaled by an even power of two to
+// order 1 for jacobi_rotation.  S, Si and P row-major, ld chi; returns whether
+// eigenvalues were dropped (P != 1).
+__device__ bool env_roots_wave(const double* M, int chi, double cutoff, double* S, double* Si, double* P) {
   const int l = threadIdx.x & 63;
   const int ne = chi + (chi & 1);
   const bool live = l < ne * ne;
@@ -52,17 +58,16 @@ __device__ void env_roots_wave(const double* M, int chi, double cutoff, double* 
   const bool in = live && i < chi && j < chi;
   double a = in ? 0.5 * (M[i + chi * j] + M[j + chi * i]) : 0.0;
   double v = (live && i == j) ? 1.0 : 0.0;
+  double mx = fabs(a);
+  for (int m = 32; m > 0; m >>= 1) mx = fmax(mx, __shfl_xor(mx, m));
+  const int ex = mx > 0 && isfinite(mx) ? ilogb(mx) & ~1 : 0;
+  a = ldexp(a, -ex);
   if (chi > 1) {
     auto rot = [&](int p, int q, double& c, double& sn) {
       const double app = __shfl(a, p * ne + p), aqq = __shfl(a, q * ne + q), apq = __shfl(a, p * ne + q);
       c = 1.0;
       sn = 0.0;
-      if (q < chi && apq != 0.0) {
-        const double zeta = (aqq - app) / (2 * apq);
-        const double t = (zeta >= 0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1 + zeta * zeta));
-        c = 1 / sqrt(1 + t * t);
-        sn = c * t;
-      }
+      if (q < chi && fabs(apq) > 1e-150) jacobi_rotation(app, aqq, apq, c, sn);
     };
     double prev = INFINITY;
     for (int sweep = 0; sweep < 40; ++sweep) {
@@ -136,7 +141,7 @@ __device__ void env_roots_wave(const double* M, int chi, double cutoff, double* 
   for (int m = 0; m < AP_ENV; ++m)
     if (m < chi && rank[m] < keep) kmask |= 1u << m;
   // S[r][c] = sum_m V[r][m] V[c][m] sqrt(l_m) over the kept m (lane (r, c) = (i, j))
-  double sv = 0, siv = 0;
+  double sv = 0, siv = 0, pv = 0;
   for (int m = 0; m < AP_ENV; ++m) {
     const int mm = m < ne ? m : 0;
     const double vr = __shfl(v, i * ne + mm), vc = __shfl(v, j * ne + mm);
@@ -144,17 +149,15 @@ __device__ void env_roots_wave(const double* M, int chi, double cutoff, double* 
       const double sq = sqrt(w[m]);  // NaN for a kept negative eigenvalue
       sv += vr * vc * sq;
       siv += vr * vc / sq;
+      pv += vr * vc;
     }
   }
   if (in) {
-    S[i * chi + j] = sv;
-    Si[i * chi + j] = siv;
+    S[i * chi + j] = ldexp(sv, ex / 2);
+    Si[i * chi + j] = ldexp(siv, -ex / 2);
+    P[i * chi + j] = pv;
   }
-}
-
-__device__ inline void wave_sync_ap() {
-  __builtin_amdgcn_s_waitcnt(0);
-  __builtin_amdgcn_wave_barrier();
+  return keep < chi;
 }
 
 struct SideGeom {
@@ -198,9 +201,6 @@ __device__ SideGeom side_geom(const VDesc& V, int j) {
   return g;
 }
 
-// the tall-skinny QR applies: four row blocks of at least n rows, n <= 16
-__device__ inline bool tsqr_ok(const SideGeom& g) { return g.n <= 16 && g.E >= 4 * g.n; }
-
 // natural offset of psi element (s, external multi-index e, bond b)
 __device__ inline int nat_off(const SideGeom& g, int s, int e, int b) {
   int off = 0, stride = g.d, rem = e;
@@ -219,820 +219,518 @@ __device__ inline int nat_off(const SideGeom& g, int s, int e, int b) {
   return s + off;
 }
 
-// mode product on external axis index pa of X (E x cols, column-major rows e):
-// Y[e with b'] = sum_b X[e with b] * Mt[b][b'] (Mt row-major, ld chi), chi <= CH
-template <int CH>
-__device__ void ext_mode_product(const SideGeom& g, int pa, const double* X, double* Y, int cols,
-                                 const double* Mt, bool transpose) {
-  const int stride = (int)g.fst[pa].d;
-  const int chi = g.dims[g.ext[pa]];
-  for (int idx = threadIdx.x; idx < g.E * cols; idx += blockDim.x) {
-    const int c = (int)g.fE.div(idx), e = idx - c * g.E;
-    const int q = (int)g.fst[pa].div(e), lo = e - q * stride;
-    const int hi = (int)g.fchi[pa].div(q), b2 = q - hi * chi;
-    double acc = 0;
-#pragma unroll
-    for (int b = 0; b < CH; ++b)
-      if (b < chi) {
-        const double m = transpose ? Mt[b2 * chi + b] : Mt[b * chi + b2];
-        acc += X[(lo + stride * (b + chi * hi)) + (long long)g.E * c] * m;
-      }
-    Y[idx] = acc;
+// ---- gates within the LDS limits ------------------------------------------------
+// Two launches over the gates of a call: k_gate_side, one workgroup per side, and
+// k_gate_pair, one per bond.  Side s of a gate leaves in work (AP_SIDE doubles):
+constexpr int AP_W_R = AP_XY;             // R, r x n
+constexpr int AP_W_TQ = AP_W_R + 1024;    // Tq, n x n: Q = X Tq
+constexpr int AP_W_SI = AP_W_TQ + 1024;   // M^{-1/2} per external bond, then P
+constexpr int AP_W_FLAG = AP_W_SI + 2 * AP_MAXEXT * AP_ENV * AP_ENV;  // bits 0 .. 2: P != 1 on that bond; 3: explicit
+static_assert(AP_W_FLAG + 1 == AP_SIDE, "layout of a side's workspace");
+// work[0 .. AP_XY): the last X_p of an explicit side (chol_pass), E x n
+
+// One side's matrix: rows e over the external bonds, columns c = s + d b.
+struct ApSide {
+  int d, chib, lay, lo, E, n, r, next;  // lay: the bond's layout (>= chib); lo: product of the bonds before it
+  int chi[AP_MAXEXT], est[AP_MAXEXT];   // external bonds: dimension, stride in e
+  long long psi_off;
+  FastDiv fd, flo, flay, fE, fper[AP_MAXEXT], fest[AP_MAXEXT];
+};
+
+__device__ void ap_side(const VDesc& V, int j, int chib, ApSide& g) {
+  g.d = V.dims[0];
+  g.chib = chib;
+  g.lay = V.dims[j];
+  g.lo = 1;
+  g.E = 1;
+  g.next = 0;
+  for (int a = 1; a <= V.k; ++a) {
+    if (a == j) continue;
+    if (a < j) g.lo *= V.dims[a];
+    g.chi[g.next] = V.dims[a];
+    g.est[g.next] = g.E;
+    g.fest[g.next++] = fast_div(g.E);
+    g.E *= V.dims[a];
   }
-  __syncthreads();
+  for (int pa = 0; pa < g.next; ++pa) g.fper[pa] = fast_div(g.E / g.chi[pa]);
+  g.n = g.d * chib;
+  g.r = g.E < g.n ? g.E : g.n;
+  g.psi_off = V.psi_off;
+  g.fd = fast_div(g.d);
+  g.flo = fast_div(g.lo);
+  g.flay = fast_div(g.lay);
+  g.fE = fast_div(g.E);
 }
 
-// Householder QR in place on X (E x n, column-major); R in the upper triangle,
-// reflector tails below, heads in vh[], betas in beta[]
-__device__ void householder_qr(double* X, int E, int n, double* vh, double* beta, double* red) {
-  const int tid = threadIdx.x;
-  const int r = E < n ? E : n;
-  for (int j = 0; j < r; ++j) {
-    double s = 0;
-    for (int i = j + tid; i < E; i += blockDim.x) s += X[i + (long long)E * j] * X[i + (long long)E * j];
-    s = block_sum_d(s, red);
-    const double xjj = X[j + (long long)E * j];
-    const double nrm = sqrt(s);
-    const double alpha = xjj >= 0 ? -nrm : nrm;
-    const double v0 = xjj - alpha;
-    const double vv = s - xjj * xjj + v0 * v0;
-    const double b = (nrm == 0.0 || vv == 0.0) ? 0.0 : 2.0 / vv;
-    if (tid == 0) {
-      vh[j] = v0;
-      beta[j] = b;
-    }
-    // apply to columns c > j: w = v . X[:, c]; X[:, c] -= b w v
-    const int w = tid >> 6, l = tid & 63;
-    for (int c = j + 1 + w; c < n; c += (int)(blockDim.x >> 6)) {
-      double dot = 0;
-      for (int i = j + l; i < E; i += 64) {
-        const double vi = (i == j) ? v0 : X[i + (long long)E * j];
-        dot += vi * X[i + (long long)E * c];
-      }
-      dot = wave_sum_d(dot);
-      for (int i = j + l; i < E; i += 64) {
-        const double vi = (i == j) ? v0 : X[i + (long long)E * j];
-        X[i + (long long)E * c] -= b * dot * vi;
-      }
-    }
-    __syncthreads();
-    if (tid == 0) X[j + (long long)E * j] = (b == 0.0) ? xjj : alpha;
-    __syncthreads();
-  }
+// pitch of a column of E rows in LDS: 2 mod 32 doubles, so that the operand
+// fragments of v_mfma_f64_16x16x4f64 (16 columns x 4 rows, 4 columns x 16 rows) meet
+// no bank twice per access
+__host__ __device__ inline int ap_pitch(int E) { return (E + 29) / 32 * 32 + 2; }
+
+// element (c, e) of the side behind entry i of the site tensor, in its memory
+// order; false for the layout's columns past chib
+__device__ inline bool ap_locate(const ApSide& g, int i, int& c, int& e, int& b) {
+  const int t = (int)g.fd.div(i), u = (int)g.flo.div(t), h = (int)g.flay.div(u);
+  b = u - h * g.lay;
+  c = i - t * g.d + g.d * b;
+  e = t - u * g.lo + g.lo * h;
+  return b < g.chib;
 }
 
-// Y (E x cols) <- H_0 ... H_{r-1} Y using the reflectors stored in X
-__device__ void apply_q(const double* X, int E, int r, const double* vh, const double* beta, double* Y,
-                        int cols) {
-  const int tid = threadIdx.x;
-  const int w = tid >> 6, l = tid & 63;
-  for (int j = r - 1; j >= 0; --j) {
-    const double b = beta[j];
-    if (b != 0.0) {
-      for (int c = w; c < cols; c += (int)(blockDim.x >> 6)) {
-        double dot = 0;
-        for (int i = j + l; i < E; i += 64) {
-          const double vi = (i == j) ? vh[j] : X[i + (long long)E * j];
-          dot += vi * Y[i + (long long)E * c];
-        }
-        dot = wave_sum_d(dot);
-        for (int i = j + l; i < E; i += 64) {
-          const double vi = (i == j) ? vh[j] : X[i + (long long)E * j];
-          Y[i + (long long)E * c] -= b * dot * vi;
-        }
-      }
-    }
-    __syncthreads();
+__device__ void ap_load(const ApSide& g, const double* __restrict__ src, double* X, int P) {
+  const int D = g.E * g.d * g.lay;
+#pragma unroll 8
+  for (int i = threadIdx.x; i < D; i += 256) {
+    const double x = src[i];
+    int c, e, b;
+    if (ap_locate(g, i, c, e, b)) X[c * P + e] = x;
   }
 }
 
-// Tall-skinny QR of a side (E x n, E >= 4 n, n <= 16), replacing the
-// workgroup-wide Householder QR there: each wave factors its quarter of the
-// rows (rows [w E / 4, (w + 1) E / 4)) with no workgroup barrier, wave 0 then
-// factors the four stacked n x n R factors (4n x n), whose R is the side's.
-// Q = diag(Q_0 .. Q_3) P Q_S (P places stacked row w n + i at block row i of
-// block w), so X = Q [R; 0] as for one Householder QR, up to the signs of R's
-// rows, which the rebuild's Q absorbs.
-//
-// Householder QR of rows x n (n <= 16) at X (column stride ld) by one wave:
-// lane (rg, c) = (l / 16, l % 16) works on rows i = rg (mod 4) of column c,
-// partial sums joined across rg by two shuffles; reflector j is
-// [vh[j]; X[j+1 .., j]] with beta[j], R in the upper triangle.  Every element
-// is read and written by its own lane, so only the diagonal element (read by
-// every lane) needs the wave to be in step.
-__device__ void wave_qr16(double* X, int ld, int rows, int n, double* vh, double* beta) {
-  const int l = threadIdx.x & 63, rg = l >> 4, c = l & 15;
-  for (int j = 0; j < n; ++j) {
-    const int i0 = j + 1 + ((rg - ((j + 1) & 3)) & 3);  // first row > j with i = rg (mod 4)
-    // four rows per iteration with independent partial sums, so that the LDS
-    // loads of an iteration are in flight together (one wave per SIMD here:
-    // nothing else hides their latency)
-    double p = 0;
-    if (c < n) {
-      const double* xj = X + (long long)ld * j;
-      const double* xc = X + (long long)ld * c;
-      double p0 = 0, p1 = 0, p2 = 0, p3 = 0;
-      int i = i0;
-      for (; i + 12 < rows; i += 16) {
-        p0 += xj[i] * xc[i];
-        p1 += xj[i + 4] * xc[i + 4];
-        p2 += xj[i + 8] * xc[i + 8];
-        p3 += xj[i + 12] * xc[i + 12];
-      }
-      for (; i < rows; i += 4) p0 += xj[i] * xc[i];
-      p = (p0 + p1) + (p2 + p3);
+// Mode product on external bond pa of the first n columns, in place: a wave owns 16
+// fibres, loads their chi <= 8 entries as B operands (B[k = b][fibre]), K stays in
+// registers as A operand (A[b'][b]); four groups of fibres in flight per iteration.
+__device__ void ap_mode(const ApSide& g, int pa, double* X, int P, int n, const double* K) {
+  const int l = threadIdx.x & 63, li = l & 15, lk = l >> 4, wv = threadIdx.x >> 6;
+  const int chi = g.chi[pa], st = g.est[pa], per = (int)g.fper[pa].d, nfib = per * n;
+  const double a0 = (lk < chi && li < chi) ? K[lk * chi + li] : 0.0;
+  const double a1 = (4 + lk < chi && li < chi) ? K[(4 + lk) * chi + li] : 0.0;
+  for (int f0 = 64 * wv; f0 < nfib; f0 += 256) {
+    double x0[4], x1[4];
+    int base[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int f = f0 + 16 * q + li;
+      if (f < nfib) {
+        const int c = (int)g.fper[pa].div(f), t = f - c * per, hi = (int)g.fest[pa].div(t);
+        base[q] = c * P + (t - hi * st) + st * chi * hi;
+      } else
+        base[q] = -1;
+      x0[q] = base[q] >= 0 && lk < chi ? X[base[q] + st * lk] : 0.0;
+      x1[q] = base[q] >= 0 && 4 + lk < chi ? X[base[q] + st * (4 + lk)] : 0.0;
     }
-    p += __shfl_xor(p, 16);
-    p += __shfl_xor(p, 32);
-    const double tail = __shfl(p, j);  // sum_{i > j} X[i][j]^2
-    const double xjj = X[j + (long long)ld * j];
-    const double s = xjj * xjj + tail;
-    const double nrm = sqrt(s);
-    const double alpha = xjj >= 0 ? -nrm : nrm;
-    const double v0 = xjj - alpha;
-    const double vv = tail + v0 * v0;
-    const double b = (nrm == 0.0 || vv == 0.0) ? 0.0 : 2.0 / vv;
-    if (c > j && c < n) {
-      const double dot = v0 * X[j + (long long)ld * c] + p;
-      const double f = b * dot;
-      if (rg == 0) X[j + (long long)ld * c] -= f * v0;
-      const double* xj = X + (long long)ld * j;
-      double* xc = X + (long long)ld * c;
-      int i = i0;
-      for (; i + 12 < rows; i += 16) {
-        const double a0 = xj[i], a1 = xj[i + 4], a2 = xj[i + 8], a3 = xj[i + 12];
-        const double c0 = xc[i], c1 = xc[i + 4], c2 = xc[i + 8], c3 = xc[i + 12];
-        xc[i] = c0 - f * a0;
-        xc[i + 4] = c1 - f * a1;
-        xc[i + 8] = c2 - f * a2;
-        xc[i + 12] = c3 - f * a3;
-      }
-      for (; i < rows; i += 4) xc[i] -= f * xj[i];
-    }
-    if (l == 0) {
-      vh[j] = v0;
-      beta[j] = b;
-    }
-    __builtin_amdgcn_s_waitcnt(0);
-    __builtin_amdgcn_wave_barrier();
-    if (l == 0) X[j + (long long)ld * j] = (b == 0.0) ? xjj : alpha;
-    __builtin_amdgcn_s_waitcnt(0);
-    __builtin_amdgcn_wave_barrier();
-  }
-}
-
-// Y[rows(i), c] <- H_0 .. H_{n-1} Y for c < cols (cols <= 16 per pass) by one
-// wave: reflector j is [vh[j]; V[j+1 .., j]] (column stride ldv) over the
-// logical rows i >= j, logical row i being Y row rowof(i); lane (rg, c) owns
-// logical rows i = rg (mod 4) of column c, and lane (0, c) the head row j.
-template <typename RowOf>
-__device__ void wave_apply_q16(const double* V, int ldv, int rows, int n, const double* vh, const double* beta,
-                               double* Y, int ldy, int cols, RowOf rowof) {
-  const int l = threadIdx.x & 63, rg = l >> 4, c16 = l & 15;
-  for (int c0 = 0; c0 < cols; c0 += 16) {
-    const int c = c0 + c16;
-    for (int j = n - 1; j >= 0; --j) {
-      const double b = beta[j];
-      if (b == 0.0) continue;
-      const int i0 = j + 1 + ((rg - ((j + 1) & 3)) & 3);
-      double p = 0;
-      const double* vj = V + (long long)ldv * j;
-      double* yc = Y + (long long)ldy * (c < cols ? c : 0);
-      if (c < cols) {
-        if (rg == 0) p = vh[j] * yc[rowof(j)];
-        double p1 = 0, p2 = 0, p3 = 0;
-        int i = i0;
-        for (; i + 12 < rows; i += 16) {
-          p += vj[i] * yc[rowof(i)];
-          p1 += vj[i + 4] * yc[rowof(i + 4)];
-          p2 += vj[i + 8] * yc[rowof(i + 8)];
-          p3 += vj[i + 12] * yc[rowof(i + 12)];
-        }
-        for (; i < rows; i += 4) p += vj[i] * yc[rowof(i)];
-        p = (p + p1) + (p2 + p3);
-      }
-      p += __shfl_xor(p, 16);
-      p += __shfl_xor(p, 32);
-      if (c < cols) {
-        const double f = b * p;
-        if (rg == 0) yc[rowof(j)] -= f * vh[j];
-        int i = i0;
-        for (; i + 12 < rows; i += 16) {
-          const double a0 = vj[i], a1 = vj[i + 4], a2 = vj[i + 8], a3 = vj[i + 12];
-          const double y0 = yc[rowof(i)], y1 = yc[rowof(i + 4)], y2 = yc[rowof(i + 8)], y3 = yc[rowof(i + 12)];
-          yc[rowof(i)] = y0 - f * a0;
-          yc[rowof(i + 4)] = y1 - f * a1;
-          yc[rowof(i + 8)] = y2 - f * a2;
-          yc[rowof(i + 12)] = y3 - f * a3;
-        }
-        for (; i < rows; i += 4) yc[rowof(i)] -= f * vj[i];
-      }
-      // row j - 1, the next head, belongs to another lane
-      __builtin_amdgcn_s_waitcnt(0);
-      __builtin_amdgcn_wave_barrier();
-    }
-  }
-}
-
-// Householder QR with column pivoting of A (M x N column-major in LDS,
-// N <= M <= 32) by one wave with A in registers, keeping R only: on return A's
-// top N x N upper triangle holds R with A P = Q R, and perm[j] is the original
-// column in position j.  Lane (c, h) = (l % 32, l / 32) holds rows
-// [16 h, 16 h + 16) of column c, as in wave_jacobi_svd32; a step finds the
-// remaining column of largest norm (ties: the smaller index), swaps it into
-// place and broadcasts the reflector by lane shuffles.  The rows below R hold
-// the reflector tails, which nothing reads.
-__device__ void wave_qrcp32(double* A, int M, int N, int* perm) {
-  const int l = threadIdx.x & 63, c = l & 31, h = l >> 5;
-  double a[16];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) a[i] = (c < N && 16 * h + i < M) ? A[16 * h + i + M * c] : 0.0;
-  int pm = c;  // original column held by this lane's column position
-  for (int j = 0; j < N; ++j) {
-    // squared norms over rows >= j of the columns c >= j
-    double part = 0;
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-      if (16 * h + i >= j) part += a[i] * a[i];
-    part += __shfl_xor(part, 32);
-    double best = (c >= j && c < N) ? part : -1.0;
-    int bi = c;
-    for (int m = 16; m > 0; m >>= 1) {
-      const double ob = __shfl_xor(best, m);
-      const int oi = __shfl_xor(bi, m);
-      if (ob > best || (ob == best && oi < bi)) {
-        best = ob;
-        bi = oi;
-      }
-    }
-    const int p = bi;  // the same in every lane
-    // swap columns j and p
-    const int src = (c == j ? p : (c == p ? j : c)) + 32 * h;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) a[i] = __shfl(a[i], src);
-    pm = __shfl(pm, src);
-    // the reflector of column j (rows >= j): v = [x_jj - alpha; x_{j+1..}]
-    double vj[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) vj[i] = __shfl(a[i], j + 32 * h);
-    double xloc = 0;
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-      if (16 * h + i == j) xloc = vj[i];
-    const double xjj = __shfl(xloc, c + 32 * (j >> 4));  // row j lives in half j / 16
-    const double nrm = sqrt(best);
-    const double alpha = xjj >= 0 ? -nrm : nrm;
-    const double v0 = xjj - alpha;
-    const double vv = best - xjj * xjj + v0 * v0;
-    const double beta = (nrm == 0.0 || vv == 0.0) ? 0.0 : 2.0 / vv;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int row = 16 * h + i;
-      vj[i] = row > j ? vj[i] : (row == j ? v0 : 0.0);
-    }
-    double dot = 0;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) dot += vj[i] * a[i];
-    dot += __shfl_xor(dot, 32);
-    if (c > j && c < N && beta != 0.0) {
-      const double f = beta * dot;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) a[i] -= f * vj[i];
-    }
-    if (c == j && beta != 0.0) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
-        if (16 * h + i == j) a[i] = alpha;
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 16; ++i)
-    if (c < N && 16 * h + i < M) A[16 * h + i + M * c] = a[i];
-  if (h == 0 && c < N) perm[c] = pm;
-}
-
-// One-sided Jacobi SVD of A (M x N column-major in LDS, N <= M <= 32) by one
-// wave with both matrices in registers: lane (c, h) = (l % 32, l / 32) holds
-// rows [16 h, 16 h + 16) of column c of A and of V.  A step fetches the
-// partner column of the round-robin schedule (rr_pair's) with lane shuffles,
-// joins the two halves' sums with one cross-half shuffle, and both lanes of a
-// pair derive the same rotation; the rotation threshold, the rounding floor and
-// the stopping rule are those of jacobi_svd.  A step needs no LDS and no
-// barrier (jacobi_svd's steps are LDS round trips with a workgroup barrier
-// each, ~1.3 us).  Writes A <- U diag(s) and, with WANT_V, V (N x N) back;
-// returns the number of sweeps.  Every lane of the wave must call it.
-template <bool WANT_V>
-__device__ int wave_jacobi_svd32(double* A, int M, int N, double* V) {
-  const int l = threadIdx.x & 63, c = l & 31, h = l >> 5;
-  double a[16], v[16];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int row = 16 * h + i;
-    a[i] = (c < N && row < M) ? A[row + M * c] : 0.0;
-    v[i] = (c < N && row == c) ? 1.0 : 0.0;
-  }
-  double fro = 0;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) fro += a[i] * a[i];
-  fro = wave_sum_d(fro);
-  const int ne = N + (N & 1);
-  const double tol = 8 * 2.220446049250313e-16 * sqrt((double)M);
-  const double floor2 = 2.220446049250313e-16 * 2.220446049250313e-16 * fro;
-  int sweep = 0;
-  for (; sweep < 60 && N > 1; ++sweep) {
-    bool rotated = false;
-    for (int st = 0; st < ne - 1; ++st) {
-      // partner of column c in step st (the inverse of rr_pair's placement)
-      int q = c;
-      if (c < ne) {
-        int t = c - 1 - st;
-        if (t < 0) t += ne - 1;
-        const int pos = c == 0 ? 0 : 1 + t;
-        const int pp = ne - 1 - pos;
-        int u = pp - 1 + st;
-        if (u >= ne - 1) u -= ne - 1;
-        q = pp == 0 ? 0 : 1 + u;
-      }
-      const int src = q + 32 * h;
-      double b[16];
-      double own = 0, oth = 0, cr = 0;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        b[i] = __shfl(a[i], src);
-        own += a[i] * a[i];
-        oth += b[i] * b[i];
-        cr += a[i] * b[i];
-      }
-      own += __shfl_xor(own, 32);
-      oth += __shfl_xor(oth, 32);
-      cr += __shfl_xor(cr, 32);
-      const bool isp = c < q;  // this lane holds the pair's first column
-      const double alpha = isp ? own : oth, beta = isp ? oth : own;
-      // first column: c a_p - s a_q; second: s a_p + c a_q (the partner is the
-      // other); a lane that does not rotate keeps c = 1, s = 0 (exact)
-      double cs = 1.0, sn = 0.0;
-      if (c < N && q < N && c != q && alpha > floor2 && beta > floor2 && fabs(cr) > tol * sqrt(alpha * beta)) {
-        const double zeta = (beta - alpha) / (2 * cr);
-        const double t = (zeta >= 0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1 + zeta * zeta));
-        cs = 1 / sqrt(1 + t * t);
-        sn = cs * t;
-        rotated = true;
-      }
-      const double sp = isp ? -sn : sn;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) a[i] = cs * a[i] + sp * b[i];
-      if (WANT_V) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const double wi = __shfl(v[i], src);
-          v[i] = cs * v[i] + sp * wi;
-        }
-      }
-    }
-    if (__ballot(rotated) == 0) break;
-  }
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int row = 16 * h + i;
-    if (c < N && row < M) A[row + M * c] = a[i];
-    if (WANT_V && c < N && row < N) V[row + N * c] = v[i];
-  }
-  return sweep + 1;
-}
-
-// out[e + E j] = sum_c X[e + E c] W[c + n j] for j < m (n <= 64), W (n x m,
-// ld n) in LDS, on the FP64 matrix cores: wave w takes the 16-row blocks
-// w, w + 4, ..; a block's A operands (A[i][k] = X[e0 + i][4 s + k], lane
-// i + 16 k, one register per step s) are loaded once and reused for every
-// 16-column tile of the output (B[k][j] = W[4 s + k][16 t + j]); rows, columns
-// and steps past E, m and n read as zero.  D[4 v + l / 16][l % 16] is value v
-// of lane l.
-__device__ void rows_times(const double* X, long long E, int n, const double* W, int m, double* out) {
-  const int l = threadIdx.x & 63, wv = threadIdx.x >> 6, li = l & 15, lk = l >> 4;
-  const int nsteps = (n + 3) >> 2;  // <= 16
-  for (long long e0 = 16LL * wv; e0 < E; e0 += 64) {
-    double av[16];
-#pragma unroll
-    for (int s = 0; s < 16; ++s) {
-      const int c = 4 * s + lk;
-      av[s] = (s < nsteps && c < n && e0 + li < E) ? X[e0 + li + E * c] : 0.0;
-    }
-    for (int t0 = 0; t0 < m; t0 += 16) {
+    for (int q = 0; q < 4; ++q) {
       f64x4 acc = {0, 0, 0, 0};
-      const int j = t0 + li;
-#pragma unroll
-      for (int s = 0; s < 16; ++s) {
-        if (s < nsteps) {
-          const int c = 4 * s + lk;
-          const double bv = (c < n && j < m) ? W[c + n * j] : 0.0;
-          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[s], bv, acc, 0, 0, 0);
-        }
-      }
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const long long e = e0 + 4 * v + lk;
-        if (e < E && j < m) out[e + E * j] = acc[v];
-      }
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, x0[q], acc, 0, 0, 0);
+      if (chi > 4) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, x1[q], acc, 0, 0, 0);
+      if (base[q] >= 0 && lk < chi) X[base[q] + st * lk] = acc[0];
+      if (base[q] >= 0 && 4 + lk < chi) X[base[q] + st * (4 + lk)] = acc[1];
     }
   }
   __syncthreads();
 }
 
-// The side matrices (E n <= AP_XY) and every small matrix in LDS, the
-// Householder reflectors of each side saved to `work` (2 AP_SIDE doubles per
-// gate).
-__global__ __launch_bounds__(256) void k_apply_gates(const ApplyItem* __restrict__ items,
-                                                     const VDesc* __restrict__ vds,
-                                                     double* __restrict__ psi,
-                                                     const double* __restrict__ msg,
-                                                     const double* __restrict__ gates, ApplyParams prm,
-                                                     double* __restrict__ work,
-                                                     double* __restrict__ truncerr,
-                                                     double* __restrict__ svals, int* __restrict__ kept,
-                                                     int* __restrict__ status) {
-  constexpr int TH = AP_TH;             // rows/cols of Theta
-  constexpr int RS = AP_ENV * AP_ENV;   // one environment root
-  extern __shared__ __align__(16) double sm[];
-  double* X = sm;               // AP_XY: QR, then SVD workspace
-  double* Y = X + AP_XY;        // AP_XY: mode-product partner, rebuild
-  double* Ru = Y + AP_XY;       // 1024: R_u (r x n), then the left factor
-  double* Rv = Ru + 1024;       // 1024: R_v, then the right factor
-  double* roots = Rv + 1024;    // 2 sides x AP_MAXEXT x (sqrt, inv sqrt) x AP_ENV^2
-  double* small = roots + 2 * AP_MAXEXT * 2 * RS;
-  double* A = X;                // Theta, then U diag(s)
-  double* VV = X + 1024;        // V of the SVD
-  double* scr_u = work + (long long)blockIdx.x * 2 * AP_SIDE;
-  double* scr_v = scr_u + AP_SIDE;
-  double* rot = small;
-  double* vh = rot + 4 * 32;
-  double* beta = vh + AP_N_BIG;
-  double* vhv = beta + AP_N_BIG;
-  double* betav = vhv + AP_N_BIG;
-  double* svec = betav + AP_N_BIG;
-  double* red = svec + TH;
-  __shared__ int sh_keep;
-  __shared__ int order[TH];
-  __shared__ int qgemm[2];  // side rebuilt as X R^{-1} F
-
-  const ApplyItem it = items[blockIdx.x];
-  const int tid = threadIdx.x;
-  // the factorisation runs on the bond as it was (columns b < chib_in); a bond
-  // grown for the kept rank only widens the layout the result is written to
-  // both sides' geometry in LDS: its arrays are indexed at run time, which
-  // would put a per-thread copy in scratch memory
-  __shared__ SideGeom sgeo[2];
-  if (tid < 2) {
-    SideGeom g = side_geom(vds[tid == 0 ? it.u : it.v], tid == 0 ? it.ju : it.jv);
-    g.chib = it.chib_in;
-    g.n = g.d * g.chib;
-    g.r = g.E < g.n ? g.E : g.n;
-    sgeo[tid] = g;
+// Gram matrix of X (NEXT: of X Tn, Tn[c][k] = Mi[k][c], which STORE writes over X) by
+// the workgroup; the element (ti + 16 a, tj + 16 b) of chol_eliminate's thread to
+// g.  sum: NT (NT + 1) / 2 tiles of 256.
+template <int NT, bool NEXT>
+__device__ void ap_gram(const ApSide& g, double* X, int P, const CholLds<NT>& L, bool store, double* sum,
+                        double (&out)[NT][NT]) {
+  constexpr int LD = CholLds<NT>::LD, NTILE = NT * (NT + 1) / 2;
+  const int tid = threadIdx.x, l = tid & 63, wv = tid >> 6, li = l & 15, lk = l >> 4;
+  const int E = g.E, n = g.n;
+  f64x4 acc[NTILE];
+#pragma unroll
+  for (int t = 0; t < NTILE; ++t) acc[t] = f64x4{0, 0, 0, 0};
+  double tn[NT][4 * NT];
+  if constexpr (NEXT) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int q = 0; q < 4 * NT; ++q) {
+        const int c = 4 * q + lk, k = 16 * t + li;
+        tn[t][q] = c < n && k < n ? L.Mi[k * LD + c] : 0.0;
+      }
+  }
+  for (int r0 = 16 * wv; r0 < E; r0 += 64) {
+    f64x4 x1[NT];
+    if constexpr (NEXT) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) x1[t] = f64x4{0, 0, 0, 0};
+#pragma unroll
+      for (int q = 0; q < 4 * NT; ++q) {
+        const double a = r0 + li < E && 4 * q + lk < n ? X[(4 * q + lk) * P + r0 + li] : 0.0;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) x1[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, tn[t][q], x1[t], 0, 0, 0);
+      }
+      if (store)  // a wave reads and writes its own rows
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            if (16 * t + li < n && r0 + 4 * v + lk < E) X[(16 * t + li) * P + r0 + 4 * v + lk] = x1[t][v];
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      double op[NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        op[t] = NEXT ? x1[t][v]
+                     : (16 * t + li < n && r0 + 4 * v + lk < E ? X[(16 * t + li) * P + r0 + 4 * v + lk] : 0.0);
+      int k = 0;
+#pragma unroll
+      for (int a = 0; a < NT; ++a)
+#pragma unroll
+        for (int b = a; b < NT; ++b, ++k)
+          acc[k] = __builtin_amdgcn_mfma_f64_16x16x4f64(op[a], op[b], acc[k], 0, 0, 0);
+    }
+  }
+  for (int q = 0; q < 4; ++q) {  // the four waves' tiles, summed in wave order
+    __syncthreads();
+    if (wv == q)
+#pragma unroll
+      for (int k = 0; k < NTILE; ++k)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          double* p = sum + k * 256 + v * 64 + l;
+          *p = (q == 0 ? 0.0 : *p) + acc[k][v];
+        }
   }
   __syncthreads();
-  const SideGeom& gu = sgeo[0];
-  const SideGeom& gv = sgeo[1];
-  phase_mark(prm, 0);
+  const int ti = tid & 15, tj = tid >> 4;
+#pragma unroll
+  for (int a = 0; a < NT; ++a)
+#pragma unroll
+    for (int b = 0; b < NT; ++b) {
+      // tile (a, b), a <= b, row i, column j: value i / 4 of lane 16 (i % 4) + j
+      const int ta = a < b ? a : b, tb = a < b ? b : a, i = a <= b ? ti : tj, j = a <= b ? tj : ti;
+      out[a][b] = sum[(ta * NT - ta * (ta - 1) / 2 + tb - ta) * 256 + (i >> 2) * 64 + (i & 3) * 16 + j];
+    }
+}
 
-  // 1. environment roots (sqrt and inverse sqrt), both sides, one environment per wave
-  {
-    const int wv = tid >> 6;
-    for (int q = wv; q < gu.next + gv.next; q += (int)blockDim.x / 64) {
-      const int side = q < gu.next ? 0 : 1;
-      const int pa = side == 0 ? q : q - gu.next;
-      const SideGeom& g = side == 0 ? gu : gv;
-      const VDesc& V = vds[side == 0 ? it.u : it.v];
-      const int a = g.ext[pa];
-      double* S = roots + ((side * AP_MAXEXT + pa) * 2) * RS;
-      env_roots_wave(msg + V.in_msg[a], g.dims[a], prm.eig_cutoff, S, S + RS);
-    }
-    __syncthreads();
+// One pass of the side's QR: R <- R_p R, the next T or (true) the final Tq.
+template <int NT, int PASS>
+__device__ bool ap_qr_pass(const ApSide& g, double* X, int P, const CholLds<NT>& L, double* T, double* R,
+                           double* Tq, bool& expl) {
+  constexpr int LD = CholLds<NT>::LD;
+  const int tid = threadIdx.x, n = g.n;
+  double a[NT][NT];
+  ap_gram<NT, (PASS > 0)>(g, X, P, L, expl, L.U, a);  // U is free here, Mi holds the last T
+  const bool fin = chol_pass<NT, PASS>(a, n, expl, L);
+  double t[NT * NT];
+#pragma unroll
+  for (int q = 0; q < NT * NT; ++q) {
+    const int i = tid + 256 * q, k = i % n, c = i / n;
+    t[q] = 0;
+    if (i >= n * n) continue;
+    if (PASS == 0)
+      t[q] = L.U[k * LD + c];
+    else
+      for (int j = k; j < n; ++j) t[q] += L.U[k * LD + j] * R[j + n * c];
   }
-  phase_mark(prm, 1);
-  // 2. X = psi with sqrt(env) on the external bonds, QR; reflectors to scratch
-  for (int side = 0; side < 2; ++side) {
-    const SideGeom& g = side == 0 ? gu : gv;
-    for (int idx = tid; idx < g.E * g.n; idx += blockDim.x) {
-      const int c = (int)g.fE.div(idx), e = idx - c * g.E;
-      const int b = (int)g.fd.div(c), s = c - b * g.d;
-      X[idx] = psi[g.psi_off + nat_off(g, s, e, b)];
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < NT * NT; ++q)
+    if (tid + 256 * q < n * n) R[tid + 256 * q] = t[q];
+  if (fin)
+    for (int i = tid; i < n * n; i += 256) {
+      const int c = i % n, k = i / n;
+      double x = 0;
+      if (expl)
+        x = L.Mi[k * LD + c];
+      else
+        for (int j = 0; j <= k; ++j) x += T[c + n * j] * L.Mi[k * LD + j];
+      Tq[i] = x;
     }
-    __syncthreads();
-    if (side == 0) phase_mark(prm, 10);
-    double* cur = X;
-    double* oth = Y;
-    for (int pa = 0; pa < g.next; ++pa) {
-      const double* S = roots + ((side * AP_MAXEXT + pa) * 2) * RS;
-      ext_mode_product<AP_ENV>(g, pa, cur, oth, g.n, S, false);
-      double* t = cur;
-      cur = oth;
-      oth = t;
-    }
-    if (cur != X) {
-      for (int i = tid; i < g.E * g.n; i += blockDim.x) X[i] = cur[i];
-      __syncthreads();
-    }
-    double* vhs = side == 0 ? vh : vhv;
-    double* bts = side == 0 ? beta : betav;
-    double* R = side == 0 ? Ru : Rv;
-    double* scr = side == 0 ? scr_u : scr_v;
-    // X itself, for a rebuild by Q = X R^{-1} (kept if the side qualifies)
-    for (int i = tid; i < g.E * g.n; i += blockDim.x) scr[i] = X[i];
-    __syncthreads();
-    if (side == 0) phase_mark(prm, 11);
-    if (tsqr_ok(g)) {
-      // the stacked R factors S (4n x n) in Y, which is free after the copy to X
-      const int n4 = 4 * g.n, wv = tid >> 6;
-      double* S = Y;
-      if (wv < 4) {
-        const int r0 = wv * g.E / 4, r1 = (wv + 1) * g.E / 4;
-        wave_qr16(X + r0, g.E, r1 - r0, g.n, vhs + wv * g.n, bts + wv * g.n);
-        for (int idx = (tid & 63); idx < g.n * g.n; idx += 64) {
-          const int i = idx % g.n, c = idx / g.n;
-          S[wv * g.n + i + n4 * c] = (i <= c) ? X[r0 + i + (long long)g.E * c] : 0.0;
-        }
-      }
-      __syncthreads();
-      double* qx = scr + AP_XY;  // S's reflectors, then their heads and betas
-      if (wv == 0) wave_qr16(S, n4, n4, g.n, qx + n4 * g.n, qx + n4 * g.n + 16);
-      __syncthreads();
-      for (int idx = tid; idx < g.r * g.n; idx += blockDim.x) {
-        const int i = idx % g.r, c = idx / g.r;
-        R[i + g.r * c] = (i <= c) ? S[i + n4 * c] : 0.0;
-      }
-      for (int i = tid; i < n4 * g.n; i += blockDim.x) qx[i] = S[i];
-    } else {
-      householder_qr(X, g.E, g.n, vhs, bts, red);
-      for (int idx = tid; idx < g.r * g.n; idx += blockDim.x) {
-        const int i = idx % g.r, c = idx / g.r;
-        R[i + g.r * c] = (i <= c) ? X[i + (long long)g.E * c] : 0.0;  // R[i][c], column-major (ld r)
-      }
-    }
-    if (side == 0) phase_mark(prm, 12);
-    // a tall side whose R has no diagonal entry below 1e-5 of its largest
-    // keeps X and R: the rebuild's Q [F; 0] is then X (R^{-1} F), one small
-    // product, instead of applying the n reflectors (latency-bound), with an
-    // orthogonality error ~eps cond(X); other sides keep their reflectors
-    __syncthreads();  // R is complete
-    if (tid == 0) {
-      bool ok = g.E >= g.n;
-      double dmax = 0, dmin = INFINITY;
-      for (int j = 0; j < g.n && ok; ++j) {
-        const double dj = fabs(R[j + g.r * j]);
-        dmax = dj > dmax ? dj : dmax;
-        dmin = dj < dmin ? dj : dmin;
-      }
-      qgemm[side] = ok && dmax > 0 && isfinite(dmax) && dmin >= 1e-5 * dmax;
-    }
-    __syncthreads();
-    if (qgemm[side]) {
-      for (int i = tid; i < g.n * g.n; i += blockDim.x) scr[AP_XY + i] = R[i];  // ld n (r = n)
-    } else {
-      for (int i = tid; i < g.E * g.n; i += blockDim.x) scr[i] = X[i];  // the reflectors
-    }
-    __syncthreads();
-    if (side == 0) phase_mark(prm, 13);
+  else if (PASS == 0)
+    for (int i = tid; i < n * n; i += 256) T[i] = L.Mi[(i / n) * LD + i % n];
+  __syncthreads();
+  return fin;
+}
+
+// Everything of a gate that concerns one side before Theta: the environments' roots
+// (one wave each), X = psi with sqrt(M) on the external bonds, X = Q R by Gram
+// matrices (chol_pass), all in LDS.  A wide side (E <= n) has R = X, Q = 1.
+//
+// Bound: latency of one workgroup's chain.  At chi = 8 (E = 512, n = 16): load and
+// roots 32 us, mode products 10, QR 19.  With Householder reflectors the products
+// and the QR took 140 to 150 us per side: every column a pass over X with
+// barriers, against two passes over X on the matrix cores in all.
+template <int NT>
+__global__ __launch_bounds__(256) void k_gate_side(const ApplyItem* __restrict__ items,
+                                                   const VDesc* __restrict__ vds, const double* __restrict__ psi,
+                                                   const double* __restrict__ msg, ApplyParams prm, int xsize,
+                                                   double* __restrict__ work) {
+  constexpr int RS = AP_ENV * AP_ENV;
+  extern __shared__ __align__(16) double sm[];
+  double* X = sm;
+  double* S = X + xsize;  // sqrt(M) per external bond
+  const CholLds<NT> L(S + AP_MAXEXT * RS);
+  double* T = S + AP_MAXEXT * RS + CholLds<NT>::bytes() / sizeof(double);
+  double* R = T + 256 * NT * NT;
+  __shared__ ApSide g;
+  __shared__ int flags;
+  const int side = blockIdx.x & 1, gate = blockIdx.x >> 1, tid = threadIdx.x, wv = tid >> 6;
+  const ApplyItem& it = items[gate];
+  const VDesc& V = vds[side == 0 ? it.u : it.v];
+  double* wk = work + (long long)blockIdx.x * AP_SIDE;
+  if (side == 0) phase_mark(prm, gate, 0);
+  if (tid == 0) {
+    ap_side(V, side == 0 ? it.ju : it.jv, it.chib_in, g);
+    flags = 0;
   }
-  phase_mark(prm, 2);
-  // 3. Theta[(ru, su'), (rv, sv')] = sum G[(su',sv'),(su,sv)] Ru[ru, su + du b] Rv[rv, sv + dv b],
-  //    stored directly in the taller orientation (X: M x N column-major), V in X + 1024
-  const int du = gu.d, dv = gv.d, chib = gu.chib;
+  __syncthreads();
+  const int P = ap_pitch(g.E);
+  ap_load(g, psi + g.psi_off, X, P);
+  if (wv < g.next) {
+    // external bond wv is axis wv + 1, or wv + 2 past the gate's bond
+    const int j = side == 0 ? it.ju : it.jv, a = wv + 1 < j ? wv + 1 : wv + 2;
+    double* Si = wk + AP_W_SI + wv * 2 * RS;
+    const bool cut = env_roots_wave(msg + V.in_msg[a], g.chi[wv], prm.eig_cutoff, S + wv * RS, Si, Si + RS);
+    if (cut && (tid & 63) == 0) atomicOr(&flags, 1 << wv);
+  }
+  __syncthreads();
+  if (side == 0) phase_mark(prm, gate, 1);
+  for (int pa = 0; pa < g.next; ++pa) ap_mode(g, pa, X, P, g.n, S + pa * RS);
+  if (side == 0) phase_mark(prm, gate, 2);
+  double* Rg = wk + AP_W_R;
+  bool expl = false;
+  if (g.E <= g.n) {
+    for (int i = tid; i < g.E * g.n; i += 256) {
+      const int c = (int)g.fE.div(i);
+      Rg[i] = X[c * P + i - c * g.E];
+    }
+  } else {
+    double* Tq = wk + AP_W_TQ;
+    if (!ap_qr_pass<NT, 0>(g, X, P, L, T, R, Tq, expl) && !ap_qr_pass<NT, 1>(g, X, P, L, T, R, Tq, expl) &&
+        !ap_qr_pass<NT, 2>(g, X, P, L, T, R, Tq, expl))
+      ap_qr_pass<NT, 3>(g, X, P, L, T, R, Tq, expl);
+    for (int i = tid; i < g.n * g.n; i += 256) Rg[i] = R[i];
+    if (expl)
+      for (int i = tid; i < g.E * g.n; i += 256) {
+        const int c = (int)g.fE.div(i);
+        wk[i] = X[c * P + i - c * g.E];
+      }
+  }
+  if (tid == 0) reinterpret_cast<int*>(wk + AP_W_FLAG)[0] = flags | (expl ? 8 : 0);
+  if (side == 0) phase_mark(prm, gate, 3);
+}
+
+// psi' of one side in X (first d keep columns) from W: psi or Q through LDS, the
+// projectors or M^{-1/2}, then X <- X W per 16 rows on the matrix cores
+template <int NT>
+__device__ void ap_rebuild(const ApSide& g, const double* wk, const double* psi, const double* W, int cols,
+                           double* X, int P) {
+  const int tid = threadIdx.x, l = tid & 63, wv = tid >> 6, li = l & 15, lk = l >> 4;
+  const int flags = reinterpret_cast<const int*>(wk + AP_W_FLAG)[0], E = g.E, n = g.n;
+  const bool expl = flags & 8;
+  if (expl) {
+    for (int i = tid; i < E * n; i += 256) {
+      const int c = (int)g.fE.div(i);
+      X[c * P + i - c * E] = wk[i];
+    }
+  } else
+    ap_load(g, psi + g.psi_off, X, P);
+  __syncthreads();
+  for (int pa = 0; pa < g.next; ++pa)
+    if (expl || (flags >> pa & 1))
+      ap_mode(g, pa, X, P, n, wk + AP_W_SI + (2 * pa + (expl ? 0 : 1)) * AP_ENV * AP_ENV);
+  for (int r0 = 16 * wv; r0 < E; r0 += 64) {
+    double av[4 * NT];
+#pragma unroll
+    for (int q = 0; q < 4 * NT; ++q)
+      av[q] = r0 + li < E && 4 * q + lk < n ? X[(4 * q + lk) * P + r0 + li] : 0.0;
+    for (int t = 0; 16 * t < cols; ++t) {
+      f64x4 acc = {0, 0, 0, 0};
+      const int col = 16 * t + li;
+#pragma unroll
+      for (int q = 0; q < 4 * NT; ++q) {
+        const double b = col < cols && 4 * q + lk < n ? W[4 * q + lk + n * col] : 0.0;
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[q], b, acc, 0, 0, 0);
+      }
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        if (col < cols && r0 + 4 * v + lk < E) X[col * P + r0 + 4 * v + lk] = acc[v];
+    }
+  }
+  __syncthreads();
+}
+
+// Theta, its SVD (gate_svd) and both sides of the bond rebuilt, one workgroup per
+// gate: psi' = (psi P) Tq F, where M^{-1/2} is never applied (X = psi sqrt(M), and
+// sqrt(M) M^{-1/2} = P, which is 1 unless eigenvalues were dropped); an explicit side
+// takes M^{-1/2} Q F, a wide one M^{-1/2} F.  Every write to psi comes after the SVD,
+// so a refused gate leaves its bond alone.
+//
+// Bound: latency, most of it the SVD's chain of Jacobi steps.  At chi = 8: Theta 15
+// us, SVD 135 (261 on one wave), factors 5, rebuilds 22 and 17 (86 and 72 by back
+// substitution and VALU products).
+template <int NT>
+__global__ __launch_bounds__(256) void k_gate_pair(const ApplyItem* __restrict__ items,
+                                                   const VDesc* __restrict__ vds, double* __restrict__ psi,
+                                                   const double* __restrict__ gates, ApplyParams prm, int wsize,
+                                                   const double* __restrict__ work, double* __restrict__ truncerr,
+                                                   double* __restrict__ svals, int* __restrict__ kept,
+                                                   int* __restrict__ status) {
+  constexpr int LD = SvdLds<AP_TH>::LD;
+  extern __shared__ __align__(16) double sm[];
+  double* Wl = sm;                // W of both sides, wsize each
+  double* body = sm + 2 * wsize;  // the SVD's buffers, then a side's columns
+  const SvdLds<AP_TH> L(body);
+  double* Ru = body + SvdLds<AP_TH>::bytes() / sizeof(double);  // R_u, then Theta
+  double* Rv = Ru + 1024;                                       // R_v, then V
+  double* F = Rv + 1024;                                        // Theta V / sqrt(S)
+  __shared__ ApSide gs[2];
+  __shared__ double red[4], sgn[AP_TH];
+  const int gate = blockIdx.x, tid = threadIdx.x, l = tid & 63, wv = tid >> 6, li = l & 15, lk = l >> 4;
+  const ApplyItem& it = items[gate];
+  const double* wk = work + (long long)gate * 2 * AP_SIDE;
+  phase_mark(prm, gate, 4);
+  if (tid == 0 || tid == 64)
+    ap_side(vds[tid == 0 ? it.u : it.v], tid == 0 ? it.ju : it.jv, it.chib_in, gs[tid >> 6]);
+  __syncthreads();
+  const ApSide& gu = gs[0];
+  const ApSide& gv = gs[1];
+  for (int i = tid; i < gu.r * gu.n; i += 256) Ru[i] = wk[AP_W_R + i];
+  for (int i = tid; i < gv.r * gv.n; i += 256) Rv[i] = wk[AP_SIDE + AP_W_R + i];
+  __syncthreads();
+  // Theta[(ru, su'), (rv, sv')] = sum G[(su',sv'),(su,sv)] Ru[ru, su + du b] Rv[rv, sv + dv b],
+  // in the taller orientation: thread (c, h) = (tid / 8, tid % 8) has rows h + 8 i of column c
+  const int du = gu.d, dv = gv.d, chib = gu.chib, dd = du * dv;
   const int Mr = gu.r * du, Nc = gv.r * dv;
-  const int dd = du * dv;
   const double* G = gates + it.gate;
   const bool tr = Mr < Nc;
   const int M = tr ? Nc : Mr, N = tr ? Mr : Nc;
-  for (int idx = tid; idx < Mr * Nc; idx += blockDim.x) {
-    const int row = idx % Mr, col = idx / Mr;
-    const int ru = row % gu.r, sup = row / gu.r;
-    const int rv = col % gv.r, svp = col / gv.r;
+  double th[AP_TH / 8], x[AP_TH / 8];
+#pragma unroll
+  for (int i = 0; i < AP_TH / 8; ++i) {
+    const int m = (tid & 7) + 8 * i, c = tid >> 3;
     double acc = 0;
-    for (int su = 0; su < du; ++su)
-      for (int sv = 0; sv < dv; ++sv) {
-        const double gval = G[(sup + du * svp) + dd * (su + du * sv)];
-        if (gval == 0.0) continue;
-        double rr = 0;
-        for (int b = 0; b < chib; ++b) rr += Ru[ru + gu.r * (su + du * b)] * Rv[rv + gv.r * (sv + dv * b)];
-        acc += gval * rr;
-      }
-    if (tr) A[col + Nc * row] = acc;
-    else A[idx] = acc;
-  }
-  __syncthreads();
-  phase_mark(prm, 3);
-  // 4. SVD
-  // QR-preconditioned one-sided Jacobi, one wave (Theta is at most 32 x 32):
-  // Theta P = Q R by a pivoted Householder QR, then Jacobi on X = R^T in
-  // registers, X <- U_x diag(s) (R^T = U_x S V_x^T, so Theta = (Q V_x) S (P U_x)^T):
-  // V_Theta = P U_x, and the kept U_Theta s = Theta V_Theta from a copy of
-  // Theta, so neither Q nor V_x is formed.  The pivoting grades X's columns and
-  // halves the sweeps (7 instead of 13-14 on a config-2 Theta).
-  int nsweeps = 0;
-  double* Th0 = A + 2048;  // a copy of Theta, then X = R^T at Th0 + 1024
-  double* Xr = Th0 + 1024;
-  __shared__ int perm[TH];
-  for (int i = tid; i < M * N; i += blockDim.x) Th0[i] = A[i];
-  __syncthreads();
-  if (tid < 64) wave_qrcp32(A, M, N, perm);
-  __syncthreads();
-  for (int i = tid; i < N * N; i += blockDim.x) {
-    const int row = i % N, col = i / N;
-    Xr[i] = col <= row ? A[col + M * row] : 0.0;  // X[row][col] = R[col][row]
-  }
-  __syncthreads();
-  if (tid < 64) nsweeps = wave_jacobi_svd32<false>(Xr, N, N, nullptr);
-  __syncthreads();
-  if (prm.ts && tid == 0) {
-    prm.ts[blockIdx.x * 16 + 8] = (unsigned long long)nsweeps;
-    prm.ts[blockIdx.x * 16 + 9] = (unsigned long long)(tsqr_ok(gu) + tsqr_ok(gv));
-  }
-  for (int j = tid; j < N; j += blockDim.x) {
-    double s = 0;
-    for (int i = 0; i < N; ++i) s += Xr[i + N * j] * Xr[i + N * j];
-    svec[j] = sqrt(s);
-  }
-  __syncthreads();
-  if (tid == 0) {
-    for (int i = 0; i < N; ++i) order[i] = i;
-    for (int i = 0; i < N; ++i)
-      for (int j = i + 1; j < N; ++j)
-        if (svec[order[j]] > svec[order[i]]) {
-          int t = order[i];
-          order[i] = order[j];
-          order[j] = t;
+    if (m < M && c < N) {
+      const int row = tr ? c : m, col = tr ? m : c;
+      const int sup = row / gu.r, a = row - sup * gu.r, svp = col / gv.r, b = col - svp * gv.r;
+      for (int su = 0; su < du; ++su)
+        for (int sv = 0; sv < dv; ++sv) {
+          const double gval = G[(sup + du * svp) + dd * (su + du * sv)];
+          if (gval == 0.0) continue;
+          double rr = 0;
+          for (int k = 0; k < chib; ++k) rr += Ru[a + gu.r * (su + du * k)] * Rv[b + gv.r * (sv + dv * k)];
+          acc += gval * rr;
         }
-    double tot = 0;
-    for (int i = 0; i < N; ++i) tot += svec[i] * svec[i];
-    int keep = N;
-    if (prm.maxdim > 0 && keep > prm.maxdim) keep = prm.maxdim;
-    double disc = 0;
-    for (int i = keep; i < N; ++i) disc += svec[order[i]] * svec[order[i]];
-    if (prm.cutoff >= 0 && tot > 0) {
-      while (keep > 1 && (disc + svec[order[keep - 1]] * svec[order[keep - 1]]) / tot <= prm.cutoff) {
-        disc += svec[order[keep - 1]] * svec[order[keep - 1]];
-        --keep;
-      }
     }
-    int st = 0;
-    if (keep > gu.dims[gu.j]) st = 1;  // more than the bond's layout holds
-    if (!isfinite(tot)) st = 2;  // non-finite Theta (a NaN or Inf in psi or the environment)
-    truncerr[it.slot] = tot > 0 ? disc / tot : (st == 2 ? tot : 0.0);
-    if (svals)
-      for (int i = 0; i < prm.max_keep; ++i)
-        svals[(long long)it.slot * prm.max_keep + i] = i < keep && i < N ? svec[order[i]] : 0.0;
-    if (kept) kept[it.slot] = keep;
-    status[it.slot] = st;
-    sh_keep = st ? -1 : keep;
+    th[i] = x[i] = acc;
   }
-  __syncthreads();
-  phase_mark(prm, 4);
-  const int keep = sh_keep;
-  // a bond whose kept rank exceeds its dimension, or whose Theta is not
-  // finite, is left untouched (the host reports the error); every write to psi
-  // comes after this point
+  phase_mark(prm, gate, 5);
+  const int keep = gate_svd<AP_TH>(x, M, N, L, prm, gu.lay, it.slot, truncerr, svals, kept, status);
+  phase_mark(prm, gate, 6);
   if (keep < 0) return;
-  // the kept singular vectors: V_o = P U_x,o = P X_o / s_o, then
-  // A_o = U_o s_o = Theta V_o (a zero singular value gets zero columns, which
-  // its sqrt(s) = 0 factor multiplies anyway)
-  for (int idx = tid; idx < N * keep; idx += blockDim.x) {
-    const int i = idx % N, o = order[idx / N];
-    const double so = svec[o];
-    VV[perm[i] + N * o] = so > 0 ? Xr[i + N * o] / so : 0.0;
+  double* Th = Ru;
+  double* Vt = Rv;
+#pragma unroll
+  for (int i = 0; i < AP_TH / 8; ++i) {
+    const int m = (tid & 7) + 8 * i, c = tid >> 3;
+    if (m < M && c < N) Th[m + M * c] = th[i];
+  }
+  for (int i = tid; i < N * keep; i += 256) {
+    const int row = i % N, k = i / N;
+    Vt[L.perm[row] + N * k] = L.X[row + LD * L.order[k]];
   }
   __syncthreads();
-  for (int idx = tid; idx < M * keep; idx += blockDim.x) {
-    const int r = idx % M, o = order[idx / M];
-    double t = 0;
-    for (int i = 0; i < N; ++i) t += Th0[r + M * i] * VV[i + N * o];
-    A[r + M * o] = t;
-  }
-  __syncthreads();
-  // left factor Lf (Mr x keep) = U sqrt(S) into Ru, right factor Rf (Nc x keep) = V sqrt(S) into Rv;
-  // A = U diag(s) (M x N), V = VV (N x N); if transposed, Theta = VV S U^T
-  for (int idx = tid; idx < Mr * keep; idx += blockDim.x) {
-    const int i = idx % Mr, j = idx / Mr;
-    const int o = order[j];
-    const double sv = svec[o];
-    Ru[idx] = !tr ? (sv > 0 ? A[i + M * o] / sqrt(sv) : 0.0) : VV[i + N * o] * sqrt(sv);
-  }
-  for (int idx = tid; idx < Nc * keep; idx += blockDim.x) {
-    const int i = idx % Nc, j = idx / Nc;
-    const int o = order[j];
-    const double sv = svec[o];
-    Rv[idx] = !tr ? VV[i + N * o] * sqrt(sv) : (sv > 0 ? A[i + M * o] / sqrt(sv) : 0.0);
-  }
-  __syncthreads();
-  phase_mark(prm, 5);
-  // 5. rebuild both sides: Y = [F as r x (d keep); 0], apply Q, then M^{-1/2};
-  //    the largest-magnitude entry of every new-bond slice of psi_u' (first in
-  //    column-major order) is made positive and the same sign applied to psi_v'
-  __shared__ double bond_sign[TH];
-  for (int side = 0; side < 2; ++side) {
-    const SideGeom& g = side == 0 ? gu : gv;
-    const double* F = side == 0 ? Ru : Rv;  // rows (r_i, s), r fastest
-    const double* scr = side == 0 ? scr_u : scr_v;
-    const int cols = g.d * keep;  // column c' = s + d b'
-    if (qgemm[side]) {
-      // W = R^{-1} F (n x cols, back substitution per column) in LDS X, Y = X_side W
-      const double* Rg = scr + AP_XY;
-      for (int cc = tid; cc < cols; cc += blockDim.x) {
-        const int b = cc / g.d, s = cc - b * g.d;
-        for (int i = g.n - 1; i >= 0; --i) {
-          double t = F[(i + g.n * s) + (long long)(g.n * g.d) * b];
-          for (int k = i + 1; k < g.n; ++k) t -= Rg[i + g.n * k] * X[k + g.n * cc];
-          X[i + g.n * cc] = t / Rg[i + g.n * i];
-        }
+  // U sqrt(S) = Theta V / sqrt(S): 16 x 16 tiles, one per wave
+  {
+    const int r0 = 16 * (wv & 1), c0 = 16 * (wv >> 1);
+    if (r0 < M && c0 < keep) {
+      f64x4 acc = {0, 0, 0, 0};
+      for (int k0 = 0; k0 < N; k0 += 4) {
+        const int k = k0 + lk;
+        const double a = (r0 + li < M && k < N) ? Th[r0 + li + M * k] : 0.0;
+        const double b = (c0 + li < keep && k < N) ? Vt[k + N * (c0 + li)] : 0.0;
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
       }
-      __syncthreads();
-      rows_times(scr, g.E, g.n, X, cols, Y);
+      if (c0 + li < keep) {
+        const double s = L.svec[L.order[c0 + li]], sc = s > 0 ? 1 / sqrt(s) : 0.0;
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          if (r0 + 4 * v + lk < M) F[r0 + 4 * v + lk + M * (c0 + li)] = acc[v] * sc;
+      }
+    }
+  }
+  __syncthreads();  // the products above read V unscaled
+  for (int i = tid; i < N * keep; i += 256) Vt[i] *= sqrt(L.svec[L.order[i / N]]);
+  __syncthreads();
+  // W = Tq F (n x d keep; F as r x d keep); a wide side's W = F (E x d keep)
+  for (int sd = 0; sd < 2; ++sd) {
+    const ApSide& g = gs[sd];
+    const double* Fs = (sd == 0) == tr ? Vt : F;
+    const double* Tq = wk + sd * AP_SIDE + AP_W_TQ;
+    double* W = Wl + sd * wsize;
+    const int n = g.n, cols = g.d * keep;
+    if (g.E <= n) {
+      for (int i = tid; i < g.E * cols; i += 256) W[i] = Fs[i];
     } else {
-      // the side's reflectors, copied back into LDS
-      for (int i = tid; i < g.E * g.n; i += blockDim.x) X[i] = scr[i];
-      for (int idx = tid; idx < g.E * cols; idx += blockDim.x) {
-        const int c = (int)g.fE.div(idx), e = idx - c * g.E;
-        const int b = (int)g.fd.div(c), s = c - b * g.d;
-        Y[idx] = e < g.r ? F[(e + g.r * s) + (long long)(g.r * g.d) * b] : 0.0;
+      for (int i = tid; i < n * cols; i += 256) {
+        const int q = i % n, c = i / n;
+        double t = 0;
+#pragma unroll 4
+        for (int k = 0; k < n; ++k) t += Tq[q + n * k] * Fs[k + n * c];
+        W[i] = t;
+      }
+    }
+  }
+  __syncthreads();
+  phase_mark(prm, gate, 7);
+  double* X = body;
+  for (int sd = 0; sd < 2; ++sd) {
+    const ApSide& g = gs[sd];
+    const int P = ap_pitch(g.E), cols = g.d * keep, E = g.E;
+    const double* W = Wl + sd * wsize;
+    if (E <= g.n) {
+      for (int i = tid; i < E * cols; i += 256) {
+        const int c = (int)g.fE.div(i);
+        X[c * P + i - c * E] = W[i];
       }
       __syncthreads();
-      if (tsqr_ok(g)) {
-        // Q [F; 0] = diag(Q_w) P Q_S [F; 0]: Q_S on the stacked rows (block w's
-        // first n rows) by wave 0, then each block's reflectors by its wave
-        const int n4 = 4 * g.n, wv = tid >> 6, E = g.E, nn = g.n;
-        const double* qx = scr + AP_XY;
-        // stacked row i -> block i / nn, row i % nn (i / nn by a multiply-high: i nn < 2^16)
-        const unsigned inv = (65536u + nn - 1) / nn;
-        if (wv == 0)
-          wave_apply_q16(qx, n4, n4, nn, qx + n4 * nn, qx + n4 * nn + 16, Y, E, cols, [=](int i) {
-            const int w = (int)(((unsigned)i * inv) >> 16);
-            return w * E / 4 + (i - w * nn);
-          });
-        __syncthreads();
-        if (wv < 4) {
-          const int r0 = wv * E / 4, r1 = (wv + 1) * E / 4;
-          const double* vb = side == 0 ? vh : vhv;
-          const double* bb = side == 0 ? beta : betav;
-          wave_apply_q16(X + r0, E, r1 - r0, nn, vb + wv * nn, bb + wv * nn, Y + r0, E, cols, [](int i) { return i; });
-        }
-        __syncthreads();
-      } else {
-        apply_q(X, g.E, g.r, side == 0 ? vh : vhv, side == 0 ? beta : betav, Y, cols);
-      }
-    }
-    // M^{-1/2}: psi'[.. b ..] = sum_b' Y[.. b' ..] Si[b][b']
-    double* cur = Y;
-    double* oth = X;
-    for (int pa = 0; pa < g.next; ++pa) {
-      const double* Si = roots + ((side * AP_MAXEXT + pa) * 2 + 1) * RS;
-      ext_mode_product<AP_ENV>(g, pa, cur, oth, cols, Si, true);
-      double* t = cur;
-      cur = oth;
-      oth = t;
-    }
-    if (side == 0) {
-      // one wave per new-bond column: the largest |entry| (ties: the smallest
-      // natural offset, so the choice does not depend on the scan order)
-      const int wv = tid >> 6, l = tid & 63, nw = (int)(blockDim.x >> 6);
-      for (int j = wv; j < keep; j += nw) {
-        double best = -1;
-        int best_off = 0x7fffffff;
-        double val = 0;
-        for (int idx = l; idx < g.E * g.d; idx += 64) {
-          const int s2 = (int)g.fE.div(idx), e = idx - s2 * g.E;
-          const double x = cur[e + (long long)g.E * (s2 + g.d * j)];
-          const int off = nat_off(g, s2, e, j);
-          if (fabs(x) > best || (fabs(x) == best && off < best_off)) {
-            best = fabs(x);
-            best_off = off;
-            val = x;
+      for (int pa = 0; pa < g.next; ++pa)
+        ap_mode(g, pa, X, P, cols, wk + sd * AP_SIDE + AP_W_SI + 2 * pa * AP_ENV * AP_ENV);
+    } else
+      ap_rebuild<NT>(g, wk + sd * AP_SIDE, psi, W, cols, X, P);
+    // the largest |entry| of every new-bond slice of the first site becomes positive
+    // (ties: the smallest offset in the site tensor), the same sign on both; one wave
+    // per slice
+    if (sd == 0) {
+      for (int j = wv; j < keep; j += 4) {
+        double best = -1, val = 0;
+        int boff = 0x7fffffff;
+        for (int i = l; i < E * g.d; i += 64) {
+          const int s = (int)g.fE.div(i), e = i - s * E, hi = (int)g.flo.div(e);
+          const double y = X[(s + g.d * j) * P + e];
+          const int off = s + g.d * (e - hi * g.lo + g.lo * (j + g.lay * hi));
+          if (fabs(y) > best || (fabs(y) == best && off < boff)) {
+            best = fabs(y);
+            boff = off;
+            val = y;
           }
         }
         for (int m = 32; m > 0; m >>= 1) {
           const double ob = __shfl_xor(best, m), ov = __shfl_xor(val, m);
-          const int oo = __shfl_xor(best_off, m);
-          if (ob > best || (ob == best && oo < best_off)) {
+          const int oo = __shfl_xor(boff, m);
+          if (ob > best || (ob == best && oo < boff)) {
             best = ob;
-            best_off = oo;
+            boff = oo;
             val = ov;
           }
         }
-        if (l == 0) bond_sign[j] = val < 0 ? -1.0 : 1.0;
+        if (l == 0) sgn[j] = val < 0 ? -1.0 : 1.0;
       }
     }
-    __syncthreads();
-    for (int idx = tid; idx < g.E * cols; idx += blockDim.x) cur[idx] *= bond_sign[g.fd.div(g.fE.div(idx))];
-    __syncthreads();
     double nrm2 = 0;
-    for (int i = tid; i < g.E * cols; i += blockDim.x) nrm2 += cur[i] * cur[i];
+    for (int i = tid; i < E * cols; i += 256) {
+      const int c = (int)g.fE.div(i);
+      const double y = X[c * P + i - c * E];
+      nrm2 += y * y;
+    }
     nrm2 = block_sum_d(nrm2, red);
     const double sc = (prm.normalize && nrm2 > 0) ? 1.0 / sqrt(nrm2) : 1.0;
-    const int ncol = g.d * g.dims[g.j];  // columns of the bond's layout
-    for (int idx = tid; idx < g.E * ncol; idx += blockDim.x) {
-      const int c = (int)g.fE.div(idx), e = idx - c * g.E;
-      const int b = (int)g.fd.div(c), s = c - b * g.d;
-      const double val = b < keep ? cur[e + (long long)g.E * (s + g.d * b)] * sc : 0.0;
-      psi[g.psi_off + nat_off(g, s, e, b)] = val;
+    double* dst = psi + g.psi_off;
+    const int D = E * g.d * g.lay;
+    for (int i = tid; i < D; i += 256) {
+      int c, e, b;
+      ap_locate(g, i, c, e, b);
+      dst[i] = b < keep ? X[c * P + e] * sgn[b] * sc : 0.0;
     }
     __syncthreads();
-    phase_mark(prm, 6 + side);
+    phase_mark(prm, gate, 8 + sd);
   }
 }
 
@@ -1071,12 +769,6 @@ __global__ __launch_bounds__(256) void k_apply_site(const int* __restrict__ vert
   for (long long i = threadIdx.x; i < V.D; i += blockDim.x) t[i] *= sc;
 }
 
-// dynamic LDS of k_apply_gates: the matrices, then rot, four reflector-head
-// vectors, the singular values and the block reduction
-size_t apply_lds_bytes() {
-  return sizeof(double) * (2 * AP_XY + 2 * 1024 + 2 * AP_MAXEXT * 2 * AP_ENV * AP_ENV + 4 * 32 + 4 * AP_N_BIG +
-                           AP_TH + 16);
-}
 // per-side sizes of a bond for the kernel limits: E (external size), n = d chi_b
 // (the bond as it is), cols = d chi (the bond's layout during the call)
 struct SideSize {
@@ -1190,7 +882,7 @@ int prepare_apply(itnbp_net* net, int n, const int* edge_ids, int maxdim, double
 }
 
 // Device memory of one apply call: launch items, gate matrices, the per-gate
-// workspace of k_apply_gates (2 AP_SIDE doubles per gate) and the per-gate outputs.
+// workspace of the LDS kernels (2 AP_SIDE doubles per gate) and the per-gate outputs.
 struct ApplyBufs {
   ApplyItem* items;
   double* gates;
@@ -1245,7 +937,7 @@ int run_apply(itnbp_net* net, int n, const std::vector<ApplyItem>& items_in, con
               int maxdim, double cutoff, int normalize, double* truncerr, double* svals, int mk, int* kept,
               const ApplyBufs& b, const std::vector<char>* big = nullptr) {
   itnbp_ctx* ctx = net->ctx;
-  // the LDS kernel's gates first, then the split pipeline's (every
+  // the LDS kernels' gates first, then the split pipeline's (every
   // output is indexed by the gate's slot, so the order is free)
   std::vector<ApplyItem> items;
   items.reserve(n);
@@ -1272,11 +964,33 @@ int run_apply(itnbp_net* net, int n, const std::vector<ApplyItem>& items_in, con
   prm.normalize = normalize;
   prm.eig_cutoff = 10 * 2.220446049250313e-16;
   prm.max_keep = mk;
-  const size_t lds = apply_lds_bytes();
-  hipError_t ea = hipFuncSetAttribute((const void*)k_apply_gates, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)lds);
-  if (ea != hipSuccess)
-    return itnbp_fail(ctx, ITNBP_ERR_HIP, std::string("apply: LDS attribute: ") + hipGetErrorString(ea));
+  // LDS of the two launches: a side's columns, both W, and the elimination of the
+  // largest tall side (NT tiles of 16 columns)
+  long long nt = 1, xside = 0, xpair = 0, wsize = 0;
+  for (int i = 0; i < nl; ++i)
+    for (int sd = 0; sd < 2; ++sd) {
+      const VDesc& V = net->vdesc[sd == 0 ? items[i].u : items[i].v];
+      const int j = sd == 0 ? items[i].ju : items[i].jv;
+      const long long d = V.dims[0], lay = V.dims[j], E = V.D / (d * lay), nn = d * items[i].chib_in;
+      const long long cols = d * std::min<long long>(lay, AP_TH);  // Theta's limit: kept rank <= 32
+      if (E > nn) nt = std::max(nt, (nn + 15) / 16);
+      xside = std::max(xside, ap_pitch((int)E) * nn);
+      xpair = std::max(xpair, ap_pitch((int)E) * std::max(nn, cols));
+      wsize = std::max(wsize, std::min(std::min(E, nn) * cols, 1024LL));  // r d <= 32, kept rank <= 32
+    }
+  const size_t lds_side = sizeof(double) * (xside + AP_MAXEXT * AP_ENV * AP_ENV + 2 * 256 * nt * nt) +
+                          (nt == 1 ? CholLds<1>::bytes() : CholLds<2>::bytes());
+  const size_t lds_pair =
+      sizeof(double) * 2 * wsize + std::max<size_t>(sizeof(double) * xpair, SvdLds<AP_TH>::bytes() + 3 * 1024 * sizeof(double));
+  const auto k_side = nt == 1 ? k_gate_side<1> : k_gate_side<2>;
+  const auto k_pair = nt == 1 ? k_gate_pair<1> : k_gate_pair<2>;
+  if (nl > 0) {
+    hipError_t ea = hipFuncSetAttribute((const void*)k_side, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_side);
+    if (ea == hipSuccess)
+      ea = hipFuncSetAttribute((const void*)k_pair, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_pair);
+    if (ea != hipSuccess)
+      return itnbp_fail(ctx, ITNBP_ERR_HIP, std::string("apply: LDS attribute: ") + hipGetErrorString(ea));
+  }
   DevBuf tsb;
   std::unique_ptr<DevBuf, void (*)(DevBuf*)> ts_guard(&tsb, [](DevBuf* x) { free_buf(*x); });
   if (getenv("ITNBP_APPLY_PHASES")) {
@@ -1308,10 +1022,14 @@ int run_apply(itnbp_net* net, int n, const std::vector<ApplyItem>& items_in, con
     ITNBP_RETCHK(ensure_buf(ctx, net->apply_big, most));
   }
   const int pm0 = prof_mark(ctx);
-  if (nl > 0)
-    hipLaunchKernelGGL(k_apply_gates, dim3(nl), dim3(256), lds, ctx->stream, (const ApplyItem*)b.items,
-                       net->d_vdesc, (double*)net->d_psi, net->d_msg[net->cur], (const double*)b.gates, prm,
-                       b.work, b.te, svals ? b.sv : nullptr, b.kept, b.st);
+  if (nl > 0) {
+    hipLaunchKernelGGL(k_side, dim3(2 * nl), dim3(256), lds_side, ctx->stream, (const ApplyItem*)b.items,
+                       net->d_vdesc, (const double*)net->d_psi, (const double*)net->d_msg[net->cur], prm, (int)xside,
+                       b.work);
+    hipLaunchKernelGGL(k_pair, dim3(nl), dim3(256), lds_pair, ctx->stream, (const ApplyItem*)b.items, net->d_vdesc,
+                       (double*)net->d_psi, (const double*)b.gates, prm, (int)wsize, (const double*)b.work, b.te,
+                       svals ? b.sv : nullptr, b.kept, b.st);
+  }
   hipError_t ek = hipGetLastError();
   prof_add(ctx, "apply_gates", pm0, prof_mark(ctx));
   if (ek == hipSuccess && nb > 0) {
@@ -1327,33 +1045,28 @@ int run_apply(itnbp_net* net, int n, const std::vector<ApplyItem>& items_in, con
     }
   }
   if (prm.ts && ek == hipSuccess) {
-    // mean duration of every phase over the LDS kernel's gates that ran to the end, in us
+    // mean duration of every phase over the LDS kernels' gates that ran to the end, in us
     std::vector<unsigned long long> ts((size_t)n * 16);
     int khz = 0;
     ek = hipMemcpyAsync(ts.data(), prm.ts, ts.size() * 8, hipMemcpyDeviceToHost, ctx->stream);
     if (ek == hipSuccess) ek = hipStreamSynchronize(ctx->stream);
     if (ek == hipSuccess) ek = hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ctx->device);
-    double mean[7] = {0, 0, 0, 0, 0, 0, 0}, sub[3] = {0, 0, 0}, load = 0, sweeps = 0, tsq = 0;
+    // intervals [p, p + 1], 3 the gap between the launches
+    double mean[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     int cnt = 0;
     for (int i = 0; i < nl && ek == hipSuccess && khz > 0; ++i) {
       const unsigned long long* t = &ts[(size_t)i * 16];
-      if (!t[7]) continue;
+      if (!t[9]) continue;
       ++cnt;
-      for (int p = 0; p < 7; ++p) mean[p] += (double)(t[p + 1] - t[p]) * 1e3 / khz;
-      sweeps += (double)t[8];
-      tsq += (double)t[9];
-      if (!t[13]) continue;
-      load += (double)(t[10] - t[1]) * 1e3 / khz;
-      for (int p = 0; p < 3; ++p) sub[p] += (double)(t[11 + p] - t[10 + p]) * 1e3 / khz;
+      for (int p = 0; p < 9; ++p) mean[p] += (double)(t[p + 1] - t[p]) * 1e3 / khz;
     }
     const double c = cnt;
     if (cnt > 0)
       fprintf(stderr,
-              "  side u of qr (us): psi load %.1f, mode products %.1f, factorisation %.1f, save %.1f\n"
-              "apply phases (us, mean over %d gates): roots %.1f, qr %.1f (%.2f tall-skinny sides), theta %.1f, "
-              "svd %.1f (%.1f sweeps), factors %.1f, rebuild_u %.1f, rebuild_v %.1f\n",
-              load / c, sub[0] / c, sub[1] / c, sub[2] / c, cnt, mean[0] / c, mean[1] / c, tsq / c, mean[2] / c,
-              mean[3] / c, sweeps / c, mean[4] / c, mean[5] / c, mean[6] / c);
+              "apply phases (us, mean over %d gates): side u: load and roots %.1f, mode products %.1f, qr %.1f; "
+              "pair: theta %.1f, svd %.1f, factors %.1f, rebuild_u %.1f, rebuild_v %.1f\n",
+              cnt, mean[0] / c, mean[1] / c, mean[2] / c, mean[4] / c, mean[5] / c, mean[6] / c, mean[7] / c,
+              mean[8] / c);
   }
   std::vector<int> st(n);
   std::vector<int> kp(n);
@@ -1394,7 +1107,7 @@ int run_apply(itnbp_net* net, int n, const std::vector<ApplyItem>& items_in, con
 // ---- workspace of itnbp_apply_gates_noalloc --------------------------------
 // At most NOALLOC_MAX_GATES gates per call, gate matrices of at most
 // NOALLOC_MAX_GATE_ELEMS elements ((d_u d_v)^2 with d <= 4) and at most
-// NOALLOC_MAX_KEEP singular values per gate: 18.4 MiB in all, held by every
+// NOALLOC_MAX_KEEP singular values per gate: 21.0 MiB in all, held by every
 // GPU the library runs on until the process ends.
 constexpr int NOALLOC_MAX_GATES = 128;
 constexpr int NOALLOC_MAX_GATE_ELEMS = 256;

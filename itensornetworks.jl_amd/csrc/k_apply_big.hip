@@ -49,7 +49,7 @@ constexpr int GB_ROWS = 64;    // external rows of one chunk
 constexpr int GB_PITCH = 66;   // LDS pitch of a chunk's columns: 2 mod 32 doubles, conflict-free MFMA operands
 constexpr int GB_N = AP_N_BIG; // 64
 constexpr int GB_ROOT = AP_ENV_BIG * AP_ENV_BIG;
-constexpr int GB_LD = GB_N + 1;
+constexpr int GB_LD = CholLds<4>::LD;
 
 struct GbSide {
   long long psi_off;             // site tensor
@@ -427,63 +427,6 @@ __global__ __launch_bounds__(256) void k_gb_gram(GbWork w) {
 }
 
 // ---- Cholesky -----------------------------------------------------------------
-// [G | 1] reduced by Gaussian elimination without exchanges, G (n x n, n <= 64)
-// symmetric: thread (ti, tj) = (tid % 16, tid / 16) holds elements (ti + 16 a,
-// tj + 16 b) of both halves in registers; only the pivot row goes through LDS,
-// one barrier per column.  With G = L D L^T: U[k][j >= k] = (D L^T)[k][j],
-// Mi = L^{-1}, piv = diag D.  A column whose pivot is not positive is skipped.
-__device__ void gb_eliminate(double (&g)[4][4], int n, double* rows, double* U, double* Mi, double* piv) {
-  const int tid = threadIdx.x, ti = tid & 15, tj = tid >> 4;
-  double m[4][4];
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = 0; b < 4; ++b) m[a][b] = ti + 16 * a == tj + 16 * b ? 1.0 : 0.0;
-  // rows: [parity][G row (64) | M row (64)]
-  if (ti == 0)
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      rows[tj + 16 * b] = g[0][b];
-      rows[64 + tj + 16 * b] = m[0][b];
-    }
-  __syncthreads();
-  for (int k = 0; k < n; ++k) {
-    const double* rg = rows + (k & 1) * 128;
-    double* nx = rows + ((k & 1) ^ 1) * 128;
-    const double p = rg[k];
-    const double inv = p > 0 ? 1 / p : 0.0;
-    if (tid < 64) {
-      U[k * GB_LD + tid] = rg[tid];
-      Mi[k * GB_LD + tid] = rg[64 + tid];
-      if (tid == 0) piv[k] = p;
-    }
-    double gj[4], mj[4];
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      gj[b] = rg[tj + 16 * b];
-      mj[b] = rg[64 + tj + 16 * b];
-    }
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      const int i = ti + 16 * a;
-      if (i <= k || i >= n) continue;
-      const double f = rg[i] * inv;
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        g[a][b] -= f * gj[b];
-        m[a][b] -= f * mj[b];
-      }
-      if (i == k + 1)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          nx[tj + 16 * b] = g[a][b];
-          nx[64 + tj + 16 * b] = m[a][b];
-        }
-    }
-    __syncthreads();
-  }
-}
-
 __device__ inline void gb_sum_parts(const GbWork& w, int side, int np, int n, double (&g)[4][4]) {
   const int ti = threadIdx.x & 15, tj = threadIdx.x >> 4;
   const double* p = w.part + (long long)side * w.nsplit * GB_SQ;
@@ -537,9 +480,8 @@ __device__ inline void gb_wide_rank(const GbWork& w, int side, int r, const doub
 }
 
 // The first factorisation of a side.  The Cholesky factor is used while its
-// pivots span at most 1e-10 (R's diagonal 1e-5, as the LDS kernel's rebuild
-// test); a side past that, rank-deficient ones among them, takes the
-// eigendecomposition G = V diag(l) V^T by one-sided Jacobi instead, dropping
+// pivots span at most 1e-10 (R's diagonal 1e-5); a side past that,
+// rank-deficient ones among them, takes the eigendecomposition G = V diag(l) V^T by one-sided Jacobi instead, dropping
 // directions with l <= n eps l_max: T = V_r l_r^{-1/2}, R0 = l_r^{1/2} V_r^T,
 // exact inverses of each other however graded l is.  A wide side keeps R = X, Q = 1
 // unless X X^T fails the same test: then R = V_r^T X and Q = V_r with its
@@ -560,10 +502,8 @@ __global__ __launch_bounds__(256) void k_gb_chol1(GbWork w) {
     }
     __syncthreads();
   }
-  double* U = sm;
-  double* Mi = U + GB_N * GB_LD;
-  double* rows = Mi + GB_N * GB_LD;
-  double* piv = rows + 256;
+  const CholLds<4> L(sm);
+  double *U = L.U, *Mi = L.Mi, *piv = L.piv;
   const int nch = (g.E + GB_ROWS - 1) / GB_ROWS, np = nch < w.nsplit ? nch : w.nsplit;
   double a[4][4];
   if (g.wide)
@@ -584,7 +524,7 @@ __global__ __launch_bounds__(256) void k_gb_chol1(GbWork w) {
     if (tid == 0) w.info[side].r = n;
     return;
   }
-  gb_eliminate(a, n, rows, U, Mi, piv);
+  chol_eliminate<4>(a, n, 0.0, L);
   double pmin = INFINITY, pmax = 0;
   for (int k = 0; k < n; ++k) {
     pmin = fmin(pmin, piv[k]);
@@ -658,14 +598,12 @@ __global__ __launch_bounds__(256) void k_gb_chol2(GbWork w) {
   const GbSide& g = w.side[side];
   if (g.wide) return;
   const int n = g.n, r = w.info[side].r;
-  double* U = sm;
-  double* Mi = U + GB_N * GB_LD;
-  double* rows = Mi + GB_N * GB_LD;
-  double* piv = rows + 256;
+  const CholLds<4> L(sm);
+  double *U = L.U, *Mi = L.Mi, *piv = L.piv;
   const int nch = (g.E + GB_ROWS - 1) / GB_ROWS, np = nch < w.nsplit ? nch : w.nsplit;
   double a[4][4];
   gb_sum_parts(w, side, np, r, a);
-  gb_eliminate(a, r, rows, U, Mi, piv);
+  chol_eliminate<4>(a, r, 0.0, L);
   // R1 and R1^{-1} in place
   for (int i = tid; i < r * r; i += 256) {
     const int k = i / r, j = i % r;
@@ -1184,7 +1122,7 @@ int apply_big_run(itnbp_net* net, const ApplyItem* items, int nb, const double* 
   const int ns = 2 * nb;
   double* psi = (double*)net->d_psi;
   const size_t lds_gram = sizeof(double) * GB_N * GB_PITCH;
-  const size_t lds_chol = sizeof(double) * (2 * GB_N * GB_LD + 256 + GB_N);
+  const size_t lds_chol = CholLds<4>::bytes();
   const size_t lds_reb = sizeof(double) * (GB_N * GB_PITCH + 4 + 6 * p.lcols + p.max_w);
   const size_t lds_svd = p.max_th <= 32 ? SvdLds<32>::bytes() : p.max_th <= 64 ? SvdLds<64>::bytes() : SvdLds<128>::bytes();
   const struct {
