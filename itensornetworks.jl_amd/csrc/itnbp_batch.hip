@@ -261,7 +261,6 @@ int update_batched(int n, itnbp_net** nets, const itnbp_update_opts* o, itnbp_up
   bool replan = true, use_small = false;
   int small_first = -1;  // vertex tasks of the first plan (reported in the path)
   bool graph_mode = false, graphed = false;
-  int tile = 0;
   // device-resident loop: every message of every instance on the per-vertex
   // kernels (chi <= 16, symmetric messages)
   DevBuf d_inst, d_active, d_out, d_ctr;
@@ -299,7 +298,6 @@ int update_batched(int n, itnbp_net** nets, const itnbp_update_opts* o, itnbp_up
     ITNBP_HIPCHK(ctx, hipMemcpyAsync(d_out.p, hout.data(), n * sizeof(BatchOut), hipMemcpyHostToDevice, ctx->stream));
     ITNBP_HIPCHK(ctx, hipMemcpyAsync(d_ctr.p, &zero, sizeof(zero), hipMemcpyHostToDevice, ctx->stream));
     ITNBP_RETCHK(small_autotune(M, acc_f64, M->d_psi, dtype, buf[M->cur], o->normalize));
-    tile = small_big_tile(M);
     small_first = small_task_count(M);
     int sweeps = 0;
     ITNBP_HIPCHK(ctx, hipEventRecord(ctx->ev0, ctx->stream));
@@ -393,7 +391,6 @@ int update_batched(int n, itnbp_net** nets, const itnbp_update_opts* o, itnbp_up
   ITNBP_HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
   if (graph_mode)
     ctx->path = std::string(graphed ? "batched-graph" : "batched-device") + " [vertex " + std::to_string(small_first) +
-                (tile ? std::string(", ") + small_big_kind(M) + " tile " + std::to_string(tile) : "") +
                 (small_queue_used(M) ? ", persistent" : "") + "]";
   else
     ctx->path = small_first > 0 ? "batched-generic [vertex " + std::to_string(small_first) + "]" : "batched-generic";

@@ -62,12 +62,9 @@ int small_task_count(itnbp_net* net);
 // batched update: the instance of every vertex and the device-side active
 // flags and sweep counter the per-vertex kernels read (null pointers: off)
 void small_set_batch(itnbp_net* net, const std::vector<int>& vinst, const int* active, const long long* sweep_ctr);
-// times the Gram tiles of the large-site kernel on scratch outputs and keeps
-// the fastest; small_big_tile reports it (0 without large sites)
+// times the two launch forms of the LDS-resident sites on scratch outputs and
+// keeps the faster
 int small_autotune(itnbp_net* net, int acc_f64, const void* psi, int psi_dtype, const void* msg_in, int normalize);
-int small_big_tile(itnbp_net* net);
-// "mfma" or "valu" for the autotuned large-site kernel ("" before tuning)
-const char* small_big_kind(itnbp_net* net);
 // the LDS-resident sites run as the persistent queue kernel
 bool small_queue_used(itnbp_net* net);
 int small_sweep(itnbp_net* net, int acc_f64, const void* psi, int psi_dtype, const void* msg_in, void* msg_out,
