@@ -31,7 +31,7 @@
 // workgroup each.  One round with the copies in and out, against one workgroup
 // per bond through all steps: 8x8 chi = 16 (4 classes of 28 gates) 44.1 -> 9.3 ms,
 // 5x4 chi = 32 (4 classes of 6 to 10) 447 -> 26.9 ms; per class there, svd 0.50 and
-// 2.05 ms, rebuild 88 and 343 us, roots 94 and 234 us, grams 89 and 347 us, chol 81
+// 2.05 ms, rebuild 88 and 343 us, roots 75 and 197 us, grams 89 and 347 us, chol 81
 // and 476 us, the three mode passes 50 and 124 us.
 #include <algorithm>
 #include <cmath>
@@ -110,84 +110,34 @@ __device__ inline int gb_nat(const GbSide& g, int s, int e, int b) {
 }
 
 // ---- environment roots -----------------------------------------------------
-// One workgroup per environment: cyclic two-sided Jacobi with the round-robin
-// pairs of rr_pair; a step derives the rotations in the first ne / 2 lanes, then
-// thread (i, j) rotates the 2 x 2 block of row pair i and column pair j and two
-// pairs of V.  Stopping rule and eigenvalue truncation of env_roots_wave.
+// One workgroup per environment (block_jacobi_eigh, M scaled to order 1 by an even
+// power of two); stopping rule and eigenvalue truncation of env_roots_wave.
 __global__ __launch_bounds__(256) void k_gb_roots(GbWork w, const double* __restrict__ msg, double cutoff) {
   const GbSide& g = w.side[blockIdx.y];
   const int pa = blockIdx.x;
   if (pa >= g.next) return;
   constexpr int LD = AP_ENV_BIG + 1;
-  __shared__ double A[AP_ENV_BIG * LD], V[AP_ENV_BIG * LD], rc[16], rs[16], red[4];
+  __shared__ double A[AP_ENV_BIG * LD], V[AP_ENV_BIG * LD], rc[16], rs[16], red[8];
   __shared__ int rank[AP_ENV_BIG], byr[AP_ENV_BIG];
-  const int tid = threadIdx.x, chi = g.ext_dim[pa], ne = chi + (chi & 1), np = ne / 2;
+  const int tid = threadIdx.x, chi = g.ext_dim[pa];
   const double* M = msg + g.msg_off[pa];
-  for (int o = tid; o < AP_ENV_BIG * AP_ENV_BIG; o += 256) {
-    const int i = o >> 5, j = o & 31;
-    A[i * LD + j] = (i < chi && j < chi) ? 0.5 * (M[i + chi * j] + M[j + chi * i]) : 0.0;
-    V[i * LD + j] = i == j ? 1.0 : 0.0;
-  }
-  __syncthreads();
-  const int pi = tid >> 4, pj = tid & 15;
-  double prev = INFINITY;
-  for (int sweep = 0; sweep < 40 && chi > 1; ++sweep) {
-    double off = 0, dg = 0;
-    for (int o = tid; o < AP_ENV_BIG * AP_ENV_BIG; o += 256) {
-      const int i = o >> 5, j = o & 31;
-      const double a = A[i * LD + j];
-      if (i != j)
-        off += a * a;
-      else
-        dg += a * a;
-    }
-    off = block_sum_d(off, red);
-    dg = block_sum_d(dg, red);
-    if (off <= 1e-30 * dg || off == 0.0 || off >= prev) break;
-    prev = off;
-    for (int st = 0; st < ne - 1; ++st) {
-      if (tid < np) {
-        int p, q;
-        rr_pair(ne, st, tid, p, q);
-        double c = 1, sn = 0;
-        const double apq = A[p * LD + q];  // the padding index of an odd chi couples to nothing
-        if (apq != 0.0) {
-          const double zeta = (A[q * LD + q] - A[p * LD + p]) / (2 * apq);
-          const double t = (zeta >= 0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1 + zeta * zeta));
-          c = 1 / sqrt(1 + t * t);
-          sn = c * t;
-        }
-        rc[tid] = c;
-        rs[tid] = sn;
-      }
-      __syncthreads();
-      if (pj < np) {
-        int p2, q2;
-        rr_pair(ne, st, pj, p2, q2);
-        const double c2 = rc[pj], s2 = rs[pj];
-        if (pi < np) {
-          int p1, q1;
-          rr_pair(ne, st, pi, p1, q1);
-          const double c1 = rc[pi], s1 = rs[pi];
-          const double app = A[p1 * LD + p2], apq = A[p1 * LD + q2], aqp = A[q1 * LD + p2], aqq = A[q1 * LD + q2];
-          const double bpp = c1 * app - s1 * aqp, bpq = c1 * apq - s1 * aqq;
-          const double bqp = s1 * app + c1 * aqp, bqq = s1 * apq + c1 * aqq;
-          A[p1 * LD + p2] = c2 * bpp - s2 * bpq;
-          A[p1 * LD + q2] = s2 * bpp + c2 * bpq;
-          A[q1 * LD + p2] = c2 * bqp - s2 * bqq;
-          A[q1 * LD + q2] = s2 * bqp + c2 * bqq;
-        }
+  double a[4], mx = 0;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int row = pi + 16 * h;
-          const double vp = V[row * LD + p2], vq = V[row * LD + q2];
-          V[row * LD + p2] = c2 * vp - s2 * vq;
-          V[row * LD + q2] = s2 * vp + c2 * vq;
-        }
-      }
-      __syncthreads();
-    }
+  for (int h = 0; h < 4; ++h) {
+    const int i = (tid >> 5) + 8 * h, j = tid & 31;
+    a[h] = (i < chi && j < chi) ? 0.5 * (M[i + chi * j] + M[j + chi * i]) : 0.0;
+    V[i * LD + j] = i == j ? 1.0 : 0.0;
+    mx = fmax(mx, fabs(a[h]));
   }
+  for (int m = 32; m > 0; m >>= 1) mx = fmax(mx, __shfl_xor(mx, m));
+  if ((tid & 63) == 0) red[tid >> 6] = mx;
+  __syncthreads();
+  mx = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+  const int ex = mx > 0 && isfinite(mx) ? ilogb(mx) & ~1 : 0;
+#pragma unroll
+  for (int h = 0; h < 4; ++h) A[((tid >> 5) + 8 * h) * LD + (tid & 31)] = ldexp(a[h], -ex);
+  __syncthreads();
+  block_jacobi_eigh<LD>(A, V, chi, 1e-30, rc, rs, red);
   // truncation: rank |lambda| descending (ties by index); drop from the small
   // end while the dropped weight / total <= cutoff (keep >= 1)
   if (tid < chi) {
@@ -227,8 +177,8 @@ __global__ __launch_bounds__(256) void k_gb_roots(GbWork w, const double* __rest
       siv += vv / sq;
       pv += vv;
     }
-    S[o] = sv;
-    S[GB_ROOT + o] = siv;
+    S[o] = ldexp(sv, ex / 2);
+    S[GB_ROOT + o] = ldexp(siv, -ex / 2);
     S[2 * GB_ROOT + o] = pv;
   }
   if (tid == 0) w.info[blockIdx.y].trunc[pa] = keep < chi;

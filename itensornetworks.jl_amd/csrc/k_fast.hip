@@ -27,6 +27,7 @@
 #include <cstdlib>
 #include <vector>
 
+#include "itnbp_jacobi.hpp"
 #include "itnbp_ops.hpp"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -1167,173 +1168,78 @@ __device__ inline void wave_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// Symmetric eigendecomposition of one 32x32 message per wave (cyclic parallel
-// Jacobi, 16 disjoint rotations per step, round-robin pairing), input
-// symmetrised as S = (M + M^T)/2.  With warm = 1 the previous sweep's
-// eigenvectors U0 (in U64) seed it: Jacobi then diagonalises U0^T S U0, which
-// is nearly diagonal once BP settles, and the rotations accumulate onto U0.
-// Stops when the off-diagonal mass is below tol2 of the diagonal's (1e-28 for
-// the FP64 pipeline, 1e-14 for the BF16 one, whose operands carry ~16 bits) or
-// stops decreasing.  grid (ceil(n/4)), 256 threads.
+// Symmetric eigendecomposition of one 32x32 message per workgroup
+// (block_jacobi_eigh), input symmetrised as S = (M + M^T)/2 and scaled to order 1 by
+// a power of two.  With warm = 1 the previous sweep's eigenvectors U0 (in U64) seed
+// it: Jacobi then diagonalises U0^T S U0, which is nearly diagonal once BP settles,
+// and the rotations accumulate onto U0.  tol2: 1e-28 for the FP64 pipeline, 1e-14
+// for the BF16 one, whose operands carry ~16 bits.  grid n, 256 threads.
+//
+// Bound: the serial chain of steps.  One wave per message, four to a workgroup, took
+// 213 us per sweep of an 8x8 lattice (LDS traffic of both triangles by one wave, and
+// a quarter of the CUs), against 87.
 template <typename TM>
-__global__ __launch_bounds__(256) void k_msg_eigh(const long long* __restrict__ moff, int n,
-                                                 const TM* __restrict__ msg, double* __restrict__ U64,
-                                                 double* __restrict__ L64, float* __restrict__ U32,
-                                                 float* __restrict__ L32, int* __restrict__ Lexp, int warm,
-                                                 double tol2) {
+__global__ __launch_bounds__(256) void k_msg_eigh(const long long* __restrict__ moff, const TM* __restrict__ msg,
+                                                 double* __restrict__ U64, double* __restrict__ L64,
+                                                 float* __restrict__ U32, float* __restrict__ L32,
+                                                 int* __restrict__ Lexp, int warm, double tol2) {
   constexpr int LD = 33;
-  __shared__ double As[4][FC * LD];
-  __shared__ double Vs[4][FC * LD];
-  __shared__ double rc[4][16], rs[4][16];
-  __shared__ int rp[4][16], rq[4][16];
-  const int wv = threadIdx.x >> 6, l = threadIdx.x & 63;
-  const int e = blockIdx.x * 4 + wv;
-  if (e >= n) return;  // whole waves only; the kernel has no workgroup barrier
-  double* A = As[wv];
-  double* V = Vs[wv];
+  __shared__ double A[FC * LD], V[FC * LD], rc[16], rs[16], red[8];
+  const int tid = threadIdx.x, l = tid & 63, wv = tid >> 6, e = blockIdx.x;
   const TM* M = msg + moff[e];
   double* u64 = U64 + (long long)e * FBLK;
-  for (int o = l; o < FBLK; o += 64) {
-    const int i = o & 31, j = o >> 5;
-    A[i * LD + j] = 0.5 * ((double)M[i + FC * j] + (double)M[j + FC * i]);
+  double a[4], mx = 0;
+#pragma unroll
+  for (int h = 0; h < 4; ++h) {
+    const int i = tid & 31, j = (tid >> 5) + 8 * h;
+    a[h] = 0.5 * ((double)M[i + FC * j] + (double)M[j + FC * i]);
     V[i * LD + j] = warm ? u64[i + FC * j] : ((i == j) ? 1.0 : 0.0);  // V[b][r] = U0[b + 32 r]
+    mx = fmax(mx, fabs(a[h]));
   }
-  wave_sync();
+  for (int m = 32; m > 0; m >>= 1) mx = fmax(mx, __shfl_xor(mx, m));
+  if (l == 0) red[wv] = mx;
+  __syncthreads();
+  mx = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+  const int ex = mx > 0 && isfinite(mx) ? ilogb(mx) : 0;
+#pragma unroll
+  for (int h = 0; h < 4; ++h) A[(tid & 31) * LD + (tid >> 5) + 8 * h] = ldexp(a[h], -ex);
+  __syncthreads();
   if (warm) {
-    // A <- U0^T S U0.  Lane l owns column j = l & 31 and rows i = (l >> 5) + 2 m
-    // (m = 0..15) of each product; the 16 accumulators are independent, so the
-    // loads of one k-step are all in flight together.
-    const int jc = l & 31, i0 = l >> 5;
-    double t[16];
+    // A <- U0^T (S U0), a 16 x 16 tile of each product per wave, the lower triangle
+    // from the upper one
+    const int li = l & 15, lg = l >> 4, r0 = 16 * (wv & 1), c0 = 16 * (wv >> 1);
+    f64x4 t = {0, 0, 0, 0};
 #pragma unroll
-    for (int m = 0; m < 16; ++m) t[m] = 0;
-#pragma unroll 2
-    for (int q = 0; q < FC; ++q) {
-      const double u = V[q * LD + jc];
+    for (int q = 0; q < 8; ++q) t = MFMA_F64(A[(r0 + li) * LD + 4 * q + lg], V[(4 * q + lg) * LD + c0 + li], t);
+    __syncthreads();
 #pragma unroll
-      for (int m = 0; m < 16; ++m) t[m] += A[(i0 + 2 * m) * LD + q] * u;  // (S U0)[i][j]
+    for (int v = 0; v < 4; ++v) A[(r0 + 4 * v + lg) * LD + c0 + li] = t[v];
+    __syncthreads();
+    t = f64x4{0, 0, 0, 0};
+#pragma unroll
+    for (int q = 0; q < 8; ++q) t = MFMA_F64(V[(4 * q + lg) * LD + r0 + li], A[(4 * q + lg) * LD + c0 + li], t);
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int i = r0 + 4 * v + lg, j = c0 + li;
+      if (i <= j) A[i * LD + j] = A[j * LD + i] = t[v];
     }
-    wave_sync();
-#pragma unroll
-    for (int m = 0; m < 16; ++m) A[(i0 + 2 * m) * LD + jc] = t[m];
-    wave_sync();
-#pragma unroll
-    for (int m = 0; m < 16; ++m) t[m] = 0;
-#pragma unroll 2
-    for (int q = 0; q < FC; ++q) {
-      const double x = A[q * LD + jc];
-#pragma unroll
-      for (int m = 0; m < 16; ++m) t[m] += V[q * LD + i0 + 2 * m] * x;  // (U0^T S U0)[i][j]
-    }
-    wave_sync();
-#pragma unroll
-    for (int m = 0; m < 16; ++m) {
-      const int i = i0 + 2 * m;
-      if (i <= jc) A[i * LD + jc] = t[m];
-    }
-    wave_sync();
-#pragma unroll
-    for (int m = 0; m < 16; ++m) {
-      const int i = i0 + 2 * m;
-      if (i > jc) A[i * LD + jc] = A[jc * LD + i];  // exact symmetry from the upper triangle
-    }
-    wave_sync();
+    __syncthreads();
   }
-  const int col = l & 31, half = l >> 5;
-  double prev = INFINITY;
-  for (int sweep = 0; sweep < 30; ++sweep) {
-    double off = 0, dg = 0;
-    for (int o = l; o < FBLK; o += 64) {
-      const int i = o >> 5, j = o & 31;
-      const double a = A[i * LD + j];
-      if (i != j) off += a * a;
-      else dg += a * a;
-    }
-    for (int m = 32; m > 0; m >>= 1) {
-      off += __shfl_xor(off, m);
-      dg += __shfl_xor(dg, m);
-    }
-    if (off <= tol2 * dg || off == 0.0 || off >= prev) break;
-    prev = off;
-    for (int st = 0; st < FC - 1; ++st) {
-      if (l < 16) {
-        auto at = [&](int pos) { return pos == 0 ? 0 : 1 + (pos - 1 + st) % (FC - 1); };
-        int p = at(l), q = at(FC - 1 - l);
-        if (p > q) {
-          const int t = p;
-          p = q;
-          q = t;
-        }
-        double c = 1, s = 0;
-        const double apq = A[p * LD + q];
-        if (apq != 0.0) {
-          const double zeta = (A[q * LD + q] - A[p * LD + p]) / (2 * apq);
-          const double t = (zeta >= 0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1 + zeta * zeta));
-          c = 1 / sqrt(1 + t * t);
-          s = c * t;
-        }
-        rc[wv][l] = c;
-        rs[wv][l] = s;
-        rp[wv][l] = p;
-        rq[wv][l] = q;
-      }
-      wave_sync();
-      // the 8 (disjoint) pairs of this lane: every operand is loaded before any
-      // store, so the LDS latency is paid once per phase rather than per pair
-      int pp[8], qq[8];
-      double cc[8], ss[8];
-#pragma unroll
-      for (int jj = 0; jj < 8; ++jj) {
-        const int i = half + 2 * jj;
-        pp[jj] = rp[wv][i];
-        qq[jj] = rq[wv][i];
-        cc[jj] = rc[wv][i];
-        ss[jj] = rs[wv][i];
-      }
-      // rows: A <- J^T A
-      double x0[8], x1[8];
-#pragma unroll
-      for (int jj = 0; jj < 8; ++jj) {
-        x0[jj] = A[pp[jj] * LD + col];
-        x1[jj] = A[qq[jj] * LD + col];
-      }
-#pragma unroll
-      for (int jj = 0; jj < 8; ++jj) {
-        A[pp[jj] * LD + col] = cc[jj] * x0[jj] - ss[jj] * x1[jj];
-        A[qq[jj] * LD + col] = ss[jj] * x0[jj] + cc[jj] * x1[jj];
-      }
-      wave_sync();
-      // columns: A <- A J, V <- V J
-      double y0[8], y1[8];
-#pragma unroll
-      for (int jj = 0; jj < 8; ++jj) {
-        x0[jj] = A[col * LD + pp[jj]];
-        x1[jj] = A[col * LD + qq[jj]];
-        y0[jj] = V[col * LD + pp[jj]];
-        y1[jj] = V[col * LD + qq[jj]];
-      }
-#pragma unroll
-      for (int jj = 0; jj < 8; ++jj) {
-        A[col * LD + pp[jj]] = cc[jj] * x0[jj] - ss[jj] * x1[jj];
-        A[col * LD + qq[jj]] = ss[jj] * x0[jj] + cc[jj] * x1[jj];
-        V[col * LD + pp[jj]] = cc[jj] * y0[jj] - ss[jj] * y1[jj];
-        V[col * LD + qq[jj]] = ss[jj] * y0[jj] + cc[jj] * y1[jj];
-      }
-      wave_sync();
-    }
-  }
+  block_jacobi_eigh<LD>(A, V, FC, tol2, rc, rs, red);
   float* u32 = U32 ? U32 + (long long)e * FBLK : nullptr;
-  for (int o = l; o < FBLK; o += 64) {
+  for (int o = tid; o < FBLK; o += 256) {
     const int b = o & 31, r = o >> 5;
     const double v = V[b * LD + r];
     u64[o] = v;  // U[b + 32 r]: column r is the eigenvector of eigenvalue r
     if (u32) u32[o] = (float)v;
   }
+  if (wv > 0) return;
   // the FP32 copy is scaled by 2^-x so that its largest |lam| lies in [1/2, 1):
   // products of eigenvalues (the Gram weights of the 16-bit kernels) then stay
   // of order one whatever the messages' scale, and the finaliser multiplies the
   // Gram back by 2^(sum of the x of the bonds it weighs)
-  const double lam = l < FC ? A[l * LD + l] : 0.0;
+  const double lam = l < FC ? ldexp(A[l * LD + l], ex) : 0.0;
   if (l < FC) L64[(long long)e * FC + l] = lam;
   if (L32) {
     double m = fabs(lam);
@@ -3709,12 +3615,12 @@ static int eig_sweep(itnbp_ctx* ctx, FastState* st, int acc_f64, const void* msg
   const int warm = (st->eig_warm && st->eig_count % 16 != 0) ? 1 : 0;
   const int e0 = prof_mark(ctx);
   if (acc_f64)
-    hipLaunchKernelGGL((k_msg_eigh<double>), dim3((ne4 + 3) / 4), dim3(256), 0, ctx->stream,
-                       (const long long*)st->d_eig_moff.p, ne4, (const double*)msg_in, (double*)st->eigU64.p,
+    hipLaunchKernelGGL((k_msg_eigh<double>), dim3(ne4), dim3(256), 0, ctx->stream,
+                       (const long long*)st->d_eig_moff.p, (const double*)msg_in, (double*)st->eigU64.p,
                        (double*)st->eigL64.p, (float*)nullptr, (float*)nullptr, (int*)nullptr, warm, 1e-28);
   else
-    hipLaunchKernelGGL((k_msg_eigh<float>), dim3((ne4 + 3) / 4), dim3(256), 0, ctx->stream,
-                       (const long long*)st->d_eig_moff.p, ne4, (const float*)msg_in, (double*)st->eigU64.p,
+    hipLaunchKernelGGL((k_msg_eigh<float>), dim3(ne4), dim3(256), 0, ctx->stream,
+                       (const long long*)st->d_eig_moff.p, (const float*)msg_in, (double*)st->eigU64.p,
                        (double*)st->eigL64.p, (float*)st->eigU32.p, (float*)st->eigL32.p, (int*)st->eigLexp.p,
                        warm, 1e-14);
   st->eig_warm = true;
@@ -3900,8 +3806,8 @@ static int rotated_sites_setup(itnbp_net* net, const std::vector<int>& want, siz
   const double* U = (const double*)st->eigU64.p;
   const double* L = (const double*)st->eigL64.p;
   // cold start: the rotations must be orthogonal to rounding
-  hipLaunchKernelGGL((k_msg_eigh<double>), dim3((ne4 + 3) / 4), dim3(256), 0, ctx->stream,
-                     (const long long*)st->d_eig_moff.p, ne4, (const double*)net->d_msg[net->cur],
+  hipLaunchKernelGGL((k_msg_eigh<double>), dim3(ne4), dim3(256), 0, ctx->stream,
+                     (const long long*)st->d_eig_moff.p, (const double*)net->d_msg[net->cur],
                      (double*)st->eigU64.p, (double*)st->eigL64.p, (float*)nullptr, (float*)nullptr, (int*)nullptr, 0,
                      1e-28);
   st->eig_warm = true;
