@@ -1509,240 +1509,298 @@ __global__ __launch_bounds__(256) void k_gram12_bf16(const EigItem* __restrict__
   }
 }
 
-// rot34, FP64: WG (256 threads) -> (s, 8 consecutive r2, ROT_NZ64 consecutive r1);
-// wave wv -> r2 = w0 + 2 wv + {0, 1}.  One block of look-ahead: the loads of the
-// next block are in flight during the 160 MFMAs of the current one.
-// grid (EIG_NPART, items) = (2 s x 4 r2 groups x 2 r1 groups)
-constexpr int ROT_NZ64 = 16;
+// Work split of a FP64 launch over n sites of `units` equal units each: workgroup w
+// of wgs takes the units [w N / wgs, (w + 1) N / wgs) of all N = n units, across
+// site boundaries, so that no launch ends with a part-filled wave of workgroups.  Its
+// Grams of a site go to partial slot w - first(site) of its `slots`; at most that many
+// workgroups touch a site.  n = 0: every slot is written.
+struct EigSplit {
+  int n, units, wgs, slots;
+  __host__ __device__ int begin(int w) const { return (int)((long long)w * n * units / wgs); }
+  __device__ int first(int b) const {
+    int w = (int)((long long)b * wgs / n);
+    while (begin(w + 1) <= b * units) ++w;
+    return w;
+  }
+  __device__ int parts(int b) const {
+    if (n == 0) return slots;
+    const int f = first(b);
+    if (b + 1 == n) return wgs - f;
+    const int g = first(b + 1);
+    return g - f + (begin(g) < (b + 1) * units ? 1 : 0);
+  }
+};
+constexpr int EIG_MAXSLOTS = 64;
+// 16, 32 or 64 partials per site: enough workgroups for two per CU
+int eig_slots(int n, int num_cu) {
+  int m = EIG_NPART;
+  while (m < EIG_MAXSLOTS && 2 * m * n <= 2 * num_cu) m *= 2;
+  return m;
+}
+// as many whole workgroups per site while all are resident (two per CU), else every
+// resident slot once, at most slots - 1 workgroups' worth per site
+EigSplit eig_split(int n, int units, int slots, int num_cu) {
+  const int resident = 2 * num_cu;
+  return EigSplit{n, units, n * slots <= resident ? n * slots : std::min(resident, n * (slots - 1)), slots};
+}
 
-// GRAM = false: rot12, as for the BF16 kernel
+// rot34, FP64: a unit is (s, 8 consecutive r2, r1); wave wv -> r2 = w0 + 2 wv + {0,
+// 1}.  A block is loaded while the products of the one before run (its registers are
+// free after V = Z U4); two workgroups per CU hide each other's staging and
+// barriers: U3 and the eigenvalues come from LDS, Y is staged with a swizzle
+// instead of padded rows.  GRAM = false: rot12, as for the BF16 kernel.
+//
+// Bound: MFMA with Grams (5 products of 32^3 per block), HBM without (2 blocks
+// moved, 2 products).  36 sites: 512 and 340 us; one workgroup per CU and 16
+// fixed parts per site (2.25 waves of them) took 665 and 420.
 template <bool GRAM>
-__global__ __launch_bounds__(256) void k_rot34_f64(const EigItem* __restrict__ items,
-                                                   const double* __restrict__ R,
-                                                   const double* __restrict__ U,
-                                                   const double* __restrict__ lam,
-                                                   double* __restrict__ Q, double* __restrict__ part) {
-  constexpr int SROW = 10;
-  __shared__ __attribute__((aligned(16))) double S[FBLK * SROW];
-  const EigItem it = items[blockIdx.y];
-  const int q = blockIdx.x;
-  const int s = q & 1, w0 = ((q >> 1) & 3) * 8, z0 = (q >> 3) * ROT_NZ64;
+__global__ __launch_bounds__(256, 2) void k_rot34_f64(const EigItem* __restrict__ items, EigSplit sp,
+                                                      const double* __restrict__ R,
+                                                      const double* __restrict__ U,
+                                                      const double* __restrict__ lam,
+                                                      double* __restrict__ Q, double* __restrict__ part) {
+  constexpr int LDU = 48;  // rows of U3 half the banks apart
+  __shared__ __attribute__((aligned(16))) double S[FBLK * 8];
+  __shared__ double U3s[FC * LDU], ls[4][FC];
   const int l = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int li = l & 15, lg = l >> 4;
-  double aU3T[2][8], bU4[8][2], lam3v[8], lam4v[8];
-#pragma unroll
-  for (int t = 0; t < 8; ++t) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      aU3T[h][t] = U[it.U[2] + (4 * t + lg) + FC * (16 * h + li)];  // U3^T[16h+li][4t+lg]
-      bU4[t][h] = U[it.U[3] + (4 * t + lg) + FC * (16 * h + li)];   // U4[4t+lg][16h+li]
-    }
-    lam3v[t] = GRAM ? lam[it.L[2] + 4 * t + lg] : 0.0;
-    lam4v[t] = GRAM ? lam[it.L[3] + 4 * t + lg] : 0.0;
-  }
+  // staging slot of element o = r4 + 32 r3, r2 = w: pairs of r2 permuted by o
+  auto slot = [](int o, int w) { return o * 8 + 2 * (((w >> 1) ^ (o >> 2) ^ (o >> 5)) & 3) + (w & 1); };
+  double bU4[8][2], cur[2][8];
   Acc32 T3, T4;
-  acc_zero(T3);
-  acc_zero(T4);
-  double cur[2][8], nxt[2][8];
-  auto fetch = [&](int j, double (&dst)[2][8]) {  // block j of this wave: z = z0 + j / 2, w = w0 + 2 wv + j % 2
-    const int z = z0 + (j >> 1), w = w0 + 2 * wv + (j & 1);
-    const double* Z = R + it.R + (long long)(s + 2 * (z + FC * w)) * FBLK;
+  const int u1 = sp.begin(blockIdx.x + 1);
+  int b = -1;
+  const EigItem* it = nullptr;
+  auto fetch = [&](int u, int i) {  // unit u, block i of this wave
+    const int rest = u & 255, s = (rest >> 5) & 1, w0 = (rest >> 6) * 8, z = rest & 31;
+    const double* Z = R + items[u >> 8].R + (long long)(s + 2 * (z + FC * (w0 + 2 * wv + i))) * FBLK;
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int t = 0; t < 8; ++t) dst[h][t] = Z[(16 * h + li) * FC + 4 * t + lg];
+      for (int t = 0; t < 8; ++t) cur[h][t] = Z[(16 * h + li) * FC + 4 * t + lg];
   };
-  fetch(0, cur);
+  auto flush = [&]() {  // the four waves' Grams of item b (S is free)
+    double* d = part + ((long long)(4 * b + 2) * sp.slots + blockIdx.x - sp.first(b)) * FBLK;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const Acc32& T = c == 0 ? T3 : T4;
+      for (int w4 = 0; w4 < 4; ++w4) {
+        if (wv == w4) {
+#pragma unroll
+          for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
+            for (int ni = 0; ni < 2; ++ni)
+#pragma unroll
+              for (int v = 0; v < 4; ++v) {
+                double* x = S + (16 * mi + 4 * v + lg) * FC + 16 * ni + li;
+                *x = (w4 == 0 ? 0.0 : *x) + T.t[mi][ni][v];
+              }
+        }
+        __syncthreads();
+      }
+      for (int o = threadIdx.x; o < FBLK; o += 256) d[(long long)c * sp.slots * FBLK + o] = S[o];
+      __syncthreads();
+    }
+  };
+  int u = sp.begin(blockIdx.x);
+  if (!GRAM && u < u1) fetch(u, 0);
 #pragma unroll 1
-  for (int zi = 0; zi < ROT_NZ64; ++zi) {
-    const int z = z0 + zi;
-    const double l1 = GRAM ? lam[it.L[0] + z] : 0.0;
+  for (; u < u1; ++u) {
+    if ((u >> 8) != b) {
+      if (GRAM && b >= 0) flush();
+      b = u >> 8;
+      it = items + b;
+      for (int o = threadIdx.x; o < FBLK; o += 256) U3s[(o & 31) * LDU + (o >> 5)] = U[it->U[2] + o];  // U3[k][j]
+      if (GRAM && threadIdx.x < 4 * FC)
+        ls[threadIdx.x >> 5][threadIdx.x & 31] = lam[it->L[threadIdx.x >> 5] + (threadIdx.x & 31)];
 #pragma unroll
+      for (int t = 0; t < 8; ++t)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) bU4[t][h] = U[it->U[3] + (4 * t + lg) + FC * (16 * h + li)];  // U4[4t+lg][16h+li]
+      acc_zero(T3);
+      acc_zero(T4);
+      __syncthreads();
+    }
+    const int rest = u & 255, s = (rest >> 5) & 1, w0 = (rest >> 6) * 8, z = rest & 31;
+#pragma unroll 1
     for (int i = 0; i < 2; ++i) {
-      const int j = 2 * zi + i;
-      if (j + 1 < 2 * ROT_NZ64) fetch(j + 1, nxt);
+      // the fences keep the LDS operands from being carried in registers between the
+      // phases, which spills
       const int wl = 2 * wv + i;
-      const double w12 = GRAM ? l1 * lam[it.L[1] + w0 + wl] : 0.0;
-      Acc32 V, Y, YT;
+      const double w12 = GRAM ? ls[0][z] * ls[1][w0 + wl] : 0.0;
+      Acc32 V, Y;
       acc_zero(V);
+      if constexpr (GRAM) fetch(u, i);
+      mm32(V, cur, bU4);  // V = Z U4
+      if constexpr (!GRAM) {
+        if (i == 0)
+          fetch(u, 1);
+        else if (u + 1 < u1)
+          fetch(u + 1, 0);
+      }
       acc_zero(Y);
-      acc_zero(YT);
-      mm32(V, cur, bU4);       // V = Z U4
-      mm32_accb(Y, aU3T, V);   // Y = U3^T V
 #pragma unroll
-      for (int t = 0; t < 8 && GRAM; ++t)  // Y^T = V^T U3
+      for (int t = 0; t < 8; ++t) {  // Y = U3^T V
+        double a[2];
 #pragma unroll
-        for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-          for (int ni = 0; ni < 2; ++ni)
-            YT.t[mi][ni] = MFMA_F64(V.t[t >> 2][mi][t & 3], aU3T[ni][t], YT.t[mi][ni]);
-#pragma unroll
-      for (int t = 0; t < 8 && GRAM; ++t)
+        for (int h = 0; h < 2; ++h) a[h] = U3s[(4 * t + lg) * LDU + 16 * h + li];
 #pragma unroll
         for (int mi = 0; mi < 2; ++mi)
 #pragma unroll
-          for (int ni = 0; ni < 2; ++ni) {
-            // T3 += Y L4 Y^T (K = r4), T4 += Y^T L3 Y (K = r3)
-            T3.t[mi][ni] = MFMA_F64(YT.t[t >> 2][mi][t & 3], w12 * lam4v[t] * YT.t[t >> 2][ni][t & 3], T3.t[mi][ni]);
-            T4.t[mi][ni] = MFMA_F64(Y.t[t >> 2][mi][t & 3], w12 * lam3v[t] * Y.t[t >> 2][ni][t & 3], T4.t[mi][ni]);
-          }
+          for (int ni = 0; ni < 2; ++ni) Y.t[mi][ni] = MFMA_F64(a[mi], V.t[t >> 2][ni][t & 3], Y.t[mi][ni]);
+      }
 #pragma unroll
       for (int mi = 0; mi < 2; ++mi)
 #pragma unroll
         for (int ni = 0; ni < 2; ++ni)
 #pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const int xb = 16 * mi + 4 * v + lg, yb = 16 * ni + li;
-            S[(yb + FC * xb) * SROW + wl] = Y.t[mi][ni][v];
-          }
+          for (int v = 0; v < 4; ++v) S[slot(16 * ni + li + FC * (16 * mi + 4 * v + lg), wl)] = Y.t[mi][ni][v];
+      if constexpr (GRAM) {
+        asm volatile("" ::: "memory");
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
+        for (int t = 0; t < 8; ++t) {  // T4 += Y^T L3 Y (K = r3)
+          const double w = w12 * ls[2][4 * t + lg];
 #pragma unroll
-        for (int t = 0; t < 8; ++t) cur[h][t] = nxt[h][t];
+          for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
+            for (int ni = 0; ni < 2; ++ni)
+              T4.t[mi][ni] = MFMA_F64(Y.t[t >> 2][mi][t & 3], w * Y.t[t >> 2][ni][t & 3], T4.t[mi][ni]);
+        }
+        asm volatile("" ::: "memory");
+        acc_zero(Y);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {  // Y^T = V^T U3
+          double a[2];
+#pragma unroll
+          for (int h = 0; h < 2; ++h) a[h] = U3s[(4 * t + lg) * LDU + 16 * h + li];
+#pragma unroll
+          for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
+            for (int ni = 0; ni < 2; ++ni) Y.t[mi][ni] = MFMA_F64(V.t[t >> 2][mi][t & 3], a[ni], Y.t[mi][ni]);
+        }
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {  // T3 += Y L4 Y^T (K = r4)
+          const double w = w12 * ls[3][4 * t + lg];
+#pragma unroll
+          for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
+            for (int ni = 0; ni < 2; ++ni)
+              T3.t[mi][ni] = MFMA_F64(Y.t[t >> 2][mi][t & 3], w * Y.t[t >> 2][ni][t & 3], T3.t[mi][ni]);
+        }
+      }
     }
     __syncthreads();
-    for (int k = threadIdx.x; k < FBLK * 4; k += blockDim.x) {
+    for (int k = threadIdx.x; k < FBLK * 4; k += 256) {
       const int o = k >> 2, pt = k & 3;
-      const int yb = o & 31, xb = o >> 5;
-      const long long qb = s + 2 * (xb + FC * yb);
-      *reinterpret_cast<double2*>(Q + it.Q + qb * FBLK + z * FC + w0 + 2 * pt) =
-          *reinterpret_cast<const double2*>(S + o * SROW + 2 * pt);
+      const long long qb = s + 2 * ((o >> 5) + FC * (o & 31));
+      *reinterpret_cast<double2*>(Q + it->Q + qb * FBLK + z * FC + w0 + 2 * pt) =
+          *reinterpret_cast<const double2*>(S + slot(o, 2 * pt));
     }
     __syncthreads();
   }
-  if (!GRAM) return;
-  double* Red = S;
-  for (int w4 = 0; w4 < 4; ++w4) {
-    if (wv == w4) {
-#pragma unroll
-      for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-        for (int ni = 0; ni < 2; ++ni)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const int rw = 16 * mi + 4 * v + lg, cl = 16 * ni + li;
-            if (w4 == 0) {
-              Red[rw * FC + cl] = T3.t[mi][ni][v];
-              Red[FBLK + rw * FC + cl] = T4.t[mi][ni][v];
-            } else {
-              Red[rw * FC + cl] += T3.t[mi][ni][v];
-              Red[FBLK + rw * FC + cl] += T4.t[mi][ni][v];
-            }
-          }
-    }
-    __syncthreads();
-  }
-  double* d3 = part + it.part + (long long)(2 * EIG_NPART + q) * FBLK;
-  double* d4 = part + it.part + (long long)(3 * EIG_NPART + q) * FBLK;
-  for (int o = threadIdx.x; o < FBLK; o += blockDim.x) {
-    d3[o] = Red[o];
-    d4[o] = Red[FBLK + o];
-  }
+  if (GRAM && b >= 0) flush();
 }
 
-// gram12, FP64: WG (256 threads) -> 4 NB consecutive Q blocks, wave -> NB.  Each
-// block is loaded once (coalesced, one block of look-ahead in registers) into a
-// per-wave LDS tile, from which both operand orientations (D for T'1, D^T for
-// T'2) are read.  grid (EIG_NPART, items)
-template <int NB>
-__global__ __launch_bounds__(256) void k_gram12_f64(const EigItem* __restrict__ items,
-                                                    const double* __restrict__ Q,
-                                                    const double* __restrict__ lam,
-                                                    double* __restrict__ part) {
+// gram12, FP64: a unit is four consecutive Q blocks, one per wave, each loaded once
+// (coalesced, one block of look-ahead in registers) into a per-wave LDS tile, from
+// which both operand orientations (D for T'1, D^T for T'2) are read.  BLOCKS: Q
+// blocks per site.  36 sites of 2048 blocks: 253 -> 206 us with the even split.
+template <int BLOCKS>
+__global__ __launch_bounds__(256, 2) void k_gram12_f64(const EigItem* __restrict__ items, EigSplit sp,
+                                                       const double* __restrict__ Q,
+                                                       const double* __restrict__ lam,
+                                                       double* __restrict__ part) {
+  constexpr int UNITS = BLOCKS / 4;
   __shared__ double Db[4][FC * LD8];
-  const EigItem it = items[blockIdx.y];
-  const int q = blockIdx.x;
   const int l = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int li = l & 15, lg = l >> 4;
   double lam1v[8], lam2v[8];
-#pragma unroll
-  for (int t = 0; t < 8; ++t) {
-    lam1v[t] = lam[it.L[0] + 4 * t + lg];
-    lam2v[t] = lam[it.L[1] + 4 * t + lg];
-  }
   Acc32 T1, T2;
-  acc_zero(T1);
-  acc_zero(T2);
-  const long long r0 = (long long)q * (4 * NB) + wv * NB;
   double* db = Db[wv];
   double2 nD[8];
+  const int u1 = sp.begin(blockIdx.x + 1);
+  int b = -1;
+  const EigItem* it = nullptr;
+  auto fetch = [&](int u) {
+    const double* D = Q + items[u / UNITS].Q + (long long)(4 * (u % UNITS) + wv) * FBLK;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) nD[j] = *reinterpret_cast<const double2*>(Q + it.Q + r0 * FBLK + 2 * l + 128 * j);
+    for (int j = 0; j < 8; ++j) nD[j] = *reinterpret_cast<const double2*>(D + 2 * l + 128 * j);
+  };
+  auto flush = [&]() {
+    __syncthreads();  // the tiles are free
+    double* Red = &Db[0][0];
+    double* d = part + ((long long)4 * b * sp.slots + blockIdx.x - sp.first(b)) * FBLK;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const int o = 2 * l + 128 * j, a = o >> 5, b = o & 31;
-    db[a * LD8 + b] = nD[j].x;
-    db[a * LD8 + b + 1] = nD[j].y;
-  }
-#pragma unroll 1
-  for (int i = 0; i < NB; ++i) {
-    __builtin_amdgcn_s_waitcnt(0);
-    __builtin_amdgcn_wave_barrier();
-    if (i + 1 < NB) {
+    for (int c = 0; c < 2; ++c) {
+      const Acc32& T = c == 0 ? T1 : T2;
+      for (int w4 = 0; w4 < 4; ++w4) {
+        if (wv == w4) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j)
-        nD[j] = *reinterpret_cast<const double2*>(Q + it.Q + (r0 + i + 1) * FBLK + 2 * l + 128 * j);
+          for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
+            for (int ni = 0; ni < 2; ++ni)
+#pragma unroll
+              for (int v = 0; v < 4; ++v) {
+                double* x = Red + (16 * mi + 4 * v + lg) * FC + 16 * ni + li;
+                *x = (w4 == 0 ? 0.0 : *x) + T.t[mi][ni][v];
+              }
+        }
+        __syncthreads();
+      }
+      for (int o = threadIdx.x; o < FBLK; o += 256) d[(long long)c * sp.slots * FBLK + o] = Red[o];
+      __syncthreads();
     }
-    const long long qb = r0 + i;
-    const int r3 = (int)((qb >> 1) & 31), r4 = (int)(qb >> 6);
-    const double w34 = lam[it.L[2] + r3] * lam[it.L[3] + r4];
-    double cr[2][8], cc[2][8];
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
+  };
+  int u = sp.begin(blockIdx.x);
+  if (u < u1) fetch(u);
+#pragma unroll 1
+  for (; u < u1; ++u) {
+    if (u / UNITS != b) {
+      if (b >= 0) flush();
+      b = u / UNITS;
+      it = items + b;
 #pragma unroll
       for (int t = 0; t < 8; ++t) {
-        cr[h][t] = db[(16 * h + li) * LD8 + 4 * t + lg];  // D[16h+li][4t+lg]
-        cc[h][t] = db[(4 * t + lg) * LD8 + 16 * h + li];  // D[4t+lg][16h+li]
+        lam1v[t] = lam[it->L[0] + 4 * t + lg];
+        lam2v[t] = lam[it->L[1] + 4 * t + lg];
       }
+      acc_zero(T1);
+      acc_zero(T2);
+    }
+    // every lane's reads of the last block were issued before the tile is overwritten
+    __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int t = 0; t < 8; ++t)
+    for (int j = 0; j < 8; ++j) {
+      const int o = 2 * l + 128 * j, a = o >> 5, c = o & 31;
+      db[a * LD8 + c] = nD[j].x;
+      db[a * LD8 + c + 1] = nD[j].y;
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __builtin_amdgcn_wave_barrier();
+    if (u + 1 < u1) fetch(u + 1);
+    const int qb = 4 * (u % UNITS) + wv;
+    const int r3 = (qb >> 1) & 31, r4 = qb >> 6;
+    const double w34 = lam[it->L[2] + r3] * lam[it->L[3] + r4];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      double cr[2], cc[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        cr[h] = db[(16 * h + li) * LD8 + 4 * t + lg];  // D[16h+li][4t+lg]
+        cc[h] = db[(4 * t + lg) * LD8 + 16 * h + li];  // D[4t+lg][16h+li]
+      }
 #pragma unroll
       for (int mi = 0; mi < 2; ++mi)
 #pragma unroll
         for (int ni = 0; ni < 2; ++ni) {
           // T1 += D L2 D^T (K = r2), T2 += D^T L1 D (K = r1)
-          T1.t[mi][ni] = MFMA_F64(cr[mi][t], w34 * lam2v[t] * cr[ni][t], T1.t[mi][ni]);
-          T2.t[mi][ni] = MFMA_F64(cc[mi][t], w34 * lam1v[t] * cc[ni][t], T2.t[mi][ni]);
+          T1.t[mi][ni] = MFMA_F64(cr[mi], w34 * lam2v[t] * cr[ni], T1.t[mi][ni]);
+          T2.t[mi][ni] = MFMA_F64(cc[mi], w34 * lam1v[t] * cc[ni], T2.t[mi][ni]);
         }
-    // every lane's reads of this block are issued before the tile is overwritten
-    __builtin_amdgcn_wave_barrier();
-    if (i + 1 < NB) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int o = 2 * l + 128 * j, a = o >> 5, b = o & 31;
-        db[a * LD8 + b] = nD[j].x;
-        db[a * LD8 + b + 1] = nD[j].y;
-      }
     }
   }
-  __syncthreads();
-  double* Red = &Db[0][0];  // 4 * 32 * 33 >= 2 * 1024
-  for (int w4 = 0; w4 < 4; ++w4) {
-    if (wv == w4) {
-#pragma unroll
-      for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-        for (int ni = 0; ni < 2; ++ni)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const int rw = 16 * mi + 4 * v + lg, cl = 16 * ni + li;
-            if (w4 == 0) {
-              Red[rw * FC + cl] = T1.t[mi][ni][v];
-              Red[FBLK + rw * FC + cl] = T2.t[mi][ni][v];
-            } else {
-              Red[rw * FC + cl] += T1.t[mi][ni][v];
-              Red[FBLK + rw * FC + cl] += T2.t[mi][ni][v];
-            }
-          }
-    }
-    __syncthreads();
-  }
-  double* d1 = part + it.part + (long long)(0 * EIG_NPART + q) * FBLK;
-  double* d2 = part + it.part + (long long)(1 * EIG_NPART + q) * FBLK;
-  for (int o = threadIdx.x; o < FBLK; o += blockDim.x) {
-    d1[o] = Red[o];
-    d2[o] = Red[FBLK + o];
-  }
+  if (b >= 0) flush();
 }
 
 // ---------------------------------------------------------------------------
@@ -2587,31 +2645,41 @@ __global__ __launch_bounds__(256) void k_rot3_d3_f64(const EigItem* __restrict__
     }
     __syncthreads();
   }
-  double* d3 = part + it.part + (long long)(2 * EIG_NPART + q) * FBLK;
+  double* d3 = part + ((long long)(4 * blockIdx.y + 2) * EIG_NPART + q) * FBLK;
   for (int o = threadIdx.x; o < FBLK; o += blockDim.x) d3[o] = Red[o];
 }
 
 // Finaliser of the eigenbasis pipeline: T'_c = sum of the partial Grams (FP64),
 // T_c = U_c T'_c U_c^T, symmetrised, normalised, message_diff / residual
-// against the previous message.  grid (4, items), 256 threads.
+// against the previous message.  sp12, sp34: how the launches of bonds 1, 2 and 3, 4
+// were split; part: the items' first partial.  grid (4, items), 256 threads.
 template <typename TP, typename TM>
 __global__ __launch_bounds__(256) void k_eig_finalize(const EigItem* __restrict__ items,
                                                       const TP* __restrict__ part,
                                                       const double* __restrict__ U64, const TM* msg_in,
                                                       TM* msg_out, MsgStat* __restrict__ stats,
                                                       int normalize, const int* __restrict__ sexp,
-                                                      const int* __restrict__ lexp) {
+                                                      const int* __restrict__ lexp, EigSplit sp12, EigSplit sp34) {
   constexpr int LD = 33;
   __shared__ double Tp[FC * LD], Us[FC * LD], X[FC * LD];
   __shared__ double red[8];
   const EigItem* itp = items + blockIdx.y;  // fields indexed by the bond: read in place
   const int cb = blockIdx.x;
-  const TP* pp = part + itp->part + (long long)cb * EIG_NPART * FBLK;
+  const EigSplit& sp = cb < 2 ? sp12 : sp34;
+  const TP* pp = part + (long long)(4 * blockIdx.y + cb) * sp.slots * FBLK + threadIdx.x;
+  const int np = sp.parts(blockIdx.y);
   const long long uoff = itp->U[cb];
-  for (int o = threadIdx.x; o < FBLK; o += blockDim.x) {
-    double sum = 0;
-    for (int ch = 0; ch < EIG_NPART; ++ch) sum += (double)pp[(long long)ch * FBLK + o];
-    Tp[(o >> 5) * LD + (o & 31)] = sum;  // T'[r][r']
+  double sum[FBLK / 256];
+#pragma unroll
+  for (int j = 0; j < FBLK / 256; ++j) sum[j] = 0;
+#pragma unroll 4
+  for (int ch = 0; ch < np; ++ch)
+#pragma unroll
+    for (int j = 0; j < FBLK / 256; ++j) sum[j] += (double)pp[(long long)ch * FBLK + 256 * j];
+#pragma unroll
+  for (int j = 0; j < FBLK / 256; ++j) {
+    const int o = threadIdx.x + 256 * j;
+    Tp[(o >> 5) * LD + (o & 31)] = sum[j];  // T'[r][r']
     const double u = U64[uoff + o];   // U[b + 32 r]
     Us[(o & 31) * LD + (o >> 5)] = u;    // Us[b][r]
   }
@@ -3411,7 +3479,9 @@ int fast_prepare(itnbp_net* net, const std::vector<int>& seq, int acc_f64, std::
   }
   // partial sums: the absorbed-pair passes need 2 items x FUSED_CHUNKS x 2 matrices
   // per bulk vertex, the eigenbasis pipeline 4 bonds x EIG_NPART per (bulk or degree-3) site
-  const size_t nparts = std::max(ni * FUSED_CHUNKS * 2, (size_t)(nb + st->e3items.size()) * 4 * EIG_NPART);
+  const size_t nparts = std::max(ni * FUSED_CHUNKS * 2,
+                                 ((size_t)nb * eig_slots(std::max(1, (int)nb), ctx->num_cu) +
+                                  st->e3items.size() * (size_t)EIG_NPART) * 4);
   if (acc_f64) {
     ITNBP_RETCHK(ensure_buf(ctx, st->P64, (size_t)2 * nb * per * 8));
     ITNBP_RETCHK(ensure_buf(ctx, st->part64, nparts * FBLK * 8));
@@ -3626,6 +3696,12 @@ static int eig_sweep(itnbp_ctx* ctx, FastState* st, int acc_f64, const void* msg
   st->eig_warm = true;
   ++st->eig_count;
   const int e1 = prof_mark(ctx);
+  const int slots = eig_slots(std::max(1, nb), ctx->num_cu);
+  const EigSplit none{0, 0, 0, EIG_NPART};
+  const EigSplit sp34 = nb > 0 ? eig_split(nb, 8 * FC, slots, ctx->num_cu) : none;
+  const EigSplit sp12 = nb > 0 ? eig_split(nb, FC * FC / 2, slots, ctx->num_cu) : none;
+  const EigSplit spd3 = n3 > 0 ? eig_split(n3, FC / 2, EIG_NPART, ctx->num_cu) : none;
+  double* part3 = (double*)st->part64.p + (long long)nb * 4 * slots * FBLK;  // the degree-3 sites' partials
   if (nb > 0) {
     // rot12.  FP64: the rot34 kernel without Grams (items k1e map U1, U2 to the
     // U[2], U[3] slots, psi layout B to R and the R buffer to Q), whose persistent
@@ -3633,7 +3709,7 @@ static int eig_sweep(itnbp_ctx* ctx, FastState* st, int acc_f64, const void* msg
     // two workgroups per CU stream faster than the rot34 loop's one.
     if (acc_f64) {
       const EigItem* k1e = (const EigItem*)st->d_k1eitems.p;
-      hipLaunchKernelGGL(k_rot34_f64<false>, dim3(EIG_NPART, nb), dim3(256), 0, ctx->stream, k1e,
+      hipLaunchKernelGGL(k_rot34_f64<false>, dim3(sp34.wgs), dim3(256), 0, ctx->stream, k1e, sp34,
                          (const double*)st->lay64.p, (const double*)st->eigU64.p, (const double*)st->eigL64.p,
                          (double*)st->P64.p, (double*)nullptr);
     } else {
@@ -3643,7 +3719,7 @@ static int eig_sweep(itnbp_ctx* ctx, FastState* st, int acc_f64, const void* msg
   const int e2 = prof_mark(ctx);
   if (nb > 0) {
     if (acc_f64)
-      hipLaunchKernelGGL(k_rot34_f64<true>, dim3(EIG_NPART, nb), dim3(256), 0, ctx->stream, ei, (const double*)st->P64.p,
+      hipLaunchKernelGGL(k_rot34_f64<true>, dim3(sp34.wgs), dim3(256), 0, ctx->stream, ei, sp34, (const double*)st->P64.p,
                          (const double*)st->eigU64.p, (const double*)st->eigL64.p, (double*)st->P64.p,
                          (double*)st->part64.p);
     else
@@ -3652,7 +3728,7 @@ static int eig_sweep(itnbp_ctx* ctx, FastState* st, int acc_f64, const void* msg
   const int e3m = prof_mark(ctx);
   if (nb > 0) {
     if (acc_f64)
-      hipLaunchKernelGGL(k_gram12_f64<32>, dim3(EIG_NPART, nb), dim3(256), 0, ctx->stream, ei,
+      hipLaunchKernelGGL(k_gram12_f64<2 * FC * FC>, dim3(sp12.wgs), dim3(256), 0, ctx->stream, ei, sp12,
                          (const double*)st->P64.p, (const double*)st->eigL64.p, (double*)st->part64.p);
     else
       eig16(ctx, st, 3, nb, n3);
@@ -3664,9 +3740,9 @@ static int eig_sweep(itnbp_ctx* ctx, FastState* st, int acc_f64, const void* msg
                          (const double*)st->eigU64.p, (double*)st->P3_64.p);
       hipLaunchKernelGGL(k_rot3_d3_f64, dim3(EIG_NPART, n3), dim3(256), 0, ctx->stream, e3,
                          (const double*)st->P3_64.p, (const double*)st->eigU64.p, (const double*)st->eigL64.p,
-                         (double*)st->P3_64.p, (double*)st->part64.p);
-      hipLaunchKernelGGL(k_gram12_f64<1>, dim3(EIG_NPART, n3), dim3(256), 0, ctx->stream, e3,
-                         (const double*)st->P3_64.p, (const double*)st->eigL64.p, (double*)st->part64.p);
+                         (double*)st->P3_64.p, part3);
+      hipLaunchKernelGGL(k_gram12_f64<2 * FC>, dim3(spd3.wgs), dim3(256), 0, ctx->stream, e3, spd3,
+                         (const double*)st->P3_64.p, (const double*)st->eigL64.p, part3);
     } else {
       eig16(ctx, st, 4, nb, n3);
     }
@@ -3676,20 +3752,22 @@ static int eig_sweep(itnbp_ctx* ctx, FastState* st, int acc_f64, const void* msg
     if (nb > 0)
       hipLaunchKernelGGL((k_eig_finalize<double, double>), dim3(4, nb), dim3(256), 0, ctx->stream, ei,
                          (const double*)st->part64.p, (const double*)st->eigU64.p, (const double*)msg_in,
-                         (double*)msg_out, stats, normalize, (const int*)nullptr, (const int*)nullptr);
+                         (double*)msg_out, stats, normalize, (const int*)nullptr, (const int*)nullptr, sp12, sp34);
     if (n3 > 0)
       hipLaunchKernelGGL((k_eig_finalize<double, double>), dim3(3, n3), dim3(256), 0, ctx->stream, e3,
-                         (const double*)st->part64.p, (const double*)st->eigU64.p, (const double*)msg_in,
-                         (double*)msg_out, stats, normalize, (const int*)nullptr, (const int*)nullptr);
+                         (const double*)part3, (const double*)st->eigU64.p, (const double*)msg_in,
+                         (double*)msg_out, stats, normalize, (const int*)nullptr, (const int*)nullptr, spd3, none);
   } else {
     if (nb > 0)
       hipLaunchKernelGGL((k_eig_finalize<float, float>), dim3(4, nb), dim3(256), 0, ctx->stream, ei,
                          (const float*)st->part32.p, (const double*)st->eigU64.p, (const float*)msg_in,
-                         (float*)msg_out, stats, normalize, (const int*)st->sexp.p, (const int*)st->eigLexp.p);
+                         (float*)msg_out, stats, normalize, (const int*)st->sexp.p, (const int*)st->eigLexp.p, none,
+                         none);
     if (n3 > 0)
       hipLaunchKernelGGL((k_eig_finalize<float, float>), dim3(3, n3), dim3(256), 0, ctx->stream, e3,
-                         (const float*)st->part32.p, (const double*)st->eigU64.p, (const float*)msg_in,
-                         (float*)msg_out, stats, normalize, (const int*)st->sexp.p, (const int*)st->eigLexp.p);
+                         (const float*)st->part32.p + (long long)nb * 4 * EIG_NPART * FBLK, (const double*)st->eigU64.p, (const float*)msg_in,
+                         (float*)msg_out, stats, normalize, (const int*)st->sexp.p, (const int*)st->eigLexp.p, none,
+                         none);
   }
   const int e6 = prof_mark(ctx);
   prof_add(ctx, "eigh", e0, e1);
@@ -3813,9 +3891,10 @@ static int rotated_sites_setup(itnbp_net* net, const std::vector<int>& want, siz
   st->eig_warm = true;
   if (nbs > 0) {
     double* P = (double*)st->P64.p;
-    hipLaunchKernelGGL(k_rot34_f64<false>, dim3(EIG_NPART, nbs), dim3(256), 0, ctx->stream, d_k1,
+    const EigSplit sp = eig_split(nbs, 8 * FC, eig_slots(nbs, ctx->num_cu), ctx->num_cu);
+    hipLaunchKernelGGL(k_rot34_f64<false>, dim3(sp.wgs), dim3(256), 0, ctx->stream, d_k1, sp,
                        (const double*)st->lay64.p, U, L, P, (double*)nullptr);
-    hipLaunchKernelGGL(k_rot34_f64<false>, dim3(EIG_NPART, nbs), dim3(256), 0, ctx->stream, d_e, (const double*)P, U,
+    hipLaunchKernelGGL(k_rot34_f64<false>, dim3(sp.wgs), dim3(256), 0, ctx->stream, d_e, sp, (const double*)P, U,
                        L, P, (double*)nullptr);
   }
   if (n3s > 0) {
