@@ -59,16 +59,19 @@ __host__ __device__ inline T zerov() {
 __device__ inline double shfl_xor_v(double v, int m) { return __shfl_xor(v, m); }
 __device__ inline cplx shfl_xor_v(cplx v, int m) { return cplx{__shfl_xor(v.x, m), __shfl_xor(v.y, m)}; }
 
-// sum over the block (256 threads); red holds 4 doubles
+constexpr int LY_THREADS = 512;
+
+// sum over the block; red holds a double per wave
 __device__ double block_sum_d(double v, double* red) {
   for (int m = 32; m > 0; m >>= 1) v += __shfl_xor(v, m);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
-  return (red[0] + red[1]) + (red[2] + red[3]);
+  double s = 0;
+#pragma unroll
+  for (int w = 0; w < LY_THREADS / 64; ++w) s += red[w];
+  return s;
 }
-
-constexpr int LY_THREADS = 256;
 
 // one site of the two-layer network
 struct LVDesc {
@@ -88,79 +91,105 @@ struct LTask {
   long long out_off, old_off;
 };
 
-// grid (tasks), 256 threads; scratch: three areas of sstride elements per workgroup
-template <typename T>
+// integers and quotients of the index loops: single-precision quotients where every
+// index is below 2^20
+template <bool SMALL>
+struct IdxDiv {
+  typedef int I;
+  SmallDiv q;
+  __device__ explicit IdxDiv(int d) : q(small_div((unsigned)d)) {}
+  __device__ int div(int x) const { return (int)q.div((unsigned)x); }
+};
+template <>
+struct IdxDiv<false> {
+  typedef long long I;
+  long long d;
+  __device__ explicit IdxDiv(long long d_) : d(d_) {}
+  __device__ long long div(long long x) const { return x / d; }
+};
+
+// grid (tasks), LY_THREADS threads; two areas of sstride elements and one of an open pair
+// per workgroup: in LDS while they fit (at most 2^20 entries per site then, by far),
+// else in scratch (three areas of sstride).
+//
+// Bound: latency; a degree-4 site of chi = 5 (complex) is 1250 entries.  With 64-bit
+// divisions per entry and the areas in global memory a sweep of a 6x6 lattice took
+// 34 us, against 16.
+template <typename T, bool LDS>
 __global__ __launch_bounds__(LY_THREADS) void k_layer_task(const LVDesc* __restrict__ vds,
                                                           const LTask* __restrict__ tasks,
                                                           const T* __restrict__ ket, const T* __restrict__ bra,
                                                           const T* msg_in, T* out, MsgStat* __restrict__ stats,
                                                           T* __restrict__ scratch, long long sstride) {
-  __shared__ double red[4];
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ double red[LY_THREADS / 64];
+  typedef IdxDiv<LDS> Div;
+  typedef typename Div::I I;
   const LTask t = tasks[blockIdx.x];
-  const LVDesc V = vds[t.v];
+  const LVDesc& V = vds[t.v];
   const int k = V.k, tid = threadIdx.x;
-  int dims[ITNBP_MAXR];
-  for (int a = 0; a <= k; ++a) dims[a] = V.kd[a];
-  long long D = V.Dk;
-  T* area = scratch + (long long)blockIdx.x * 3 * sstride;
+  I D = (I)V.Dk;
+  T* area = LDS ? reinterpret_cast<T*>(smem) : scratch + (long long)blockIdx.x * 3 * sstride;
   const T* X = ket + V.ket_off;
   int cur = -1;
   // 1. absorb every incoming message but the open bond's: axis a goes from the
-  //    ket dimension to the bra dimension
+  //    ket dimension to the bra dimension (A: product of the axes before it)
+  I A = V.kd[0], Aj = 1;
   for (int a = 1; a <= k; ++a) {
-    if (a == t.j) continue;
     const int nk = V.kd[a], nb = V.bd[a];
+    if (a == t.j) {
+      Aj = A;
+      A *= nk;
+      continue;
+    }
     const T* M = msg_in + V.in_msg[a];
-    long long A = 1;
-    for (int b = 0; b < a; ++b) A *= dims[b];
-    const long long B = D / (A * nk);
-    const long long Dn = A * nb * B;
+    const I Dn = D / nk * nb;
     T* Y = area + (long long)((cur + 1) & 1) * sstride;
-    for (long long i = tid; i < Dn; i += LY_THREADS) {
-      const long long lo = i % A, rest = i / A;
-      const int c = (int)(rest % nb);
-      const long long hi = rest / nb;
-      const long long base = lo + A * nk * hi;
+    const Div dA(A), dnb(nb);
+    for (I i = tid; i < Dn; i += LY_THREADS) {
+      const I rest = dA.div(i), lo = i - rest * A, hi = dnb.div(rest);
+      const int c = (int)(rest - hi * nb);
+      const T* x = X + lo + A * nk * hi;
+      const T* m = M + nk * c;
       T acc = zerov<T>();
-      for (int x = 0; x < nk; ++x) acc += X[base + A * x] * M[x + (long long)nk * c];
+#pragma unroll 4
+      for (int b = 0; b < nk; ++b) acc += x[A * b] * m[b];
       Y[i] = acc;
     }
     __threadfence_block();
     __syncthreads();
     X = Y;
     cur = (cur + 1) & 1;
-    dims[a] = nb;
+    A *= nb;
     D = Dn;
   }
   // 2. contract with conj(bra) over every index but the open one:
   //    T[o] = sum_r X[offx(row) + roff(r)] conj(bra[offy(col) + roff(r)])
   const T* P = bra + V.bra_off;
-  long long Aj, nrow, ncol;
+  int nrow, ncol;
   if (t.j >= 1) {
-    Aj = 1;
-    for (int b = 0; b < t.j; ++b) Aj *= dims[b];
     nrow = V.kd[t.j];
     ncol = V.bd[t.j];
   } else if (t.j == 0) {
-    Aj = 1;
     nrow = ncol = V.kd[0];
   } else {
-    Aj = 1;
     nrow = ncol = 1;
   }
-  const long long R = D / nrow;  // summed elements per output
-  const int P2 = (int)(nrow * ncol);
+  const I R = D / nrow;  // summed elements per output
+  const int P2 = nrow * ncol;
   T* Tb = area + 2 * sstride;
   int G = 1;
   while (G * 2 * P2 <= LY_THREADS && G < 64) G *= 2;
   const int per = LY_THREADS / G;
+  const Div dAj(Aj);
   for (int ob = 0; ob < P2; ob += per) {
     const int o = ob + tid / G, gi = tid % G;
     T acc = zerov<T>();
     if (o < P2) {
-      const long long row = o % nrow, col = o / nrow;
-      for (long long r = gi; r < R; r += G) {
-        const long long lo = r % Aj, hi = r / Aj;
+      const int row = o % nrow, col = o / nrow;
+#pragma unroll 4
+      for (I r = gi; r < R; r += G) {
+        const I hi = dAj.div(r), lo = r - hi * Aj;
         acc += X[lo + Aj * (row + nrow * hi)] * conjv(P[lo + Aj * (col + ncol * hi)]);
       }
     }
@@ -285,26 +314,39 @@ itnbp_graph::Topo topo_of(const itnbp_lnet* n) {
   return itnbp_graph::Topo{n->nv, n->ne, n->edges.data(), n->inc_ptr.data(), n->inc_edge.data()};
 }
 
-// launch the tasks (scratch sized for them); msg_in/out may be the same buffer
-// when no task reads a message another task of the launch writes
+// LDS of a task, or 0 if it does not fit
+size_t layer_lds(const itnbp_lnet* L) {
+  const size_t b = (2 * (size_t)L->maxD + L->maxP2) * L->es;
+  return b <= 160 * 1024 - 256 ? b : 0;
+}
+
+template <typename T>
+int launch_layer_tasks_t(itnbp_lnet* L, const LTask* tasks, size_t n, const void* msg_in, void* out, MsgStat* stats) {
+  itnbp_ctx* ctx = L->ctx;
+  const size_t lds = layer_lds(L);
+  const long long sstride = lds ? L->maxD : std::max<long long>(L->maxD, L->maxP2);
+  if (!lds) ITNBP_RETCHK(ensure_buf(ctx, L->scratch, n * 3 * (size_t)sstride * L->es));
+  const auto kern = lds ? k_layer_task<T, true> : k_layer_task<T, false>;
+  if (lds) ITNBP_HIPCHK(ctx, hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  hipLaunchKernelGGL(kern, dim3((unsigned)n), dim3(LY_THREADS), lds, ctx->stream, (const LVDesc*)L->d_vdesc.p, tasks,
+                     (const T*)L->d_ket, (const T*)L->d_bra, (const T*)msg_in, (T*)out, stats, (T*)L->scratch.p, sstride);
+  ITNBP_HIPCHK(ctx, hipGetLastError());
+  return ITNBP_OK;
+}
+int launch_layer_tasks(itnbp_lnet* L, const LTask* tasks, size_t n, const void* msg_in, void* out, MsgStat* stats) {
+  return L->cplx ? launch_layer_tasks_t<cplx>(L, tasks, n, msg_in, out, stats)
+                 : launch_layer_tasks_t<double>(L, tasks, n, msg_in, out, stats);
+}
+
+// launch the tasks; msg_in/out may be the same buffer when no task reads a message
+// another task of the launch writes
 int run_layer_tasks(itnbp_lnet* L, const std::vector<LTask>& tasks, const void* msg_in, void* out, MsgStat* stats) {
   itnbp_ctx* ctx = L->ctx;
   if (tasks.empty()) return ITNBP_OK;
-  const long long sstride = std::max<long long>(L->maxD, L->maxP2);
   const size_t n = tasks.size();
   ITNBP_RETCHK(ensure_buf(ctx, L->tasks, n * sizeof(LTask)));
-  ITNBP_RETCHK(ensure_buf(ctx, L->scratch, n * 3 * (size_t)sstride * L->es));
   ITNBP_HIPCHK(ctx, hipMemcpyAsync(L->tasks.p, tasks.data(), n * sizeof(LTask), hipMemcpyHostToDevice, ctx->stream));
-  if (L->cplx)
-    hipLaunchKernelGGL(k_layer_task<cplx>, dim3((unsigned)n), dim3(LY_THREADS), 0, ctx->stream,
-                       (const LVDesc*)L->d_vdesc.p, (const LTask*)L->tasks.p, (const cplx*)L->d_ket,
-                       (const cplx*)L->d_bra, (const cplx*)msg_in, (cplx*)out, stats, (cplx*)L->scratch.p, sstride);
-  else
-    hipLaunchKernelGGL(k_layer_task<double>, dim3((unsigned)n), dim3(LY_THREADS), 0, ctx->stream,
-                       (const LVDesc*)L->d_vdesc.p, (const LTask*)L->tasks.p, (const double*)L->d_ket,
-                       (const double*)L->d_bra, (const double*)msg_in, (double*)out, stats,
-                       (double*)L->scratch.p, sstride);
-  ITNBP_HIPCHK(ctx, hipGetLastError());
+  ITNBP_RETCHK(launch_layer_tasks(L, (const LTask*)L->tasks.p, n, msg_in, out, stats));
   // the task table is reused by the next call: finish this launch first
   ITNBP_HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
   return ITNBP_OK;
