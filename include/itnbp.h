@@ -287,6 +287,8 @@ int itnbp_lnet_fold_operator(itnbp_lnet* lnet, const double* psi, const int* psi
 int itnbp_lnet_get_ket(itnbp_lnet* lnet, double* ket);
 int itnbp_lnet_set_message(itnbp_lnet* lnet, int msg_id, const double* data);
 int itnbp_lnet_get_message(itnbp_lnet* lnet, int msg_id, double* data);
+/* every message in id order, set or not (itnbp_lnet_msg_numel elements) */
+int itnbp_lnet_get_messages(itnbp_lnet* lnet, double* data);
 int itnbp_lnet_message_is_set(itnbp_lnet* lnet, int msg_id);
 /* delta(b_ket, b_bra) on every message (equal bond dimensions only) */
 int itnbp_lnet_init_identity_messages(itnbp_lnet* lnet);

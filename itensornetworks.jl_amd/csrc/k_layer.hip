@@ -18,6 +18,7 @@
 // matrix, and with nothing open the vertex scalar (beliefpropagationcache.jl:107-113).
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <memory>
 #include <numeric>
 #include <string>
@@ -120,7 +121,8 @@ __global__ __launch_bounds__(LY_THREADS) void k_layer_task(const LVDesc* __restr
                                                           const LTask* __restrict__ tasks,
                                                           const T* __restrict__ ket, const T* __restrict__ bra,
                                                           const T* msg_in, T* out, MsgStat* __restrict__ stats,
-                                                          T* __restrict__ scratch, long long sstride) {
+                                                          int* __restrict__ badflag, T* __restrict__ scratch,
+                                                          long long sstride) {
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ double red[LY_THREADS / 64];
   typedef IdxDiv<LDS> Div;
@@ -238,6 +240,7 @@ __global__ __launch_bounds__(LY_THREADS) void k_layer_task(const LVDesc* __restr
     st.norm = nrm;
     st.bad = (bad > 0 || !isfinite(nrm)) ? 1.0 : 0.0;
     stats[t.slot] = st;
+    if (st.bad > 0) *badflag = 1;  // every writer stores the same value
   }
 }
 
@@ -321,7 +324,8 @@ size_t layer_lds(const itnbp_lnet* L) {
 }
 
 template <typename T>
-int launch_layer_tasks_t(itnbp_lnet* L, const LTask* tasks, size_t n, const void* msg_in, void* out, MsgStat* stats) {
+int launch_layer_tasks_t(itnbp_lnet* L, const LTask* tasks, size_t n, const void* msg_in, void* out, MsgStat* stats,
+                         int* bad) {
   itnbp_ctx* ctx = L->ctx;
   const size_t lds = layer_lds(L);
   const long long sstride = lds ? L->maxD : std::max<long long>(L->maxD, L->maxP2);
@@ -329,27 +333,22 @@ int launch_layer_tasks_t(itnbp_lnet* L, const LTask* tasks, size_t n, const void
   const auto kern = lds ? k_layer_task<T, true> : k_layer_task<T, false>;
   if (lds) ITNBP_HIPCHK(ctx, hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   hipLaunchKernelGGL(kern, dim3((unsigned)n), dim3(LY_THREADS), lds, ctx->stream, (const LVDesc*)L->d_vdesc.p, tasks,
-                     (const T*)L->d_ket, (const T*)L->d_bra, (const T*)msg_in, (T*)out, stats, (T*)L->scratch.p, sstride);
+                     (const T*)L->d_ket, (const T*)L->d_bra, (const T*)msg_in, (T*)out, stats, bad, (T*)L->scratch.p,
+                     sstride);
   ITNBP_HIPCHK(ctx, hipGetLastError());
   return ITNBP_OK;
 }
-int launch_layer_tasks(itnbp_lnet* L, const LTask* tasks, size_t n, const void* msg_in, void* out, MsgStat* stats) {
-  return L->cplx ? launch_layer_tasks_t<cplx>(L, tasks, n, msg_in, out, stats)
-                 : launch_layer_tasks_t<double>(L, tasks, n, msg_in, out, stats);
+int launch_layer_tasks(itnbp_lnet* L, const LTask* tasks, size_t n, const void* msg_in, void* out, MsgStat* stats,
+                       int* bad) {
+  return L->cplx ? launch_layer_tasks_t<cplx>(L, tasks, n, msg_in, out, stats, bad)
+                 : launch_layer_tasks_t<double>(L, tasks, n, msg_in, out, stats, bad);
 }
 
-// launch the tasks; msg_in/out may be the same buffer when no task reads a message
-// another task of the launch writes
-int run_layer_tasks(itnbp_lnet* L, const std::vector<LTask>& tasks, const void* msg_in, void* out, MsgStat* stats) {
-  itnbp_ctx* ctx = L->ctx;
+// densities and scalars: upload and launch the tasks
+int run_layer_tasks(itnbp_lnet* L, const std::vector<LTask>& tasks, const void* msg_in, void* out) {
   if (tasks.empty()) return ITNBP_OK;
-  const size_t n = tasks.size();
-  ITNBP_RETCHK(ensure_buf(ctx, L->tasks, n * sizeof(LTask)));
-  ITNBP_HIPCHK(ctx, hipMemcpyAsync(L->tasks.p, tasks.data(), n * sizeof(LTask), hipMemcpyHostToDevice, ctx->stream));
-  ITNBP_RETCHK(launch_layer_tasks(L, (const LTask*)L->tasks.p, n, msg_in, out, stats));
-  // the task table is reused by the next call: finish this launch first
-  ITNBP_HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-  return ITNBP_OK;
+  ITNBP_RETCHK(upload(L->ctx, L->tasks, tasks.data(), tasks.size() * sizeof(LTask)));
+  return launch_layer_tasks(L, (const LTask*)L->tasks.p, tasks.size(), msg_in, out, nullptr, nullptr);
 }
 
 int axis_into(const itnbp_lnet* L, int v, int e) {
@@ -396,39 +395,52 @@ int lnet_update(itnbp_lnet* L, const itnbp_update_opts* o, itnbp_update_result* 
   if (const int rc = itnbp_graph::check_sequence(tp, L->msg_set, seq, seqsched, need_old, why))
     return itnbp_fail(ctx, rc, why);
   const size_t nseq = seq.size();
-  ITNBP_RETCHK(ensure_buf(ctx, L->stats, nseq * sizeof(MsgStat)));
+  // statistics, then a flag that a sweep without a read-back raises on a non-finite
+  // message
+  ITNBP_RETCHK(ensure_buf(ctx, L->stats, (nseq + 1) * sizeof(MsgStat)));
+  MsgStat* stats = (MsgStat*)L->stats.p;
+  int* bad = (int*)(stats + nseq);
   std::vector<std::pair<int, int>> runs{{0, (int)nseq}};
   std::vector<int> order(nseq);
   std::iota(order.begin(), order.end(), 0);
   if (seqsched) itnbp_graph::sequential_levels(tp, seq, order, runs);
-  std::vector<MsgStat> hs(nseq);
+  // the tasks in launch order, uploaded once: a table for the first sweep, whose
+  // messages may not all be set, and one for the later sweeps
+  std::vector<LTask> tasks(2 * nseq);
+  std::vector<char> covered(2 * L->ne, 0);
+  for (const auto& run : runs) {
+    for (int k = run.first; k < run.second; ++k) {
+      const int m = seq[order[k]];
+      tasks[k] = message_task_l(L, m, order[k], L->msg_set[m] || (seqsched && covered[m]), o->normalize);
+      tasks[nseq + k] = message_task_l(L, m, order[k], true, o->normalize);
+    }
+    for (int k = run.first; k < run.second; ++k) covered[seq[order[k]]] = 1;
+  }
+  const bool all = std::count(covered.begin(), covered.end(), 1) == 2 * L->ne;
+  ITNBP_RETCHK(upload(ctx, L->tasks, tasks.data(), tasks.size() * sizeof(LTask)));
+  std::vector<MsgStat> hs(nseq + 1);
   itnbp_update_result r{};
+  ITNBP_HIPCHK(ctx, hipMemsetAsync(bad, 0, sizeof(int), ctx->stream));
   ITNBP_HIPCHK(ctx, hipEventRecord(ctx->ev0, ctx->stream));
   for (int it = 1; it <= o->maxiter; ++it) {
     void* cur = L->d_msg[L->cur];
     void* nxt = seqsched ? cur : L->d_msg[1 - L->cur];
-    if (!seqsched)
+    if (!seqsched && !all)  // messages outside the sequence keep their values
       ITNBP_HIPCHK(ctx, hipMemcpyAsync(nxt, cur, L->msg_total * L->es, hipMemcpyDeviceToDevice, ctx->stream));
-    for (const auto& run : runs) {
-      std::vector<LTask> tasks;
-      for (int k = run.first; k < run.second; ++k) {
-        const int i = order[k], m = seq[i];
-        tasks.push_back(message_task_l(L, m, i, L->msg_set[m] != 0, o->normalize));
-      }
-      ITNBP_RETCHK(run_layer_tasks(L, tasks, cur, nxt, (MsgStat*)L->stats.p));
-      if (seqsched)
-        for (int k = run.first; k < run.second; ++k) L->msg_set[seq[order[k]]] = 1;
-    }
-    if (!seqsched) {
-      L->cur = 1 - L->cur;
-      for (int m : seq) L->msg_set[m] = 1;
-    }
-    ITNBP_HIPCHK(ctx, hipMemcpyAsync(hs.data(), L->stats.p, nseq * sizeof(MsgStat), hipMemcpyDeviceToHost,
-                                     ctx->stream));
+    const LTask* table = (const LTask*)L->tasks.p + (it == 1 ? 0 : nseq);
+    for (const auto& run : runs)
+      ITNBP_RETCHK(launch_layer_tasks(L, table + run.first, run.second - run.first, cur, nxt, stats, bad));
+    for (int m : seq) L->msg_set[m] = 1;
+    if (!seqsched) L->cur = 1 - L->cur;
+    // without a stopping rule only the last sweep's statistics are wanted
+    if (!need_old && it < o->maxiter) continue;
+    ITNBP_HIPCHK(ctx, hipMemcpyAsync(hs.data(), stats, hs.size() * sizeof(MsgStat), hipMemcpyDeviceToHost, ctx->stream));
     ITNBP_HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    int hbad = 0;
+    std::memcpy(&hbad, &hs[nseq], sizeof(int));
+    if (hbad) return itnbp_fail(ctx, ITNBP_ERR_NONFINITE, "non-finite message");
     double sd = 0, mr = 0;
     for (size_t i = 0; i < nseq; ++i) {
-      if (hs[i].bad > 0) return itnbp_fail(ctx, ITNBP_ERR_NONFINITE, "non-finite message");
       sd += hs[i].diff;
       mr = std::max(mr, hs[i].res2);
     }
@@ -463,7 +475,7 @@ int lnet_region_scalars(itnbp_lnet* L, double* vert, double* edge) {
   std::vector<LTask> tasks(L->nv);
   for (int v = 0; v < L->nv; ++v) tasks[v] = LTask{v, -1, -1, 0, (long long)v, -1};
   const void* msg = L->d_msg[L->cur];
-  ITNBP_RETCHK(run_layer_tasks(L, tasks, msg, L->small_out.p, nullptr));
+  ITNBP_RETCHK(run_layer_tasks(L, tasks, msg, L->small_out.p));
   if (L->ne > 0) {
     char* eo = (char*)L->small_out.p + (size_t)L->nv * L->es;
     if (L->cplx)
@@ -689,6 +701,16 @@ int itnbp_lnet_get_message(itnbp_lnet* L, int m, double* data) {
   });
 }
 
+int itnbp_lnet_get_messages(itnbp_lnet* L, double* data) {
+  if (!L || !data) return ITNBP_ERR_ARG;
+  itnbp_ctx* ctx = L->ctx;
+  return itnbp_guarded(ctx, [&]() -> int {
+    ITNBP_HIPCHK(ctx, hipMemcpyAsync(data, L->d_msg[L->cur], L->msg_total * L->es, hipMemcpyDeviceToHost, ctx->stream));
+    ITNBP_HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    return ITNBP_OK;
+  });
+}
+
 int itnbp_lnet_message_is_set(itnbp_lnet* L, int m) {
   if (!L || m < 0 || m >= 2 * L->ne) return -1;
   return L->msg_set[m] ? 1 : 0;
@@ -763,7 +785,7 @@ int itnbp_lnet_rdm1(itnbp_lnet* L, int n, const int* verts, double* out) {
       tot += (long long)L->phys[v] * L->phys[v];
     }
     ITNBP_RETCHK(ensure_buf(ctx, L->small_out, tot * L->es));
-    ITNBP_RETCHK(run_layer_tasks(L, tasks, L->d_msg[L->cur], L->small_out.p, nullptr));
+    ITNBP_RETCHK(run_layer_tasks(L, tasks, L->d_msg[L->cur], L->small_out.p));
     ITNBP_HIPCHK(ctx, hipMemcpyAsync(out, L->small_out.p, tot * L->es, hipMemcpyDeviceToHost, ctx->stream));
     ITNBP_HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     return ITNBP_OK;

@@ -103,6 +103,7 @@ SIGNATURES = {
     "itnbp_lnet_get_ket": (_I, [_P, _DP]),
     "itnbp_lnet_set_message": (_I, [_P, _I, _DP]),
     "itnbp_lnet_get_message": (_I, [_P, _I, _DP]),
+    "itnbp_lnet_get_messages": (_I, [_P, _DP]),
     "itnbp_lnet_message_is_set": (_I, [_P, _I]),
     "itnbp_lnet_init_identity_messages": (_I, [_P]),
     "itnbp_lnet_update": (_I, [_P, C.POINTER(UpdateOpts), C.POINTER(UpdateResult)]),

@@ -154,11 +154,17 @@ class LayeredBPCache:
 
     def messages(self):
         g = self.graph
-        out = {}
+        flat = np.empty(int(self.lib.itnbp_lnet_msg_numel(self.h)), dtype=self.dtype)
+        if g.ne:
+            self.ctx.check(self.lib.itnbp_lnet_get_messages(self.h, L.dptr(flat.view(np.float64))))
+        out, off = {}, 0
+        kchi, bchi = self.kchi.tolist(), self.bchi.tolist()
         for m in range(2 * g.ne):
+            k, b = kchi[m >> 1], bchi[m >> 1]
             if self.lib.itnbp_lnet_message_is_set(self.h, m) == 1:
-                e = g.message_edge(m)
-                out[e] = self.message(e)
+                # a buffer of its own, as from message()
+                out[g.message_edge(m)] = flat[off:off + k * b].copy().reshape((k, b), order="F")
+            off += k * b
         return out
 
     def folded_ket(self):
