@@ -113,6 +113,11 @@ __device__ void finalize_task(const OcTask& t, const TA* Tb, int P2, const TM* m
 // ---------------------------------------------------------------------------
 // small path
 // ---------------------------------------------------------------------------
+// One workgroup per task, everything in LDS (D elements twice, so every index is below
+// 2^20 for SmallDiv).  Bound: latency of the contraction's loop, R terms per output.
+// With integer divisions and psi from global memory in it, the halves of a pair
+// density matrix on a 16x16 chi = 8 lattice (P = 16, R = 512) took 212 us a launch,
+// against 91.
 template <typename TP, typename TM, typename TA>
 __global__ __launch_bounds__(ITNBP_BLOCK) void k_oc_small(const VDesc* __restrict__ vds,
                                                           const OcTask* __restrict__ tasks,
@@ -146,18 +151,21 @@ __global__ __launch_bounds__(ITNBP_BLOCK) void k_oc_small(const VDesc* __restric
     __syncthreads();
     TA* Y = bufp((cur + 1) & 1);
     const int An = A * n;
+    const SmallDiv dA = small_div(A), dn = small_div(n);
     for (int i = tid; i < D; i += blockDim.x) {
-      const int lo = i % A;
-      const int rest = i / A;
-      const int c = rest % n;
-      const int hi = rest / n;
+      const int rest = (int)dA.div(i);
+      const int lo = i - rest * A;
+      const int hi = (int)dn.div(rest);
+      const int c = rest - hi * n;
       const int base = lo + An * hi;
       const TA* Mc = Mst + n * c;
       TA acc = 0;
       if (cur < 0) {
+#pragma unroll 4
         for (int x = 0; x < n; ++x) acc += load_as<TA>(ps, base + A * x) * Mc[x];
       } else {
         const TA* X = bufp(cur);
+#pragma unroll 4
         for (int x = 0; x < n; ++x) acc += X[base + A * x] * Mc[x];
       }
       Y[i] = acc;
@@ -166,12 +174,18 @@ __global__ __launch_bounds__(ITNBP_BLOCK) void k_oc_small(const VDesc* __restric
     __syncthreads();
   }
 
-  // T[row, col] = sum_r Phi[offx(row) + roff(r)] * psi[offx(col) + roff(r)]
+  // T[row, col] = sum_r Phi[offx(row) + roff(r)] * psi[offx(col) + roff(r)], psi from
+  // the buffer that is free
+  TA* Ps = bufp((cur + 1) & 1);
+#pragma unroll 4
+  for (int i = tid; i < D; i += blockDim.x) Ps[i] = load_as<TA>(ps, i);
+  __syncthreads();
   const int P2 = g.P * g.P;
   int G = 1;
   while (G * 2 * P2 <= (int)blockDim.x && G < 64) G *= 2;
   const int per = blockDim.x / G;
-  const TA* Phi = cur < 0 ? nullptr : bufp(cur);
+  const TA* Phi = cur < 0 ? Ps : bufp(cur);
+  const SmallDiv dlo = small_div(g.lo_n);
   const int strideHi = g.Aj * g.nj;
   for (int ob = 0; ob < P2; ob += per) {
     const int o = ob + tid / G;
@@ -181,11 +195,11 @@ __global__ __launch_bounds__(ITNBP_BLOCK) void k_oc_small(const VDesc* __restric
       const int row = o % g.P, col = o / g.P;
       const int offx = (row % g.ds) + g.Aj * (row / g.ds);
       const int offy = (col % g.ds) + g.Aj * (col / g.ds);
+#pragma unroll 4
       for (int r = gi; r < g.R; r += G) {
-        const int lo = r % g.lo_n, hi = r / g.lo_n;
+        const int hi = (int)dlo.div(r), lo = r - hi * g.lo_n;
         const int roff = g.ds * lo + strideHi * hi;
-        const TA ph = Phi ? Phi[offx + roff] : load_as<TA>(ps, offx + roff);
-        acc += ph * load_as<TA>(ps, offy + roff);
+        acc += Phi[offx + roff] * Ps[offy + roff];
       }
     }
     for (int m = G / 2; m > 0; m >>= 1) acc += __shfl_xor(acc, m);
