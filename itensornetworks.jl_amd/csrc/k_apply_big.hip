@@ -825,13 +825,15 @@ __global__ __launch_bounds__(256) void k_gb_rebuild(GbWork w, double* psi) {
         const int c0 = b0 * g.d, nc = bs * g.d;
         __syncthreads();  // tile read (first pass) or written out
         for (int t = 0; 16 * t < nc; ++t) {
+          // the last tile's columns past nc (d = 3, 5, 6, 7) belong to the next pass
           const int cc = c0 + 16 * t + li;
+          const bool in = 16 * t + li < nc && cc < cols;
           f64x4 acc = {0, 0, 0, 0};
 #pragma unroll
           for (int q = 0; q < 16; ++q)
             if (q < nq) {
               const int c = 4 * q + lk;
-              const double b = (c < n && cc < cols) ? Wl[c + n * cc] : 0.0;
+              const double b = (c < n && in) ? Wl[c + n * cc] : 0.0;
               acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[q], b, acc, 0, 0, 0);
             }
           double best = 0;
@@ -841,7 +843,7 @@ __global__ __launch_bounds__(256) void k_gb_rebuild(GbWork w, double* psi) {
             const int r = 16 * wv + 4 * v + lk, e = e0 + r;
             if (16 * t + li < GB_ROWS) tile[(16 * t + li) * GB_PITCH + r] = acc[v];
             nrm2 += acc[v] * acc[v];
-            if (first && e < g.E && cc < cols) {
+            if (first && e < g.E && in) {
               const int b = (int)g.fd.div(cc);
               gb_better(best, boff, acc[v], gb_nat(g, cc - b * g.d, e, b));
             }
@@ -849,7 +851,7 @@ __global__ __launch_bounds__(256) void k_gb_rebuild(GbWork w, double* psi) {
           if (first) {
             gb_better(best, boff, __shfl_xor(best, 16), __shfl_xor(boff, 16));
             gb_better(best, boff, __shfl_xor(best, 32), __shfl_xor(boff, 32));
-            if (lk == 0 && cc < cols) gb_better(cv[wv * lcols + cc], co[wv * lcols + cc], best, boff);
+            if (lk == 0 && in) gb_better(cv[wv * lcols + cc], co[wv * lcols + cc], best, boff);
           }
         }
         __syncthreads();
