@@ -348,6 +348,7 @@ __global__ __launch_bounds__(SV_THREADS) void k_big_pass(const BigSite* __restri
   }
   V4 acca = {0, 0, 0, 0}, accb = {0, 0, 0, 0};
   double ga[4] = {0, 0, 0, 0}, gb[4] = {0, 0, 0, 0};
+  int run = 0;  // r in acca, accb; on across chunks, which may hold fewer than 4 per wave
   for (int c = blockIdx.x; c < P.nchunk; c += gridDim.x) {
     const int ch = c / P.ncl, cl = c - ch * P.ncl;
     const int lo0 = cl * P.L, nl = min(P.L, sa - lo0), hi0 = ch * P.H, nh = min(P.H, P.nhi - hi0);
@@ -391,7 +392,6 @@ __global__ __launch_bounds__(SV_THREADS) void k_big_pass(const BigSite* __restri
       wr[tid] = (TA)w;
     }
     __syncthreads();
-    int run = 0;
     for (int r = wv; r < nr; r += 4) {
       TA* x = slab + r * BIG_T;
       const TA w = grams ? wr[r] : (TA)0;
