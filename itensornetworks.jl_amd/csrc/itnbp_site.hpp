@@ -17,7 +17,7 @@ struct SiteTask {
   int lsh;    // 16 >> lsh blocks share one 16 x 16 tile
   int want;   // bit 0: message on p, bit 1: on q
   long long psi_off;
-  long long mp, mq;      // messages into the site on p and q (mq < 0: none)
+  long long mp, mq;      // messages into the site on p (for the output on q) and q (< 0: not read)
   long long out[2];      // messages out on p and q
   long long old[2];      // previous messages out (-1: none to compare with)
   int slot[2];           // statistics slots (-1: none)

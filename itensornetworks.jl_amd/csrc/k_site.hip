@@ -63,7 +63,8 @@ __device__ inline double site_wave_sum(double v) {
 }
 
 // A operand of a product with the message at msg (n x n, column-major):
-// A[b'][b] = M[b][b'] for output row b' = a_row(lane) and K-steps b = 4 q + l / 16
+// A[b'][b] = M[b][b'] for output row b' = a_row(lane) and K-steps b = 4 q + l / 16.
+// msg < 0: none, ones (the missing second bond of a site of one; else not used)
 template <typename TA, typename TM>
 __device__ inline void site_msg(const TM* msg_in, long long msg, int n, TA (&a)[4]) {
   const int l = threadIdx.x & 63, lk = l >> 4, r = Mf<TA>::a_row(l & 15);
@@ -487,8 +488,10 @@ SiteTask site_task(const VDesc& V, int p, int want, int elem_bytes) {
   t.fsp = fast_div((unsigned)sp);
   t.sps = sp + site_padding(sp, t.np, t.nq, lsh, elem_bytes);
   t.Ds = V.D / sp * t.sps;
-  t.mp = V.in_msg[p];
-  t.mq = q ? V.in_msg[q] : -1;
+  // only what an output absorbs: another workgroup of the launch may be writing the
+  // message into the site on a lone output's own bond
+  t.mp = (want & 2) ? V.in_msg[p] : -1;
+  t.mq = q && (want & 1) ? V.in_msg[q] : -1;
   t.slot[0] = t.slot[1] = -1;
   t.old[0] = t.old[1] = -1;
   int st = V.dims[0];
