@@ -304,8 +304,10 @@ __global__ __launch_bounds__(SV_THREADS) void k_big_eigh(const BigSite* __restri
               rq + 8 * wv);
 }
 
+// grid ns nsplit, nsplit consecutive workgroups per site (in x: a batched set may hold
+// more sites than a grid has rows)
 template <typename TS, typename TA, bool GRAM>
-__global__ __launch_bounds__(SV_THREADS) void k_big_pass(const BigSite* __restrict__ sites, int pass,
+__global__ __launch_bounds__(SV_THREADS) void k_big_pass(const BigSite* __restrict__ sites, int nsplit, int pass,
                                                          const TS* __restrict__ psi, TA* __restrict__ scratch,
                                                          const double* __restrict__ seeds,
                                                          const double* __restrict__ lam, double* __restrict__ part,
@@ -315,11 +317,12 @@ __global__ __launch_bounds__(SV_THREADS) void k_big_pass(const BigSite* __restri
   __shared__ TA slab[R * BIG_T];
   __shared__ TA wr[R];
   __shared__ double ls[ITNBP_MAXK][SV_MAXCHI];
-  const BigSite& t = sites[blockIdx.y];
+  const int site = blockIdx.x / nsplit, wg = blockIdx.x - site * nsplit;
+  const BigSite& t = sites[site];
   // a site's last pair gets its Grams with the rotation
   if (pass >= (GRAM ? t.m - 1 : t.m) || (active && !active[t.inst])) return;
   const BigPair& P = t.pr[pass];
-  if ((int)blockIdx.x >= P.nchunk) return;
+  if (wg >= P.nchunk) return;
   const bool grams = GRAM || pass == t.m - 1;
   const int tid = threadIdx.x, l = tid & 63, wv = tid >> 6, li = l & 15, lk = l >> 4;
   const int na = P.na, nb = P.nb, nab = na * nb, sa = P.sa;
@@ -349,7 +352,7 @@ __global__ __launch_bounds__(SV_THREADS) void k_big_pass(const BigSite* __restri
   V4 acca = {0, 0, 0, 0}, accb = {0, 0, 0, 0};
   double ga[4] = {0, 0, 0, 0}, gb[4] = {0, 0, 0, 0};
   int run = 0;  // r in acca, accb; on across chunks, which may hold fewer than 4 per wave
-  for (int c = blockIdx.x; c < P.nchunk; c += gridDim.x) {
+  for (int c = wg; c < P.nchunk; c += nsplit) {
     const int ch = c / P.ncl, cl = c - ch * P.ncl;
     const int lo0 = cl * P.L, nl = min(P.L, sa - lo0), hi0 = ch * P.H, nh = min(P.H, P.nhi - hi0);
     const SmallDiv fl = nl == P.L ? P.fL : P.fLr, fab = P.fab, fa = P.fa;
@@ -461,7 +464,7 @@ __global__ __launch_bounds__(SV_THREADS) void k_big_pass(const BigSite* __restri
     for (int v = 0; v < 4; ++v)
       sum[wv * 256 + 16 * Mma<TA>::drow(lk, v) + li] = b == 0 ? ga[v] + (double)acca[v] : gb[v] + (double)accb[v];
     __syncthreads();
-    part[t.part + ((long long)(P.a - 1 + b) * gridDim.x + blockIdx.x) * 256 + tid] =
+    part[t.part + ((long long)(P.a - 1 + b) * nsplit + wg) * 256 + tid] =
         (sum[tid] + sum[256 + tid]) + (sum[512 + tid] + sum[768 + tid]);
   }
 }
@@ -615,13 +618,13 @@ hipError_t launch_big_sites(itnbp_net* net, SmallState* st, const void* psi, con
   TA* y = (TA*)st->ybuf.p;
   hipLaunchKernelGGL(k_big_eigh<TM>, dim3(ns), dim3(SV_THREADS), 0, stream, sites, (const TM*)msg_in, seeds, lam, warm,
                      st->active, st->sweep_ctr);
-  const dim3 grid(st->bsplit, ns);
+  const dim3 grid((unsigned)ns * (unsigned)st->bsplit);
   for (int p = 0; p < st->bpairs; ++p)
-    hipLaunchKernelGGL((k_big_pass<TS, TA, false>), grid, dim3(SV_THREADS), 0, stream, sites, p, (const TS*)psi, y,
-                       (const double*)seeds, (const double*)lam, part, st->active);
+    hipLaunchKernelGGL((k_big_pass<TS, TA, false>), grid, dim3(SV_THREADS), 0, stream, sites, st->bsplit, p,
+                       (const TS*)psi, y, (const double*)seeds, (const double*)lam, part, st->active);
   for (int p = 0; p + 1 < st->bpairs; ++p)
-    hipLaunchKernelGGL((k_big_pass<TS, TA, true>), grid, dim3(SV_THREADS), 0, stream, sites, p, (const TS*)psi, y,
-                       (const double*)seeds, (const double*)lam, part, st->active);
+    hipLaunchKernelGGL((k_big_pass<TS, TA, true>), grid, dim3(SV_THREADS), 0, stream, sites, st->bsplit, p,
+                       (const TS*)psi, y, (const double*)seeds, (const double*)lam, part, st->active);
   hipLaunchKernelGGL(k_big_final<TM>, dim3((unsigned)st->bonds.size()), dim3(SV_THREADS), 0, stream, sites, bonds,
                      st->bsplit, (const double*)seeds, (const double*)part, (const TM*)msg_in, (TM*)msg_out, stats,
                      normalize, st->active);
