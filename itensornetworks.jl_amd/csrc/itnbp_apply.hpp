@@ -3,6 +3,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <vector>
+
 #include "itnbp_internal.hpp"
 #include "itnbp_jacobi.hpp"
 
@@ -576,6 +578,8 @@ __device__ int gate_svd(double (&a)[NP / 8], int M, int N, const SvdLds<NP>& L, 
 // device workspace of nb gates (host items) of one launch sequence, in bytes
 size_t apply_big_bytes(const itnbp_net* net, const ApplyItem* items, int nb);
 // launches the gates: outputs per slot as the LDS kernel's; work holds
-// apply_big_bytes bytes
+// apply_big_bytes bytes.  The uploaded table is added to tables, which the caller keeps
+// until it has waited for the stream
 int apply_big_run(itnbp_net* net, const ApplyItem* items, int nb, const double* d_gates, const ApplyParams& prm,
-                  void* work, double* truncerr, double* svals, int* kept, int* status);
+                  void* work, double* truncerr, double* svals, int* kept, int* status,
+                  std::vector<std::vector<char>>& tables);

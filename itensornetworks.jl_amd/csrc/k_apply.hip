@@ -954,6 +954,16 @@ int run_apply(itnbp_net* net, int n, const std::vector<ApplyItem>& items_in, con
   std::vector<char> up(sz[0] + (size_t)goff * 8);
   std::memcpy(up.data(), items.data(), n * sizeof(ApplyItem));
   std::memcpy(up.data() + sz[0], gates, (size_t)goff * 8);
+  // host memory of the call's copies (up, the split pipeline's tables): every way out
+  // waits for the stream before it goes
+  std::vector<std::vector<char>> tables;
+  struct Wait {
+    hipStream_t s;
+    bool on = true;
+    ~Wait() {
+      if (on) (void)hipStreamSynchronize(s);
+    }
+  } wait{ctx->stream};
   if ((char*)b.gates != (char*)b.items + sz[0])
     return itnbp_fail(ctx, ITNBP_ERR_HIP, "apply: workspace layout");
   if (hipMemcpyAsync(b.items, up.data(), up.size(), hipMemcpyHostToDevice, ctx->stream) != hipSuccess)
@@ -1036,11 +1046,8 @@ int run_apply(itnbp_net* net, int n, const std::vector<ApplyItem>& items_in, con
     int c0 = nl;
     for (int c1 : chunk_end) {
       const int rc = apply_big_run(net, items.data() + c0, c1 - c0, b.gates, prm, net->apply_big.p, b.te,
-                                   svals ? b.sv : nullptr, b.kept, b.st);
-      if (rc != ITNBP_OK) {
-        (void)hipStreamSynchronize(ctx->stream);
-        return rc;
-      }
+                                   svals ? b.sv : nullptr, b.kept, b.st, tables);
+      if (rc != ITNBP_OK) return rc;
       c0 = c1;
     }
   }
@@ -1078,6 +1085,7 @@ int run_apply(itnbp_net* net, int n, const std::vector<ApplyItem>& items_in, con
     return itnbp_fail(ctx, ITNBP_ERR_HIP, "apply: workspace layout");
   if (ek == hipSuccess) ek = hipMemcpyAsync(dn.data(), b.te, dn.size(), hipMemcpyDeviceToHost, ctx->stream);
   if (ek == hipSuccess) ek = hipStreamSynchronize(ctx->stream);
+  wait.on = ek != hipSuccess;
   if (net->apply_big.bytes > APPLY_BIG_KEEP) free_buf(net->apply_big);
   if (ek != hipSuccess) return itnbp_fail(ctx, ITNBP_ERR_HIP, std::string("apply: ") + hipGetErrorString(ek));
   std::memcpy(truncerr, dn.data(), (size_t)n * 8);

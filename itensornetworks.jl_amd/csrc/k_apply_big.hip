@@ -1036,7 +1036,8 @@ size_t apply_big_bytes(const itnbp_net* net, const ApplyItem* items, int nb) {
 }
 
 int apply_big_run(itnbp_net* net, const ApplyItem* items, int nb, const double* d_gates, const ApplyParams& prm,
-                  void* work, double* truncerr, double* svals, int* kept, int* status) {
+                  void* work, double* truncerr, double* svals, int* kept, int* status,
+                  std::vector<std::vector<char>>& tables) {
   itnbp_ctx* ctx = net->ctx;
   GbPlan p;
   gb_plan(net, items, nb, p);
@@ -1067,7 +1068,8 @@ int apply_big_run(itnbp_net* net, const ApplyItem* items, int nb, const double* 
   w.mcols = p.mcols;
   w.lcols = p.lcols;
   hipStream_t s = ctx->stream;
-  std::vector<char> up(p.off[2]);
+  tables.emplace_back(p.off[2]);
+  std::vector<char>& up = tables.back();
   std::memcpy(up.data(), p.side.data(), p.side.size() * sizeof(GbSide));
   std::memcpy(up.data() + p.off[1], p.gate.data(), p.gate.size() * sizeof(GbGate));
   ITNBP_HIPCHK(ctx, hipMemcpyAsync(base, up.data(), up.size(), hipMemcpyHostToDevice, s));

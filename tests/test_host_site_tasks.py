@@ -7,10 +7,10 @@ import subprocess
 from helpers import LIB, ROOT
 
 
-def build_driver(tmp_path, name):
+def build_driver(tmp_path, name, *flags):
     exe = str(tmp_path / name)
     libdir = os.path.dirname(LIB)
-    r = subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+    r = subprocess.run(["g++", "-std=c++17", "-O1", *flags, "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
                         "-I" + os.path.join(ROOT, "include"), os.path.join(ROOT, "tests", "cpp", name + ".cpp"),
                         "-o", exe, "-L" + libdir, "-litnbp", "-Wl,-rpath," + libdir], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
