@@ -3084,6 +3084,7 @@ struct FastState {
   DevBuf sexp, pmax;
   // one-site density matrices: item lists, partial sums and request tables
   DevBuf rdm;
+  std::vector<std::vector<char>> rdm_tables;  // host memory of the uploads into rdm (upload_rdm)
 };
 
 FastState* state_of(itnbp_net* net) { return reinterpret_cast<FastState*>(net->fast); }
@@ -3823,6 +3824,14 @@ struct RotSites {
   char* tail = nullptr;       // device scratch after the item lists
 };
 
+// Uploads a table into the density matrices' buffer; the state holds its host memory
+// until the next request has waited for the stream (rotated_sites_setup).
+static int upload_rdm(itnbp_ctx* ctx, FastState* st, void* dst, const void* src, size_t bytes) {
+  st->rdm_tables.emplace_back((const char*)src, (const char*)src + bytes);
+  ITNBP_HIPCHK(ctx, hipMemcpyAsync(dst, st->rdm_tables.back().data(), bytes, hipMemcpyHostToDevice, ctx->stream));
+  return ITNBP_OK;
+}
+
 static int rotated_sites_setup(itnbp_net* net, const std::vector<int>& want, size_t tail_bytes, RotSites& rs,
                                bool& ok) {
   itnbp_ctx* ctx = net->ctx;
@@ -3873,9 +3882,13 @@ static int rotated_sites_setup(itnbp_net* net, const std::vector<int>& want, siz
   for (int k = 0; k < nbs; ++k) all.push_back(st->k1eitems[bidx[rs.sb[k]]]);
   const size_t b_items = all.size() * sizeof(EigItem);
   const size_t at_tail = (b_items + 255) / 256 * 256;
+  if (!st->rdm_tables.empty()) {
+    ITNBP_HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    st->rdm_tables.clear();
+  }
   ITNBP_RETCHK(ensure_buf(ctx, st->rdm, at_tail + tail_bytes));
   char* base = (char*)st->rdm.p;
-  ITNBP_HIPCHK(ctx, hipMemcpyAsync(base, all.data(), b_items, hipMemcpyHostToDevice, ctx->stream));
+  ITNBP_RETCHK(upload_rdm(ctx, st, base, all.data(), b_items));
   rs.tail = base + at_tail;
   const EigItem* d_e = (const EigItem*)base;
   const EigItem* d_3 = d_e + nbs;
@@ -3941,8 +3954,8 @@ int fast_site_rdm(itnbp_net* net, int n, const int* verts, const long long* offs
   char* tb = rs.tail + (size_t)(nbs + n3s) * RHO_NPART * 3 * 8;
   long long* d_off = (long long*)tb;
   int* d_item = (int*)(tb + (size_t)nr * 8);
-  ITNBP_HIPCHK(ctx, hipMemcpyAsync(d_off, roff.data(), nr * 8, hipMemcpyHostToDevice, ctx->stream));
-  ITNBP_HIPCHK(ctx, hipMemcpyAsync(d_item, ritem.data(), nr * 4, hipMemcpyHostToDevice, ctx->stream));
+  ITNBP_RETCHK(upload_rdm(ctx, st, d_off, roff.data(), nr * 8));
+  ITNBP_RETCHK(upload_rdm(ctx, st, d_item, ritem.data(), nr * 4));
   const EigItem* d_e = (const EigItem*)st->rdm.p;
   const double* L = (const double*)st->eigL64.p;
   if (nbs > 0)
@@ -3997,7 +4010,7 @@ int fast_pair_halves(itnbp_net* net, int n, const int* sites, const int* axes, c
   if (nt == 0) return ITNBP_OK;
   PairTask* d_t = (PairTask*)rs.tail;
   double* part = (double*)(rs.tail + ((size_t)nt * sizeof(PairTask) + 255) / 256 * 256);
-  ITNBP_HIPCHK(ctx, hipMemcpyAsync(d_t, tasks.data(), nt * sizeof(PairTask), hipMemcpyHostToDevice, ctx->stream));
+  ITNBP_RETCHK(upload_rdm(ctx, st, d_t, tasks.data(), nt * sizeof(PairTask)));
   hipLaunchKernelGGL(k_pair_gram_f64, dim3(PG_NPART, nt), dim3(256), 0, ctx->stream, (const PairTask*)d_t,
                      (const double*)st->P64.p, (const double*)st->P3_64.p, (const double*)st->eigL64.p, part);
   hipLaunchKernelGGL(k_pair_finalize, dim3(nt), dim3(256), 0, ctx->stream, (const PairTask*)d_t, (const double*)part,
