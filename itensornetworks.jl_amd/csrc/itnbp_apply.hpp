@@ -575,10 +575,13 @@ __device__ int gate_svd(double (&a)[NP / 8], int M, int N, const SvdLds<NP>& L, 
 }
 
 // ---- the split pipeline (k_apply_big.hip) -----------------------------------
-// device workspace of nb gates (host items) of one launch sequence, in bytes
-size_t apply_big_bytes(const itnbp_net* net, const ApplyItem* items, int nb);
+// The launch sequences of nb gates (host items): the end of each, as many gates as its
+// device workspace may take of budget bytes (at least one; a sequence's grids have two
+// rows per gate, and a gate takes 0.7 MiB, so 16 GiB stay within 65535 rows).  bytes: the
+// largest workspace.  One pass over the gates.
+std::vector<int> apply_big_chunks(const itnbp_net* net, const ApplyItem* items, int nb, size_t budget, size_t& bytes);
 // launches the gates: outputs per slot as the LDS kernel's; work holds
-// apply_big_bytes bytes.  The uploaded table is added to tables, which the caller keeps
+// the bytes of apply_big_chunks.  The uploaded table is added to tables, which the caller keeps
 // until it has waited for the stream
 int apply_big_run(itnbp_net* net, const ApplyItem* items, int nb, const double* d_gates, const ApplyParams& prm,
                   void* work, double* truncerr, double* svals, int* kept, int* status,

@@ -1010,25 +1010,13 @@ int run_apply(itnbp_net* net, int n, const std::vector<ApplyItem>& items_in, con
   }
   // the split pipeline's workspace first, so that a failed allocation leaves
   // every tensor of the call untouched
-  std::vector<int> chunk_end;  // ends of the launch sequences of items [nl, n)
+  std::vector<int> chunk_end;  // ends of the launch sequences, from item nl on
   if (nb > 0) {
     size_t fr = 0, tot = 0;
     if (hipMemGetInfo(&fr, &tot) != hipSuccess) fr = 0;
     const size_t budget = std::min<size_t>(fr / 2 + net->apply_big.bytes, 16ULL << 30);
     size_t most = 0;
-    for (int c0 = nl; c0 < n;) {
-      int c1 = c0 + 1;
-      size_t bytes = apply_big_bytes(net, items.data() + c0, 1);
-      while (c1 < n) {
-        const size_t more = apply_big_bytes(net, items.data() + c0, c1 + 1 - c0);
-        if (more > budget) break;
-        bytes = more;
-        ++c1;
-      }
-      most = std::max(most, bytes);
-      chunk_end.push_back(c1);
-      c0 = c1;
-    }
+    chunk_end = apply_big_chunks(net, items.data() + nl, nb, budget, most);
     ITNBP_RETCHK(ensure_buf(ctx, net->apply_big, most));
   }
   const int pm0 = prof_mark(ctx);
@@ -1043,9 +1031,9 @@ int run_apply(itnbp_net* net, int n, const std::vector<ApplyItem>& items_in, con
   hipError_t ek = hipGetLastError();
   prof_add(ctx, "apply_gates", pm0, prof_mark(ctx));
   if (ek == hipSuccess && nb > 0) {
-    int c0 = nl;
+    int c0 = 0;
     for (int c1 : chunk_end) {
-      const int rc = apply_big_run(net, items.data() + c0, c1 - c0, b.gates, prm, net->apply_big.p, b.te,
+      const int rc = apply_big_run(net, items.data() + nl + c0, c1 - c0, b.gates, prm, net->apply_big.p, b.te,
                                    svals ? b.sv : nullptr, b.kept, b.st, tables);
       if (rc != ITNBP_OK) return rc;
       c0 = c1;

@@ -932,73 +932,71 @@ __global__ __launch_bounds__(256) void k_gb_scale(GbWork w, double* __restrict__
 }
 
 // ---- host ------------------------------------------------------------------------
+// what the workspace's layout depends on
+struct GbNeed {
+  int gates = 0, mcols = 1, lcols = 1, max_th = 1, max_w = 1;  // max_w: the most entries of a tall side's W
+  long long xtot = 0, maxD = 1, maxE = 1;
+};
 struct GbPlan {
   std::vector<GbSide> side;
   std::vector<GbGate> gate;
-  int nsplit, gxr, mcols, lcols, max_th, max_w;  // max_w: the most entries of a tall side's W
-  long long xtot, maxD;
+  GbNeed need;
+  int nsplit, gxr;
   size_t off[20], total;
 };
 
-void gb_plan(const itnbp_net* net, const ApplyItem* items, int nb, GbPlan& p) {
-  p.side.assign(2 * nb, GbSide{});
-  p.gate.assign(nb, GbGate{});
-  p.xtot = 0;
-  p.maxD = 1;
-  p.mcols = 1;
-  p.lcols = 1;
-  p.max_th = 1;
-  p.max_w = 1;
-  long long maxE = 1;
-  for (int i = 0; i < nb; ++i) {
-    p.gate[i].gate_off = items[i].gate;
-    p.gate[i].slot = items[i].slot;
-    for (int sd = 0; sd < 2; ++sd) {
-      GbSide& g = p.side[2 * i + sd];
-      const VDesc& V = net->vdesc[sd == 0 ? items[i].u : items[i].v];
-      const int j = sd == 0 ? items[i].ju : items[i].jv;
-      g.psi_off = V.psi_off;
-      g.x_off = p.xtot;
-      p.xtot += (V.D + 31) & ~31LL;
-      g.d = V.dims[0];
-      g.chib = items[i].chib_in;
-      g.lay = V.dims[j];
-      g.lo = 1;
-      g.E = 1;
-      int st = g.d;
-      for (int a = 1; a <= V.k; ++a) {
-        if (a < j) g.lo *= V.dims[a];
-        if (a != j) {
-          g.ext_dim[g.next] = V.dims[a];
-          g.ext_st[g.next] = st;
-          g.ext_est[g.next] = g.E;
-          g.msg_off[g.next++] = V.in_msg[a];
-          g.E *= V.dims[a];
-        }
-        st *= V.dims[a];
-      }
-      g.n = g.d * g.chib;
-      g.wide = g.E <= g.n;
-      g.D = V.D;
-      g.fd = fast_div(g.d);
-      g.fn = fast_div(g.n);
-      g.flo = fast_div(g.lo);
-      g.fdlo = fast_div(g.d * g.lo);
-      g.flay = fast_div(g.lay);
-      maxE = std::max<long long>(maxE, g.E);
-      p.maxD = std::max<long long>(p.maxD, g.D);
-      const int cols = g.d * std::min(g.lay, AP_KEEP_BIG);
-      p.mcols = std::max(p.mcols, cols);
-      if (!g.wide) {  // n d <= 128 (Theta's limit), so n cols <= GB_W
-        p.lcols = std::max(p.lcols, cols);
-        p.max_w = std::max(p.max_w, g.n * cols);
-      }
-      p.max_th = std::max(p.max_th, std::min(g.E, g.n) * g.d);
+// side sd of a gate; x_off is left to the caller
+GbSide gb_side(const itnbp_net* net, const ApplyItem& it, int sd) {
+  GbSide g{};
+  const VDesc& V = net->vdesc[sd == 0 ? it.u : it.v];
+  const int j = sd == 0 ? it.ju : it.jv;
+  g.psi_off = V.psi_off;
+  g.d = V.dims[0];
+  g.chib = it.chib_in;
+  g.lay = V.dims[j];
+  g.lo = 1;
+  g.E = 1;
+  int st = g.d;
+  for (int a = 1; a <= V.k; ++a) {
+    if (a < j) g.lo *= V.dims[a];
+    if (a != j) {
+      g.ext_dim[g.next] = V.dims[a];
+      g.ext_st[g.next] = st;
+      g.ext_est[g.next] = g.E;
+      g.msg_off[g.next++] = V.in_msg[a];
+      g.E *= V.dims[a];
     }
+    st *= V.dims[a];
   }
+  g.n = g.d * g.chib;
+  g.wide = g.E <= g.n;
+  g.D = V.D;
+  g.fd = fast_div(g.d);
+  g.fn = fast_div(g.n);
+  g.flo = fast_div(g.lo);
+  g.fdlo = fast_div(g.d * g.lo);
+  g.flay = fast_div(g.lay);
+  return g;
+}
+
+void gb_count(const GbSide& g, GbNeed& q) {
+  q.xtot += (g.D + 31) & ~31LL;
+  q.maxE = std::max<long long>(q.maxE, g.E);
+  q.maxD = std::max<long long>(q.maxD, g.D);
+  const int cols = g.d * std::min(g.lay, AP_KEEP_BIG);
+  q.mcols = std::max(q.mcols, cols);
+  if (!g.wide) {  // n d <= 128 (Theta's limit), so n cols <= GB_W
+    q.lcols = std::max(q.lcols, cols);
+    q.max_w = std::max(q.max_w, g.n * cols);
+  }
+  q.max_th = std::max(q.max_th, std::min(g.E, g.n) * g.d);
+}
+
+void gb_layout(const GbNeed& q, GbPlan& p) {
+  p.need = q;
   // row blocks per side: about two workgroups per CU over all sides, at most one
   // per chunk and 48 partial Grams (one workgroup sums them)
-  const int ns = 2 * nb, nch = (int)((maxE + GB_ROWS - 1) / GB_ROWS);
+  const int nb = q.gates, ns = 2 * nb, nch = (int)((q.maxE + GB_ROWS - 1) / GB_ROWS);
   p.nsplit = std::max(1, std::min({512 / ns + 1, 48, nch}));
   p.gxr = std::max(1, std::min({512 / ns + 1, 128, nch}));
   size_t at = 0;
@@ -1012,27 +1010,51 @@ void gb_plan(const itnbp_net* net, const ApplyItem* items, int nb, GbPlan& p) {
   take(ns * sizeof(GbInfo));
   take(nb * sizeof(GbOut));
   take((size_t)ns * AP_MAXEXT * 3 * GB_ROOT * 8);
-  for (int q = 0; q < 4; ++q) take((size_t)ns * GB_SQ * 8);  // T, R0, R, Tq
+  for (int q4 = 0; q4 < 4; ++q4) take((size_t)ns * GB_SQ * 8);  // T, R0, R, Tq
   take((size_t)ns * GB_W * 8);
   take((size_t)nb * AP_TH_BIG * AP_TH_BIG * 8);
   take((size_t)nb * GB_W * 8);
   take((size_t)nb * AP_KEEP_BIG * 8);
   take((size_t)ns * p.nsplit * GB_SQ * 8);
   take((size_t)ns * p.gxr * 8);
-  take((size_t)nb * p.gxr * p.mcols * 8);
-  take((size_t)nb * p.gxr * p.mcols * 4);
+  take((size_t)nb * p.gxr * q.mcols * 8);
+  take((size_t)nb * p.gxr * q.mcols * 4);
   take((size_t)nb * AP_KEEP_BIG * 8);
   take((size_t)ns * 8);
-  take((size_t)p.xtot * 8);
+  take((size_t)q.xtot * 8);
   p.total = at;
 }
 
 }  // namespace
 
-size_t apply_big_bytes(const itnbp_net* net, const ApplyItem* items, int nb) {
+std::vector<int> apply_big_chunks(const itnbp_net* net, const ApplyItem* items, int nb, size_t budget, size_t& bytes) {
+  std::vector<int> ends;
+  GbNeed have;
   GbPlan p;
-  gb_plan(net, items, nb, p);
-  return p.total;
+  size_t last = 0;
+  bytes = 0;
+  for (int i = 0; i < nb; ++i) {
+    const GbSide u = gb_side(net, items[i], 0), v = gb_side(net, items[i], 1);
+    for (;;) {
+      GbNeed q = have;
+      gb_count(u, q);
+      gb_count(v, q);
+      ++q.gates;
+      gb_layout(q, p);
+      if (have.gates > 0 && p.total > budget) {  // a new sequence starts with this gate
+        ends.push_back(i);
+        bytes = std::max(bytes, last);
+        have = GbNeed{};
+        continue;
+      }
+      have = q;
+      last = p.total;
+      break;
+    }
+  }
+  if (nb > 0) ends.push_back(nb);
+  bytes = std::max(bytes, last);
+  return ends;
 }
 
 int apply_big_run(itnbp_net* net, const ApplyItem* items, int nb, const double* d_gates, const ApplyParams& prm,
@@ -1040,7 +1062,23 @@ int apply_big_run(itnbp_net* net, const ApplyItem* items, int nb, const double* 
                   std::vector<std::vector<char>>& tables) {
   itnbp_ctx* ctx = net->ctx;
   GbPlan p;
-  gb_plan(net, items, nb, p);
+  GbNeed need;
+  p.side.reserve(2 * nb);
+  p.gate.reserve(nb);
+  for (int i = 0; i < nb; ++i) {
+    for (int sd = 0; sd < 2; ++sd) {
+      GbSide g = gb_side(net, items[i], sd);
+      g.x_off = need.xtot;
+      gb_count(g, need);
+      p.side.push_back(g);
+    }
+    GbGate gt{};
+    gt.gate_off = items[i].gate;
+    gt.slot = items[i].slot;
+    p.gate.push_back(gt);
+    ++need.gates;
+  }
+  gb_layout(need, p);
   char* base = (char*)work;
   GbWork w;
   w.side = (const GbSide*)(base + p.off[0]);
@@ -1065,8 +1103,8 @@ int apply_big_run(itnbp_net* net, const ApplyItem* items, int nb, const double* 
   w.X = (double*)(base + p.off[19]);
   w.nsplit = p.nsplit;
   w.gxr = p.gxr;
-  w.mcols = p.mcols;
-  w.lcols = p.lcols;
+  w.mcols = need.mcols;
+  w.lcols = need.lcols;
   hipStream_t s = ctx->stream;
   tables.emplace_back(p.off[2]);
   std::vector<char>& up = tables.back();
@@ -1077,8 +1115,8 @@ int apply_big_run(itnbp_net* net, const ApplyItem* items, int nb, const double* 
   double* psi = (double*)net->d_psi;
   const size_t lds_gram = sizeof(double) * GB_N * GB_PITCH;
   const size_t lds_chol = CholLds<4>::bytes();
-  const size_t lds_reb = sizeof(double) * (GB_N * GB_PITCH + 4 + 6 * p.lcols + p.max_w);
-  const size_t lds_svd = p.max_th <= 32 ? SvdLds<32>::bytes() : p.max_th <= 64 ? SvdLds<64>::bytes() : SvdLds<128>::bytes();
+  const size_t lds_reb = sizeof(double) * (GB_N * GB_PITCH + 4 + 6 * need.lcols + need.max_w);
+  const size_t lds_svd = need.max_th <= 32 ? SvdLds<32>::bytes() : need.max_th <= 64 ? SvdLds<64>::bytes() : SvdLds<128>::bytes();
   const struct {
     const void* f;
     size_t lds;
@@ -1094,7 +1132,7 @@ int apply_big_run(itnbp_net* net, const ApplyItem* items, int nb, const double* 
   const int pm0 = prof_mark(ctx);
   hipLaunchKernelGGL(k_gb_roots, dim3(AP_MAXEXT, ns), dim3(256), 0, s, w, (const double*)net->d_msg[net->cur],
                      prm.eig_cutoff);
-  const dim3 gmode((unsigned)std::max<long long>(1, std::min<long long>((p.maxD / 16 + 63) / 64, 2048 / ns + 1)), ns);
+  const dim3 gmode((unsigned)std::max<long long>(1, std::min<long long>((need.maxD / 16 + 63) / 64, 2048 / ns + 1)), ns);
   for (int pa = 0; pa < AP_MAXEXT; ++pa)
     hipLaunchKernelGGL(k_gb_mode<false>, gmode, dim3(256), 0, s, w, (const double*)psi, pa);
   hipLaunchKernelGGL(k_gb_gram<false>, dim3(p.nsplit, ns), dim3(256), lds_gram, s, w);
@@ -1102,9 +1140,9 @@ int apply_big_run(itnbp_net* net, const ApplyItem* items, int nb, const double* 
   hipLaunchKernelGGL(k_gb_gram<true>, dim3(p.nsplit, ns), dim3(256), 2 * lds_gram, s, w);
   hipLaunchKernelGGL(k_gb_chol2, dim3(ns), dim3(256), lds_chol, s, w);
   hipLaunchKernelGGL(k_gb_theta, dim3(16, nb), dim3(256), 2 * GB_SQ * sizeof(double), s, w, d_gates);
-  if (p.max_th <= 32)
+  if (need.max_th <= 32)
     hipLaunchKernelGGL(k_gb_svd<32>, dim3(nb), dim3(256), lds_svd, s, w, prm, truncerr, svals, kept, status);
-  else if (p.max_th <= 64)
+  else if (need.max_th <= 64)
     hipLaunchKernelGGL(k_gb_svd<64>, dim3(nb), dim3(512), lds_svd, s, w, prm, truncerr, svals, kept, status);
   else
     hipLaunchKernelGGL(k_gb_svd<128>, dim3(nb), dim3(1024), lds_svd, s, w, prm, truncerr, svals, kept, status);
@@ -1114,7 +1152,7 @@ int apply_big_run(itnbp_net* net, const ApplyItem* items, int nb, const double* 
   hipLaunchKernelGGL(k_gb_rebuild, dim3(p.gxr, ns), dim3(256), lds_reb, s, w, psi);
   hipLaunchKernelGGL(k_gb_signs, dim3(nb), dim3(256), 0, s, w, prm.normalize);
   hipLaunchKernelGGL(k_gb_scale,
-                     dim3((unsigned)std::max<long long>(1, std::min<long long>((p.maxD + 1023) / 1024, 2048 / ns + 1)), ns),
+                     dim3((unsigned)std::max<long long>(1, std::min<long long>((need.maxD + 1023) / 1024, 2048 / ns + 1)), ns),
                      dim3(256), 0, s, w, psi);
   ITNBP_HIPCHK(ctx, hipGetLastError());
   prof_add(ctx, "apply_gates_split", pm0, prof_mark(ctx));
