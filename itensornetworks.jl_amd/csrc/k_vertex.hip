@@ -239,6 +239,7 @@ __device__ inline double block_sum(double v, double* red) {
 // One workgroup per site through every step (12 passes over Y, their latency
 // exposed) took 970 us.
 constexpr int BIG_R32 = 32, BIG_R64 = 16;  // r per chunk
+constexpr int BIG_ROWS = 32768;            // sites per plane of a pass's grid
 constexpr int BIG_Q = 17, BIG_T = 16 * BIG_Q + 1;  // LDS pitch of q, of r
 
 template <typename TA>
@@ -304,10 +305,10 @@ __global__ __launch_bounds__(SV_THREADS) void k_big_eigh(const BigSite* __restri
               rq + 8 * wv);
 }
 
-// grid ns nsplit, nsplit consecutive workgroups per site (in x: a batched set may hold
-// more sites than a grid has rows)
+// grid (workgroups per site, rows of sites, planes): a batched set may hold more sites
+// than a grid has rows
 template <typename TS, typename TA, bool GRAM>
-__global__ __launch_bounds__(SV_THREADS) void k_big_pass(const BigSite* __restrict__ sites, int nsplit, int pass,
+__global__ __launch_bounds__(SV_THREADS) void k_big_pass(const BigSite* __restrict__ sites, int nsites, int pass,
                                                          const TS* __restrict__ psi, TA* __restrict__ scratch,
                                                          const double* __restrict__ seeds,
                                                          const double* __restrict__ lam, double* __restrict__ part,
@@ -317,12 +318,13 @@ __global__ __launch_bounds__(SV_THREADS) void k_big_pass(const BigSite* __restri
   __shared__ TA slab[R * BIG_T];
   __shared__ TA wr[R];
   __shared__ double ls[ITNBP_MAXK][SV_MAXCHI];
-  const int site = blockIdx.x / nsplit, wg = blockIdx.x - site * nsplit;
+  const int site = blockIdx.y + gridDim.y * blockIdx.z;
+  if (site >= nsites) return;
   const BigSite& t = sites[site];
   // a site's last pair gets its Grams with the rotation
   if (pass >= (GRAM ? t.m - 1 : t.m) || (active && !active[t.inst])) return;
   const BigPair& P = t.pr[pass];
-  if (wg >= P.nchunk) return;
+  if ((int)blockIdx.x >= P.nchunk) return;
   const bool grams = GRAM || pass == t.m - 1;
   const int tid = threadIdx.x, l = tid & 63, wv = tid >> 6, li = l & 15, lk = l >> 4;
   const int na = P.na, nb = P.nb, nab = na * nb, sa = P.sa;
@@ -351,8 +353,7 @@ __global__ __launch_bounds__(SV_THREADS) void k_big_pass(const BigSite* __restri
   }
   V4 acca = {0, 0, 0, 0}, accb = {0, 0, 0, 0};
   double ga[4] = {0, 0, 0, 0}, gb[4] = {0, 0, 0, 0};
-  int run = 0;  // r in acca, accb; on across chunks, which may hold fewer than 4 per wave
-  for (int c = wg; c < P.nchunk; c += nsplit) {
+  for (int c = blockIdx.x; c < P.nchunk; c += gridDim.x) {
     const int ch = c / P.ncl, cl = c - ch * P.ncl;
     const int lo0 = cl * P.L, nl = min(P.L, sa - lo0), hi0 = ch * P.H, nh = min(P.H, P.nhi - hi0);
     const SmallDiv fl = nl == P.L ? P.fL : P.fLr, fab = P.fab, fa = P.fa;
@@ -395,6 +396,7 @@ __global__ __launch_bounds__(SV_THREADS) void k_big_pass(const BigSite* __restri
       wr[tid] = (TA)w;
     }
     __syncthreads();
+    int run = 0;
     for (int r = wv; r < nr; r += 4) {
       TA* x = slab + r * BIG_T;
       const TA w = grams ? wr[r] : (TA)0;
@@ -443,6 +445,15 @@ __global__ __launch_bounds__(SV_THREADS) void k_big_pass(const BigSite* __restri
         }
       }
     }
+    // a chunk of fewer r, or what is left of one
+    if (grams && sizeof(TA) == 4 && run > 0) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        ga[v] += (double)acca[v];
+        gb[v] += (double)accb[v];
+        acca[v] = accb[v] = 0;
+      }
+    }
     if constexpr (!GRAM) {
       __syncthreads();
 #pragma unroll 8
@@ -464,7 +475,7 @@ __global__ __launch_bounds__(SV_THREADS) void k_big_pass(const BigSite* __restri
     for (int v = 0; v < 4; ++v)
       sum[wv * 256 + 16 * Mma<TA>::drow(lk, v) + li] = b == 0 ? ga[v] + (double)acca[v] : gb[v] + (double)accb[v];
     __syncthreads();
-    part[t.part + ((long long)(P.a - 1 + b) * nsplit + wg) * 256 + tid] =
+    part[t.part + ((long long)(P.a - 1 + b) * gridDim.x + blockIdx.x) * 256 + tid] =
         (sum[tid] + sum[256 + tid]) + (sum[512 + tid] + sum[768 + tid]);
   }
 }
@@ -618,13 +629,14 @@ hipError_t launch_big_sites(itnbp_net* net, SmallState* st, const void* psi, con
   TA* y = (TA*)st->ybuf.p;
   hipLaunchKernelGGL(k_big_eigh<TM>, dim3(ns), dim3(SV_THREADS), 0, stream, sites, (const TM*)msg_in, seeds, lam, warm,
                      st->active, st->sweep_ctr);
-  const dim3 grid((unsigned)ns * (unsigned)st->bsplit);
+  const int rows = std::min(ns, BIG_ROWS);
+  const dim3 grid(st->bsplit, rows, (ns + rows - 1) / rows);
   for (int p = 0; p < st->bpairs; ++p)
-    hipLaunchKernelGGL((k_big_pass<TS, TA, false>), grid, dim3(SV_THREADS), 0, stream, sites, st->bsplit, p,
-                       (const TS*)psi, y, (const double*)seeds, (const double*)lam, part, st->active);
+    hipLaunchKernelGGL((k_big_pass<TS, TA, false>), grid, dim3(SV_THREADS), 0, stream, sites, ns, p, (const TS*)psi,
+                       y, (const double*)seeds, (const double*)lam, part, st->active);
   for (int p = 0; p + 1 < st->bpairs; ++p)
-    hipLaunchKernelGGL((k_big_pass<TS, TA, true>), grid, dim3(SV_THREADS), 0, stream, sites, st->bsplit, p,
-                       (const TS*)psi, y, (const double*)seeds, (const double*)lam, part, st->active);
+    hipLaunchKernelGGL((k_big_pass<TS, TA, true>), grid, dim3(SV_THREADS), 0, stream, sites, ns, p, (const TS*)psi,
+                       y, (const double*)seeds, (const double*)lam, part, st->active);
   hipLaunchKernelGGL(k_big_final<TM>, dim3((unsigned)st->bonds.size()), dim3(SV_THREADS), 0, stream, sites, bonds,
                      st->bsplit, (const double*)seeds, (const double*)part, (const TM*)msg_in, (TM*)msg_out, stats,
                      normalize, st->active);
