@@ -197,7 +197,10 @@ int itnbp_normalize(itnbp_net* net);
  * other gates were applied.  Limits: degree <= 4, external bonds <= 32,
  * d chi <= 64 on the gate's bond, Theta <= 128 x 128, kept rank <= 64
  * (bonds with external bonds <= 8 and Theta <= 32 x 32 run on the LDS
- * kernel, the others on the split pipeline). */
+ * kernel, the others on the split pipeline).  Of a side (external bonds against
+ * physical index and gate bond, environments applied) the LDS kernel keeps every
+ * direction, the split pipeline those above about 1e-7 of the largest singular
+ * value.  The net keeps up to 256 MiB of device workspace for its next call. */
 int itnbp_apply_gates(itnbp_net* net, int n, const int* edge_ids, const double* gates,
                       int maxdim, double cutoff, int normalize, double* truncerr,
                       double* svals, int max_keep, int* kept);

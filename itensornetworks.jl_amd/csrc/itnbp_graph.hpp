@@ -63,7 +63,8 @@ void default_sequence(const Topo& t, bool parallel, std::vector<int>& seq);
 
 // Consecutive runs [begin, end) of seq in which no message reads another one
 // of the run (or repeats it): each run can be updated in one launch and still
-// give the result of the one-by-one sequential update.
+// give the result of the one-by-one sequential update.  The sweeps launch by the
+// levels below, of which the tests find no more than there are runs.
 std::vector<std::pair<int, int>> sequential_runs(const Topo& t, const std::vector<int>& seq);
 
 // Launch levels of a sequential sweep: positions of seq grouped so that no

@@ -53,9 +53,11 @@ bool site_enabled();
 // with psi staged in LDS (shortest task: no global load after the first).  More
 // tasks than that are bound by throughput: psi is read from global memory a second
 // time, so that more workgroups share a CU, in launches of similar LDS need (below
-// 2048 elements 256 threads; P of at most 40, 80 and 160 KB 512 threads).  16x16
-// chi = 8 (512 tasks) 46 us a sweep staged, 39 us unstaged; heavy-hex 9x7 FP32 (188
-// tasks) 15 us staged, 31 us unstaged.
+// 2048 elements 256 threads; P of at most 40, 80 and 160 KB 512 threads).  A sweep,
+// staged / unstaged: FP64 chi = 8 grids of 158 to 260 tasks 18.6 / 27.5 us, 308 20.5 / 27.6,
+// 388 35.1 / 36.2, 508 36.9 / 36.9; FP32 chi = 16 heavy-hex lattices of 165 to 340 tasks
+// 16.3 / 22.2, 625 26.3 / 28.9; FP64 chi = 4 grids 8.5 / 8.3 at every size.  The line at one
+// task per CU is on the safe side: the forms meet between 1.3 and 2.
 constexpr int SITE_CLASSES = 4;
 struct SiteLaunch {
   size_t begin, count;

@@ -929,9 +929,12 @@ ApplyBufs carve_apply_bufs(char* base, int n, long long goff, int mk) {
 // pipeline's workspace comes from b.  Gates marked in big run on the split
 // pipeline after the others, in chunks whose workspace fits the device's free
 // memory (at most 16 GiB).  The network keeps a workspace of up to
-// APPLY_BIG_KEEP bytes for its next call (a round is a call per colour class,
-// and an allocation of this size costs more than a launch sequence at small
-// bonds); a larger one is freed at the end of the call.
+// APPLY_BIG_KEEP bytes for its next call (a round is a call per colour class); a
+// larger one is freed at the end of the call, so that a network does not hold
+// gigabytes.  The line bounds what every network may hold; what it costs past it: a
+// chi = 16 round with the workspace freed per class, and kept, 8x8 (32 gates a class)
+// 5.5 and 4.3 ms, 12x12 6.6 and 5.7, 16x16 (past the line) 8.9 and 8.4, 24x24 19.8 and
+// 19.7.
 constexpr size_t APPLY_BIG_KEEP = 256ULL << 20;
 int run_apply(itnbp_net* net, int n, const std::vector<ApplyItem>& items_in, const double* gates, long long goff,
               int maxdim, double cutoff, int normalize, double* truncerr, double* svals, int mk, int* kept,

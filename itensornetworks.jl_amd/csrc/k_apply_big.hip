@@ -29,9 +29,9 @@
 // (three read + write passes, two Gram reads, rebuild, scale) and are HBM-bound
 // at chi = 32; the per-gate kernels (roots, chol, svd) are latency-bound, one
 // workgroup each.  One round with the copies in and out, against one workgroup
-// per bond through all steps: 8x8 chi = 16 (4 classes of 28 gates) 44.1 -> 9.3 ms,
-// 5x4 chi = 32 (4 classes of 6 to 10) 447 -> 26.9 ms; per class there, svd 0.50 and
-// 2.05 ms, rebuild 88 and 343 us, roots 75 and 197 us, grams 89 and 347 us, chol 81
+// per bond through all steps: 8x8 chi = 16 (4 classes of 28 gates) 44.1 -> 8.9 ms,
+// 5x4 chi = 32 (4 classes of 6 to 10) 447 -> 26.6 ms; per class there, svd 0.51 and
+// 2.12 ms, rebuild 88 and 343 us, roots 75 and 197 us, grams 89 and 347 us, chol 81
 // and 476 us, the three mode passes 50 and 124 us.
 #include <algorithm>
 #include <cmath>

@@ -418,6 +418,17 @@ int site_class(long long D, int elem_bytes) {
   return D < 2048 ? 0 : b <= 40 * 1024 ? 1 : b <= 80 * 1024 ? 2 : 3;
 }
 
+// Workgroup size by the tensor's elements: below 2048 four waves have their blocks, and
+// unstaged tasks want many workgroups per CU; one staged workgroup has its CU to
+// itself.  Sweeps of 10x10 (staged) and 24x24 (unstaged) FP64 grids, us:
+//   D (chi)      staged 256 / 512 / 1024 threads   unstaged 256 / 512
+//   512 (4)       8.6 /  8.2 /  8.5                13.3 / 20.0
+//   1250 (5)     15.1 / 11.9 / 12.6                25.5 / 31.0
+//   2592 (6)     20.3 / 15.0 / 13.7                43.6 / 46.0
+//   4802 (7)     27.2 / 19.1 / 17.2                78.5 / 60.2
+//   8192 (8)     29.1 / 20.8 / 18.8                77.7 / 65.2
+// The lines suit the unstaged form; staged tasks would gain from 512 threads at 1250 and
+// 1024 at 2592 elements.
 int site_threads(long long D, bool staged) { return D < 2048 ? 256 : staged && D >= 4096 ? 1024 : 512; }
 
 size_t site_lds_bytes(long long D, int elem_bytes, bool staged) {

@@ -207,7 +207,7 @@ def test_bond_takes_the_kept_dimension():
 @pytest.mark.parametrize("chi", [16, 32])
 def test_large_bonds_run_on_the_global_memory_kernel(chi):
     """Bonds past the LDS kernel's limits (external bonds above 8, Theta up to
-    128 x 128) run on its global-memory variant: on a 3x3 chi = 16 or 32 PEPS a
+    128 x 128) run on the split pipeline: on a 3x3 chi = 16 or 32 PEPS a
     bulk bond (the centre's side has E = chi^3 external rows against n = 2 chi,
     the tall QR; at chi = 32 Theta is 128 x 128) and a corner bond (E = chi < n,
     the wide QR), truncated to maxdim = chi, against the oracle (apply.jl:33-95):
@@ -239,7 +239,7 @@ def test_large_bonds_run_on_the_global_memory_kernel(chi):
 def test_mixed_small_and_large_bonds_and_a_rank_deficient_side():
     """One call with gates on both kernels on a 4x4 PEPS whose bonds at (2,2)
     have chi = 12 and all others 4: the gates next to (2,2) run on the
-    global-memory variant, the far ones in LDS.  One large side is
+    split pipeline, the far ones in LDS.  One large side is
     rank-deficient (the slices b >= 6 of (2,2)'s gate bond vanish, so X has rank
     n / 2 with E >> n: the Gram QR drops the null directions where the oracle's
     Householder QR keeps zero rows).  Tensors, singular values and truncation
@@ -258,7 +258,7 @@ def test_mixed_small_and_large_bonds_and_a_rank_deficient_side():
     opsi = oracle_psi(psi)
     msgs = to_index(g, bpc.messages())
     deg = {v: g.degree(v) for v in g.vertices}
-    # global-memory variant: the first two; LDS kernel: the last two
+    # split pipeline: the first two; LDS kernel: the last two
     bonds = [((2, 2), (2, 3)), ((1, 1), (1, 2)), ((3, 4), (4, 4)), ((4, 1), (4, 2))]
     gates = [O.expm_sym(O.two_site(O.X, O.Z) + O.ising_bond_hamiltonian(2.5, deg[u], deg[v]), -0.3) for u, v in bonds]
     svals = []
@@ -276,7 +276,7 @@ def test_mixed_small_and_large_bonds_and_a_rank_deficient_side():
 
 
 def test_large_bonds_with_physical_dimension_three():
-    """The global-memory variant at d = 3 (qutrits): a 3x3 chi = 12 PEPS, a bulk
+    """The split pipeline at d = 3 (qutrits): a 3x3 chi = 12 PEPS, a bulk
     bond and one next to a corner (E = 12 < n = 36, the wide side) with random
     symmetric gates exp(-0.2 H) (9 x 9), truncated to maxdim = 12, against the
     oracle."""

@@ -6,7 +6,7 @@ rank-deficient sides against the state itself.
 
 Tolerances: FP64 results to 1e-10 relative, the bar of the other gate tests; the
 state to 1e-13 (products of n x n factors and E-row sums, ~sqrt(n) eps each, through
-roots of messages of condition 3.4, rotations to 8 eps sqrt(N); a few times their sum).
+roots of messages of condition 3.4, rotations to eps sqrt(N); a few times their sum).
 """
 import numpy as np
 import pytest

@@ -173,7 +173,7 @@ def test_rank_deficient_pairs_keep_the_state(chie, chib, rank, gate):
     side of low rank (wide: E <= n, tall: E = 32 > n = 20), whose kept rank is the
     rank's bound, or a gate that halves Theta's rank, whose bond keeps noise
     values.  Bound: products of n x n factors and E-row sums, ~sqrt(n) eps each,
-    and rotations to 8 eps sqrt(N): 1e-13 is a few times their sum."""
+    and rotations to eps sqrt(N): 1e-13 is a few times their sum."""
     rng = np.random.default_rng(66)
     g, n = itnbp.path_graph(4), 2 * chib
     psi = itnbp.random_tensornetwork(rng, np.float64, g, link_space=[chie, chib, chie])

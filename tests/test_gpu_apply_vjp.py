@@ -197,7 +197,7 @@ def test_gradient_of_a_tebd_step(checkpoint):
 
 def test_apply_vjp_refuses_bonds_past_the_lds_kernel():
     """The adjoint covers the forward's LDS kernel only: a bond with an external
-    bond of dimension 12 (the forward runs it on the global-memory variant) is
+    bond of dimension 12 (the forward runs it on the split pipeline) is
     refused with ITNBP_ERR_UNSUPPORTED, and the cache is left as it was."""
     g = itnbp.named_grid((3, 3))
     psi = itnbp.random_tensornetwork(np.random.default_rng(91), np.float64, g, link_space=12)

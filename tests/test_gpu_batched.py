@@ -35,7 +35,7 @@ def test_batched_matches_per_instance_oracle(dtype, prec, tol):
         assert max(np.abs(got[e] - ref[e]).max() for e in ref) < tol
     # instances converge at different sweeps and drop out
     assert len({r["iterations"] for r in res}) > 1
-    # small-chi sites on the per-vertex kernel, the chi = 16 degree-4 centre on the generic one
+    # sites in LDS on the site kernel, the chi = 16 degree-4 centre on the passes over large sites
     assert "[vertex " in res[0]["path"], res[0]["path"]
 
 
@@ -77,8 +77,7 @@ def run_batched(inst, monkeypatch, graph, **kw):
                                 dict(maxiter=30, tol=1e-10, precision="f32")])
 def test_graph_loop_matches_the_host_loop(monkeypatch, kw):
     """The device-resident loop (eight sweeps captured in a HIP graph and
-    replayed, per-instance convergence and drop-out decided on the device, the
-    large-site Gram tile autotuned) stops every instance at the sweep the
+    replayed, per-instance convergence and drop-out decided on the device) stops every instance at the sweep the
     host-driven loop does, with the same messages; without a tolerance every
     instance runs maxiter sweeps, also when maxiter is not a multiple of eight."""
     inst = instances(np.float32 if kw["precision"] == "f32" else np.float64)
@@ -99,26 +98,27 @@ def test_graph_loop_matches_the_host_loop(monkeypatch, kw):
                                                  abs=1e-14 if f64 else 1e-7)
 
 
-@pytest.mark.parametrize("tile", ["1", "2", "4", "192"])
-def test_large_site_kernel_variants_match_the_oracle(monkeypatch, tile):
-    """Every variant of the large-site kernel (k_vertex_big: sites whose tensor
-    does not fit in LDS), forced through ITNBP_VERTEX_BIG_TILE: the FP32 MFMA
-    kernel with 1, 2 or 4 tiles in flight per wave and the VALU kernel with a
-    192-fibre Gram tile, on the chi = 16 degree-4 centre of a 3x3 grid and the
-    four chi = 12 degree-4 sites of a 4x4 grid, FP32, against the oracle."""
-    monkeypatch.setenv("ITNBP_VERTEX_BIG_TILE", tile)
+@pytest.mark.parametrize("copies", [1, 8, 64])
+def test_large_site_kernel_variants_match_the_oracle(monkeypatch, copies):
+    """Both splits of the passes over sites too large for LDS (k_big_pass): one
+    workgroup per chunk (5 sites) and with fewer workgroups than chunks (40 and 320
+    sites: about 8 workgroups per CU over all of them), on the chi = 16 degree-4
+    centre of a 3x3 grid and the four chi = 12 degree-4 sites of a 4x4 grid, FP32,
+    against the oracle; every copy agrees bit for bit."""
     rng = np.random.default_rng(17)
     inst = []
     for g, chi in [(itnbp.named_grid((3, 3)), 16), (itnbp.named_grid((4, 4)), 12)]:
         inst.append((g, itnbp.random_tensornetwork(rng, np.float32, g, link_space=chi, scale=1 / np.sqrt(chi))))
-    res, got = run_batched(inst, monkeypatch, True, maxiter=12, precision="f32")
+    res, got = run_batched(inst * copies, monkeypatch, True, maxiter=12, precision="f32")
     assert "[vertex " in res[0]["path"], res[0]["path"]
+    for i, m in enumerate(got):
+        assert all(np.array_equal(m[e], got[i % 2][e]) for e in m)
     for r, m, (g, psi) in zip(res, got, inst):
         og, opsi = oracle_graph(g), oracle_psi(psi)
         ref, _, _, _ = O.bp_update(og, opsi, O.identity_messages(og, opsi), maxiter=r["iterations"],
                                    schedule="parallel")
         err = max(np.abs(m[e] - ref[e]).max() for e in ref)
-        print(f"tile {tile}: {g.nv} sites, {r['iterations']} sweeps, max abs err {err:.2e}, path {r['path']}",
+        print(f"{copies} copies: {g.nv} sites, {r['iterations']} sweeps, max abs err {err:.2e}, path {r['path']}",
               flush=True)
         assert err < 2e-5
 

@@ -214,7 +214,7 @@ def test_vertex_kernel_matches_generic_kernels(precision, monkeypatch):
     chi = 6 (degrees 2..4) and a 2x6 grid at chi = 16 (degrees 2..3) in LDS; the
     degree-4 sites of a 3x4 grid at chi = 12 and a 3x3 grid at chi = 16 and the
     degree-6 centre of a 3x3 triangular lattice at chi = 6, too large for LDS
-    (scratch tensors in global memory, k_vertex_big)."""
+    (scratch tensors in global memory, k_big_pass)."""
     g0 = itnbp.named_grid((3, 3))
     tri = itnbp.NamedGraph(g0.vertices, list(g0.edges) + [((i, j), (i + 1, j + 1)) for i in (1, 2) for j in (1, 2)])
     assert max(tri.degree(v) for v in tri.vertices) == 6
