@@ -1705,7 +1705,8 @@ __global__ __launch_bounds__(256, 2) void k_rot34_f64(const EigItem* __restrict_
 // gram12, FP64: a unit is four consecutive Q blocks, one per wave, each loaded once
 // (coalesced, one block of look-ahead in registers) into a per-wave LDS tile, from
 // which both operand orientations (D for T'1, D^T for T'2) are read.  BLOCKS: Q
-// blocks per site.  36 sites of 2048 blocks: 253 -> 206 us with the even split.
+// blocks per site.  With the even split 36 sites of 2048 blocks take 253 -> 206 us, and 900
+// sites, where every CU is busy either way, 4.55 -> 4.77 ms.
 template <int BLOCKS>
 __global__ __launch_bounds__(256, 2) void k_gram12_f64(const EigItem* __restrict__ items, EigSplit sp,
                                                        const double* __restrict__ Q,
