@@ -1531,10 +1531,15 @@ struct EigSplit {
   }
 };
 constexpr int EIG_MAXSLOTS = 64;
-// 16, 32 or 64 partials per site: enough workgroups for two per CU
+// 16, 32 or 64 partials per site: more while the device has room for them and an even
+// share of the resident workgroups (eig_split) holds fewer of a site's 8 FC rotation units
+// than one of m whole parts.  A sweep, whole parts -> even shares: 9 sites 507 -> 426 us,
+// 12 531 -> 500, 20 924 -> 729, 25 951 -> 875, 30 1049 -> 1020 (16 parts per site and one
+// workgroup per CU 1030); 15 sites, of the same share either way, 551 -> 591: left whole.
 int eig_slots(int n, int num_cu) {
+  const int resident = 2 * num_cu, share = (8 * FC * n + resident - 1) / resident;
   int m = EIG_NPART;
-  while (m < EIG_MAXSLOTS && 2 * m * n <= 2 * num_cu) m *= 2;
+  while (m < EIG_MAXSLOTS && n * m < resident && share < 8 * FC / m) m *= 2;
   return m;
 }
 // as many whole workgroups per site while all are resident (two per CU), else every

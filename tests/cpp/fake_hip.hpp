@@ -17,7 +17,12 @@ namespace fake {
 struct Launch {
   dim3 grid, block;
   size_t lds;
+  const char* kernel;  // mangled name
 };
+inline std::map<const void*, const char*>& kernels() {  // the library registers them before main
+  static std::map<const void*, const char*> k;
+  return k;
+}
 inline std::vector<Launch> config, launches;
 inline std::vector<std::function<void()>> pending;
 inline std::map<void*, size_t> allocated;
@@ -117,7 +122,7 @@ hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void*, int
   return hipSuccess;
 }
 hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t lds, hipStream_t) {
-  fake::config.push_back({grid, block, lds});
+  fake::config.push_back({grid, block, lds, ""});
   return hipSuccess;
 }
 hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* lds, hipStream_t* s) {
@@ -128,8 +133,17 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* lds, hipSt
   fake::config.pop_back();
   return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void*, dim3 grid, dim3 block, void**, size_t lds, hipStream_t) {
-  fake::launches.push_back({grid, block, lds});
+void** __hipRegisterFatBinary(const void*) {
+  static void* module;
+  return &module;
+}
+void __hipUnregisterFatBinary(void**) {}
+void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
+void __hipRegisterFunction(void**, const void* f, char*, const char* name, unsigned, void*, void*, dim3*, dim3*, int*) {
+  fake::kernels()[f] = name;
+}
+hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void**, size_t lds, hipStream_t) {
+  fake::launches.push_back({grid, block, lds, fake::kernels()[f]});
   return hipSuccess;
 }
 }
