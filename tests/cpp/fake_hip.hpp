@@ -113,7 +113,17 @@ hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpyKind, h
   return hipSuccess;
 }
 hipError_t hipMemsetAsync(void* dst, int v, size_t n, hipStream_t) {
-  fake::pending.push_back([=] { std::memset(dst, v, n); });
+  fake::pending.push_back([=] {
+    char* a = (char*)(((size_t)dst + 4095) & ~(size_t)4095);  // zeroed pages go back to the system
+    char* e = (char*)(((size_t)dst + n) & ~(size_t)4095);
+    if (v != 0 || a >= e) {
+      std::memset(dst, v, n);
+      return;
+    }
+    std::memset(dst, 0, a - (char*)dst);
+    madvise(a, e - a, MADV_DONTNEED);
+    std::memset(e, 0, (char*)dst + n - e);
+  });
   return hipSuccess;
 }
 hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
